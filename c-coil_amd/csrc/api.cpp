@@ -167,6 +167,7 @@ std::string pack_coils(const ccoil_coils *c, bool need_len, bool need_freq, std:
         d.inv_rmax2 = 1.0 / (d.rmax * d.rmax);
         d.far_d2 = 0.0;
         d.mp_terms = 0;
+        set_rule_limits(d);
         out[(size_t)i] = d;
         return "";
     };
@@ -270,14 +271,14 @@ ccoil_status ccoil_create(int device, ccoil_ctx *out)
         return bail(e, "hipHostMalloc");
     if ((e = scratch_address(device, &ctx->scratch)) != hipSuccess) return bail(e, "hipGetSymbolAddress(scratch)");
     if (const char *tf = std::getenv("CCOIL_TUNING_FILE")) load_tuning_file(ctx, tf);
-    const size_t nd = sizeof(double) * kTableSize, nf = sizeof(float) * kTableSize;
+    const size_t nf = sizeof(float) * kTableSize;
     double **dp[11] = {&ctx->gl_x, &ctx->gl_w, &ctx->gl_cos, &ctx->gl_omc, &ctx->gl_rcos, &ctx->gl_rsin, &ctx->gl_wcos,
                        &ctx->gl_opc, &ctx->gl_ws, &ctx->gl_ws2, &ctx->gl_wcs};
     float **fp[7] = {&ctx->gl_xf, &ctx->gl_wf, &ctx->gl_cosf, &ctx->gl_omcf, &ctx->gl_wcosf, &ctx->gl_opcf,
                      &ctx->gl_wcsf};
-    for (auto p : dp)   // x and w also hold the series' length rule (kTableSizeXW)
-        if ((e = hipMalloc((void **)p, p == &ctx->gl_x || p == &ctx->gl_w ? sizeof(double) * kTableSizeXW : nd)) !=
-            hipSuccess)
+    // x and w also hold the series' length rule, w and the angular tables the reduced rules (kTableSizeAng)
+    for (auto p : dp)
+        if ((e = hipMalloc((void **)p, sizeof(double) * kTableSizeAng)) != hipSuccess)
             return bail(e, "hipMalloc(tables)");
     for (auto p : fp)
         if ((e = hipMalloc((void **)p, nf)) != hipSuccess) return bail(e, "hipMalloc(tables)");
@@ -287,6 +288,15 @@ ccoil_status ccoil_create(int device, ccoil_ctx *out)
     launch_angular_tables(ctx->stream, ctx->gl_x, ctx->gl_w, ctx->gl_cos, ctx->gl_omc, ctx->gl_wcos, ctx->gl_wcosf,
                           ctx->gl_opc, ctx->gl_opcf, ctx->gl_ws, ctx->gl_ws2, ctx->gl_wcs, ctx->gl_wcsf);
     if ((e = hipGetLastError()) != hipSuccess) return bail(e, "angular_table_kernel launch");
+    RedTables red;
+    reduced_tables(red);
+    const std::pair<double *, const double *> rt[7] = {{ctx->gl_w, red.w}, {ctx->gl_omc, red.omc}, {ctx->gl_opc, red.opc},
+                                                       {ctx->gl_wcos, red.wcos}, {ctx->gl_ws, red.ws},
+                                                       {ctx->gl_ws2, red.ws2}, {ctx->gl_wcs, red.wcs}};
+    for (const auto &t : rt)
+        if ((e = hipMemcpyAsync(t.first + kRedOffset, t.second, sizeof(double) * kRedNodes, hipMemcpyHostToDevice,
+                                ctx->stream)) != hipSuccess)
+            return bail(e, "hipMemcpy(reduced rules)");
     if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return bail(e, "gl_table_kernel");
     *out = ctx;
     return CCOIL_OK;

@@ -13,6 +13,27 @@ constexpr int kTableSize = kMaxOrder * (kMaxOrder + 1) / 2;
 constexpr int kSeriesLenNodes = 126;
 constexpr int kSeriesLenOffset = kTableSize;
 constexpr int kTableSizeXW = kTableSize + kSeriesLenNodes;
+
+// Reduced rules: the node sets that replace a rule's Gauss-Legendre angular or thickness sum where that sum has
+// converged to rounding (reduced_rules.cpp: the bounds, the tables and what they measured).
+//
+// Angular class k (1..kRedAng) serves the pairs whose angular integrand is analytic in the strip |Im phi| < eta for an
+// eta of at least kRedEta[k - 1]; its kRedAngN[k - 1] nodes lie in the angular double tables at kRedOffset. Class 0 is
+// the coil's own rule.
+constexpr int kRedAng = 6;
+constexpr int kRedAngN[kRedAng] = {20, 16, 12, 10, 8, 6};
+constexpr double kRedEta[kRedAng] = {0.1, 0.3, 0.75, 1.0, 1.8, 3.2};
+constexpr int kRedNodes = 20 + 16 + 12 + 10 + 8 + 6;
+constexpr int kRedOffset = kTableSizeXW;
+constexpr int kTableSizeAng = kRedOffset + kRedNodes;   // the w, omc, wcos, opc, ws, ws2 and wcs tables
+// Thickness class t (1..kRedThk): the Gauss-Legendre rule of kRedThkN[t - 1] nodes, for points outside the ellipse with
+// foci at the winding's inner and outer radius whose parameter is (kRedThkC / kRedTol)^(1 / (2 n)). Class 0 is the
+// coil's own rule.
+constexpr int kRedThk = 6;
+constexpr int kRedThkN[kRedThk] = {22, 17, 13, 10, 8, 6};
+constexpr double kRedThkC = 200.0;
+constexpr double kRedTol = 3e-16;
+constexpr int kRuleClasses = (kRedAng + 1) * (kRedThk + 1);   // class = (kRedThk + 1) angular class + thickness class
 constexpr double kPi = 3.14159265358979323846;
 constexpr double kMuReduced = 1e-7;                    // mu0 / (4 pi), g_MiReduced (CalculateFieldsFast.cxx:10)
 constexpr double kGpuAxisRatio = 1e-5;                 // on-axis branch of the GPU gradient (FieldGGroup.cu:134)
@@ -44,10 +65,15 @@ struct alignas(64) CoilDev {
     int32_t blk_ang, blk_thk, blk_len;
     int32_t near_key; // FP32C near pass: the coil's place in the evaluation order (most nodes first)
     int32_t mp_terms; // highest order of the far-field series a pair of this call can use (0: no series)
+    // Reduced rules: the least cosh(eta) - 1 and the least ellipse parameter sum (d1 + d2) / (a / 2) at which the
+    // coil's angular and thickness rules may be replaced (FLT_MAX: never), and the winding's geometry in float
+    // (inner and outer radius, half length, 2 / a).
+    float red_x, red_s;
+    float r0f, r1f, hbf, ia2f;
 };
 
 // Gauss-Legendre tables for orders 1..100 at offset table_offset(n), generated in FP64 on the device (x and w also
-// hold the series' length rule at kSeriesLenOffset).
+// hold the series' length rule at kSeriesLenOffset, and the double angular tables the reduced rules at kRedOffset).
 struct Tables {
     const double *x;      // nodes, ascending
     const double *w;      // weights
@@ -211,6 +237,69 @@ __device__ inline bool is_near(const CoilDev &c, double z, double r, bool axis)
 __device__ inline bool near_pass_pair(const CoilDev &c, double z, double r, bool axis)
 {
     return !is_far(c, z, r) && is_near(c, z, r, axis);
+}
+
+// The node sets of one evaluation: offset and count of its angular and thickness rules in the tables.
+struct RuleSel {
+    int oa, na, ot, nt;
+};
+
+__device__ inline RuleSel full_rule(const CoilDev &c)
+{
+    return {table_offset(c.n_ang), c.n_ang, table_offset(c.n_thk), c.n_thk};
+}
+
+__device__ inline RuleSel class_rule(const CoilDev &c, int cls)
+{
+    const int k = cls / (kRedThk + 1), t = cls - k * (kRedThk + 1);
+    RuleSel s = full_rule(c);
+    int off = kRedOffset;
+#pragma unroll
+    for (int i = 0; i < kRedAng; ++i) {
+        if (k == i + 1) {
+            s.oa = off;
+            s.na = kRedAngN[i];
+        }
+        off += kRedAngN[i];
+    }
+#pragma unroll
+    for (int i = 0; i < kRedThk; ++i)
+        if (t == i + 1) {
+            s.nt = kRedThkN[i];
+            s.ot = table_offset(kRedThkN[i]);
+        }
+    return s;
+}
+
+// The class of the cheapest rule whose value at local (z, r) is that of the coil's own rule to rounding
+// (reduced_rules.cpp). With zd the point's distance beyond the winding's axial span, the angular integrand of the
+// ring at radius rho is analytic for |Im phi| < eta, cosh(eta) = 1 + ((rho - r)^2 + zd^2) / (2 rho r), least at the
+// winding's radius nearest to sqrt(r^2 + zd^2); the thickness integrand is analytic outside the point (r, zd) and its
+// mirror, whose ellipse about [R, R + a] has the distance sum d1 + d2. Every operation is a float operation rounded on
+// its own, so every kernel gives a pair the same class; the thresholds carry margins far above float rounding.
+__device__ inline int rule_class(const CoilDev &c, double z, double r)
+{
+#pragma clang fp contract(off)
+    const float rf = (float)r, zd = fmaxf((float)fabs(z) - c.hbf, 0.0f), zd2 = zd * zd;
+    const float rho = fminf(fmaxf(__builtin_amdgcn_sqrtf(rf * rf + zd2), c.r0f), c.r1f);
+    const float dr = rho - rf, num = dr * dr + zd2, den = 2.0f * rho * rf;
+    int k = 0, t = 0;
+    if (num >= c.red_x * den) {
+        constexpr float kX[kRedAng] = {0.0050042f, 0.0453385f, 0.2946833f, 0.5430806f, 2.1074632f, 11.2864665f};
+        k = 1;   // red_x is at least the first class's threshold
+#pragma unroll
+        for (int i = 1; i < kRedAng; ++i) k += num >= kX[i] * den ? 1 : 0;
+    }
+    const float e0 = rf - c.r0f, e1 = rf - c.r1f;
+    const float s = (__builtin_amdgcn_sqrtf(e0 * e0 + zd2) + __builtin_amdgcn_sqrtf(e1 * e1 + zd2)) * c.ia2f;
+    if (s >= c.red_s) {
+        // rho_B + 1 / rho_B, rho_B = (kRedThkC / kRedTol)^(1 / (2 n))
+        constexpr float kS[kRedThk] = {2.935256f, 3.643171f, 5.054480f, 7.913130f, 13.079747f, 30.607902f};
+        t = 1;
+#pragma unroll
+        for (int i = 1; i < kRedThk; ++i) t += s >= kS[i] ? 1 : 0;
+    }
+    return (kRedThk + 1) * k + t;
 }
 
 }  // namespace ccoil

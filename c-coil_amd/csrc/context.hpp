@@ -124,6 +124,12 @@ double far_cost_floor(int n_ang, int n_thk, bool fast, double log_tol);
 // precision's tolerance (fp64: kFarToleranceFP64, else kFarTolerance) from the cost floor on (cost_floor: launches
 // with one lane per point or secondary node), else from 2.
 double far_distance(const CoilDev &c, bool fp64, bool cost_floor);
+// Reduced rules (reduced_rules.cpp): a packed coil's thresholds, and the angular tables' entries from kRedOffset on.
+void set_rule_limits(CoilDev &c);
+struct RedTables {
+    double w[kRedNodes], omc[kRedNodes], opc[kRedNodes], wcos[kRedNodes], ws[kRedNodes], ws2[kRedNodes], wcs[kRedNodes];
+};
+void reduced_tables(RedTables &t);
 // Runs fn(i0, i1) over ranges that cover [0, n) once: on up to 16 host threads for large n, else on the caller.
 void host_parallel_for(int64_t n, const std::function<void(int64_t, int64_t)> &fn);
 // The highest order a series evaluated beyond y r_max can use (multipole_terms there, with a margin; 0 if y is 0).

@@ -122,7 +122,7 @@ void field_kernel(FieldParams p)
         to_local(c, px, py, pz, z, r, cph, sph);
         Local L = {0, 0, 0, 0, 0, 0, 0};
         if constexpr (PREC == kFP64IEEE) {
-            eval_stable<double, WA, WB, WG>(c, p.tab, z, r, lane, SPLIT, L);
+            eval_stable<double, WA, WB, WG>(c, p.tab, full_rule(c), z, r, lane, SPLIT, 0, 1, L);
         } else if constexpr (PREC == kFP64Reference) {
             eval_plain<double, WA, WB, WG>(c, p.tab, z, r, lane, SPLIT, L);
         } else if constexpr (PREC == kFP32) {
@@ -134,8 +134,8 @@ void field_kernel(FieldParams p)
             const bool far = is_far(c, z, r);
             const int kind = record_kind(p, c, z, r, WG);
             if (!far && kind < 0) {
-                if constexpr (PREC == kFP64) eval_stable<f64s, WA, WB, WG>(c, p.tab, z, r, lane, SPLIT, L);
-                else eval_stable<float, WA, WB, WG>(c, p.tab, z, r, lane, SPLIT, L);
+                if constexpr (PREC == kFP64) eval_stable<f64s, WA, WB, WG>(c, p.tab, full_rule(c), z, r, lane, SPLIT, 0, 1, L);
+                else eval_stable<float, WA, WB, WG>(c, p.tab, full_rule(c), z, r, lane, SPLIT, 0, 1, L);
             }
             if (kind >= 0) ++n_near;
             if (__ballot(far)) {
@@ -197,9 +197,9 @@ void field_series_kernel(FieldParams p)
     // the loop would keep the compiler from loading the coil records through the scalar cache.
     extern __shared__ uint32_t key_counts[];   // [kind][coil of the chunk]
     const bool count = series_counts_keys(p);
-    const int n_kinds = p.float_records ? 2 : 1, cpc = p.coils_per_chunk;
+    const int cpc = p.coils_per_chunk, words = series_key_words(p);
     if (count)
-        for (int i = threadIdx.x; i < n_kinds * cpc; i += kFieldBlock) key_counts[i] = 0u;
+        for (int i = threadIdx.x; i < words; i += kFieldBlock) key_counts[i] = 0u;
     __syncthreads();
     for (int ci = c0; ci < c1; ++ci) {
         const CoilDev &c = p.coils[ci];
@@ -208,11 +208,17 @@ void field_series_kernel(FieldParams p)
         const bool far = is_far(c, z, r);
         const int kind = active ? record_kind(p, c, z, r, WG) : -1;
         if (kind >= 0) ++n_near;
-        if (count)
-            for (int k = 0; k < n_kinds; ++k) {
-                const uint64_t m = __ballot(kind == k);
-                if (m && lane == __builtin_ctzll(m)) atomicAdd(&key_counts[k * cpc + (ci - c0)], (unsigned)__popcll(m));
+        if (count && __ballot(kind >= 0)) {
+            // [slot][coil of the chunk], one LDS atomic per distinct key of the wave
+            const uint32_t slot = kind < 0 ? 0u : record_slot(p, c, kind, z, r);
+            uint64_t todo = __ballot(kind >= 0);
+            while (todo) {
+                const uint32_t k = __builtin_amdgcn_readfirstlane(__shfl(slot, __builtin_ctzll(todo)));
+                const uint64_t m = __ballot(kind >= 0 && slot == k);
+                if (lane == __builtin_ctzll(m)) atomicAdd(&key_counts[k * cpc + (ci - c0)], (unsigned)__popcll(m));
+                todo &= ~m;
             }
+        }
         if (__ballot(far)) {
             const int own = far ? multipole_terms(r * r + z * z, c.inv_rmax2,
                                                   PREC == kFP64 ? kMpLogTolFP64 : kMpLogTolFP32C) : 0;
@@ -227,7 +233,7 @@ void field_series_kernel(FieldParams p)
     }
     __syncthreads();
     if (count)
-        for (int i = threadIdx.x; i < n_kinds * cpc; i += kFieldBlock) {
+        for (int i = threadIdx.x; i < words; i += kFieldBlock) {
             const uint32_t v = key_counts[i];
             const int k = i / cpc, ci = c0 + i % cpc;
             if (v && ci < c1) atomicAdd(&p.near_hist[k * p.n_coils + p.coils[ci].near_key], v);
@@ -331,7 +337,7 @@ template <int PREC, bool WA, bool WB, bool WG>
 static void launch_series_q(hipStream_t s, const FieldParams &p)
 {
     const dim3 grid((unsigned)((p.n_pts + kFieldBlock - 1) / kFieldBlock), (unsigned)p.n_chunks);
-    const size_t lds = series_counts_keys(p) ? sizeof(uint32_t) * (p.float_records ? 2 : 1) * p.coils_per_chunk : 0;
+    const size_t lds = series_counts_keys(p) ? sizeof(uint32_t) * (size_t)series_key_words(p) : 0;
     hipLaunchKernelGGL((field_series_kernel<PREC, WA, WB, WG>), grid, dim3(kFieldBlock), lds, s, p);
 }
 

@@ -150,7 +150,9 @@ ccoil_status near_buffers(ccoil_ctx ctx, FieldLaunch &L, int64_t cap, int width,
     ccoil_status st;
     if ((st = call_buffer(ctx, ctx->ncounts, arena, sizeof(int64_t) * (size_t)n, &counts)) != CCOIL_OK) return st;
     if ((st = call_buffer(ctx, ctx->noffsets, arena, sizeof(int64_t) * (size_t)n, &offsets)) != CCOIL_OK) return st;
-    if ((st = call_buffer(ctx, ctx->nhist, arena, 2 * sizeof(uint32_t) * ((size_t)p.n_keys + 2), &hist)) != CCOIL_OK)
+    // the cursors replace the counts in place in the fixed scratch, whose calls never run the record pass again
+    const size_t key_words = (size_t)p.n_keys + 2, key_arrays = arena && arena->fixed ? 1 : 2;
+    if ((st = call_buffer(ctx, ctx->nhist, arena, key_arrays * sizeof(uint32_t) * key_words, &hist)) != CCOIL_OK)
         return st;
     if ((st = call_buffer(ctx, ctx->nstate, arena, sizeof(NearState), &state)) != CCOIL_OK) return st;
     if ((st = call_buffer(ctx, ctx->ntemp, arena, tb > 0 ? tb : 1, &temp)) != CCOIL_OK) return st;
@@ -165,7 +167,7 @@ ccoil_status near_buffers(ccoil_ctx ctx, FieldLaunch &L, int64_t cap, int width,
     p.near_counts = (int64_t *)counts;
     p.near_offsets = (const int64_t *)offsets;
     p.near_hist = (uint32_t *)hist;
-    p.near_cursor = p.near_hist + ((size_t)p.n_keys + 2);
+    p.near_cursor = p.near_hist + (key_arrays - 1) * key_words;
     p.near_state = (NearState *)state;
     p.near_cap = cap;
     p.near_keys = (uint32_t *)keys;
@@ -305,7 +307,9 @@ ccoil_status fields_prepare(ccoil_ctx ctx, const ccoil_coils *coils, const doubl
                                hipMemcpyHostToDevice, ctx->stream));
     p.coils = (const CoilDev *)coil_mem;
     p.n_coils = (int32_t)hc.size();
-    p.n_keys = p.n_coils * (p.float_records ? 2 : 1);
+    // the fixed scratch keeps its room for records, and thousands of coils would have a few records per key: two slots
+    p.n_slots = arena && arena->fixed ? 2 : !uniform_records(p) ? 4 : hc.size() > 2048 ? 2 : kRuleClasses;
+    p.n_keys = p.n_coils * (p.n_slots + (p.float_records ? 1 : 0));
     p.near_coil = (const uint32_t *)((const char *)coil_mem + coil_bytes);
     p.tab = ctx_tables(ctx);
     if (!dev) {

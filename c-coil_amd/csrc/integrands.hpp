@@ -7,7 +7,8 @@
 // eval_stable<T>: the same integrands, algebraically rearranged so that no subtraction cancels; per-node
 //   work in T (float: FP32C; double: the accurate FP64 mode), per-row work and row sums in FP64.
 //
-// Both evaluate thickness rows j = row0, row0 + rstep, ... so several lanes can share one point.
+// Both evaluate thickness rows j = row0, row0 + rstep, ... so several lanes can share one point; eval_stable takes
+// its node sets from the caller (the coil's own rule or a reduced one) and angular nodes i = node0, node0 + nstep, ...
 #pragma once
 
 #include "common.hpp"
@@ -305,21 +306,22 @@ struct AdjA {
 template <typename T, bool WA> constexpr int kStableUnroll = (sizeof(T) == 4 && !WA) ? 2 : 4;
 
 template <typename P, bool WA, bool WB, bool WG, bool AD = false, bool ADA = false, bool LEAN = false>
-__device__ inline void eval_stable(const CoilDev &c, const Tables &tab, double zd, double rd, int row0, int rstep,
-                                   Local &L, AdjLocal *ad = nullptr, AdjA *ada = nullptr)
+__device__ inline void eval_stable(const CoilDev &c, const Tables &tab, const RuleSel &rule, double zd, double rd,
+                                   int row0, int rstep, int node0, int nstep, Local &L, AdjLocal *ad = nullptr,
+                                   AdjA *ada = nullptr)
 {
     static_assert(!AD || (WB && WG), "the adjoint needs B and the gradient terms");
     static_assert(!ADA || (WA && WB), "the pair adjoint needs A and B");
     using T = real_t<P>;
-    const double *xt = tab.x + table_offset(c.n_thk);
-    const double *wt = tab.w + table_offset(c.n_thk);
-    const T *st = tab_omc<T>(tab) + table_offset(c.n_ang);
-    const T *wa = tab_w<T>(tab) + table_offset(c.n_ang);
-    const T *wct = tab_wcos<T>(tab) + table_offset(c.n_ang);   // w cos
-    const T *opt = tab_opc<T>(tab) + table_offset(c.n_ang);    // 1 + cos
-    const T *wcst = tab_wcs<T>(tab) + table_offset(c.n_ang);     // w cos (1 - cos)
-    const double *wsd = tab.ws + table_offset(c.n_ang);          // w (1 - cos), double fast instances without G
-    const int na = c.n_ang, nt = c.n_thk;
+    const double *xt = tab.x + rule.ot;
+    const double *wt = tab.w + rule.ot;
+    const T *st = tab_omc<T>(tab) + rule.oa;
+    const T *wa = tab_w<T>(tab) + rule.oa;
+    const T *wct = tab_wcos<T>(tab) + rule.oa;   // w cos
+    const T *opt = tab_opc<T>(tab) + rule.oa;    // 1 + cos
+    const T *wcst = tab_wcs<T>(tab) + rule.oa;     // w cos (1 - cos)
+    const double *wsd = tab.ws + rule.oa;          // w (1 - cos), double fast instances without G
+    const int na = rule.na, nt = rule.nt;
     double aA = 0, aBh = 0, aBz = 0, aRR = 0, aRZ = 0, aZZ = 0;
     double hR0 = 0, hR1 = 0, ha0 = 0, ha1 = 0, hb0 = 0, hb1 = 0;   // adjoint row sums
     double qR = 0, qa = 0, qb = 0, qAr = 0;                         // pair adjoint row sums (A_phi)
@@ -366,7 +368,7 @@ __device__ inline void eval_stable(const CoilDev &c, const Tables &tab, double z
                 T eA = 0;           // pair adjoint: end rings of A, sum w cos (K1 + K2)
                 T rAr = 0;          // pair adjoint: sum w cos (r - rho cos) dgM
 #pragma unroll kStableUnroll<T, WA>
-                for (int i = 0; i < na; ++i) {
+                for (int i = node0; i < na; i += nstep) {
                     const T s = st[i], w = wa[i], wc = wct[i];
                     const T M = fma_<T>(q, s, base);
                     const T J1 = M + z1s, J2 = M + z2s;
@@ -567,10 +569,10 @@ __device__ inline void eval_stable(const CoilDev &c, const Tables &tab, double z
                 // are at most quadratic in s. The combinations cancel no more than the per-node sums they replace
                 // (the cos-weighted first harmonic). The weights w s and w s^2 are tabulated, so each moment is one
                 // FMA per node.
-                const double *wst = tab.ws + table_offset(c.n_ang), *ws2t = tab.ws2 + table_offset(c.n_ang);
+                const double *wst = tab.ws + rule.oa, *ws2t = tab.ws2 + rule.oa;
                 T b0 = 0, b1 = 0, b2 = 0, g0 = 0, g1 = 0, g2 = 0;
 #pragma unroll kStableUnroll<T, WA>
-                for (int i = 0; i < na; ++i) {
+                for (int i = node0; i < na; i += nstep) {
                     const T s = st[i], w = wa[i];
                     const T J = fma_<T>(q, s, baseJ);
                     const T K = prsq<P>(J);
@@ -597,7 +599,7 @@ __device__ inline void eval_stable(const CoilDev &c, const Tables &tab, double z
                 rRZ = fma_<T>(k0, g0, -fma_<T>(k1, g1, k2 * g2));  // sum w (k0 - k1 s - k2 s^2) K^5
             } else {
 #pragma unroll kStableUnroll<T, WA>
-                for (int i = 0; i < na; ++i) {
+                for (int i = node0; i < na; i += nstep) {
                     const T s = st[i], w = wa[i], wc = wct[i];
                     const T J = fma_<T>(q, s, baseJ);
                     const T K = prsq<P>(J);

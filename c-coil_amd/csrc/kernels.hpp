@@ -15,6 +15,7 @@ struct NearState {
     unsigned int overflow;      // total > near_cap: the pass was skipped
     unsigned int mismatch;      // near_fill classified a pair differently from field_kernel
     unsigned long long fp64;    // records of kind 0 (FP64 rule)
+    unsigned long long split;   // records of kind 0 that are split over more lanes (the first ones)
 };
 
 struct FieldParams {
@@ -29,9 +30,10 @@ struct FieldParams {
     // Rule records (the series modes, large calls): field_kernel evaluates only the series and defers every other
     // (coil, point) pair to the record pass below, which runs the rule on waves of one coil each. A record's kind is
     // 0 for the FP64 rule (FP32C's near pairs; every rule pair in FP64) and 1 for the float rule (FP32C's others);
-    // its key is kind * n_coils + CoilDev::near_key, n_keys = n_coils * (1 + float_records).
+    // its key is record_key below; n_keys = n_coils * (n_slots + float_records).
     int32_t rule_records;
     int32_t float_records;
+    int32_t n_slots;       // key slots of a coil's FP64 records: kRuleClasses, 4 or 2 (record_slot)
     int32_t n_keys;
     // FP32C far field: the recurrence header and each coil's moments (kMpHeader + n_coils * kMpCoil doubles,
     // multipole.hpp); a coil with CoilDev::far_d2 > 0 takes its series beyond that distance. NULL: no coil does.
@@ -70,6 +72,8 @@ struct FieldParams {
     double *partial;
 };
 
+constexpr int64_t kUniformRecordPoints = (int64_t)1 << 17;
+
 // What becomes of a (coil, point) pair: -1 field_kernel evaluates it (the series beyond the far-field distance, or
 // the rule in the kernel), 0 an FP64-rule record, 1 a float-rule record. field_kernel, near_count and near_fill all
 // classify with this, bitwise alike (to_local and the tests round operation by operation).
@@ -79,6 +83,45 @@ __device__ inline int record_kind(const FieldParams &p, const CoilDev &c, double
     const bool near = p.near_fp64 && is_near(c, z, r, axis);
     if (p.rule_records) return (p.float_records && !near) ? 1 : 0;
     return near ? 0 : -1;
+}
+
+// Whether near_eval gives each wave one coil and class at a time (uniform control flow, scalar loads: calls whose
+// records are many per key) or each group of lanes its own record (calls with few records, where a wave would hold a
+// dozen keys and take them in series: 128 coils at 16,411 points measured 640 us that way, 60 us in groups, while at
+// 2^20 points the groups' vector loads are the slower way).
+__host__ __device__ inline bool uniform_records(const FieldParams &p)
+{
+    return p.n_pts >= kUniformRecordPoints;
+}
+
+// The sort key of a record: slot, then coil (most nodes first). FP64 records whose serial chain of nodes would outlast
+// the rest of the launch come first, and near_eval splits them over more lanes; with two slots that is all. Else
+// uniform records are sorted by rule class, the costliest first, so that a wave holds one coil's records of one
+// class: the split ones, with the coil's own angular rule and at least kRecordSplit thickness rows, take the first
+// kSplitSlots slots. Grouped records are sorted by their node count in steps of four, the split ones with kGroupSplit
+// nodes or more. Float records follow by coil.
+constexpr int kRecordSplit = 8;
+constexpr int kSplitSlots = kRedThk;
+constexpr int kGroupSplit = 640;
+static_assert(kRedThkN[kRedThk - 1] < kRecordSplit && kRedThkN[kRedThk - 2] >= kRecordSplit, "record_slot");
+__device__ inline uint32_t record_slot(const FieldParams &p, const CoilDev &c, int kind, double z, double r)
+{
+    if (kind) return (uint32_t)p.n_slots;
+    const int cls = rule_class(c, z, r);
+    if (uniform_records(p)) {
+        const int k = cls / (kRedThk + 1), t = cls - k * (kRedThk + 1);
+        const bool rows = t == 0 ? c.n_thk >= kRecordSplit : t < kRedThk;   // at least kRecordSplit
+        if (p.n_slots == 2) return k == 0 && rows ? 0u : 1u;
+        return (uint32_t)(rows ? cls : k * (kRedThk + 1) + kRedThk);
+    }
+    const RuleSel s = class_rule(c, cls);
+    const int n = s.na * s.nt;
+    if (p.n_slots == 2) return n >= kGroupSplit ? 0u : 1u;
+    return n >= kGroupSplit ? 0u : n >= kGroupSplit / 4 ? 1u : n >= kGroupSplit / 16 ? 2u : 3u;
+}
+__device__ inline uint32_t record_key(const FieldParams &p, const CoilDev &c, int kind, double z, double r)
+{
+    return record_slot(p, c, kind, z, r) * (uint32_t)p.n_coils + (uint32_t)c.near_key;
 }
 
 // Adjoint of the summed B field: per-coil gradients of sum_x dL/dB(x) . B(x), 9 per coil in the order
@@ -111,11 +154,16 @@ void launch_field(hipStream_t s, const FieldParams &p, int precision, int split)
 void launch_field_reduce(hipStream_t s, const FieldParams &p);   // after launch_field when n_chunks > 1
 // Resident 256-thread blocks per CU of the field kernel instance (0 if the runtime cannot tell).
 int field_blocks_per_cu(uint32_t q, int precision, int split);
-// Whether the series-only kernel counts the record pass's keys (in LDS, 4 bytes per coil of a chunk and kind), so
-// that near_count_kernel is not launched: calls with rule records whose coil chunks fit.
+// Whether the series-only kernel counts the record pass's keys (in LDS, 4 bytes per coil of a chunk and slot), so
+// that near_count_kernel is not launched: calls with rule records whose coil chunks fit 40 KB, where the kernel's four
+// blocks per CU still share the LDS.
+__host__ __device__ inline int series_key_words(const FieldParams &p)
+{
+    return p.coils_per_chunk * (p.n_slots + (p.float_records ? 1 : 0));
+}
 __host__ __device__ inline bool series_counts_keys(const FieldParams &p)
 {
-    return p.rule_records && p.coils_per_chunk <= 4096;
+    return p.rule_records && series_key_words(p) <= 10240;
 }
 // Resident 256-thread blocks per CU of the series-only kernel (the launch of calls with rule records).
 int field_series_blocks_per_cu(uint32_t q, int precision);

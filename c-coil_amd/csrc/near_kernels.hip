@@ -11,6 +11,7 @@
 // its slot; near_add_kernel adds a point's slots to the outputs in coil order. A slot's value depends only on its
 // (coil, point), and every sum has a fixed order, so FP32C results are bitwise reproducible although the order of the
 // records within a coil is not. Nothing here is read back by the host before the work is done.
+#include <algorithm>
 #include <cstddef>
 
 #include "kernels.hpp"
@@ -50,9 +51,8 @@ __device__ inline uint32_t record_candidates(const CoilDev *coils, int n_coils, 
     return m;
 }
 
-// Calls with fewer points than kNearSplitPoints split each near record's thickness rows over kNearSplit lanes.
+// Calls with fewer points than kNearSplitPoints split each float record's thickness rows over kRecordSplit lanes.
 constexpr int64_t kNearSplitPoints = (int64_t)1 << 17;
-constexpr int kNearSplit = 8;
 
 // Per coil key, the near points (points with near pairs only; the coil loop is wave-uniform, so each coil's count
 // in a wave is one ballot and one atomic).
@@ -71,32 +71,50 @@ __global__ __launch_bounds__(256) void near_count_kernel(FieldParams p)
             double z, r, cph, sph;
             to_local(c, px, py, pz, z, r, cph, sph);
             const int kind = record_kind(p, c, z, r, p.q & (Q_G | Q_GJ));   // the field kernel's test, bitwise
-            for (int k = 0; k <= p.float_records; ++k) {
-                const uint64_t m = __ballot(kind == k);
-                if (m && lane == __builtin_ctzll(m))
-                    atomicAdd(&p.near_hist[k * p.n_coils + c.near_key], (unsigned)__popcll(m));
+            const uint32_t key = kind < 0 ? 0u : record_key(p, c, kind, z, r);
+            uint64_t todo = __ballot(kind >= 0);
+            while (todo) {
+                const uint32_t k = __builtin_amdgcn_readfirstlane(__shfl(key, __builtin_ctzll(todo)));
+                const uint64_t m = __ballot(kind >= 0 && key == k);
+                if (lane == __builtin_ctzll(m)) atomicAdd(&p.near_hist[k], (unsigned)__popcll(m));
+                todo &= ~m;
             }
         }
 }
 
-// One workgroup: cursor = exclusive prefix sum of near_hist over the n_coils + 1 keys, and the call's total.
-__global__ __launch_bounds__(256) void near_key_scan_kernel(FieldParams p)
+// One workgroup: cursor = exclusive prefix sum of near_hist over the keys, and the call's total. Four keys per thread
+// and iteration, scanned by waves: a call's few thousand keys (coils x rule classes) take two iterations.
+constexpr int kKeyScanThreads = 1024;
+__global__ __launch_bounds__(kKeyScanThreads) void near_key_scan_kernel(FieldParams p)
 {
-    __shared__ uint32_t part[256];
-    const int t = threadIdx.x, nk = p.n_keys + 1;
+    __shared__ uint32_t wsum[kKeyScanThreads / 64];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nk = p.n_keys + 1;
     uint32_t carry = 0;
-    for (int base = 0; base < nk; base += 256) {
-        const uint32_t v = base + t < nk ? p.near_hist[base + t] : 0u;
-        part[t] = v;
-        __syncthreads();
-        for (int d = 1; d < 256; d <<= 1) {   // inclusive Hillis-Steele scan
-            const uint32_t add = t >= d ? part[t - d] : 0u;
-            __syncthreads();
-            part[t] += add;
-            __syncthreads();
+    for (int base = 0; base < nk; base += 4 * kKeyScanThreads) {
+        const int i0 = base + 4 * t;
+        uint32_t v[4], own = 0;
+        for (int k = 0; k < 4; ++k) {
+            v[k] = i0 + k < p.n_keys ? p.near_hist[i0 + k] : 0u;
+            own += v[k];
         }
-        if (base + t < nk) p.near_cursor[base + t] = carry + part[t] - v;
-        carry += part[255];
+        uint32_t incl = own;   // inclusive scan of the wave's threads
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t add = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += add;
+        }
+        if (lane == 63) wsum[wave] = incl;
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+        for (int w = 0; w < kKeyScanThreads / 64; ++w) {
+            if (w < wave) before += wsum[w];
+            all += wsum[w];
+        }
+        uint32_t run = carry + before + incl - own;
+        for (int k = 0; k < 4; ++k) {
+            if (i0 + k < nk) p.near_cursor[i0 + k] = run;
+            run += v[k];
+        }
+        carry += all;
         __syncthreads();
     }
     if (t == 0) {
@@ -104,8 +122,12 @@ __global__ __launch_bounds__(256) void near_key_scan_kernel(FieldParams p)
             (unsigned long long)(p.near_offsets[p.n_pts - 1] + p.near_counts[p.n_pts - 1]);
         p.near_state->total = total;
         p.near_state->overflow = total > (unsigned long long)p.near_cap ? 1u : 0u;
-        p.near_state->fp64 = p.near_cursor[p.n_coils];   // the kind-0 keys come first
     }
+    // the threads that wrote these cursors: the kind-0 keys come first, and of those the split ones
+    const int64_t k_fp64 = (int64_t)p.n_slots * p.n_coils;
+    const int64_t k_split = (int64_t)(p.n_slots == kRuleClasses ? kSplitSlots : 1) * p.n_coils;
+    if (k_fp64 / 4 % kKeyScanThreads == t) p.near_state->fp64 = p.near_cursor[k_fp64];
+    if (k_split / 4 % kKeyScanThreads == t) p.near_state->split = p.near_cursor[k_split];
 }
 
 __global__ __launch_bounds__(256) void near_fill_kernel(FieldParams p)
@@ -131,18 +153,23 @@ __global__ __launch_bounds__(256) void near_fill_kernel(FieldParams p)
             double z, r, cph, sph;
             to_local(c, px, py, pz, z, r, cph, sph);
             const int kind = record_kind(p, c, z, r, p.q & (Q_G | Q_GJ));   // the field kernel's test, bitwise
-            // the wave's records of this coil and kind take consecutive places from one atomic on the key's cursor
-            for (int k = 0; k <= p.float_records; ++k) {
-                const bool mine = kind == k;
+            // the wave's records of one key take consecutive places from one atomic on the key's cursor; the keys'
+            // leading lanes issue theirs together, so a coil costs one round trip
+            const uint32_t key = kind < 0 ? 0u : record_key(p, c, kind, z, r);
+            uint64_t todo = __ballot(kind >= 0), same = 0;
+            while (todo) {
+                const uint32_t k = __builtin_amdgcn_readfirstlane(__shfl(key, __builtin_ctzll(todo)));
+                const bool mine = kind >= 0 && key == k;
                 const uint64_t m = __ballot(mine);
-                if (!m) continue;
-                const int leader = __builtin_ctzll(m);
-                const uint32_t key = (uint32_t)(k * p.n_coils + c.near_key);
-                uint32_t base = 0;
-                if (lane == leader) base = atomicAdd(&p.near_cursor[key], (unsigned)__popcll(m));
-                base = __shfl(base, leader);
-                if (!mine) continue;
-                const uint64_t pos = base + (uint64_t)__popcll(m & ((1ull << lane) - 1ull));
+                if (mine) same = m;
+                todo &= ~m;
+            }
+            const int leader = kind < 0 ? lane : __builtin_ctzll(same);
+            uint32_t base = 0;
+            if (kind >= 0 && lane == leader) base = atomicAdd(&p.near_cursor[key], (unsigned)__popcll(same));
+            base = __shfl(base, leader);
+            if (kind >= 0) {
+                const uint64_t pos = base + (uint64_t)__popcll(same & ((1ull << lane) - 1ull));
                 // a pair classified differently from the series or field kernel: report it, write nothing
                 if (slot >= end || pos >= total) {
                     bad = true;
@@ -157,84 +184,133 @@ __global__ __launch_bounds__(256) void near_fill_kernel(FieldParams p)
     if (bad || slot != end) atomicOr(&p.near_state->mismatch, 1u);
 }
 
-// Records sorted by coil: S consecutive lanes take one record (thickness rows sub, sub + S, ..., combined by a
-// fixed xor butterfly, so every lane of the group holds the same sum); its value goes to the record's slot. S > 1 on
-// calls with few points, where the records are too few to fill the chip one lane each and one lane's serial chain
-// of nodes sets the kernel's duration; the lanes then stride over the records (a group's value does not depend on
-// the grid). FLOAT: the kind-1 records [fp64, total) by the float rule, at 5 waves per SIMD as field_kernel's float
-// instances; else the kind-0 records [0, fp64) by the FP64 rule.
-template <bool WA, bool WB, bool WG, bool FLOAT, int S, bool LOOP>
+// Sum over the S lanes of a record by a fixed xor butterfly, so every lane of the group holds the same sum.
+__device__ inline void reduce_record(Local &L, int S)
+{
+    for (int m = 1; m < S; m <<= 1) {
+        L.A += __shfl_xor(L.A, m, 64);
+        L.Bh += __shfl_xor(L.Bh, m, 64);
+        L.Bz += __shfl_xor(L.Bz, m, 64);
+        L.RP += __shfl_xor(L.RP, m, 64);
+        L.RR += __shfl_xor(L.RR, m, 64);
+        L.RZ += __shfl_xor(L.RZ, m, 64);
+        L.ZZ += __shfl_xor(L.ZZ, m, 64);
+    }
+}
+
+// Records sorted by rule class and coil. S consecutive lanes of a wave take one record (thickness rows sub, sub + S,
+// ...); its value goes to the record's slot. FLOAT: the kind-1 records [fp64, total) by the float rule, at 5 waves per
+// SIMD as field_kernel's float instances, S = kRecordSplit in calls with few points, where the records are too few to
+// fill the chip one lane each; else the kind-0 records [0, fp64) by the FP64 rule, S = kRecordSplit for the first
+// `split` of them (record_slot) and 1 for the others, whose reduced rules have at most a few hundred nodes. S follows
+// from the record and the call's shape alone, so a record's value does not depend on its wave.
+template <bool WA, bool WB, bool WG, bool FLOAT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FLOAT ? 5 : 1)))
 void near_eval_kernel(FieldParams p)
 {
     if (p.near_state->overflow) return;
     const int64_t total = (int64_t)p.near_state->total, fp64 = (int64_t)p.near_state->fp64;
-    const int64_t lo = FLOAT ? fp64 : 0, hi = FLOAT ? total : fp64;
-    const int sub = (int)(threadIdx.x % S);
-    auto record = [&](int64_t e) {
+    const int64_t hi = FLOAT ? total : fp64;
+    // waves of split records first; a split wave at the end of its range is part empty
+    const int64_t wave = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6;
+    const int64_t first = FLOAT ? fp64 : 0;
+    const int64_t n_split = FLOAT ? (p.n_pts < kNearSplitPoints ? total - fp64 : 0) : (int64_t)p.near_state->split;
+    const int64_t split_waves = (n_split * kRecordSplit + 63) >> 6;
+    const int S = __builtin_amdgcn_readfirstlane(wave < split_waves ? kRecordSplit : 1);
+    const int lane = (int)(threadIdx.x & 63), sub = lane % S;
+    const int64_t e = S > 1 ? first + wave * (64 / kRecordSplit) + lane / kRecordSplit
+                            : first + n_split + ((wave - split_waves) << 6) + lane;
+    if (e >= (S > 1 ? first + n_split : hi)) return;
+    const uint32_t key = p.near_keys[e];
+    const uint64_t rec = p.near_recs[e];
+    const int64_t pi = (int64_t)(rec >> 32), slot = (int64_t)(rec & 0xffffffffu);
+    // only a near_fill that reported a mismatch leaves records unwritten; never follow one out of bounds
+    if (pi >= p.n_pts || slot >= total) return;
+    double *o = p.near_vals + slot * p.near_width;
+    // A wave holds one coil's records, or two or more at the boundaries of the sorted keys: it takes its keys one at a
+    // time (the key of the lowest lane still to do, read into a scalar register), and every lane evaluates that coil
+    // at its point, keeping the value only if the key is its own. The control flow stays uniform and no store
+    // precedes the loads, so the coil's fields and the quadrature tables are scalar loads, as in field_kernel; a
+    // divergent branch would take the same issue time. todo is wave-uniform and loses at least one lane on every pass;
+    // a group's lanes share their key, so a group is always active as a whole.
+    const double px = p.pts[3 * pi], py = p.pts[3 * pi + 1], pz = p.pts[3 * pi + 2];
+    Cart acc;
+    for (int j = 0; j < 3; ++j) { acc.A[j] = 0.0; acc.E[j] = 0.0; acc.B[j] = 0.0; }
+    for (int j = 0; j < 9; ++j) acc.G[j] = 0.0;
+    uint64_t todo = __ballot(1);
+    while (todo) {
+        const uint32_t k = __builtin_amdgcn_readfirstlane(__shfl(key, __builtin_ctzll(todo)));
+        const bool mine = key == k;
+        todo &= ~(uint64_t)__ballot(mine);
+        // only a reported mismatch can leave a key outside the range's kind
+        const uint32_t slot_of = k / (uint32_t)p.n_coils;
+        if (k >= (uint32_t)p.n_keys || (slot_of == (uint32_t)p.n_slots) != FLOAT) continue;
+        const CoilDev &c = p.coils[p.near_coil[k - slot_of * (uint32_t)p.n_coils]];
+        double z, r, cph, sph;
+        to_local(c, px, py, pz, z, r, cph, sph);
+        // FP64 records take their rule classes one at a time too (a slot holds one class, but for the coils of few
+        // rows): the rule's node sets stay uniform, hence scalar loads
+        const int cls = FLOAT ? 0 : rule_class(c, z, r);
+        uint64_t left = __ballot(mine);
+        while (left) {
+            const int q = FLOAT ? 0 : __builtin_amdgcn_readfirstlane(__shfl(cls, __builtin_ctzll(left)));
+            const bool sel = mine && cls == q;
+            left &= ~(uint64_t)__ballot(sel);
+            Local L;
+            if (FLOAT) eval_stable<float, WA, WB, WG>(c, p.tab, full_rule(c), z, r, sub, S, 0, 1, L);
+            else eval_stable<f64s, WA, WB, WG>(c, p.tab, class_rule(c, q), z, r, sub, S, 0, 1, L);
+            reduce_record(L, S);
+            if (sel) accumulate_global(c, L, r, cph, sph, p.q, acc);
+        }
+    }
+    if (sub == 0) {
+        if (p.A) { for (int j = 0; j < 3; ++j) o[j] = acc.A[j]; o += 3; }
+        if (p.E) { for (int j = 0; j < 3; ++j) o[j] = acc.E[j]; o += 3; }
+        if (p.B) { for (int j = 0; j < 3; ++j) o[j] = acc.B[j]; o += 3; }
+        if (p.G) for (int j = 0; j < 9; ++j) o[j] = acc.G[j];
+    }
+}
+
+// The kind-0 records of calls with few of them: a group of consecutive lanes takes a record of its own coil and rule
+// class, a whole wave for the first `split` of them (kGroupSplit nodes or more) and kRecordSplit lanes for the others.
+// The lanes split the rows in four (two) and the rows' nodes: 80 x 20 nodes take 25 steps of a wave. Coil and tables
+// are vector loads; a wave takes as long as its longest record, and the records are sorted by node count.
+template <bool WA, bool WB, bool WG>
+__global__ __launch_bounds__(256) void near_eval_group_kernel(FieldParams p)
+{
+    if (p.near_state->overflow) return;
+    const int64_t n_split = (int64_t)p.near_state->split, fp64 = (int64_t)p.near_state->fp64;
+    const int64_t waves = n_split + (fp64 - n_split + 64 / kRecordSplit - 1) / (64 / kRecordSplit);
+    const int lane = (int)(threadIdx.x & 63);
+    // a bounded grid strides over the waves' worth of records; the bound is wave-uniform
+    for (int64_t wave = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6; wave < waves; wave += (int64_t)gridDim.x * 4) {
+        const int group = __builtin_amdgcn_readfirstlane(wave < n_split ? 64 : kRecordSplit);
+        const int sub = lane % group;
+        const int64_t e = group == 64 ? wave : n_split + (wave - n_split) * (64 / kRecordSplit) + lane / kRecordSplit;
+        if (e >= fp64) continue;   // whole groups, in the last wave only
         const uint32_t key = p.near_keys[e];
         const uint64_t rec = p.near_recs[e];
         const int64_t pi = (int64_t)(rec >> 32), slot = (int64_t)(rec & 0xffffffffu);
         // only a near_fill that reported a mismatch leaves records unwritten; never follow one out of bounds
-        if (pi >= p.n_pts || slot >= total) return;
-        double *o = p.near_vals + slot * p.near_width;
-        // A wave holds one coil's records, or two or more at the boundaries of the sorted keys: it takes its keys
-        // one at a time (the key of the lowest lane still to do, read into a scalar register), and every lane
-        // evaluates that coil at its point, keeping the value only if the key is its own. The control flow stays
-        // uniform and no store precedes the loads, so the coil's fields and the quadrature tables are scalar loads,
-        // as in field_kernel; a divergent branch would take the same issue time. todo is wave-uniform and loses at
-        // least one lane on every pass; a group's lanes share their key, so a group is always active as a whole.
-        const double px = p.pts[3 * pi], py = p.pts[3 * pi + 1], pz = p.pts[3 * pi + 2];
+        if (pi >= p.n_pts || slot >= (int64_t)p.near_state->total || key >= (uint32_t)(p.n_slots * p.n_coils)) continue;
+        const CoilDev &c = p.coils[p.near_coil[key % (uint32_t)p.n_coils]];
+        double z, r, cph, sph;
+        to_local(c, p.pts[3 * pi], p.pts[3 * pi + 1], p.pts[3 * pi + 2], z, r, cph, sph);
+        const RuleSel rule = class_rule(c, rule_class(c, z, r));
+        const int sr = rule.nt == 1 ? 1 : group == 64 ? 4 : 2;
+        Local L;
+        eval_stable<f64s, WA, WB, WG>(c, p.tab, rule, z, r, sub & (sr - 1), sr, sub / sr, group / sr, L);
+        reduce_record(L, group);
+        if (sub) continue;
         Cart acc;
         for (int j = 0; j < 3; ++j) { acc.A[j] = 0.0; acc.E[j] = 0.0; acc.B[j] = 0.0; }
         for (int j = 0; j < 9; ++j) acc.G[j] = 0.0;
-        uint64_t todo = __ballot(1);
-        while (todo) {
-            const uint32_t k = __builtin_amdgcn_readfirstlane(__shfl(key, __builtin_ctzll(todo)));
-            const bool mine = key == k;
-            todo &= ~(uint64_t)__ballot(mine);
-            // only a reported mismatch can leave a key outside the range's kind
-            const uint32_t kind = k / (uint32_t)p.n_coils;
-            if (k >= (uint32_t)p.n_keys || kind != (FLOAT ? 1u : 0u)) continue;
-            const CoilDev &c = p.coils[p.near_coil[k - kind * (uint32_t)p.n_coils]];
-            double z, r, cph, sph;
-            to_local(c, px, py, pz, z, r, cph, sph);
-            Local L;
-            if (FLOAT) eval_stable<float, WA, WB, WG>(c, p.tab, z, r, sub, S, L);
-            else eval_stable<f64s, WA, WB, WG>(c, p.tab, z, r, sub, S, L);
-            if constexpr (S > 1) {
-#pragma unroll
-                for (int m = 1; m < S; m <<= 1) {
-                    L.A += __shfl_xor(L.A, m, 64);
-                    L.Bh += __shfl_xor(L.Bh, m, 64);
-                    L.Bz += __shfl_xor(L.Bz, m, 64);
-                    L.RP += __shfl_xor(L.RP, m, 64);
-                    L.RR += __shfl_xor(L.RR, m, 64);
-                    L.RZ += __shfl_xor(L.RZ, m, 64);
-                    L.ZZ += __shfl_xor(L.ZZ, m, 64);
-                }
-            }
-            if (mine) accumulate_global(c, L, r, cph, sph, p.q, acc);
-        }
-        if (sub == 0) {
-            if (p.A) { for (int j = 0; j < 3; ++j) o[j] = acc.A[j]; o += 3; }
-            if (p.E) { for (int j = 0; j < 3; ++j) o[j] = acc.E[j]; o += 3; }
-            if (p.B) { for (int j = 0; j < 3; ++j) o[j] = acc.B[j]; o += 3; }
-            if (p.G) for (int j = 0; j < 9; ++j) o[j] = acc.G[j];
-        }
-    };
-    const int64_t e0 = lo + ((int64_t)blockIdx.x * 256 + threadIdx.x) / S;
-    if constexpr (!LOOP) {
-        // the grid covers the capacity, one record per group; with no store before the loads, the coil records
-        // and the tables are scalar loads
-        if (e0 < hi) record(e0);
-    } else {
-        // a bounded grid strides over a larger capacity (the stores in the loop make the loads vector loads). A
-        // wave's groups hold consecutive records, so the loop's exit is wave-uniform once no lane has a record
-        // left, and a group is active or idle as a whole
-        const int64_t stride = (int64_t)gridDim.x * (256 / S);
-        for (int64_t e = e0; __ballot(e < hi); e += stride)
-            if (e < hi) record(e);
+        accumulate_global(c, L, r, cph, sph, p.q, acc);
+        double *o = p.near_vals + slot * p.near_width;
+        if (p.A) { for (int j = 0; j < 3; ++j) o[j] = acc.A[j]; o += 3; }
+        if (p.E) { for (int j = 0; j < 3; ++j) o[j] = acc.E[j]; o += 3; }
+        if (p.B) { for (int j = 0; j < 3; ++j) o[j] = acc.B[j]; o += 3; }
+        if (p.G) for (int j = 0; j < 9; ++j) o[j] = acc.G[j];
     }
 }
 
@@ -353,7 +429,7 @@ hipError_t near_scan(hipStream_t s, const int64_t *counts, int64_t *offsets, int
 void launch_near_key_scan(hipStream_t s, const FieldParams &p)
 {
     if (p.n_pts <= 0) return;
-    hipLaunchKernelGGL(near_key_scan_kernel, dim3(1), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(near_key_scan_kernel, dim3(1), dim3(kKeyScanThreads), 0, s, p);
 }
 
 void launch_near_count(hipStream_t s, const FieldParams &p)
@@ -368,49 +444,47 @@ void launch_near_fill(hipStream_t s, const FieldParams &p)
     hipLaunchKernelGGL(near_fill_kernel, dim3((unsigned)((p.n_pts + 255) / 256)), dim3(256), 0, s, p);
 }
 
-template <bool FLOAT, int S, bool LOOP>
+template <bool FLOAT>
 static void launch_near_eval_g(hipStream_t s, const FieldParams &p, unsigned blocks)
 {
     const bool wa = p.q & (Q_A | Q_E), wb = p.q & Q_B, wg = p.q & (Q_G | Q_GJ);
     const dim3 g(blocks), b(256);
     switch ((wa ? 4 : 0) | (wb ? 2 : 0) | (wg ? 1 : 0)) {
-        case 1: hipLaunchKernelGGL((near_eval_kernel<false, false, true, FLOAT, S, LOOP>), g, b, 0, s, p); break;
-        case 2: hipLaunchKernelGGL((near_eval_kernel<false, true, false, FLOAT, S, LOOP>), g, b, 0, s, p); break;
-        case 3: hipLaunchKernelGGL((near_eval_kernel<false, true, true, FLOAT, S, LOOP>), g, b, 0, s, p); break;
-        case 4: hipLaunchKernelGGL((near_eval_kernel<true, false, false, FLOAT, S, LOOP>), g, b, 0, s, p); break;
-        case 5: hipLaunchKernelGGL((near_eval_kernel<true, false, true, FLOAT, S, LOOP>), g, b, 0, s, p); break;
-        case 6: hipLaunchKernelGGL((near_eval_kernel<true, true, false, FLOAT, S, LOOP>), g, b, 0, s, p); break;
-        default: hipLaunchKernelGGL((near_eval_kernel<true, true, true, FLOAT, S, LOOP>), g, b, 0, s, p); break;
+        case 1: hipLaunchKernelGGL((near_eval_kernel<false, false, true, FLOAT>), g, b, 0, s, p); break;
+        case 2: hipLaunchKernelGGL((near_eval_kernel<false, true, false, FLOAT>), g, b, 0, s, p); break;
+        case 3: hipLaunchKernelGGL((near_eval_kernel<false, true, true, FLOAT>), g, b, 0, s, p); break;
+        case 4: hipLaunchKernelGGL((near_eval_kernel<true, false, false, FLOAT>), g, b, 0, s, p); break;
+        case 5: hipLaunchKernelGGL((near_eval_kernel<true, false, true, FLOAT>), g, b, 0, s, p); break;
+        case 6: hipLaunchKernelGGL((near_eval_kernel<true, true, false, FLOAT>), g, b, 0, s, p); break;
+        default: hipLaunchKernelGGL((near_eval_kernel<true, true, true, FLOAT>), g, b, 0, s, p); break;
     }
 }
 
-// S = 1: one lane per record of the capacity. S > 1: S lanes per record of the capacity while that is at most 2^21
-// lanes, else a grid of 2^21 lanes striding over the records.
-template <bool FLOAT, int S>
-static void launch_near_eval_k(hipStream_t s, const FieldParams &p)
+static void launch_near_eval_group(hipStream_t s, const FieldParams &p, unsigned blocks)
 {
-    const int64_t lanes = p.near_cap * S, max_lanes = (int64_t)1 << 21;
-    if constexpr (S == 1) {
-        launch_near_eval_g<FLOAT, 1, false>(s, p, (unsigned)((lanes + 255) / 256));
-    } else {
-        if (lanes <= max_lanes) launch_near_eval_g<FLOAT, S, false>(s, p, (unsigned)((lanes + 255) / 256));
-        else launch_near_eval_g<FLOAT, S, true>(s, p, (unsigned)(max_lanes / 256));
+    const bool wa = p.q & (Q_A | Q_E), wb = p.q & Q_B, wg = p.q & (Q_G | Q_GJ);
+    const dim3 g(blocks), b(256);
+    switch ((wa ? 4 : 0) | (wb ? 2 : 0) | (wg ? 1 : 0)) {
+        case 1: hipLaunchKernelGGL((near_eval_group_kernel<false, false, true>), g, b, 0, s, p); break;
+        case 2: hipLaunchKernelGGL((near_eval_group_kernel<false, true, false>), g, b, 0, s, p); break;
+        case 3: hipLaunchKernelGGL((near_eval_group_kernel<false, true, true>), g, b, 0, s, p); break;
+        case 4: hipLaunchKernelGGL((near_eval_group_kernel<true, false, false>), g, b, 0, s, p); break;
+        case 5: hipLaunchKernelGGL((near_eval_group_kernel<true, false, true>), g, b, 0, s, p); break;
+        case 6: hipLaunchKernelGGL((near_eval_group_kernel<true, true, false>), g, b, 0, s, p); break;
+        default: hipLaunchKernelGGL((near_eval_group_kernel<true, true, true>), g, b, 0, s, p); break;
     }
 }
 
-// Each grid covers the capacity; threads beyond their kind's range (read on the device) return at once. Calls with
-// fewer than 2^17 points split each record's rows over 8 lanes (a choice made from the call's shape alone, so a
-// call and its captured plan run the same split).
+// Each grid covers the capacity with every record split (float records of large calls: none); the waves beyond the
+// records there are (read on the device) return at once.
 void launch_near_eval(hipStream_t s, const FieldParams &p)
 {
     if (p.near_cap <= 0) return;
-    if (p.n_pts < kNearSplitPoints) {
-        launch_near_eval_k<false, kNearSplit>(s, p);
-        if (p.float_records) launch_near_eval_k<true, kNearSplit>(s, p);
-    } else {
-        launch_near_eval_k<false, 1>(s, p);
-        if (p.float_records) launch_near_eval_k<true, 1>(s, p);
-    }
+    const unsigned split = (unsigned)((p.near_cap * kRecordSplit + 255) / 256 + 1);
+    if (uniform_records(p)) launch_near_eval_g<false>(s, p, split);
+    else launch_near_eval_group(s, p, (unsigned)std::min<int64_t>((p.near_cap + 3) / 4, 8192));
+    if (p.float_records)
+        launch_near_eval_g<true>(s, p, p.n_pts < kNearSplitPoints ? split : (unsigned)((p.near_cap + 255) / 256));
 }
 
 void launch_near_add(hipStream_t s, const FieldParams &p)

@@ -31,23 +31,23 @@ __device__ inline void eval_prim(const CoilDev &pc, const Tables &tab, double z,
                                  Local &L, AdjA *ada)
 {
     if constexpr (GR) {   // gradients of M: A, B and the pair adjoint extras; FP64, FP64_IEEE or FP32C far nodes
-        if constexpr (PREC == 4) eval_stable<double, true, true, false, false, true>(pc, tab, z, r, row0, rstep, L, nullptr, ada);
-        else if constexpr (PREC == 1) eval_stable<float, true, true, false, false, true>(pc, tab, z, r, row0, rstep, L, nullptr, ada);
-        else eval_stable<f64s, true, true, false, false, true>(pc, tab, z, r, row0, rstep, L, nullptr, ada);
+        if constexpr (PREC == 4) eval_stable<double, true, true, false, false, true>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L, nullptr, ada);
+        else if constexpr (PREC == 1) eval_stable<float, true, true, false, false, true>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L, nullptr, ada);
+        else eval_stable<f64s, true, true, false, false, true>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L, nullptr, ada);
         return;
     }
     if constexpr (PREC == 0) {
-        eval_stable<f64s, WM, WF, false, false, false, true>(pc, tab, z, r, row0, rstep, L);
+        eval_stable<f64s, WM, WF, false, false, false, true>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L);
     } else if constexpr (PREC == 4) {
-        eval_stable<double, WM, WF, false>(pc, tab, z, r, row0, rstep, L);
+        eval_stable<double, WM, WF, false>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L);
     } else if constexpr (PREC == 2) {
         eval_plain<float, WM, WF, false>(pc, tab, z, r, row0, rstep, L);
     } else if constexpr (PREC == 3) {
         eval_plain<double, WM, WF, false>(pc, tab, z, r, row0, rstep, L);
     } else if (is_near(pc, z, r, false)) {
-        eval_stable<f64s, WM, WF, false>(pc, tab, z, r, row0, rstep, L);
+        eval_stable<f64s, WM, WF, false>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L);
     } else {
-        eval_stable<float, WM, WF, false>(pc, tab, z, r, row0, rstep, L);
+        eval_stable<float, WM, WF, false>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L);
     }
 }
 
@@ -272,13 +272,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pa
                         Local L = {0, 0, 0, 0, 0, 0, 0};
                         if constexpr (GR) {
                             AdjA q;
-                            eval_stable<float, true, true, false, false, true>(pc, p.tab, n.z, n.r, rg, pd.row_groups,
+                            eval_stable<float, true, true, false, false, true>(pc, p.tab, full_rule(pc), n.z, n.r, rg, pd.row_groups, 0, 1,
                                                                                L, nullptr, &q);
                             accumulate_grad(n, L, q);
                         } else {
                             AdjA q;
-                            eval_stable<float, WM || WD, WF || WD, false, false, WD, true>(pc, p.tab, n.z, n.r, rg,
-                                                                                     pd.row_groups, L, nullptr, &q);
+                            eval_stable<float, WM || WD, WF || WD, false, false, WD, true>(pc, p.tab, full_rule(pc), n.z, n.r, rg,
+                                                                                     pd.row_groups, 0, 1, L, nullptr, &q);
                             accumulate(n, L, q);
                         }
                     }
@@ -294,13 +294,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pa
                         Local L = {0, 0, 0, 0, 0, 0, 0};
                         if constexpr (GR) {
                             AdjA q;
-                            eval_stable<f64s, true, true, false, false, true>(pc, p.tab, n.z, n.r, rg, pd.row_groups,
+                            eval_stable<f64s, true, true, false, false, true>(pc, p.tab, full_rule(pc), n.z, n.r, rg, pd.row_groups, 0, 1,
                                                                               L, nullptr, &q);
                             accumulate_grad(n, L, q);
                         } else {
                             AdjA q;
-                            eval_stable<f64s, WM || WD, WF || WD, false, false, WD, true>(pc, p.tab, n.z, n.r, rg,
-                                                                                    pd.row_groups, L, nullptr, &q);
+                            eval_stable<f64s, WM || WD, WF || WD, false, false, WD, true>(pc, p.tab, full_rule(pc), n.z, n.r, rg,
+                                                                                    pd.row_groups, 0, 1, L, nullptr, &q);
                             accumulate(n, L, q);
                         }
                         qh = (qh + 64) & 127;
@@ -315,13 +315,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pa
                 Local L = {0, 0, 0, 0, 0, 0, 0};
                 if constexpr (GR) {
                     AdjA q;
-                    eval_stable<f64s, true, true, false, false, true>(pc, p.tab, n.z, n.r, rg, pd.row_groups, L,
+                    eval_stable<f64s, true, true, false, false, true>(pc, p.tab, full_rule(pc), n.z, n.r, rg, pd.row_groups, 0, 1, L,
                                                                       nullptr, &q);
                     accumulate_grad(n, L, q);
                 } else {
                     AdjA q;
-                    eval_stable<f64s, WM || WD, WF || WD, false, false, WD, true>(pc, p.tab, n.z, n.r, rg,
-                                                                                  pd.row_groups, L, nullptr, &q);
+                    eval_stable<f64s, WM || WD, WF || WD, false, false, WD, true>(pc, p.tab, full_rule(pc), n.z, n.r, rg,
+                                                                                  pd.row_groups, 0, 1, L, nullptr, &q);
                     accumulate(n, L, q);
                 }
             }

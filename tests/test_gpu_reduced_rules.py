@@ -1,0 +1,83 @@
+"""The reduced rules against the coil's own rule.
+
+CCOIL_FP64 replaces a coil's angular or thickness sum by one of fewer nodes where the rule has converged to rounding;
+CCOIL_FP64_IEEE sums the coil's own rule at every pair. Points around the winding at distances from a hundredth to
+thirty times its cross-section cross every class boundary, inside the bore, beyond the ends, outside and on the axis.
+
+Tolerance, per point and relative to the coil's own field: the reduced and the own rule each err by at most 1e-15 of the
+sum of the node terms' magnitudes, and both sums carry rounding of a few ulps of it. That sum exceeds the field by at
+most about (1 + y)^2 (y = D / r_max: the terms cancel to the far field) times 10 for A and B and 100 for the gradient
+where eta >= 0.1 (its terms grow like eta^-4): 2e-14 (1 + y)^2 and 2e-13 (1 + y)^2. Closer points keep the own angular
+rule and differ from CCOIL_FP64_IEEE as before: 1e-11 for A and B, 1e-6 for the gradient. Pairs that take the far-field
+series are held to its 1e-13 of the coil's field at their distance instead.
+"""
+import numpy as np
+import pytest
+
+import ccoil_abi as abi
+import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+COILS = [("RECTANGULAR", 0.1, 0.1, 0.1, 59, 27), ("RECTANGULAR", 0.02, 0.2, 0.01, 48, 34), ("THIN", 0.3, 0.0, 0.2, 80, 1),
+         ("THIN", 0.05, 0.0, 0.005, 12, 1), ("FLAT", 0.1, 0.05, 0.0, 80, 20), ("FLAT", 0.4, 0.2, 0.0, 100, 100),
+         ("FILAMENT", 0.25, 0.0, 0.0, 80, 1), ("FILAMENT", 0.25, 0.0, 0.0, 6, 1), ("RECTANGULAR", 0.2, 0.02, 0.3, 21, 2),
+         ("FLAT", 0.1, 0.05, 0.0, 20, 7)]
+
+
+def _row(typ, R, a, b, n_ang, n_thk):
+    p = dict(type=typ, R=R, a=a, b=b, N=250, I=3.0, pos=np.array([0.03, -0.02, 0.05]), alpha=0.7, beta=1.9)
+    row = W.coil_row(W.make_coil(p))
+    row.update(n_ang=n_ang, n_thk=n_thk, blocks=(1, 1, 1))
+    return row
+
+
+def _points(rng, row, n):
+    """Global points around the winding, and their r, z in the coil's frame."""
+    R, a, b = row["R"], row["a"], row["b"]
+    size = max(a, b, 0.05 * R)
+    d = size * 10.0 ** rng.uniform(-2.0, 1.5, n)
+    t = rng.uniform(0.0, 2.0 * np.pi, n)
+    r = np.abs(R + a * rng.uniform(0.0, 1.0, n) + d * np.cos(t))
+    z = b * rng.uniform(-0.5, 0.5, n) + d * np.sin(t)
+    r[: n // 20] = R * 10.0 ** rng.uniform(-9.0, -2.0, n // 20)   # the axis
+    phi = rng.uniform(0.0, 2.0 * np.pi, n)
+    loc = np.stack([r * np.cos(phi), r * np.sin(phi), z], axis=1)
+    return np.asarray(row["pos"]) + loc @ W.rotation(row["alpha"], row["beta"]).T, r, z
+
+
+def check(ctx, row, n, prec, flags, seed):
+    rng = np.random.default_rng(seed)
+    pts, r, z = _points(rng, row, n)
+    cs = abi.CoilSet.from_rows([row])
+    q = abi.A | abi.B | abi.G
+    ref, _ = ctx.fields(cs, pts, q, abi.FP64_IEEE)
+    got, _ = ctx.fields(cs, pts, q, prec, flags)
+    R, a, hb = row["R"], row["a"], 0.5 * row["b"] if row["use_fast"] else 0.0
+    zd = np.maximum(np.abs(z) - hb, 0.0)
+    rho = np.clip(np.hypot(r, zd), R, R + a)
+    eta = np.arccosh(1.0 + ((rho - r) ** 2 + zd * zd) / (2.0 * rho * r))
+    y = np.hypot(r, z) / np.hypot(R + a, hb)
+    worst = {}
+    for k, near, far in (("A", 1e-11, 2e-14), ("B", 1e-11, 2e-14), ("G", 1e-6, 2e-13)):
+        err = np.linalg.norm(got[k] - ref[k], axis=1)
+        scale = np.linalg.norm(ref[k], axis=1)
+        # near the axis A and B_rho vanish like r while their sums' terms do not: those are of the size of B R for A
+        # and of B for B_rho, which the gradient divides by r (down to 1e-5 R)
+        b = np.linalg.norm(ref["B"], axis=1)
+        scale += b * R if k == "A" else b / np.maximum(r, 1e-5 * R) if k == "G" else 0.0
+        e = err / scale
+        tol = np.where(eta > 0.1, far * (1.0 + y) ** 2, near)
+        if flags & abi.FAR_FIELD:
+            tol = np.maximum(tol, 1e-12)
+        worst[k] = float(np.max(e / tol))
+        i = int(np.argmax(e / tol))
+        assert e[i] <= tol[i], (row["n_ang"], row["n_thk"], k, n, e[i], tol[i], eta[i], y[i], r[i], z[i])
+    return worst
+
+
+@pytest.mark.parametrize("n", [16500, 131500])
+@pytest.mark.parametrize("coil", COILS, ids=lambda c: f"{c[0]}-{c[4]}x{c[5]}")
+def test_records_match_the_own_rule(ctx, coil, n):
+    """The record pass of the series mode: lanes grouped per record (few points), and uniform waves (many)."""
+    print(f"\n{coil} n={n}: worst error over tolerance {check(ctx, _row(*coil), n, abi.FP64, abi.FAR_FIELD, 5)}")
