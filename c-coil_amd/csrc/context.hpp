@@ -114,6 +114,8 @@ constexpr int64_t kOrderMinPoints = 16384;
 // in the record pass (waves of one coil) instead of beside the series; larger calls are split into pieces of
 // kRecordMaxPoints points by ccoil_fields.
 constexpr int64_t kRecordMaxPoints = (int64_t)1 << 20;
+// CCOIL_FP64 calls of the rule alone take one lane per point, in a spatial visit order, from this many points on.
+constexpr int64_t kSortedPoints = 65536;
 // Whether a field call of this precision, flags and size has a record pass, and whether it has rule records.
 bool field_record_pass(int32_t precision, uint32_t flags, int64_t n_points, bool fixed_arena, bool *rule_records);
 double far_threshold(int n_ang, double q, double tol, double ylo);

@@ -93,6 +93,59 @@ __device__ inline void reduce_local(Local &L)
     }
 }
 
+// Rules with at least kCoopNodes nodes are summed by the whole wave, one point after the other (eval_classes).
+template <int SPLIT> constexpr int kCoopNodes = SPLIT == 1 ? 256 : SPLIT == 4 ? 128 : SPLIT == 16 ? 512 : 1 << 30;
+
+__device__ inline double lane_value(double v, int src)   // src: wave-uniform
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)u, src), hi = __builtin_amdgcn_readlane((uint32_t)(u >> 32), src);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// The FP64 rule of one coil at the wave's points that need it, by each point's rule class (rule_class); all lanes of the
+// wave call. The SPLIT lanes of a point get shares of its sums (reduce_local adds them).
+//
+// A wave's points are of one to three classes at most coils. With one lane per point the classes are taken one at a
+// time, so their node sets and tables stay uniform (scalar loads); with SPLIT lanes per point each point's rows and
+// nodes are split over its lanes, whatever its class. A point whose rule has hundreds of nodes -- next to the
+// winding, where the coil's own 80 x 20 nodes stay -- would hold the other 63 lanes up for as long: the whole wave sums
+// it, 25 nodes a lane, and hands the sums to the point's first lane. How a point is summed follows from its class
+// alone, so its value does not depend on its wave.
+template <bool WA, bool WB, bool WG, int SPLIT>
+__device__ inline void eval_classes(const CoilDev &c, const Tables &tab, double z, double r, bool need, Local &L)
+{
+    const int lane = threadIdx.x & 63;
+    const int cls = need ? rule_class(c, z, r) : -1;
+    const RuleSel own = class_rule(c, need ? cls : 0);
+    const bool coop = need && own.na * own.nt >= kCoopNodes<SPLIT>;
+    if constexpr (SPLIT == 1) {
+        uint64_t todo = __ballot(need && !coop);
+        while (todo) {
+            const int q = __builtin_amdgcn_readlane(cls, __builtin_ctzll(todo));
+            const bool sel = need && !coop && cls == q;
+            todo &= ~(uint64_t)__ballot(sel);
+            // every lane evaluates, the class's lanes keep the sums: under a branch on cls == q the compiler would put
+            // the lane's cls for the uniform q, and load the tables lane by lane
+            Local M;
+            eval_stable<f64s, WA, WB, WG>(c, tab, class_rule(c, q), z, r, 0, 1, 0, 1, M);
+            if (sel) L = M;
+        }
+    } else if (SPLIT < 64 && need && !coop) {
+        const int sub = lane % SPLIT, sr = own.nt == 1 ? 1 : SPLIT >= 16 ? 4 : 2;
+        eval_shared<WA, WB, WG>(c, tab, own, z, r, sub & (sr - 1), sr, sub / sr, SPLIT / sr, L);
+    }
+    uint64_t left = __ballot((SPLIT == 64 ? need : coop) && lane % SPLIT == 0);
+    while (left) {
+        const int src = __builtin_ctzll(left);
+        left &= left - 1;
+        Local M;
+        eval_wave<WA, WB, WG>(c, tab, class_rule(c, __builtin_amdgcn_readlane(cls, src)), lane_value(z, src),
+                              lane_value(r, src), lane, M);
+        if (lane == src) L = M;
+    }
+}
+
 // Minimum waves per SIMD: 5 for the float instances (at most 102 VGPRs; the spills this costs sit at the coil
 // level, outside the node loops; the FP32C headline kernel measured 7.6 % faster than at the allocator's 4 waves),
 // the allocator's choice for the double instances (forcing more waves there was slower).
@@ -133,9 +186,10 @@ void field_kernel(FieldParams p)
             // pair) nothing here: the record pass adds them; elsewhere the rule
             const bool far = is_far(c, z, r);
             const int kind = record_kind(p, c, z, r, WG);
-            if (!far && kind < 0) {
-                if constexpr (PREC == kFP64) eval_stable<f64s, WA, WB, WG>(c, p.tab, full_rule(c), z, r, lane, SPLIT, 0, 1, L);
-                else eval_stable<float, WA, WB, WG>(c, p.tab, full_rule(c), z, r, lane, SPLIT, 0, 1, L);
+            if constexpr (PREC == kFP64) {
+                eval_classes<WA, WB, WG, SPLIT>(c, p.tab, z, r, !far && kind < 0, L);
+            } else if (!far && kind < 0) {
+                eval_stable<float, WA, WB, WG>(c, p.tab, full_rule(c), z, r, lane, SPLIT, 0, 1, L);
             }
             if (kind >= 0) ++n_near;
             if (__ballot(far)) {
@@ -149,7 +203,7 @@ void field_kernel(FieldParams p)
                                                lo, own, L);
             }
         }
-        if (SPLIT > 1) reduce_local<SPLIT>(L);
+        if (SPLIT > 1 && SPLIT < 64) reduce_local<SPLIT>(L);   // a whole wave's sums are whole
         accumulate_global(c, L, r, cph, sph, p.q, acc);
     }
     if (!active || lane != 0) return;
@@ -330,7 +384,10 @@ static void launch_field_q(hipStream_t s, const FieldParams &p, int split)
     const dim3 grid((unsigned)((threads + kFieldBlock - 1) / kFieldBlock), (unsigned)p.n_chunks);
     if (split == 1) hipLaunchKernelGGL((field_kernel<PREC, WA, WB, WG, 1>), grid, dim3(kFieldBlock), 0, s, p);
     else if (split == 4) hipLaunchKernelGGL((field_kernel<PREC, WA, WB, WG, 4>), grid, dim3(kFieldBlock), 0, s, p);
-    else hipLaunchKernelGGL((field_kernel<PREC, WA, WB, WG, 16>), grid, dim3(kFieldBlock), 0, s, p);
+    else if (split == 16 || PREC != kFP64)
+        hipLaunchKernelGGL((field_kernel<PREC, WA, WB, WG, 16>), grid, dim3(kFieldBlock), 0, s, p);
+    else if constexpr (PREC == kFP64)
+        hipLaunchKernelGGL((field_kernel<PREC, WA, WB, WG, 64>), grid, dim3(kFieldBlock), 0, s, p);
 }
 
 template <int PREC, bool WA, bool WB, bool WG>

@@ -17,7 +17,10 @@ namespace ccoil {
 // every SIMD of the 256 CUs several waves, and over 16 lanes when even one chunk per coil would leave the launch
 // below one wave per SIMD (few points and few coils: then each lane's serial chain of nodes, not the issue rate,
 // sets the kernel's duration; one coil at 4,096 points measured 46 us at 4 lanes and 25 us at 16, while at 65,536
-// points 16 lanes were slower). Split the coils into chunks (grid y, summed in order by field_reduce_kernel) while
+// points 16 lanes were slower). The FP64 kernel takes a whole wave per point where that is at most four waves per SIMD:
+// a point next to the winding has 20 times the nodes of the others, and four points of a wave would wait for one
+// another (one coil at 4,096 points around it: 30 us at 16 lanes, 20 us at 64; below 512 points there is nothing
+// to gain). Split the coils into chunks (grid y, summed in order by field_reduce_kernel) while
 // the launch still has fewer than about 8 waves per SIMD. Large launches take 1-4 chunks, whichever makes the last
 // round of resident waves fullest: every wave does the same work, so with R rounds of resident waves the launch
 // runs ceil(R) rounds.
@@ -25,8 +28,9 @@ FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n, int64_t n_coils, uint32_t 
 {
     FieldShape sh;
     const int64_t target = (int64_t)256 * 4 * 8;
-    sh.split = n < (int64_t)256 * 4 * 64 * 4 ? 4 : 1;
+    sh.split = n < (precision == CCOIL_FP64 ? kSortedPoints : (int64_t)256 * 4 * 64 * 4) ? 4 : 1;
     if (sh.split == 4 && (n * 4 + 63) / 64 * n_coils < (int64_t)256 * 4) sh.split = 16;
+    if (sh.split == 16 && precision == CCOIL_FP64 && n >= 512 && n * n_coils <= (int64_t)256 * 4 * 4) sh.split = 64;
     if (series_only) sh.split = 1;   // no rows to split
     const int64_t waves = std::max<int64_t>(1, (n * sh.split + 63) / 64);
     int64_t chunks = waves >= target ? 1 : std::min<int64_t>(n_coils, (target + waves - 1) / waves);
@@ -280,7 +284,8 @@ ccoil_status fields_prepare(ccoil_ctx ctx, const ccoil_coils *coils, const doubl
     if (n == 0 || hc.empty()) return CCOIL_OK;   // nothing to evaluate, or every field zero
     const FieldShape sh = shape ? *shape : field_shape_rule(ctx, n, (int64_t)hc.size(), quantities, precision,
                                                             rule_records);
-    if (sh.split != 1 && sh.split != 4 && sh.split != 16) return fail(ctx, CCOIL_ERR_ARGUMENT, "split must be 1, 4 or 16");
+    if (shape && sh.split != 1 && sh.split != 4 && sh.split != 16)
+        return fail(ctx, CCOIL_ERR_ARGUMENT, "split must be 1, 4 or 16");
     L.split = rule_records ? 1 : sh.split;   // the series-only kernel runs one lane per point
     if (far)
         for (auto &c : hc) {
@@ -333,30 +338,33 @@ ccoil_status fields_prepare(ccoil_ctx ctx, const ccoil_coils *coils, const doubl
         if (st != CCOIL_OK) return st;
         p.partial = (double *)partial;
     }
-    if (far) {
-        // the series' moments, and the visit order when there are enough points for the spatial sort to pay
-        L.far_bytes = sizeof(double) * ((size_t)kMpHeader + (size_t)kMpCoil * hc.size()) + 256;
+    if (far) {   // the series' moments
+        const size_t mb = sizeof(double) * ((size_t)kMpHeader + (size_t)kMpCoil * hc.size());
+        L.far_bytes = mb + 256;
         void *mp = nullptr;
-        st = call_buffer(ctx, ctx->fmp, arena, sizeof(double) * ((size_t)kMpHeader + (size_t)kMpCoil * hc.size()), &mp);
+        st = call_buffer(ctx, ctx->fmp, arena, mb, &mp);
         if (st != CCOIL_OK) return st;
         p.mp = (const double *)mp;
-        if (n >= kOrderMinPoints) {
-            // about 16-32 points per cell: 2^bits cells per axis, bits = log8(n / 16), between 3 and 6
-            int bits = 3;
-            while (bits < 6 && ((int64_t)1 << (3 * (bits + 1))) * 16 <= n) ++bits;
-            const int64_t cells = (int64_t)1 << (3 * bits);
-            size_t sb = 0;
-            CC_HIP(ctx, near_scan(ctx->stream, nullptr, nullptr, cells, nullptr, sb));
-            const size_t ob = sizeof(uint32_t) * (size_t)n, tb = visit_order_bytes(n, bits, sb);
-            void *order = nullptr, *temp = nullptr;
-            if ((st = call_buffer(ctx, ctx->forder, arena, ob, &order)) != CCOIL_OK) return st;
-            if ((st = call_buffer(ctx, ctx->ftemp, arena, tb, &temp)) != CCOIL_OK) return st;
-            L.far_bytes += ob + tb + 2 * 256;
-            p.order = (const uint32_t *)order;
-            L.order_temp = temp;
-            L.order_scan_bytes = sb;
-            L.order_bits = bits;
-        }
+    }
+    // The visit order, when there are enough points for the spatial sort to pay: the series modes, and the FP64 rule
+    // with one lane per point (no result depends on it, so the fixed scratch, which has no room to spare, goes without)
+    const bool sorted_rule = precision == CCOIL_FP64 && L.split == 1 && n >= kSortedPoints && !(arena && arena->fixed);
+    if ((far && n >= kOrderMinPoints) || sorted_rule) {
+        // about 16-32 points per cell: 2^bits cells per axis, bits = log8(n / 16), between 3 and 6
+        int bits = 3;
+        while (bits < 6 && ((int64_t)1 << (3 * (bits + 1))) * 16 <= n) ++bits;
+        const int64_t cells = (int64_t)1 << (3 * bits);
+        size_t sb = 0;
+        CC_HIP(ctx, near_scan(ctx->stream, nullptr, nullptr, cells, nullptr, sb));
+        const size_t ob = sizeof(uint32_t) * (size_t)n, tb = visit_order_bytes(n, bits, sb);
+        void *order = nullptr, *temp = nullptr;
+        if ((st = call_buffer(ctx, ctx->forder, arena, ob, &order)) != CCOIL_OK) return st;
+        if ((st = call_buffer(ctx, ctx->ftemp, arena, tb, &temp)) != CCOIL_OK) return st;
+        L.far_bytes += ob + tb + 2 * 256;
+        p.order = (const uint32_t *)order;
+        L.order_temp = temp;
+        L.order_scan_bytes = sb;
+        L.order_bits = bits;
     }
     if (L.near) {
         // Buffers for the records: every (coil, point) pair when that is small, else a capacity kept from earlier

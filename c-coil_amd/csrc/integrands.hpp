@@ -177,11 +177,13 @@ template <> __device__ inline float log1p_<float>(float x) { return log1pf(x); }
 
 // Arithmetic policies of eval_stable: float (FP32C), double (IEEE division and square root), and f64s:
 // double arithmetic whose reciprocals and reciprocal square roots come from the hardware FP64
-// approximations (v_rcp_f64, v_rsq_f64; relative error below 2^-24 on gfx950) refined by one Newton step.
-// The refined value errs by about (3/8) e^2 for the reciprocal square root and e^2 for the reciprocal, i.e.
-// below 1e-15 relative, so f64s is accurate to a few ulp per operation while avoiding the scaled division and
-// square-root sequences (FP64 FMA issues at the FP32 rate on CDNA3/4; those sequences dominate the IEEE
-// double kernel's time). Its domain is that of the approximations: normal, finite operands.
+// approximations (v_rcp_f64, v_rsq_f64; relative error below 2^-24 on gfx950) refined by one step, of second order
+// (Newton) for the reciprocal and of third for the reciprocal square root: errors of e^2, below 4e-15, and of e^3, so
+// f64s is accurate to a few ulp per operation while avoiding the scaled division and square-root sequences, which
+// dominate the IEEE double kernel's time. (A Newton step for the reciprocal square root too leaves up to 1.3e-15 of one
+// sign, which the far field's cancelling sums of few nodes do not average out: the gradient of a thin coil at seven
+// r_max erred by 9.8e-14 of its field with it and by 3.6e-14 without, for one more operation per root.) Its domain is
+// that of the approximations: normal, finite operands.
 struct f64s {};
 template <typename P> struct Real { using type = P; };
 template <> struct Real<f64s> { using type = double; };
@@ -192,7 +194,7 @@ template <> __device__ inline double prsq<f64s>(double x)
 {
     const double y = __builtin_amdgcn_rsq(x);
     const double e = fma(-(x * y), y, 1.0);               // 1 - x y^2
-    return fma(0.5 * y, e, y);                            // y (1 + e/2)
+    return fma(y * e, fma(0.375, e, 0.5), y);             // y (1 + e/2 + 3 e^2 / 8)
 }
 template <typename P> __device__ inline real_t<P> prcp(real_t<P> x) { return rcp_<real_t<P>>(x); }
 template <> __device__ inline double prcp<f64s>(double x)
@@ -673,6 +675,192 @@ __device__ inline void eval_stable(const CoilDev &c, const Tables &tab, const Ru
         L.RZ = aRZ;
         L.ZZ = -3.0 * zd * aZZ;
     }
+}
+
+// eval_stable<f64s> for lanes that share one point's sums (row0, rstep, node0, nstep differ between lanes): a lane keeps
+// one angular node at a time and runs over its rows two at a time, so the tables' vector loads are one set per node
+// instead of one per node and row, and two rows' evaluations overlap. Launches that split a point run about a wave per
+// SIMD, where those latencies are the duration; the row constants cost a third more operations per node than
+// eval_stable. The same integrands, with each term weighted at its node; values differ from eval_stable's in the last
+// bits.
+struct SharedSums {
+    double A, Bh, Bz, RR, RZ, ZZ;
+};
+
+// One node (1 - cos: s, 1 + cos: op; cos(phi) enters with the weight) of the row at radius rho, with weights Ww and
+// Wc = Ww cos(phi); zs: the coil's half-length geometry at the point (z1, z2 of eval_stable).
+template <bool WA, bool WB, bool WG, bool FAST>
+__device__ inline void shared_node(double rho, double r, double s, double op, double Ww, double Wc, double b, double z1,
+                                   double z2, double tbz, bool same, double zz, SharedSums &a)
+{
+    const double d = rho - r, base = d * d, qh = rho * r;
+    const double M = fma(2.0 * qh, s, base), rmc = fma(r, s, d), rr = fma(rho, s, -d);   // rho - r cos, r - rho cos
+    if constexpr (FAST) {
+        const double J1 = fma(z1, z1, M), J2 = fma(z2, z2, M), K1 = prsq<f64s>(J1), K2 = prsq<f64s>(J2);
+        double Nx = 0, Da = 1, Ea = 1, Re = 0;
+        if (WA) {
+            const double sJ1 = J1 * K1, sJ2 = J2 * K2, sum = sJ1 + sJ2;
+            Da = sum * (same ? z2 + sJ2 : M);
+            Nx = fma(b, sum, tbz) * (same ? 1.0 : sJ2 - z2);
+            Ea = fma(Da, 2.0, Nx);
+        }
+        if (WB || WG) {
+            const double K12 = K1 * K2, tP2 = tbz * (K12 * K12), g2 = z2 * K2;
+            const double gs = fma(z1, K1, g2), gsel = same ? gs : 1.0, Y = M * gsel, Ks = K1 + K2, KsY = Ks * Y;
+            const double R = prcp<f64s>(WA ? KsY * Ea : KsY), Rb = WA ? Ea * R : R;
+            if (WA) Re = KsY * R;
+            const double Rr = Ks * Rb, mdK = tP2 * (Y * Rb), invM = gsel * Rr;   // mdK = K2 - K1
+            const double dgM = (same ? tP2 * M : fma(z1, K1, -g2)) * Rr;         // (z1 K1 - z2 K2) / M
+            a.Bh = fma(Wc, mdK, a.Bh);
+            const double wr = Ww * rmc;
+            if (WB) a.Bz = fma(wr, dgM, a.Bz);
+            if (WG) {
+                const double mdL = mdK * fma(Ks, Ks, -K12);   // K2^3 - K1^3
+                a.RR = fma(-Wc * rr, mdL, a.RR);
+                a.ZZ = fma(-wr, mdL, a.ZZ);
+                const double hM = fma(dgM, K1 * K1, -(tP2 * g2) * invM);
+                // cos (rho^2 + r^2) - 2 rho r, and eval_stable's polynomial N in s
+                const double O = fma(op, base, -M);
+                const double n1 = base * fma(2.0, qh, -base), n2 = -3.0 * qh * base, n3 = -2.0 * qh * qh;
+                const double N = fma(s, fma(s, fma(s, n3, n2), n1), base * base);
+                a.RZ = fma(Ww, fma(O, dgM, N * hM) * invM, a.RZ);
+            }
+        } else {
+            Re = prcp<f64s>(Ea);
+        }
+        if (WA) a.A = fma(Wc, log1p_ratio<f64s>(Nx, Nx * Re, [&] { return Da; }), a.A);
+    } else {
+        const double K = prsq<f64s>(M + zz);
+        if (WB || WG) {
+            const double K2 = K * K, K3 = K2 * K, wr = Ww * rmc;
+            a.Bh = fma(Wc, K3, a.Bh);
+            if (WB) a.Bz = fma(wr, K3, a.Bz);
+            if (WG) {
+                const double K5 = K3 * K2, k0 = fma(2.0, base, -zz);
+                a.RR = fma(Wc * rr, K5, a.RR);
+                a.ZZ = fma(wr, K5, a.ZZ);
+                a.RZ = fma(Ww, (k0 - s * fma(qh, s, fma(2.0, qh, k0))) * K5, a.RZ);
+            }
+        }
+        if (WA) a.A = fma(Wc, K, a.A);
+    }
+}
+
+template <bool WA, bool WB, bool WG, bool FAST>
+__device__ inline void shared_sums(const CoilDev &c, const Tables &tab, const RuleSel &rule, double z, double r, int row0,
+                                   int rstep, int node0, int nstep, SharedSums &a)
+{
+    const double *xt = tab.x + rule.ot, *wt = tab.w + rule.ot;
+    const double *st = tab.omc + rule.oa, *wa = tab.w + rule.oa, *wct = tab.wcos + rule.oa, *opt = tab.opc + rule.oa;
+    const double zm = fabs(z), z1 = zm + 0.5 * c.b, z2 = zm - 0.5 * c.b, tbz = 2.0 * c.b * zm, zz = z * z, ha = 0.5 * c.a;
+    const bool same = z2 > 0.0;
+    // rows in pairs, each pair's table entries loaded while the pair before it is evaluated; past the last row: that
+    // row again, at weight zero
+    const int last = rule.nt - 1, jf = row0 < last ? row0 : last, jf2 = row0 + rstep < last ? row0 + rstep : last;
+    const double xf0 = xt[jf], xf1 = xt[jf2], wf0 = row0 <= last ? wt[jf] : 0.0, wf1 = row0 + rstep <= last ? wt[jf2] : 0.0;
+    for (int i = node0; i < rule.na; i += nstep) {
+        const double s = st[i], w = wa[i], wc = wct[i], op = WG && FAST ? opt[i] : 0.0;
+        double x0 = xf0, x1 = xf1, w0 = wf0, w1 = wf1;
+        for (int j = row0 + 2 * rstep;; j += 2 * rstep) {
+            const int n0 = j < last ? j : last, n1 = j + rstep < last ? j + rstep : last;
+            const double nx0 = xt[n0], nx1 = xt[n1], nw0 = wt[n0], nw1 = wt[n1];
+            const double rho0 = fma(ha, 1.0 + x0, c.R), rho1 = fma(ha, 1.0 + x1, c.R);
+            const double W0 = c.cf * w0 * rho0, W1 = c.cf * w1 * rho1;
+            shared_node<WA, WB, WG, FAST>(rho0, r, s, op, W0 * w, W0 * wc, c.b, z1, z2, tbz, same, zz, a);
+            shared_node<WA, WB, WG, FAST>(rho1, r, s, op, W1 * w, W1 * wc, c.b, z1, z2, tbz, same, zz, a);
+            if (j > last) break;
+            x0 = nx0;
+            x1 = nx1;
+            w0 = nw0;
+            w1 = j + rstep <= last ? nw1 : 0.0;
+        }
+    }
+}
+
+__device__ inline void shared_local(const CoilDev &c, double z, double r, const SharedSums &a, Local &L)
+{
+    const double odd = c.use_fast ? (z < 0.0 ? -1.0 : 1.0) : z, odd3 = c.use_fast ? odd : -3.0 * z;
+    L.A = a.A;
+    L.Bh = odd * a.Bh;
+    L.Bz = a.Bz;
+    L.RP = L.Bh / r;
+    L.RR = odd3 * a.RR;
+    L.RZ = a.RZ;
+    L.ZZ = odd3 * a.ZZ;
+}
+
+template <bool WA, bool WB, bool WG>
+__device__ inline void eval_shared(const CoilDev &c, const Tables &tab, const RuleSel &rule, double z, double r, int row0,
+                                   int rstep, int node0, int nstep, Local &L)
+{
+    SharedSums a = {0, 0, 0, 0, 0, 0};
+    if (c.use_fast) shared_sums<WA, WB, WG, true>(c, tab, rule, z, r, row0, rstep, node0, nstep, a);
+    else shared_sums<WA, WB, WG, false>(c, tab, rule, z, r, row0, rstep, node0, nstep, a);
+    shared_local(c, z, r, a, L);
+}
+
+// The sums of one point by all 64 lanes of a wave (z, r and rule wave-uniform): the lanes split the rows in four (two
+// where the angular rule has more than 80 nodes) and a row's nodes over the rest; a lane's nodes, five at most, stay in
+// registers while it runs over its rows, so a row's constants serve all of them. Every lane gets its share of the
+// sums.
+constexpr int kWaveNodes = 5;
+template <bool WA, bool WB, bool WG, bool FAST>
+__device__ inline void wave_sums(const CoilDev &c, const Tables &tab, const RuleSel &rule, double z, double r, int lane,
+                                 SharedSums &a)
+{
+    const int sr = rule.nt == 1 ? 1 : rule.na <= 16 * kWaveNodes ? 4 : 2, sn = 64 / sr, row0 = lane % sr, node0 = lane / sr;
+    static_assert(2 * 16 * kWaveNodes >= kMaxOrder, "the nodes of a row fit the lanes' registers");
+    const int m = (rule.na + sn - 1) / sn;   // nodes of a lane, the last at weight zero beyond the rule's
+    double s[kWaveNodes], w[kWaveNodes], wc[kWaveNodes], op[kWaveNodes];
+#pragma unroll
+    for (int k = 0; k < kWaveNodes; ++k) {
+        const int i = node0 + k * sn;
+        const bool in = i < rule.na;
+        const int e = rule.oa + (in ? i : rule.na - 1);
+        s[k] = tab.omc[e];
+        w[k] = in ? tab.w[e] : 0.0;
+        wc[k] = in ? tab.wcos[e] : 0.0;
+        op[k] = WG && FAST ? tab.opc[e] : 0.0;
+    }
+    const double *xt = tab.x + rule.ot, *wt = tab.w + rule.ot;
+    const double zm = fabs(z), z1 = zm + 0.5 * c.b, z2 = zm - 0.5 * c.b, tbz = 2.0 * c.b * zm, zz = z * z, ha = 0.5 * c.a;
+    const bool same = z2 > 0.0;
+    for (int j = row0; j < rule.nt; j += sr) {
+        const double rho = fma(ha, 1.0 + xt[j], c.R), W = c.cf * wt[j] * rho;
+        SharedSums b = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < kWaveNodes; ++k)
+            if (k < m)
+                shared_node<WA, WB, WG, FAST>(rho, r, s[k], op[k], w[k], wc[k], c.b, z1, z2, tbz, same, zz, b);
+        a.A = fma(W, b.A, a.A);
+        a.Bh = fma(W, b.Bh, a.Bh);
+        a.Bz = fma(W, b.Bz, a.Bz);
+        a.RR = fma(W, b.RR, a.RR);
+        a.RZ = fma(W, b.RZ, a.RZ);
+        a.ZZ = fma(W, b.ZZ, a.ZZ);
+    }
+}
+
+// Every lane returns the point's whole sums (a fixed xor butterfly).
+template <bool WA, bool WB, bool WG>
+__device__ inline void eval_wave(const CoilDev &c, const Tables &tab, const RuleSel &rule, double z, double r, int lane,
+                                 Local &L)
+{
+    SharedSums a = {0, 0, 0, 0, 0, 0};
+    if (c.use_fast) wave_sums<WA, WB, WG, true>(c, tab, rule, z, r, lane, a);
+    else wave_sums<WA, WB, WG, false>(c, tab, rule, z, r, lane, a);
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+        if (WA) a.A += __shfl_xor(a.A, m, 64);
+        if (WB || WG) a.Bh += __shfl_xor(a.Bh, m, 64);
+        if (WB) a.Bz += __shfl_xor(a.Bz, m, 64);
+        if (WG) {
+            a.RR += __shfl_xor(a.RR, m, 64);
+            a.RZ += __shfl_xor(a.RZ, m, 64);
+            a.ZZ += __shfl_xor(a.ZZ, m, 64);
+        }
+    }
+    shared_local(c, z, r, a, L);
 }
 
 }  // namespace ccoil

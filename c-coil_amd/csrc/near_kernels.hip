@@ -297,10 +297,18 @@ __global__ __launch_bounds__(256) void near_eval_group_kernel(FieldParams p)
         double z, r, cph, sph;
         to_local(c, p.pts[3 * pi], p.pts[3 * pi + 1], p.pts[3 * pi + 2], z, r, cph, sph);
         const RuleSel rule = class_rule(c, rule_class(c, z, r));
-        const int sr = rule.nt == 1 ? 1 : group == 64 ? 4 : 2;
         Local L;
-        eval_stable<f64s, WA, WB, WG>(c, p.tab, rule, z, r, sub & (sr - 1), sr, sub / sr, group / sr, L);
-        reduce_record(L, group);
+        if (group == 64) {
+            // one record: the wave's control flow and loads are uniform
+            const int k = __builtin_amdgcn_readfirstlane(key);
+            const CoilDev &cu = p.coils[p.near_coil[(uint32_t)k % (uint32_t)p.n_coils]];
+            eval_wave<WA, WB, WG>(cu, p.tab, class_rule(cu, __builtin_amdgcn_readfirstlane(rule_class(c, z, r))), z, r, lane,
+                                  L);
+        } else {
+            const int sr = rule.nt == 1 ? 1 : 2;
+            eval_shared<WA, WB, WG>(c, p.tab, rule, z, r, sub & (sr - 1), sr, sub / sr, kRecordSplit / sr, L);
+            reduce_record(L, kRecordSplit);
+        }
         if (sub) continue;
         Cart acc;
         for (int j = 0; j < 3; ++j) { acc.A[j] = 0.0; acc.E[j] = 0.0; acc.B[j] = 0.0; }

@@ -77,9 +77,9 @@ ccoil_status tune_fields(ccoil_ctx ctx, const ccoil_coils *coils, const double *
         for (int64_t c : {(int64_t)1, (int64_t)2, (int64_t)3, (int64_t)4, (int64_t)rule.chunks,
                           (int64_t)std::max(1, rule.chunks / 2), (int64_t)rule.chunks * 2})
             if (c >= 1 && c <= nc && c <= 65535) cand.insert({s, (int)c});
-    cand.insert({rule.split, rule.chunks});
+    cand.insert({std::min(rule.split, 16), rule.chunks});
     double best = 1e300;
-    FieldShape best_shape = rule;
+    FieldShape best_shape = rule;   // every candidate is timed, so one of them replaces it
     for (const auto &c : cand) {
         FieldShape sh;
         sh.split = c.first;

@@ -81,3 +81,13 @@ def check(ctx, row, n, prec, flags, seed):
 def test_records_match_the_own_rule(ctx, coil, n):
     """The record pass of the series mode: lanes grouped per record (few points), and uniform waves (many)."""
     print(f"\n{coil} n={n}: worst error over tolerance {check(ctx, _row(*coil), n, abi.FP64, abi.FAR_FIELD, 5)}")
+
+
+@pytest.mark.parametrize("n,split", [(300, 16), (600, 64), (5000, 16), (20000, 4), (70000, 1)])
+@pytest.mark.parametrize("coil", COILS, ids=lambda c: f"{c[0]}-{c[4]}x{c[5]}")
+def test_field_kernel_matches_the_own_rule(ctx, coil, n, split):
+    """The rule alone at every launch shape: a whole wave, 16 or 4 lanes per point, one lane per point."""
+    row = _row(*coil)
+    _, rep = ctx.fields(abi.CoilSet.from_rows([row]), np.zeros((n, 3)), abi.B, abi.FP64)
+    assert rep.split == split
+    print(f"\n{coil} n={n}: worst error over tolerance {check(ctx, row, n, abi.FP64, 0, 7)}")
