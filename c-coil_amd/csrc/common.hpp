@@ -244,12 +244,12 @@ struct RuleSel {
     int oa, na, ot, nt;
 };
 
-__device__ inline RuleSel full_rule(const CoilDev &c)
+__host__ __device__ inline RuleSel full_rule(const CoilDev &c)
 {
     return {table_offset(c.n_ang), c.n_ang, table_offset(c.n_thk), c.n_thk};
 }
 
-__device__ inline RuleSel class_rule(const CoilDev &c, int cls)
+__host__ __device__ inline RuleSel class_rule(const CoilDev &c, int cls)
 {
     const int k = cls / (kRedThk + 1), t = cls - k * (kRedThk + 1);
     RuleSel s = full_rule(c);
@@ -277,12 +277,12 @@ __device__ inline RuleSel class_rule(const CoilDev &c, int cls)
 // winding's radius nearest to sqrt(r^2 + zd^2); the thickness integrand is analytic outside the point (r, zd) and its
 // mirror, whose ellipse about [R, R + a] has the distance sum d1 + d2. Every operation is a float operation rounded on
 // its own, so every kernel gives a pair the same class; the thresholds carry margins far above float rounding.
-__device__ inline int rule_class(const CoilDev &c, double z, double r)
+//
+// class_of: the class at num = (rho - r)^2 + zd^2, den = 2 rho r and s = (d1 + d2) / (a / 2), or at bounds of them
+// (num / den and s from below).
+__host__ __device__ inline int class_of(const CoilDev &c, float num, float den, float s)
 {
 #pragma clang fp contract(off)
-    const float rf = (float)r, zd = fmaxf((float)fabs(z) - c.hbf, 0.0f), zd2 = zd * zd;
-    const float rho = fminf(fmaxf(__builtin_amdgcn_sqrtf(rf * rf + zd2), c.r0f), c.r1f);
-    const float dr = rho - rf, num = dr * dr + zd2, den = 2.0f * rho * rf;
     int k = 0, t = 0;
     if (num >= c.red_x * den) {
         constexpr float kX[kRedAng] = {0.0050042f, 0.0453385f, 0.2946833f, 0.5430806f, 2.1074632f, 11.2864665f};
@@ -290,8 +290,6 @@ __device__ inline int rule_class(const CoilDev &c, double z, double r)
 #pragma unroll
         for (int i = 1; i < kRedAng; ++i) k += num >= kX[i] * den ? 1 : 0;
     }
-    const float e0 = rf - c.r0f, e1 = rf - c.r1f;
-    const float s = (__builtin_amdgcn_sqrtf(e0 * e0 + zd2) + __builtin_amdgcn_sqrtf(e1 * e1 + zd2)) * c.ia2f;
     if (s >= c.red_s) {
         // rho_B + 1 / rho_B, rho_B = (kRedThkC / kRedTol)^(1 / (2 n))
         constexpr float kS[kRedThk] = {2.935256f, 3.643171f, 5.054480f, 7.913130f, 13.079747f, 30.607902f};
@@ -300,6 +298,16 @@ __device__ inline int rule_class(const CoilDev &c, double z, double r)
         for (int i = 1; i < kRedThk; ++i) t += s >= kS[i] ? 1 : 0;
     }
     return (kRedThk + 1) * k + t;
+}
+__device__ inline int rule_class(const CoilDev &c, double z, double r)
+{
+#pragma clang fp contract(off)
+    const float rf = (float)r, zd = fmaxf((float)fabs(z) - c.hbf, 0.0f), zd2 = zd * zd;
+    const float rho = fminf(fmaxf(__builtin_amdgcn_sqrtf(rf * rf + zd2), c.r0f), c.r1f);
+    const float dr = rho - rf, num = dr * dr + zd2, den = 2.0f * rho * rf;
+    const float e0 = rf - c.r0f, e1 = rf - c.r1f;
+    const float s = (__builtin_amdgcn_sqrtf(e0 * e0 + zd2) + __builtin_amdgcn_sqrtf(e1 * e1 + zd2)) * c.ia2f;
+    return class_of(c, num, den, s);
 }
 
 }  // namespace ccoil

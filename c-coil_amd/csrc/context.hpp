@@ -132,6 +132,9 @@ struct RedTables {
     double w[kRedNodes], omc[kRedNodes], opc[kRedNodes], wcos[kRedNodes], ws[kRedNodes], ws2[kRedNodes], wcs[kRedNodes];
 };
 void reduced_tables(RedTables &t);
+// Nodes of the rule class that serves every point at least dist from the coil's centre (the coil's own rule within the
+// sphere that holds its winding).
+int64_t rule_nodes_beyond(const CoilDev &c, double dist);
 // Runs fn(i0, i1) over ranges that cover [0, n) once: on up to 16 host threads for large n, else on the caller.
 void host_parallel_for(int64_t n, const std::function<void(int64_t, int64_t)> &fn);
 // The highest order a series evaluated beyond y r_max can use (multipole_terms there, with a margin; 0 if y is 0).

@@ -141,7 +141,7 @@ __device__ inline void eval_classes(const CoilDev &c, const Tables &tab, double 
         left &= left - 1;
         Local M;
         eval_wave<WA, WB, WG>(c, tab, class_rule(c, __builtin_amdgcn_readlane(cls, src)), lane_value(z, src),
-                              lane_value(r, src), lane, M);
+                              lane_value(r, src), lane, 0, 1, M);
         if (lane == src) L = M;
     }
 }

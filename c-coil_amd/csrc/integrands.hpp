@@ -806,9 +806,9 @@ __device__ inline void eval_shared(const CoilDev &c, const Tables &tab, const Ru
 constexpr int kWaveNodes = 5;
 template <bool WA, bool WB, bool WG, bool FAST>
 __device__ inline void wave_sums(const CoilDev &c, const Tables &tab, const RuleSel &rule, double z, double r, int lane,
-                                 SharedSums &a)
+                                 int first_row, int row_step, SharedSums &a)
 {
-    const int sr = rule.nt == 1 ? 1 : rule.na <= 16 * kWaveNodes ? 4 : 2, sn = 64 / sr, row0 = lane % sr, node0 = lane / sr;
+    const int sr = rule.nt == 1 ? 1 : rule.na <= 16 * kWaveNodes ? 4 : 2, sn = 64 / sr, node0 = lane / sr;
     static_assert(2 * 16 * kWaveNodes >= kMaxOrder, "the nodes of a row fit the lanes' registers");
     const int m = (rule.na + sn - 1) / sn;   // nodes of a lane, the last at weight zero beyond the rule's
     double s[kWaveNodes], w[kWaveNodes], wc[kWaveNodes], op[kWaveNodes];
@@ -825,7 +825,7 @@ __device__ inline void wave_sums(const CoilDev &c, const Tables &tab, const Rule
     const double *xt = tab.x + rule.ot, *wt = tab.w + rule.ot;
     const double zm = fabs(z), z1 = zm + 0.5 * c.b, z2 = zm - 0.5 * c.b, tbz = 2.0 * c.b * zm, zz = z * z, ha = 0.5 * c.a;
     const bool same = z2 > 0.0;
-    for (int j = row0; j < rule.nt; j += sr) {
+    for (int j = first_row + row_step * (lane % sr); j < rule.nt; j += row_step * sr) {
         const double rho = fma(ha, 1.0 + xt[j], c.R), W = c.cf * wt[j] * rho;
         SharedSums b = {0, 0, 0, 0, 0, 0};
 #pragma unroll
@@ -841,14 +841,14 @@ __device__ inline void wave_sums(const CoilDev &c, const Tables &tab, const Rule
     }
 }
 
-// Every lane returns the point's whole sums (a fixed xor butterfly).
+// Every lane returns the sums of the rows first_row, first_row + row_step, ... (a fixed xor butterfly).
 template <bool WA, bool WB, bool WG>
 __device__ inline void eval_wave(const CoilDev &c, const Tables &tab, const RuleSel &rule, double z, double r, int lane,
-                                 Local &L)
+                                 int first_row, int row_step, Local &L)
 {
     SharedSums a = {0, 0, 0, 0, 0, 0};
-    if (c.use_fast) wave_sums<WA, WB, WG, true>(c, tab, rule, z, r, lane, a);
-    else wave_sums<WA, WB, WG, false>(c, tab, rule, z, r, lane, a);
+    if (c.use_fast) wave_sums<WA, WB, WG, true>(c, tab, rule, z, r, lane, first_row, row_step, a);
+    else wave_sums<WA, WB, WG, false>(c, tab, rule, z, r, lane, first_row, row_step, a);
 #pragma unroll
     for (int m = 1; m < 64; m <<= 1) {
         if (WA) a.A += __shfl_xor(a.A, m, 64);

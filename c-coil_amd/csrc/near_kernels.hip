@@ -303,7 +303,7 @@ __global__ __launch_bounds__(256) void near_eval_group_kernel(FieldParams p)
             const int k = __builtin_amdgcn_readfirstlane(key);
             const CoilDev &cu = p.coils[p.near_coil[(uint32_t)k % (uint32_t)p.n_coils]];
             eval_wave<WA, WB, WG>(cu, p.tab, class_rule(cu, __builtin_amdgcn_readfirstlane(rule_class(c, z, r))), z, r, lane,
-                                  L);
+                                  0, 1, L);
         } else {
             const int sr = rule.nt == 1 ? 1 : 2;
             eval_shared<WA, WB, WG>(c, p.tab, rule, z, r, sub & (sr - 1), sr, sub / sr, kRecordSplit / sr, L);

@@ -30,24 +30,46 @@ template <int PREC, bool WM, bool WF, bool GR>
 __device__ inline void eval_prim(const CoilDev &pc, const Tables &tab, double z, double r, int row0, int rstep,
                                  Local &L, AdjA *ada)
 {
-    if constexpr (GR) {   // gradients of M: A, B and the pair adjoint extras; FP64, FP64_IEEE or FP32C far nodes
-        if constexpr (PREC == 4) eval_stable<double, true, true, false, false, true>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L, nullptr, ada);
-        else if constexpr (PREC == 1) eval_stable<float, true, true, false, false, true>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L, nullptr, ada);
-        else eval_stable<f64s, true, true, false, false, true>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L, nullptr, ada);
-        return;
-    }
-    if constexpr (PREC == 0) {
-        eval_stable<f64s, WM, WF, false, false, false, true>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L);
-    } else if constexpr (PREC == 4) {
-        eval_stable<double, WM, WF, false>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L);
+    if constexpr (PREC == 4) {
+        if constexpr (GR) eval_stable<double, true, true, false, false, true>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L, nullptr, ada);
+        else eval_stable<double, WM, WF, false>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L);
     } else if constexpr (PREC == 2) {
         eval_plain<float, WM, WF, false>(pc, tab, z, r, row0, rstep, L);
-    } else if constexpr (PREC == 3) {
-        eval_plain<double, WM, WF, false>(pc, tab, z, r, row0, rstep, L);
-    } else if (is_near(pc, z, r, false)) {
-        eval_stable<f64s, WM, WF, false>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L);
     } else {
-        eval_stable<float, WM, WF, false>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L);
+        static_assert(PREC == 3, "FP64 and FP32C take eval_pair");
+        eval_plain<double, WM, WF, false>(pc, tab, z, r, row0, rstep, L);
+    }
+}
+
+// The FP64 rule of the primary at a wave's nodes (z, r of each lane), by one rule for all of them: the cheapest that
+// serves every lane in `lanes` (rule_class; own: the coil's own angular rule). Every lane evaluates, so loops and
+// tables stay uniform; the lanes outside `lanes` get values of no use. A node's value so depends on its wave, as it
+// does through the lean loop (eval_stable): in rounding only, and a pair's waves are fixed by its schedule.
+template <bool WA, bool WB, bool ADA>
+__device__ inline void eval_pair(const CoilDev &pc, const Tables &tab, double z, double r, bool lanes, int cls, bool own,
+                                 int row0, int rstep, Local &L, AdjA *ada)
+{
+    const int k = cls / (kRedThk + 1), t = cls - k * (kRedThk + 1);
+    const int kw = own ? 0 : 7 - wave_max_bits<3>(lanes ? 7 - k : 0), tw = 7 - wave_max_bits<3>(lanes ? 7 - t : 0);
+    const RuleSel rule = class_rule(pc, kw * (kRedThk + 1) + tw);
+    eval_stable<f64s, WA, WB, false, false, ADA, !ADA>(pc, tab, rule, z, r, row0, rstep, 0, 1, L, nullptr, ada);
+}
+
+// One node (wave-uniform) by the coil's own angular rule, its rows and nodes split over the wave's lanes.
+template <bool WA, bool WB, bool ADA>
+__device__ inline void eval_pair_wave(const CoilDev &pc, const Tables &tab, double z, double r, int cls, int lane, int row0,
+                                      int rstep, Local &L, AdjA *ada)
+{
+    const RuleSel rule = class_rule(pc, cls);
+    if constexpr (!ADA) {
+        eval_wave<WA, WB, false>(pc, tab, rule, z, r, lane, row0, rstep, L);
+    } else {
+        const int sr = rule.nt == 1 ? 1 : 4;
+        eval_stable<f64s, WA, WB, false, false, true>(pc, tab, rule, z, r, row0 + rstep * (lane % sr), rstep * sr, lane / sr,
+                                                      64 / sr, L, nullptr, ada);
+        double *v[7] = {&L.A, &L.Bh, &L.Bz, &ada->dR, &ada->da, &ada->db, &ada->Ar};
+#pragma unroll
+        for (int q = 0; q < 7; ++q) *v[q] = wave_sum(*v[q]);
     }
 }
 
@@ -88,8 +110,36 @@ __device__ inline void grad_m_term(const CoilDev &pc, const Local &L, double Ar,
         }
 }
 
+// A wave-uniform value in scalar registers.
+__device__ inline double scalar(double v)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u), hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// x / d for a wave-uniform d, leaving the remainder in x: the float quotient is within one of it (x < 2^24, or x < 2 d).
+__device__ inline uint32_t divide(uint32_t &x, uint32_t d)
+{
+    uint32_t q = (uint32_t)((float)x * __builtin_amdgcn_rcpf((float)d));
+    int64_t r = (int64_t)x - (int64_t)q * d;
+    if (r < 0) {
+        --q;
+        r += d;
+    } else if (r >= (int64_t)d) {
+        ++q;
+        r -= d;
+    }
+    x = (uint32_t)r;
+    return q;
+}
+
+// Minimum waves per SIMD: the FP64 kernels' short rules leave the spills of node generation in the way (8,192 pairs,
+// M and F: 16.3 ms at four waves, 15.5 at three, 15.7 at two; the gradient of 256 pairs 2.22, 1.84, 1.72 ms).
+template <int PREC, bool GR> constexpr int kPairWaves = PREC != 0 ? 4 : GR ? 2 : 3;
+
 template <int PREC, bool WM, bool WF, bool WD, bool GR = false>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pair_kernel(PairParams p)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPairWaves<PREC, GR>))) void pair_kernel(PairParams p)
 {
     static_assert(!GR || (WM && !WF && !WD), "the gradient instance evaluates M and its derivatives");
     const int lane = threadIdx.x;
@@ -110,11 +160,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pa
         const int64_t n1 = min(n0 + (int64_t)pd.nodes_per_item, pd.n_nodes);
         const int NA = sc.blk_ang * sc.n_ang, NT = sc.blk_thk * sc.n_thk;
         const bool table_ring = sc.blk_ang == 1 && pd.half_ring == 0 && pd.ring_offset == 0.0;
-        const double ang_blk = (pd.half_ring ? kPi : 2.0 * kPi) / sc.blk_ang;
-        const double tbs = sc.a / sc.blk_thk, lbs = sc.b / sc.blk_len;
-        const double ax[3] = {sc.sa * sc.cb, sc.sa * sc.sb, sc.ca};
-        const double u[3] = {sc.cb * sc.ca, sc.sb * sc.ca, -sc.sa};
-        const double v[3] = {-sc.sb, sc.cb, 0.0};
+        const double ang_blk = scalar((pd.half_ring ? kPi : 2.0 * kPi) / sc.blk_ang);
+        const double tbs = scalar(sc.a / sc.blk_thk), lbs = scalar(sc.b / sc.blk_len);
+        // the ring frame, wave-uniform: kept in scalar registers, as the kernel has no vector register to spare
+        const double ax[3] = {scalar(sc.sa * sc.cb), scalar(sc.sa * sc.sb), sc.ca};
+        const double u[3] = {scalar(sc.cb * sc.ca), scalar(sc.sb * sc.ca), scalar(-sc.sa)};
+        const double v[3] = {scalar(-sc.sb), sc.cb, 0.0};
         const int oa = table_offset(sc.n_ang), ot = table_offset(sc.n_thk), ol = table_offset(sc.n_len);
         double m = 0.0, f0 = 0.0, f1 = 0.0, f2 = 0.0, t0 = 0.0, t1 = 0.0, t2 = 0.0, d0 = 0.0, d1 = 0.0, d2 = 0.0;
         double gs[kPairGradTerms - 1] = {};   // GR: the derivative sums after M
@@ -125,30 +176,37 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pa
             double w, arm[3], tan[3], z, r, pcph, psph;
             double cs, ss, rho, ell, ht, hl;
         };
-        auto node = [&](int64_t k, Node &n) {
-            const int ia = (int)(k % NA);
-            const int64_t rest = k / NA;
-            const int it = (int)(rest % NT);
-            const int il = (int)(rest / NT);
-            const int i = ia % sc.n_ang, j = it % sc.n_thk, l = il % sc.n_len;
+        // (angular, thickness, length) digits of the item's first node; the item's node j (at most a few thousand) is
+        // j steps on, so the lanes' digits take 32-bit divisions by uniform divisors
+        const int64_t first_rest = n0 / NA;
+        const uint32_t ia0 = (uint32_t)(n0 % NA), it0 = (uint32_t)(first_rest % NT), il0 = (uint32_t)(first_rest / NT);
+        const int n_item = (int)(n1 - n0);
+        auto node = [&](int j0, Node &n) {
+            uint32_t ia = ia0 + (uint32_t)j0, it, il, ba = 0, bt = 0, bl = 0;
+            it = it0 + divide(ia, (uint32_t)NA);
+            il = il0 + divide(it, (uint32_t)NT);
+            uint32_t i = ia, j = it, l = il;   // within the block
+            if (sc.blk_ang > 1) ba = divide(i, (uint32_t)sc.n_ang);
+            if (sc.blk_thk > 1) bt = divide(j, (uint32_t)sc.n_thk);
+            if (sc.blk_len > 1) bl = divide(l, (uint32_t)sc.n_len);
             double cph, sph;
             if (table_ring) {
                 cph = p.tab.rcos[oa + i];
                 sph = p.tab.rsin[oa + i];
             } else {
-                const double phi = pd.ring_offset + ang_blk * ((ia / sc.n_ang) + 0.5) + 0.5 * ang_blk * p.tab.x[oa + i];
+                const double phi = pd.ring_offset + ang_blk * ((double)ba + 0.5) + 0.5 * ang_blk * p.tab.x[oa + i];
                 sincos(phi, &sph, &cph);
             }
-            const double rho = sc.R + tbs * ((it / sc.n_thk) + 0.5) + 0.5 * tbs * p.tab.x[ot + j];
-            const double ell = -0.5 * sc.b + lbs * ((il / sc.n_len) + 0.5) + 0.5 * lbs * p.tab.x[ol + l];
+            const double rho = sc.R + tbs * ((double)bt + 0.5) + 0.5 * tbs * p.tab.x[ot + j];
+            const double ell = -0.5 * sc.b + lbs * ((double)bl + 0.5) + 0.5 * lbs * p.tab.x[ol + l];
             n.w = 0.125 * rho * p.tab.w[ol + l] * p.tab.w[ot + j] * p.tab.w[oa + i];
             if constexpr (GR) {
                 n.cs = cph;
                 n.ss = sph;
                 n.rho = rho;
                 n.ell = ell;
-                n.ht = ((it / sc.n_thk) + 0.5 + 0.5 * p.tab.x[ot + j]) / sc.blk_thk;
-                n.hl = -0.5 + ((il / sc.n_len) + 0.5 + 0.5 * p.tab.x[ol + l]) / sc.blk_len;
+                n.ht = ((double)bt + 0.5 + 0.5 * p.tab.x[ot + j]) / sc.blk_thk;
+                n.hl = -0.5 + ((double)bl + 0.5 + 0.5 * p.tab.x[ol + l]) / sc.blk_len;
             }
             for (int q = 0; q < 3; ++q) {
                 n.arm[q] = ell * ax[q] + rho * (cph * u[q] + sph * v[q]);
@@ -238,106 +296,111 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pa
         // in row group 0 (the other groups of a pair skip them). The loop runs to the wave's largest term count and
         // each lane stops adding at its own, so a node's value does not depend on its wave. Not in the gradient
         // instance (the series carries no derivatives with respect to the primary's R, a, b).
-        auto series = [&](const Node &n, bool far) {
+        constexpr bool kA = WM || WD || GR, kB = WF || WD || GR, kAda = GR || WD;
+        auto series = [&](const Node &n, bool far, Local &L, AdjA &q) {
             if constexpr (!GR) {
-                if (!__ballot(far)) return;
+                if (rg != 0 || !__ballot(far)) return;
                 const int own = far ? multipole_terms(n.z * n.z + n.r * n.r, pc.inv_rmax2,
                                                       PREC == 1 ? kMpLogTolFP32C : kMpLogTolFP64) : 0;
                 const int terms = wave_max_small(own), lo = wave_min_small(own, far);
-                if (far && rg == 0) {
-                    Local L = {0, 0, 0, 0, 0, 0, 0};
+                if (far) {
                     double aor = 0.0;
-                    eval_multipole_pair<WM || WD, WF || WD>(p.mp + kMpHeader + (size_t)pd.prim * kMpCoil, p.mp,
-                                                            pc.rmax, n.z, n.r, terms, lo, own, L, aor);
-                    AdjA q = {0.0, 0.0, 0.0, L.Bz - aor};   // dA_phi/dr = B_z - A_phi / r
-                    accumulate(n, L, q);
+                    eval_multipole_pair<kA, kB>(p.mp + kMpHeader + (size_t)pd.prim * kMpCoil, p.mp, pc.rmax, n.z, n.r,
+                                                terms, lo, own, L, aor);
+                    q = {0.0, 0.0, 0.0, L.Bz - aor};   // dA_phi/dr = B_z - A_phi / r
                 }
             }
         };
-        if constexpr (PREC == 1) {
-            // FP32C: far nodes in FP32 as they come; nodes in the primary's near-winding shell are queued (ring of
-            // 128 in LDS, wave-uniform head and count) and evaluated in FP64 64 at a time, so the FP64 evaluation
-            // runs with full waves instead of beside the FP32 one in every wave that holds a near node.
-            __shared__ int64_t queue[128];
-            int qh = 0, qn = 0;
-            for (int64_t base = n0; base < n1; base += 64) {
-                const int64_t k = base + lane;
-                Node n;
-                bool near = false, far = false;
-                if (k < n1) {
-                    node(k, n);
-                    far = !GR && p.mp && is_far(pc, n.z, n.r);
-                    near = !far && is_near(pc, n.z, n.r, WD || GR);   // the position gradient divides A by r
-                    if (!near && !far) {
-                        Local L = {0, 0, 0, 0, 0, 0, 0};
-                        if constexpr (GR) {
-                            AdjA q;
-                            eval_stable<float, true, true, false, false, true>(pc, p.tab, full_rule(pc), n.z, n.r, rg, pd.row_groups, 0, 1,
-                                                                               L, nullptr, &q);
-                            accumulate_grad(n, L, q);
-                        } else {
-                            AdjA q;
-                            eval_stable<float, WM || WD, WF || WD, false, false, WD, true>(pc, p.tab, full_rule(pc), n.z, n.r, rg,
-                                                                                     pd.row_groups, 0, 1, L, nullptr, &q);
-                            accumulate(n, L, q);
-                        }
-                    }
-                }
-                series(n, far);
-                const unsigned long long mask = __ballot(near);
-                if (mask) {
-                    if (near) queue[(qh + qn + __popcll(mask & ((1ull << lane) - 1ull))) & 127] = k;
-                    qn += __popcll(mask);
-                    __syncthreads();
-                    if (qn >= 64) {
-                        node(queue[(qh + lane) & 127], n);
-                        Local L = {0, 0, 0, 0, 0, 0, 0};
-                        if constexpr (GR) {
-                            AdjA q;
-                            eval_stable<f64s, true, true, false, false, true>(pc, p.tab, full_rule(pc), n.z, n.r, rg, pd.row_groups, 0, 1,
-                                                                              L, nullptr, &q);
-                            accumulate_grad(n, L, q);
-                        } else {
-                            AdjA q;
-                            eval_stable<f64s, WM || WD, WF || WD, false, false, WD, true>(pc, p.tab, full_rule(pc), n.z, n.r, rg,
-                                                                                    pd.row_groups, 0, 1, L, nullptr, &q);
-                            accumulate(n, L, q);
-                        }
-                        qh = (qh + 64) & 127;
-                        qn -= 64;
-                    }
-                    __syncthreads();
-                }
-            }
-            if (qn > 0 && lane < qn) {
-                Node n;
-                node(queue[(qh + lane) & 127], n);
-                Local L = {0, 0, 0, 0, 0, 0, 0};
-                if constexpr (GR) {
-                    AdjA q;
-                    eval_stable<f64s, true, true, false, false, true>(pc, p.tab, full_rule(pc), n.z, n.r, rg, pd.row_groups, 0, 1, L,
-                                                                      nullptr, &q);
-                    accumulate_grad(n, L, q);
+        auto add = [&](const Node &n, const Local &L, const AdjA &q) {
+            if constexpr (GR) accumulate_grad(n, L, q);
+            else accumulate(n, L, q);
+        };
+        if constexpr (PREC == 0 || PREC == 1) {
+            // FP64: nodes with a reduced angular rule as they come, by one rule for the wave; FP32C: nodes outside the
+            // primary's near-winding shell in FP32 as they come, the others by the FP64 rule. Nodes next to the winding,
+            // which keep the coil's own angular rule with ten times the nodes, are queued (FP32C's other FP64 nodes in a
+            // second queue; rings of 128 in LDS, wave-uniform heads and counts) and evaluated 64 at a time, so that
+            // those evaluations run with full waves instead of beside the cheaper ones in every wave that holds such a
+            // node. One loop and one copy of its code serve all three: a small batch runs through each instruction a few
+            // times only, and waits for it to be fetched.
+            __shared__ int queue[PREC == 1 ? 256 : 128];   // the hard nodes, then FP32C's others
+            int h0 = 0, c0 = 0, h1 = 0, c1 = 0;                // head and count of either ring
+            const int own = pc.n_ang * ((pc.n_thk + pd.row_groups - 1) / pd.row_groups);
+            const bool reducible = pc.red_x < 1e30f;   // else every node keeps the own rule
+            auto push = [&](int ring, int head, int &count, bool mine, int k) {
+                const unsigned long long mask = __ballot(mine);
+                if (mine) queue[ring + ((head + count + __popcll(mask & ((1ull << lane) - 1ull))) & 127)] = k;
+                count += __popcll(mask);
+            };
+            for (int base = 0;;) {
+                // 0: the next 64 nodes, 1: the hard queue, 2: the other; each queue when it is full, and at the end what
+                // is left but for the last few hard nodes
+                int mode;
+                if (c0 >= 64) mode = 1;
+                else if (PREC == 1 && c1 >= 64) mode = 2;
+                else if (base < n_item) mode = 0;
+                else if (c0 * (own / 64 + 8) > own || (c0 > 0 && own < 256)) mode = 1;
+                else if (PREC == 1 && c1 > 0) mode = 2;
+                else break;
+                int k = base + lane;
+                bool sel = k < n_item;
+                if (mode == 0) {
+                    if (!sel) k = n_item - 1;   // lanes past the end shadow the last node
+                    base += 64;
                 } else {
-                    AdjA q;
-                    eval_stable<f64s, WM || WD, WF || WD, false, false, WD, true>(pc, p.tab, full_rule(pc), n.z, n.r, rg,
-                                                                                  pd.row_groups, 0, 1, L, nullptr, &q);
-                    accumulate(n, L, q);
+                    int &head = mode == 1 ? h0 : h1, &count = mode == 1 ? c0 : c1;
+                    const int take = count < 64 ? count : 64;
+                    sel = lane < take;
+                    k = queue[(mode == 1 ? 0 : 128) + ((head + (sel ? lane : 0)) & 127)];
+                    head += take;
+                    count -= take;
                 }
-            }
-        } else {
-            for (int64_t k = n0 + lane; k < n1; k += 64) {
                 Node n;
                 node(k, n);
-                const bool far = !GR && p.mp && is_far(pc, n.z, n.r);
-                if (!far) {
-                    Local L = {0, 0, 0, 0, 0, 0, 0};
-                    AdjA q;
-                    eval_prim<PREC, WM || WD, WF || WD, GR || WD>(pc, p.tab, n.z, n.r, rg, pd.row_groups, L, &q);
-                    if constexpr (GR) accumulate_grad(n, L, q);
-                    else accumulate(n, L, q);
+                const int cls = rule_class(pc, n.z, n.r);
+                Local L = {0, 0, 0, 0, 0, 0, 0};
+                AdjA q;
+                bool far = false, single = false, hard = false, other = false;
+                if (mode == 0) {
+                    far = sel && !GR && p.mp && is_far(pc, n.z, n.r);
+                    // the position gradient divides A by r, so its near nodes include the axis cone
+                    const bool fp64 = sel && !far && (PREC == 0 || is_near(pc, n.z, n.r, WD || GR));
+                    single = sel && !far && !fp64;
+                    hard = fp64 && cls <= kRedThk && reducible;   // the coil's own angular rule
+                    other = PREC == 1 && fp64 && !hard;
+                    sel = PREC == 0 && fp64 && !hard;
                 }
-                series(n, far);
+                if ((PREC == 0 || mode != 0) && __ballot(sel)) {
+                    // all lanes write L; the others' values are dropped or overwritten below
+                    eval_pair<kA, kB, kAda>(pc, p.tab, n.z, n.r, sel, cls, mode == 1, rg, pd.row_groups, L, &q);
+                }
+                if (PREC == 1 && single)
+                    eval_stable<float, kA, kB, false, false, kAda, !kAda>(pc, p.tab, full_rule(pc), n.z, n.r, rg,
+                                                                          pd.row_groups, 0, 1, L, nullptr, &q);
+                series(n, far, L, q);
+                if (sel || single || (far && rg == 0)) add(n, L, q);
+                push(0, h0, c0, hard, k);
+                if constexpr (PREC == 1) push(128, h1, c1, other, k);
+                __syncthreads();
+            }
+            // the last few hard nodes of a large rule: one at a time over the whole wave, which is the shorter way
+            for (int i = 0; i < c0; ++i) {
+                Node n;
+                node(queue[(h0 + i) & 127], n);
+                const int cls = __builtin_amdgcn_readfirstlane(rule_class(pc, n.z, n.r));
+                Local L = {0, 0, 0, 0, 0, 0, 0};
+                AdjA q;
+                eval_pair_wave<kA, kB, kAda>(pc, p.tab, n.z, n.r, cls, lane, rg, pd.row_groups, L, &q);
+                if (lane == 0) add(n, L, q);
+            }
+        } else {
+            for (int k = lane; k < n_item; k += 64) {
+                Node n;
+                node(k, n);
+                Local L = {0, 0, 0, 0, 0, 0, 0};
+                AdjA q;
+                eval_prim<PREC, kA, kB, kAda>(pc, p.tab, n.z, n.r, rg, pd.row_groups, L, &q);
+                add(n, L, q);
             }
         }
         if constexpr (GR) {

@@ -11,30 +11,42 @@ using namespace ccoil;
 
 namespace {
 
-// Primary-node evaluations per lane and work item. Large batches give every lane about 8192 (each item's
-// fixed costs, the wave reduction and the partial, stay small); a batch with too little work to give the 1,024
-// SIMDs about 4 waves each at that size lowers it, down to 256, so that a single pair or a few pairs still spread
-// over the chip instead of running one long chain per lane. Powers of two only.
-int64_t lane_target(int64_t node_pairs)
+// Primary-node evaluations per lane and work item. Large batches give every lane about 8192 of the planned rule's
+// (each item's fixed costs, the wave reduction and the partial, stay small); a batch with too little work to give the
+// 1,024 SIMDs about 4 waves each at that size lowers it, down to 256, so that a single pair or a few pairs still spread
+// over the chip instead of running one long chain per lane. Powers of two only. The FP64 kernels, which evaluate
+// reduced rules, count those rules' nodes (rule_nodes_of), of which a lane takes up to 2048 and down to 16.
+int64_t lane_target(int64_t node_pairs, bool reduced)
 {
-    int64_t t = 8192;
-    while (t > 256 && node_pairs < (int64_t)64 * 4096 * t) t >>= 1;
+    const int64_t most = reduced ? 2048 : 8192, least = reduced ? 16 : 256;
+    int64_t t = most;
+    while (t > least && node_pairs < (int64_t)64 * 4096 * t) t >>= 1;
     return t;
+}
+
+// Nodes of the rule that an FP64 pair evaluates at most of its secondary's nodes: the class beyond the nearest that
+// the secondary comes to the primary's centre, and where its nodes come near the winding, a quarter of the planned
+// rule (the nodes next to the winding, with all of it, weigh as much as all others).
+int64_t rule_nodes_of(const CoilDev &p, const CoilDev &s)
+{
+    const double d[3] = {s.pos[0] - p.pos[0], s.pos[1] - p.pos[1], s.pos[2] - p.pos[2]};
+    const double near = std::sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]) - std::hypot(s.R + s.a, 0.5 * s.b);
+    const int64_t own = (int64_t)p.n_ang * p.n_thk, beyond = rule_nodes_beyond(p, near);
+    return beyond < own ? beyond : p.red_x < 1e30f ? std::max<int64_t>(1, own / 4) : own;
 }
 
 // Work decomposition of one pair for a lane target: secondary nodes per item (64 lanes times nodes per lane)
 // and the number of groups the primary's thickness rows are split into. Small primaries take several secondary
 // nodes per lane; a primary with more nodes than the target splits its rows.
-void decompose(int64_t target, int n_ang, int n_thk, int &nodes_per_item, int &row_groups)
+void decompose(int64_t target, int64_t prim_nodes, int n_thk, int &nodes_per_item, int &row_groups)
 {
-    const int64_t prim_nodes = (int64_t)n_ang * n_thk;
     if (prim_nodes <= target) {
         const int64_t per_lane = std::max<int64_t>(1, std::min<int64_t>(64, (target + prim_nodes - 1) / prim_nodes));
         nodes_per_item = (int)(64 * per_lane);
         row_groups = 1;
     } else {
         nodes_per_item = 64;
-        const int64_t rows_per_group = std::max<int64_t>(1, target / n_ang);
+        const int64_t rows_per_group = std::max<int64_t>(1, target * n_thk / prim_nodes);
         row_groups = (int)std::min<int64_t>(n_thk, (n_thk + rows_per_group - 1) / rows_per_group);
     }
 }
@@ -92,7 +104,11 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
         host_parallel_for((int64_t)hp.size(), [&](int64_t i0, int64_t i1) {
             for (int64_t i = i0; i < i1; ++i) {
                 CoilDev &c = hp[(size_t)i];
-                const double y = far_distance(c, precision == CCOIL_FP64, true);
+                // the slow method's reduced rules take no longer than its series at any distance (18 operations a node;
+                // flat primaries measured 10.6k cycles per 64 nodes either way at three radii, filaments 7.4k against
+                // 9.0k), so FP64 keeps the rule there and saves the moments
+                const bool rule = precision == CCOIL_FP64 && !c.use_fast && c.red_x < 1e30f;
+                const double y = rule ? 0.0 : far_distance(c, precision == CCOIL_FP64, true);
                 c.far_d2 = y > 0.0 ? (y * c.rmax) * (y * c.rmax) : 0.0;
                 c.mp_terms = far_terms(y, precision == CCOIL_FP64);
             }
@@ -100,16 +116,21 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
 
     // Pair table, longest work item first (LPT order of the persistent queue).
     std::vector<PairDev> pd((size_t)n_pairs);
-    int64_t node_pairs = 0;
+    const bool reduced = precision == CCOIL_FP64;
+    std::vector<int64_t> prim_nodes((size_t)n_pairs);   // that an item evaluates per secondary node
+    int64_t node_pairs = 0, work = 0;
     const bool ref_scale = flags & CCOIL_FORCE_REFERENCE_SCALE;
     for (int64_t k = 0; k < n_pairs; ++k) {
         const int64_t pi = prim_index ? prim_index[k] : k, si = sec_index ? sec_index[k] : k;
         if (pi < 0 || pi >= (int64_t)hp.size() || si < 0 || si >= (int64_t)hs.size())
             return fail(ctx, CCOIL_ERR_ARGUMENT, "pair " + std::to_string(k) + ": coil index out of range");
         const CoilDev &p = hp[(size_t)pi], &s = hs[(size_t)si];
-        node_pairs += (int64_t)s.blk_ang * s.n_ang * s.blk_thk * s.n_thk * s.blk_len * s.n_len * p.n_ang * p.n_thk;
+        const int64_t sec_nodes = (int64_t)s.blk_ang * s.n_ang * s.blk_thk * s.n_thk * s.blk_len * s.n_len;
+        node_pairs += sec_nodes * p.n_ang * p.n_thk;
+        prim_nodes[(size_t)k] = series_only(p, s) ? kSeriesNodes : reduced ? rule_nodes_of(p, s) : (int64_t)p.n_ang * p.n_thk;
+        work += sec_nodes * (reduced ? prim_nodes[(size_t)k] : (int64_t)p.n_ang * p.n_thk);
     }
-    const int64_t target = target_override > 0 ? target_override : lane_target(node_pairs);
+    const int64_t target = target_override > 0 ? target_override : lane_target(work, reduced);
     out.target = target;
     int max_row_groups = 1;
     for (int64_t k = 0; k < n_pairs; ++k) {
@@ -121,8 +142,7 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
         d.sec = (int32_t)si;
         d.out = (int32_t)k;
         d.n_nodes = (int64_t)s.blk_ang * s.n_ang * s.blk_thk * s.n_thk * s.blk_len * s.n_len;
-        if (series_only(p, s)) decompose(target, kSeriesNodes, 1, d.nodes_per_item, d.row_groups);
-        else decompose(target, p.n_ang, p.n_thk, d.nodes_per_item, d.row_groups);
+        decompose(target, prim_nodes[(size_t)k], series_only(p, s) ? 1 : p.n_thk, d.nodes_per_item, d.row_groups);
         max_row_groups = std::max(max_row_groups, d.row_groups);
         d.ring_offset = ring_offset ? ring_offset[k] : 0.0;
         d.half_ring = half_ring ? (half_ring[k] ? 1 : 0) : 0;
@@ -138,10 +158,9 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
     for (int64_t k = 0; k < n_pairs; ++k) {
         const PairDev &d = pd[(size_t)k];
         const CoilDev &p = hp[(size_t)d.prim];
-        const int64_t rows = (p.n_thk + d.row_groups - 1) / d.row_groups;
-        cost[(size_t)k] = series_only(p, hs[(size_t)d.sec])
-                              ? std::min<int64_t>(d.nodes_per_item, d.n_nodes) * kSeriesNodes
-                              : std::min<int64_t>(d.nodes_per_item, d.n_nodes) * p.n_ang * rows * (p.use_fast ? 2 : 1);
+        cost[(size_t)k] = std::min<int64_t>(d.nodes_per_item, d.n_nodes) *
+                          ((prim_nodes[(size_t)k] + d.row_groups - 1) / d.row_groups) *
+                          (p.use_fast && !series_only(p, hs[(size_t)d.sec]) ? 2 : 1);
     }
     std::vector<int32_t> order((size_t)n_pairs);
     std::iota(order.begin(), order.end(), 0);

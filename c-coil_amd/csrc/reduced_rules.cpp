@@ -129,6 +129,17 @@ void set_rule_limits(CoilDev &c)
     c.ia2f = c.red_s < FLT_MAX ? (float)(2.0 / c.a) : 0.0f;
 }
 
+int64_t rule_nodes_beyond(const CoilDev &c, double dist)
+{
+    // every ring element lies within rmax of the centre, so a point at D >= dist is at least gap = D - rmax from it,
+    // and r rho <= D (R + a)
+    const double gap = dist - c.rmax;
+    if (!(gap > 0.0)) return (int64_t)c.n_ang * c.n_thk;
+    const RuleSel s = class_rule(c, class_of(c, (float)(gap * gap), (float)(2.0 * dist * (c.R + c.a)),
+                                             (float)(2.0 * gap) * c.ia2f));
+    return (int64_t)s.na * s.nt;
+}
+
 void reduced_tables(RedTables &t)
 {
     int e = 0;

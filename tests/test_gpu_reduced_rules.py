@@ -91,3 +91,44 @@ def test_field_kernel_matches_the_own_rule(ctx, coil, n, split):
     _, rep = ctx.fields(abi.CoilSet.from_rows([row]), np.zeros((n, 3)), abi.B, abi.FP64)
     assert rep.split == split
     print(f"\n{coil} n={n}: worst error over tolerance {check(ctx, row, n, abi.FP64, 0, 7)}")
+
+
+@pytest.mark.parametrize("blocks", [(1, 1, 1), (3, 2, 2)])
+@pytest.mark.parametrize("coil", COILS, ids=lambda c: f"{c[0]}-{c[4]}x{c[5]}")
+def test_pairs_match_the_own_rule(ctx, coil, blocks):
+    """M, F, T, dM and the gradient of M of one primary with secondaries from inside its bore and across its winding to
+    twenty radii away, CCOIL_FP64 against CCOIL_FP64_IEEE, alone (a few work items) and as a batch. Each sum's terms
+    exceed it by at most about a thousand here (M relative to its size over the pose's neighbourhood), and both rules
+    round each term to a few ulps: 1e-12, and 1e-10 where the secondary crosses the primary's winding. The derivatives
+    with respect to the primary's geometry cancel once more like the field they come from, by (1 + y)^2 / 10 beyond."""
+    row = _row(*coil)
+    rng = np.random.default_rng(11)
+    size = np.hypot(row["R"] + row["a"], 0.5 * row["b"])
+    secs = []
+    ys = np.array([0.3, 0.9, 1.6, 2.5, 4.0, 8.0, 20.0])
+    for y in ys:
+        d = rng.standard_normal(3)
+        s = _row("RECTANGULAR", 0.3 * row["R"], 0.1 * row["R"], 0.2 * row["R"], 14, 3)
+        s.update(pos=tuple(np.asarray(row["pos"]) + y * size * d / np.linalg.norm(d)), alpha=rng.uniform(0, 3.0),
+                 beta=rng.uniform(0, 6.0), n_len=5, blocks=blocks)
+        secs.append(s)
+    P, S, n = abi.CoilSet.from_rows([row]), abi.CoilSet.from_rows(secs), len(secs)
+    what, prim = abi.PAIR_M | abi.PAIR_FT | abi.PAIR_DM, np.zeros(n, dtype=np.int64)
+    ref, _ = ctx.pairs(P, S, n, what, abi.FP64_IEEE, prim_index=prim)
+    got, _ = ctx.pairs(P, S, n, what, abi.FP64, prim_index=prim)
+    Mr, Gr, _ = ctx.pairs_grad(P, S, n, abi.FP64_IEEE, prim_index=prim)
+    Mg, Gg, _ = ctx.pairs_grad(P, S, n, abi.FP64, prim_index=prim)
+    one, _ = ctx.pairs(P, S, 1, what, abi.FP64, prim_index=prim[:1], sec_index=np.array([3]))
+    norm = np.linalg.norm
+    dist = np.array([norm(np.array(s["pos"]) - np.array(row["pos"])) for s in secs])
+    mscale = np.abs(ref["M"]) + norm(ref["dM"], axis=1) * dist
+    errs = {"M": np.abs(got["M"] - ref["M"]) / mscale, "M of grad": np.abs(Mg - Mr) / mscale,
+            "grad": norm(Gg - Gr, axis=1) / norm(Gr, axis=1)}
+    for k in ("F", "T", "dM"):
+        errs[k] = norm(got[k] - ref[k], axis=1) / norm(ref[k], axis=1)
+    print(f"\n{coil} {blocks}: " + ", ".join(f"{k} {v.max():.2g}" for k, v in errs.items()))
+    for k, v in errs.items():
+        tol = np.where(ys < 1.0, 1e-10, 1e-12 * (np.maximum(1.0, (1.0 + ys) ** 2 / 10.0) if k == "grad" else 1.0))
+        assert np.all(v <= tol), (k, v, tol)
+    assert abs(one["M"][0] - ref["M"][3]) <= 1e-12 * mscale[3]
+    assert norm(one["F"][0] - ref["F"][3]) <= 1e-12 * norm(ref["F"][3])
