@@ -45,8 +45,11 @@ __global__ __launch_bounds__(kGradBlock) void field_grad_kernel(GradParams p)
         to_local(c, p.pts[3 * pi], p.pts[3 * pi + 1], p.pts[3 * pi + 2], z, r, cph, sph);
         Local L = {0, 0, 0, 0, 0, 0, 0};
         AdjLocal ad;
+        // the wave's points by one rule that serves them all (reduced rules; next to a winding the coil's own): a
+        // pair's rounding so depends on its wave, as explained below
+        const RuleSel rule = class_rule(c, wave_rule_class(rule_class(c, z, r)));
         if constexpr (PREC == kFP64) {
-            eval_stable<f64s, false, true, true, true>(c, p.tab, full_rule(c), z, r, 0, 1, 0, 1, L, &ad);
+            eval_stable<f64s, false, true, true, true>(c, p.tab, rule, z, r, 0, 1, 0, 1, L, &ad);
         } else if constexpr (PREC == kFP64IEEE) {
             eval_stable<double, false, true, true, true>(c, p.tab, full_rule(c), z, r, 0, 1, 0, 1, L, &ad);
         } else {
@@ -54,7 +57,7 @@ __global__ __launch_bounds__(kGradBlock) void field_grad_kernel(GradParams p)
             // the FP64 one would add its own issue time. A pair's value thus depends on its wave, which the
             // point order and the grid fix, as they fix the order of the sums over points.
             if (__ballot(is_near(c, z, r, true)))
-                eval_stable<f64s, false, true, true, true>(c, p.tab, full_rule(c), z, r, 0, 1, 0, 1, L, &ad);
+                eval_stable<f64s, false, true, true, true>(c, p.tab, rule, z, r, 0, 1, 0, 1, L, &ad);
             else
                 eval_stable<float, false, true, true, true>(c, p.tab, full_rule(c), z, r, 0, 1, 0, 1, L, &ad);
         }

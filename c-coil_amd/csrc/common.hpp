@@ -310,4 +310,21 @@ __device__ inline int rule_class(const CoilDev &c, double z, double r)
     return class_of(c, num, den, s);
 }
 
+// Largest v over the wave for 0 <= v < 2^BITS (lanes not executing count as 0): its bits from the top, one ballot each.
+template <int BITS> __device__ inline int wave_max_bits(int v)
+{
+    int m = 0;
+#pragma unroll
+    for (int b = 1 << (BITS - 1); b >= 1; b >>= 1)
+        if (__ballot(v >= (m | b))) m |= b;
+    return m;
+}
+// The cheapest rule class that serves every executing lane of the wave (cls: the lane's own).
+__device__ inline int wave_rule_class(int cls)
+{
+    const int k = cls / (kRedThk + 1), t = cls - k * (kRedThk + 1);
+    return (7 - wave_max_bits<3>(7 - k)) * (kRedThk + 1) + 7 - wave_max_bits<3>(7 - t);
+}
+static_assert(kRedAng < 8 && kRedThk < 8, "three bits each");
+
 }  // namespace ccoil

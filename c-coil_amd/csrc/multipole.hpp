@@ -55,15 +55,7 @@ __device__ inline int multipole_terms(double D2, double inv_rmax2, float log_tol
     return L < 4 ? 4 : (L > kMpTerms ? kMpTerms : L);
 }
 
-// Largest v over the wave for 0 <= v < 2^BITS (every lane active): its bits from the top, one ballot each.
-template <int BITS> __device__ inline int wave_max_bits(int v)
-{
-    int m = 0;
-#pragma unroll
-    for (int b = 1 << (BITS - 1); b >= 1; b >>= 1)
-        if (__ballot(v >= (m | b))) m |= b;
-    return m;
-}
+// Largest v over the wave for 0 <= v < 256 (every lane active).
 __device__ inline int wave_max_small(int v) { return wave_max_bits<8>(v); }
 
 // Smallest v over the lanes with active set, for 0 <= v < 256 (every lane of the wave executing); 255 if none is.
