@@ -2,6 +2,7 @@
 #include "context.hpp"
 #include "zaxis.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
@@ -11,19 +12,115 @@ namespace {
 
 constexpr double kMu = 1e-7;   // g_MiReduced (CalculateMInductanceZAxis.cxx:12)
 
+// Distance sum, in units of half the length, from the points (x, y), x in [x0, x1], to the ends of the segment
+// [lo, lo + len] of the x axis: the least over them.
+double ellipse_sum(double lo, double len, double x0, double x1, double y)
+{
+    const double mid = lo + 0.5 * len, x = std::fmin(std::fmax(mid, x0), x1);   // the nearest to the middle is the least
+    const double d0 = x - lo, d1 = d0 - len;
+    return 2.0 * (std::sqrt(d0 * d0 + y * y) + std::sqrt(d1 * d1 + y * y)) / len;
+}
+
+// The reduced rules of a pair's M and force sums (na == 0: none); t, r 0: the coil's own nodes.
+struct PairRule { int na, a_off, l, t, r; };
+
+// Reduced rules (reduced_rules.cpp) for two coaxial coils clear of each other: R, a, h: the inner radii, thicknesses and
+// half-lengths of the primary and the secondary, c the distance of their centres; n_ang, n_thk, n_rad their nodes.
+//
+// With g the axial and q the radial gap of the windings, the angular integrand at radii t, r is analytic for |Im phi| <
+// eta, cosh(eta) = 1 + ((t - r)^2 + g^2) / (2 t r) (the terms singular at t = r alone cancel between the four
+// offsets where the coils are axially apart); the thickness and radial integrands are analytic outside the other coil's
+// nearest point in the meridian plane, as in the field rules; and the force and inductance of a sheet of half-length H
+// at an offset l along the shorter coil (half-length h <= H) outside l = -c +- H +- i D, D >= q the in-plane distance.
+// A rule of several blocks converges no later than one block of it. Coils that the angular or the length nodes do not
+// serve (72 of a table of 1,500 random pairs) keep their rules.
+PairRule pair_rule(double Rp, double ap, double hp, double Rs, double as, double hs, double c, int n_ang, int n_thk, int n_rad)
+{
+    PairRule rule = {0, 0, 0, 0, 0};
+    const double g = std::fmax(0.0, std::fabs(c) - hp - hs);
+    const double q = std::fmax(0.0, std::fmax(Rp - (Rs + as), Rs - (Rp + ap)));
+    if (!(q + g > 0.0)) return rule;
+    CoilDev d;
+    d.R = Rp;
+    d.a = ap;
+    d.b = 2.0 * hp;
+    d.use_fast = 1;
+    d.n_ang = n_ang;
+    d.n_thk = n_thk;
+    set_rule_limits(d);
+    const float num = (float)(q * q + g * g), den = (float)(2.0 * (Rp + ap) * (Rs + as));
+    const int cls = class_of(d, num, den, (float)ellipse_sum(Rp, ap, Rs, Rs + as, g));
+    const int k = cls / (kRedThk + 1), t = cls % (kRedThk + 1);
+    const double H = std::fmax(hp, hs), h = std::fmin(hp, hs), x0 = -c + H, x1 = -c - H;
+    d.n_thk = n_rad;
+    set_rule_limits(d);
+    const int r = class_of(d, num, den, (float)ellipse_sum(Rs, as, Rp, Rp + ap, g)) % (kRedThk + 1);
+    d.n_thk = kMaxOrder;
+    set_rule_limits(d);
+    const double sl = std::fmin(ellipse_sum(-h, 2.0 * h, x0, x0, q), ellipse_sum(-h, 2.0 * h, x1, x1, q));
+    const int l = class_of(d, num, den, (float)sl) % (kRedThk + 1);
+    if (k == 0 || l == 0) return rule;
+    rule.na = kRedAngN[k - 1];
+    rule.a_off = kRedOffset;
+    for (int i = 0; i < k - 1; ++i) rule.a_off += kRedAngN[i];
+    rule.l = kRedThkN[l - 1];
+    rule.t = t ? kRedThkN[t - 1] : 0;
+    rule.r = r ? kRedThkN[r - 1] : 0;
+    return rule;
+}
+
+// Rewrites a pair's item with its reduced rules.
+void reduce_item(ZItemDev &it, const PairRule &rule)
+{
+    it.constant *= kPi * std::fmin(it.hp, it.hs) / it.a_width;
+    it.a_blk = 1;
+    it.a_inc = (int16_t)rule.na;
+    it.a_off = (int16_t)rule.a_off;
+    it.l_inc = (int16_t)rule.l;
+    if (rule.t) {
+        it.constant *= it.t_blk;
+        it.t_width *= it.t_blk;
+        it.t_blk = 1;
+        it.t_inc = (int16_t)rule.t;
+    }
+    if (rule.r) {
+        it.constant *= it.r_blk;
+        it.r_width *= it.r_blk;
+        it.r_blk = 1;
+        it.r_inc = (int16_t)rule.r;
+    }
+}
+
+// Sets the item's units from its rules.
+void set_units(ZItemDev &it)
+{
+    it.t_split = (int16_t)((it.t_inc + kZNodes - 1) / kZNodes);
+    it.units = (int64_t)it.r_blk * it.r_inc * it.a_blk * it.a_inc * std::max<int>(it.l_inc, 1) * it.t_split;
+    it.n_wg = (it.units + kZBlock - 1) / kZBlock;
+}
+
 bool valid_rule(int32_t blocks, int32_t inc) { return blocks >= 1 && inc >= 1 && inc <= kMaxOrder; }
 
-// Upload the items, run the node kernel and the ordered reduction, copy n_out results back.
-ccoil_status run_items(ccoil_ctx ctx, std::vector<ZItemDev> &items, size_t n_out, uint32_t flags, double *out_host,
-                       double *out_dev, int64_t node_evals, ccoil_report *report)
+// Upload the items, run the node kernel and the ordered reduction for `modes` quantities from `mode` on, copy n_out
+// results back.
+ccoil_status run_items(ccoil_ctx ctx, std::vector<ZItemDev> &items, int32_t mode, int32_t modes, size_t n_out,
+                       uint32_t flags, double *out_host, double *out_dev, int64_t node_evals, ccoil_report *report)
 {
     int64_t wg = 0;
     for (auto &it : items) {
         it.first_wg = wg;
-        wg += (it.units + kZBlock - 1) / kZBlock;
+        wg += modes * it.n_wg;
     }
     if (wg > INT32_MAX) return fail(ctx, CCOIL_ERR_ARGUMENT, "coaxial batch needs more than 2^31 - 1 workgroups");
     CC_HIP(ctx, hipSetDevice(ctx->device));
+    // the items, then each workgroup's item
+    const size_t n_items = items.size();
+    const bool mapped = wg <= kZMapped;
+    if (mapped) {
+        items.resize(n_items + ((size_t)wg * sizeof(int32_t) + sizeof(ZItemDev) - 1) / sizeof(ZItemDev));
+        int32_t *wg_item = reinterpret_cast<int32_t *>(items.data() + n_items);
+        for (size_t i = 0; i < n_items; ++i) wg_item = std::fill_n(wg_item, modes * items[i].n_wg, (int32_t)i);
+    }
     CC_HIP(ctx, ensure(ctx->zitems, sizeof(ZItemDev) * items.size()));
     CC_HIP(ctx, ensure(ctx->zpartial, sizeof(double) * (size_t)wg));
     CC_HIP(ctx, hipMemcpyAsync(ctx->zitems.p, items.data(), sizeof(ZItemDev) * items.size(), hipMemcpyHostToDevice,
@@ -31,7 +128,11 @@ ccoil_status run_items(ccoil_ctx ctx, std::vector<ZItemDev> &items, size_t n_out
     ZParams zp;
     std::memset(&zp, 0, sizeof zp);
     zp.items = (const ZItemDev *)ctx->zitems.p;
-    zp.n_items = (int32_t)items.size();
+    zp.wg_item = mapped ? (const int32_t *)(zp.items + n_items) : nullptr;
+    zp.n_items = (int32_t)n_items;
+    zp.mode = mode;
+    zp.n_modes = modes;
+    zp.out_stride = modes > 1 ? (int64_t)n_out / modes : 0;
     zp.n_wg = wg;
     zp.partial = (double *)ctx->zpartial.p;
     zp.tab = ctx_tables(ctx);
@@ -101,76 +202,71 @@ extern "C" ccoil_status ccoil_pairs_zaxis(ccoil_ctx ctx, const ccoil_coils *prim
     if (n_pairs == 0) return CCOIL_OK;
     if (prim->n == 0 || sec->n == 0) return fail(ctx, CCOIL_ERR_ARGUMENT, "pairs given but a coil array is empty");
 
-    std::vector<ZItemDev> items;
+    std::vector<ZItemDev> items, reduced;   // full rules are launched first: their workgroups run longest
+    items.reserve((size_t)n_pairs + 1);
+    reduced.reserve((size_t)n_pairs);
     int64_t evals = 0;
-    const int modes[2] = {kZMutual, kZForce};
-    for (int m = 0; m < 2; ++m) {
-        if (!(what & (m == 0 ? CCOIL_PAIR_M : CCOIL_PAIR_FT))) continue;
-        for (int64_t k = 0; k < n_pairs; ++k) {
-            const int64_t i = prim_index ? prim_index[k] : k, j = sec_index ? sec_index[k] : k;
-            if (i < 0 || i >= prim->n || j < 0 || j >= sec->n)
-                return fail(ctx, CCOIL_ERR_ARGUMENT, "pair " + std::to_string(k) + ": coil index out of range");
-            ZItemDev it;
-            std::memset(&it, 0, sizeof it);
-            it.mode = modes[m];
-            it.out = (int32_t)(m * n_pairs + k);
-            it.a_blk = prim->blocks ? prim->blocks[3 * i] : 1;
-            it.t_blk = prim->blocks ? prim->blocks[3 * i + 1] : 1;
-            it.r_blk = sec->blocks ? sec->blocks[3 * j + 1] : 1;
-            it.a_inc = prim->n_ang[i];
-            it.t_inc = prim->n_thk[i];
-            it.r_inc = sec->n_thk[j];
-            const double t_width = prim->a[i] / it.t_blk, a_width = kPi / it.a_blk, r_width = sec->a[j] / it.r_blk;
-            it.t_inner = prim->R[i];
-            it.t_width = t_width;
-            it.a_width = a_width;
-            it.r_inner = sec->R[j];
-            it.r_width = r_width;
-            it.constant = kMu * prim->J[i] * sec->J[j] * t_width * a_width * r_width * 0.125;
-            const double d = sec->pos[3 * j + 2] - prim->pos[3 * i + 2];
-            const double hs = sec->b[j] * 0.5, hp = prim->b[i] * 0.5;
-            it.z[0] = d + hs + hp;
-            it.z[1] = d + hs - hp;
-            it.z[2] = d - hs - hp;
-            it.z[3] = d - hs + hp;
-            for (int q = 0; q < 4; ++q) it.zsq[q] = it.z[q] * it.z[q];
-            if (it.mode == kZMutual) {
-                if (prim->current[i] == 0.0 || sec->current[j] == 0.0)
-                    return fail(ctx, CCOIL_ERR_ARGUMENT, "pair " + std::to_string(k) + ": mutual inductance needs "
-                                                         "non-zero currents (M = sum * 2 pi / (I1 I2))");
-                it.mul = 2.0 * kPi;
-                it.mul2 = 1.0;
-                it.div = prim->current[i] * sec->current[j];
-            } else {
-                it.mul = -2.0 * kPi;
-                it.mul2 = 1.0;
-                it.div = 1.0;
-            }
-            it.units = (int64_t)it.r_blk * it.r_inc * it.a_blk * it.a_inc;
-            evals += it.units * it.t_blk * it.t_inc;
-            items.push_back(it);
+    const int modes = (what & CCOIL_PAIR_M ? 1 : 0) + (what & CCOIL_PAIR_FT ? 1 : 0);
+    for (int64_t k = 0; k < n_pairs; ++k) {
+        const int64_t i = prim_index ? prim_index[k] : k, j = sec_index ? sec_index[k] : k;
+        if (i < 0 || i >= prim->n || j < 0 || j >= sec->n)
+            return fail(ctx, CCOIL_ERR_ARGUMENT, "pair " + std::to_string(k) + ": coil index out of range");
+        ZItemDev it;
+        std::memset(&it, 0, sizeof it);
+        it.out = (int32_t)k;
+        it.a_blk = prim->blocks ? prim->blocks[3 * i] : 1;
+        it.t_blk = prim->blocks ? prim->blocks[3 * i + 1] : 1;
+        it.r_blk = sec->blocks ? sec->blocks[3 * j + 1] : 1;
+        it.a_inc = (int16_t)prim->n_ang[i];
+        it.t_inc = (int16_t)prim->n_thk[i];
+        it.r_inc = (int16_t)sec->n_thk[j];
+        const double t_width = prim->a[i] / it.t_blk, a_width = kPi / it.a_blk, r_width = sec->a[j] / it.r_blk;
+        it.t_inner = prim->R[i];
+        it.t_width = t_width;
+        it.a_width = a_width;
+        it.r_inner = sec->R[j];
+        it.r_width = r_width;
+        it.constant = kMu * prim->J[i] * sec->J[j] * t_width * a_width * r_width * 0.125;
+        it.z = sec->pos[3 * j + 2] - prim->pos[3 * i + 2];
+        it.hs = sec->b[j] * 0.5;
+        it.hp = prim->b[i] * 0.5;
+        if (what & CCOIL_PAIR_M) {
+            if (prim->current[i] == 0.0 || sec->current[j] == 0.0)
+                return fail(ctx, CCOIL_ERR_ARGUMENT, "pair " + std::to_string(k) + ": mutual inductance needs "
+                                                     "non-zero currents (M = sum * 2 pi / (I1 I2))");
+            it.div = prim->current[i] * sec->current[j];
         }
+        evals += (int64_t)modes * it.r_blk * it.r_inc * it.a_blk * it.a_inc * it.t_blk * it.t_inc;
+        const PairRule rule = pair_rule(it.t_inner, prim->a[i], it.hp, it.r_inner, sec->a[j], it.hs, it.z, it.a_inc,
+                                        it.t_inc, it.r_inc);
+        const bool reduce = rule.na && it.r_blk <= 1 << 10;   // a reduced item's units are counted in 32 bits
+        if (reduce) reduce_item(it, rule);
+        set_units(it);
+        (reduce ? reduced : items).push_back(it);
     }
-    const size_t n_out = (size_t)n_pairs * 2;
-    // host results: M then Fz, staged in one device buffer of 2 n_pairs values
-    std::vector<double> host(n_out, 0.0);
+    items.insert(items.end(), reduced.begin(), reduced.end());
+    const int32_t mode = what & CCOIL_PAIR_M ? kZMutual : kZForce;
+    // results: M, then Fz, of what is asked for, staged in one device buffer
+    const size_t n_out = (size_t)n_pairs * (size_t)modes;
+    const size_t f_at = modes > 1 ? (size_t)n_pairs : 0;
     const bool dev = flags & CCOIL_DEVICE_POINTERS;
     if (dev) {
         // device outputs are written in place: route M and Fz through one staging buffer, then copy on device
         CC_HIP(ctx, ensure(ctx->zout, sizeof(double) * n_out));
-        ccoil_status st = run_items(ctx, items, n_out, flags, nullptr, (double *)ctx->zout.p, evals, report);
+        ccoil_status st = run_items(ctx, items, mode, modes, n_out, flags, nullptr, (double *)ctx->zout.p, evals, report);
         if (st != CCOIL_OK) return st;
         const size_t s1 = sizeof(double) * (size_t)n_pairs;
         if (what & CCOIL_PAIR_M) CC_HIP(ctx, hipMemcpyAsync(M, ctx->zout.p, s1, hipMemcpyDeviceToDevice, ctx->stream));
         if (what & CCOIL_PAIR_FT)
-            CC_HIP(ctx, hipMemcpyAsync(Fz, (double *)ctx->zout.p + n_pairs, s1, hipMemcpyDeviceToDevice, ctx->stream));
+            CC_HIP(ctx, hipMemcpyAsync(Fz, (double *)ctx->zout.p + f_at, s1, hipMemcpyDeviceToDevice, ctx->stream));
         CC_HIP(ctx, hipStreamSynchronize(ctx->stream));
         return CCOIL_OK;
     }
-    ccoil_status st = run_items(ctx, items, n_out, flags, host.data(), nullptr, evals, report);
+    std::vector<double> host(n_out);
+    ccoil_status st = run_items(ctx, items, mode, modes, n_out, flags, host.data(), nullptr, evals, report);
     if (st != CCOIL_OK) return st;
     if (what & CCOIL_PAIR_M) std::memcpy(M, host.data(), sizeof(double) * (size_t)n_pairs);
-    if (what & CCOIL_PAIR_FT) std::memcpy(Fz, host.data() + n_pairs, sizeof(double) * (size_t)n_pairs);
+    if (what & CCOIL_PAIR_FT) std::memcpy(Fz, host.data() + f_at, sizeof(double) * (size_t)n_pairs);
     return CCOIL_OK;
 }
 
@@ -195,14 +291,13 @@ extern "C" ccoil_status ccoil_self_inductance(ccoil_ctx ctx, const ccoil_coils *
                                                  "current (L = sum * 2 pi N / (I l))");
         ZItemDev it;
         std::memset(&it, 0, sizeof it);
-        it.mode = kZSelf;
         it.out = (int32_t)i;
         it.a_blk = coils->blocks ? coils->blocks[3 * i] : 1;
         it.t_blk = coils->blocks ? coils->blocks[3 * i + 1] : 1;
         it.r_blk = radial[2 * i];
-        it.a_inc = coils->n_ang[i];
-        it.t_inc = coils->n_thk[i];
-        it.r_inc = radial[2 * i + 1];
+        it.a_inc = (int16_t)coils->n_ang[i];
+        it.t_inc = (int16_t)coils->n_thk[i];
+        it.r_inc = (int16_t)radial[2 * i + 1];
         const double a = coils->a[i], len = coils->b[i];
         const double t_width = a / it.t_blk, a_width = kPi / it.a_blk, r_unit = 1.0 / it.r_blk;
         it.t_inner = coils->R[i];
@@ -211,14 +306,12 @@ extern "C" ccoil_status ccoil_self_inductance(ccoil_ctx ctx, const ccoil_coils *
         it.r_inner = coils->R[i];
         it.r_width = r_unit * a;   // the radial nodes span the thickness; the constant keeps the unit block
         it.constant = kMu * coils->J[i] * t_width * a_width * r_unit * 2 * 0.125;
-        it.z[0] = len;
-        it.zsq[0] = len * len;
-        it.mul = 2.0 * kPi;
-        it.mul2 = coils->turns[i];
+        it.z = len;
+        it.mul = coils->turns[i];
         it.div = coils->current[i] * len;
-        it.units = (int64_t)it.r_blk * it.r_inc * it.a_blk * it.a_inc;
-        evals += it.units * it.t_blk * it.t_inc;
+        evals += (int64_t)it.r_blk * it.r_inc * it.a_blk * it.a_inc * it.t_blk * it.t_inc;
+        set_units(it);
         items.push_back(it);
     }
-    return run_items(ctx, items, (size_t)coils->n, flags, L, L, evals, report);
+    return run_items(ctx, items, kZSelf, 1, (size_t)coils->n, flags, L, L, evals, report);
 }

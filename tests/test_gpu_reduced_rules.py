@@ -15,6 +15,7 @@ import numpy as np
 import pytest
 
 import ccoil_abi as abi
+import oracle as O
 import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -156,3 +157,38 @@ def test_adjoint_matches_the_own_rule(ctx, coil, n):
                                          np.array([row["current"], R, max(a, 1e-3 * R), max(row["b"], 1e-3 * R), R, R, R, 1, 1]))
     print(f"\n{coil} {len(pts)} points: {err.max():.2g}")
     assert err.max() <= 1e-10
+
+
+COAXIAL = [(0.1, 0.05, 0.12, 0.1, 0.03, 0.05), (0.05, 0.0, 0.2, 0.07, 0.04, 0.01), (0.2, 0.1, 0.02, 0.02, 0.0, 0.3),
+           (0.1, 0.01, 0.1, 0.12, 0.02, 0.1), (0.03, 0.02, 0.1, 0.2, 0.1, 0.1)]   # R, a, b of both
+
+
+@pytest.mark.parametrize("apart", [0, 1])
+@pytest.mark.parametrize("i", range(len(COAXIAL)))
+def test_coaxial_pairs(ctx, i, apart):
+    """M and axial force against the long double sum of the coils' own rules, single and of several blocks, at axial gaps
+    of a hundredth to thirty radii, and side by side (nested) at small offsets. The angular sum cancels to at most some
+    1/100 of its terms, the offsets keep the force off its zero at the middle: 1e-12 of the value. The oracle's long double
+    sum itself cancels from eight terms of up to z log(2 z / D) (force: of four logarithms), weights 2 t r: some 2^-60 of
+    20 |z| (20) times them."""
+    R, a, b, R2, a2, b2 = COAXIAL[i]
+    rows, orders, coils = ([], []), [], ([], [])
+    gaps = np.geomspace(0.01, 30.0, 24) * max(R, R2) + 0.5 * (b + b2) if apart else np.linspace(0.3, 0.9, 8) * max(b, b2)
+    for n, d in enumerate(gaps):
+        p = O.make_coil(R, a, b, 250, 3.0, pos=(0, 0, 0.1))
+        s = O.make_coil(R2, a2, b2, 100, -2.0, pos=(0, 0, 0.1 + (d if n % 2 else -d)))
+        blocks = 1 + n % 3 // 2
+        args = np.array([blocks, blocks if a else 1, 1, 80, 20 if a else 1, 20] + [1, blocks if a2 else 1, 1, 80, 20 if a2 else 1, 20])
+        orders.append(args)
+        for c, part, half in ((p, 0, args[:6]), (s, 1, args[6:])):
+            coils[part].append(c)
+            rows[part].append(dict(use_fast=int(c.use_fast), n_ang=int(half[3]), n_thk=int(half[4]), n_len=int(half[5]),
+                                   blocks=tuple(int(v) for v in half[:3]), R=c.R, a=c.a, b=c.b, J=c.J, current=c.I,
+                                   turns=float(c.N), frequency=c.freq, pos=tuple(c.pos), alpha=0.0, beta=0.0))
+    P, S = (abi.CoilSet.from_rows(r) for r in rows)
+    out, _ = ctx.pairs_zaxis(P, S, len(orders), abi.PAIR_M | abi.PAIR_FT)
+    for k, (p, s, args) in enumerate(zip(*coils, orders)):
+        m, f = O.mutual_inductance_zaxis_fast(p, s, args, True), O.force_zaxis_fast(p, s, args, True)
+        lost = 2.0 ** -60 * 20.0 * 2e-7 * np.pi ** 2 * abs(p.J * s.J) * p.a * s.a * (p.R + p.a) * (s.R + s.a)
+        assert abs(out["M"][k] - m) <= 1e-12 * abs(m) + lost * gaps[k] / abs(p.I * s.I), (k, gaps[k])
+        assert abs(out["Fz"][k] - f) <= 1e-12 * abs(f) + lost, (k, gaps[k])
