@@ -276,7 +276,7 @@ ccoil_status ccoil_create(int device, ccoil_ctx *out)
                        &ctx->gl_opc, &ctx->gl_ws, &ctx->gl_ws2, &ctx->gl_wcs};
     float **fp[7] = {&ctx->gl_xf, &ctx->gl_wf, &ctx->gl_cosf, &ctx->gl_omcf, &ctx->gl_wcosf, &ctx->gl_opcf,
                      &ctx->gl_wcsf};
-    // x and w also hold the series' length rule, w and the angular tables the reduced rules (kTableSizeAng)
+    // w and the angular tables also hold the reduced rules (kTableSizeAng)
     for (auto p : dp)
         if ((e = hipMalloc((void **)p, sizeof(double) * kTableSizeAng)) != hipSuccess)
             return bail(e, "hipMalloc(tables)");

@@ -8,11 +8,6 @@ namespace ccoil {
 
 constexpr int kMaxOrder = 100;                        // Legendre::maxLegendreOrder (LegendreMatrix.h:9)
 constexpr int kTableSize = kMaxOrder * (kMaxOrder + 1) / 2;
-// The far-field series' length nodes: a Gauss-Legendre rule of kSeriesLenNodes nodes (exact to degree 251), stored in
-// the x and w tables after the orders 1..kMaxOrder, at kSeriesLenOffset.
-constexpr int kSeriesLenNodes = 126;
-constexpr int kSeriesLenOffset = kTableSize;
-constexpr int kTableSizeXW = kTableSize + kSeriesLenNodes;
 
 // Reduced rules: the node sets that replace a rule's Gauss-Legendre angular or thickness sum where that sum has
 // converged to rounding (reduced_rules.cpp: the bounds, the tables and what they measured).
@@ -24,7 +19,7 @@ constexpr int kRedAng = 6;
 constexpr int kRedAngN[kRedAng] = {20, 16, 12, 10, 8, 6};
 constexpr double kRedEta[kRedAng] = {0.1, 0.3, 0.75, 1.0, 1.8, 3.2};
 constexpr int kRedNodes = 20 + 16 + 12 + 10 + 8 + 6;
-constexpr int kRedOffset = kTableSizeXW;
+constexpr int kRedOffset = kTableSize;
 constexpr int kTableSizeAng = kRedOffset + kRedNodes;   // the w, omc, wcos, opc, ws, ws2 and wcs tables
 // Thickness class t (1..kRedThk): the Gauss-Legendre rule of kRedThkN[t - 1] nodes, for points outside the ellipse with
 // foci at the winding's inner and outer radius whose parameter is (kRedThkC / kRedTol)^(1 / (2 n)). Class 0 is the
@@ -72,8 +67,8 @@ struct alignas(64) CoilDev {
     float r0f, r1f, hbf, ia2f;
 };
 
-// Gauss-Legendre tables for orders 1..100 at offset table_offset(n), generated in FP64 on the device (x and w also
-// hold the series' length rule at kSeriesLenOffset, and the double angular tables the reduced rules at kRedOffset).
+// Gauss-Legendre tables for orders 1..100 at offset table_offset(n), generated in FP64 on the device (w and the double
+// angular tables also hold the reduced rules at kRedOffset).
 struct Tables {
     const double *x;      // nodes, ascending
     const double *w;      // weights

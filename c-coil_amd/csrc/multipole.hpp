@@ -12,8 +12,9 @@
 //
 // The rings are the field rule's own: its thickness nodes (the rule's Gauss-Legendre nodes over [R, R + a], so the
 // series reproduces the rule's thickness sum exactly, whatever its order), and over the length either the exact
-// average (the fast rule integrates the length in closed form; 126 Gauss-Legendre nodes are exact for l <= 250) or
-// the mid-plane alone (the slow rule's flat sheet). What the series leaves out is then the angular rule's own error
+// average (the fast rule integrates the length in closed form; dV_(l+1)/dz0 = (l + 2) V_l, as for all solid harmonics,
+// so the average over |z0| <= h is V_(l+1)(h) / ((l + 2) h) for odd l) or the mid-plane alone (the slow rule's flat
+// sheet: the limit h = 0). What the series leaves out is then the angular rule's own error
 // and the truncation. With s = sin theta, u = 1 / D and q_l = (r_max / D)^(l+1), and the moments normalised as
 // m_l = mu0 M_l / r_max^(l+1):
 //   A_phi = s sum m_l q_l P'_l / l           B_z  = u sum (l + 1) m_l q_l P_(l+1)
@@ -33,12 +34,8 @@ constexpr int kMpTerms = 250;               // highest order l (below 256, the r
 constexpr int kMpStride = 256;              // doubles per coefficient array (index l), one per thread of a block
 constexpr int kMpCoil = 4 * kMpStride;      // per coil: m_l / l, m_l, (l + 1) m_l, (l + 1)(l + 2) m_l
 constexpr int kMpHeader = 3 * kMpStride;    // recurrence coefficients (2l + 5) / (l + 3), (l + 2) / (l + 3), 2l + 5
-constexpr int kMpLenNodes = kSeriesLenNodes; // Gauss-Legendre nodes over the length of a fast-rule coil: exact to
-                                             // degree 251, and V_l has degree l - 1 in the ring's height
 static_assert(kMpTerms < 256 && kMpTerms < kMpStride && kMpStride <= 256, "series orders and their arrays");
-static_assert(2 * kMpLenNodes - 1 >= kMpTerms - 1, "the length rule integrates V_l exactly");
-// Every coil's winding is symmetric about its mid-plane (the length rule's nodes come in pairs +-z0, a slow-rule
-// coil is a mid-plane sheet), so its moments of even order are zero: multipole_moments_kernel writes them as exact
+// Every coil's winding is symmetric about its mid-plane (a slow-rule coil is a mid-plane sheet), so its moments of even order are zero: multipole_moments_kernel writes them as exact
 // zeros, and the series loops add only the odd orders.
 constexpr bool kMpEvenZero = true;
 

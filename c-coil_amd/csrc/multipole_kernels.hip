@@ -1,7 +1,7 @@
 // Far-field moments of the coils and the spatial visit order of the points (gfx950).
 //
-// multipole_moments_kernel: one workgroup per coil sums the zonal-harmonic moments of the coil's rings (the field
-// rule's thickness nodes times the length nodes, multipole.hpp) in FP64, with a fixed reduction order.
+// multipole_moments_kernel: one workgroup per coil sums the zonal-harmonic moments of the coil's sheets (the field
+// rule's thickness nodes, their length in closed form, multipole.hpp) in FP64, with a fixed reduction order.
 //
 // The visit order: the points' bounding box, a cell of a 2^k x 2^k x 2^k grid for every point (Morton order of the
 // cells), a counting sort of the point indices by cell. field_kernel reads its points in that order, so the 64
@@ -13,115 +13,79 @@
 
 namespace ccoil {
 
-constexpr int kMpChunks = kMpStride / 64;   // blocks of 64 orders per coil
-constexpr int kMomThreads = 512;            // threads of a moments block (8 waves; at most 2 per SIMD by registers)
-constexpr int kMomWaves = kMomThreads / 64;
-static_assert(kMpChunks == 4, "multipole_moments_kernel dispatches four chunks");
+constexpr int kMomThreads = 128;   // one sheet a thread
+constexpr int kMomOrders = 32;     // odd orders summed at a time
+constexpr int kMomStride = kMaxOrder + 1;   // odd, so that a column of orders crosses the LDS banks
+static_assert(kMaxOrder <= kMomThreads && kMomStride % 2 == 1 && kMpStride % (2 * kMomOrders) == 0, "moments block");
 
-__device__ inline double wave_sum(double v)
-{
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-    return v;
-}
-
-// Adds w V_l of one ring (radius^2 c2, height z0, both in units of r_max) to acc[l - L0] for the orders l of the
-// chunk [L0, L0 + 64) up to kMpTerms. The recurrence runs from l = 1 with compile-time indices, so acc stays in
-// registers (each chunk repeats the recurrence below it).
-template <int L0>
-__device__ inline void ring_moments(double w, double z0, double c2, double *acc)
-{
-    constexpr int kEnd = L0 + 64 < kMpTerms + 1 ? L0 + 64 : kMpTerms + 1;   // orders below kEnd
-    double Um = 1.0, U = z0;     // U_(l-1), U_l
-    double Vm = 0.0, V = 1.0;    // V_(l-1), V_l
-    if constexpr (L0 <= 1) acc[1 - L0] += w;
-#pragma unroll
-    for (int l = 1; l + 1 < kEnd; ++l) {
-        const double Un = ((2.0 * l + 1.0) * z0 * U - l * c2 * Um) * (1.0 / (l + 1.0));
-        const double Vn = c2 * Vm + (2.0 * l + 1.0) * U;
-        Um = U;
-        U = Un;
-        Vm = V;
-        V = Vn;
-        if (l + 1 >= L0) acc[l + 1 - L0] += w * V;
-    }
-}
-
-// The moments of orders [L0, L0 + 64) of coil c into out (a block of kMomThreads threads over the coil's rings).
-// The length rule is symmetric about the mid-plane and V_l(rho, -z0) = (-1)^(l-1) V_l(rho, z0) (every operation of
-// the recurrence flips sign exactly with z0), so a node pair adds 2 V_l for odd l and exactly nothing for even l:
-// the rings take the nodes z0 > 0 at twice their weight, and the even orders of a coil with a length rule are zero.
-// (A slow-rule coil's mid-plane ring has V_l = 0 for even l by itself.)
-template <int L0>
-__device__ inline void chunk_moments(const CoilDev &c, const Tables &tab, double *out, double (*part)[64])
-{
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const double inv = 1.0 / c.rmax;
-    static_assert(kMpLenNodes % 2 == 0, "the length rule's nodes come in pairs +-z0");
-    const int nt = c.n_thk, nz = c.use_fast ? kMpLenNodes / 2 : 1;
-    const double *xt = tab.x + table_offset(nt), *wt = tab.w + table_offset(nt);
-    // the upper half of the ascending length nodes: z0 > 0
-    const double *xz = tab.x + kSeriesLenOffset + kMpLenNodes / 2, *wz = tab.w + kSeriesLenOffset + kMpLenNodes / 2;
-    double acc[64];
-#pragma unroll
-    for (int l = 0; l < 64; ++l) acc[l] = 0.0;
-    for (int k = t; k < nt * nz; k += kMomThreads) {
-        const int j = k / nz, i = k - j * nz;
-        // ring (rho, z0) in units of r_max, weight: its share of the current (the weights sum to 1)
-        const double rho = (c.R + 0.5 * c.a * (1.0 + xt[j])) * inv;
-        const double z0 = nz > 1 ? 0.5 * c.b * xz[i] * inv : 0.0;
-        const double w = 0.5 * wt[j] * (nz > 1 ? wz[i] : 1.0) * rho * rho;   // 2 x (1/2) wz for the node pair
-        ring_moments<L0>(w, z0, rho * rho + z0 * z0, acc);
-    }
-#pragma unroll
-    for (int l = 0; l < 64; ++l) {
-        const double v = wave_sum(acc[l]);
-        if (lane == 0) part[wave][l] = v;
-    }
-    __syncthreads();
-    // m_l = mu0 N I sum / (2 (l + 1)), mu0 = 4 pi 1e-7
-    const double ni = c.ni * (4.0 * kPi * kMuReduced);
-    if (t < 64 && L0 + t < kMpStride) {
-        const int l = L0 + t;
-        double m = 0.0;
-        if (l >= 1 && l <= kMpTerms && (l % 2 == 1 || !c.use_fast)) {
-            const double s = ((part[0][t] + part[1][t]) + (part[2][t] + part[3][t])) +
-                             ((part[4][t] + part[5][t]) + (part[6][t] + part[7][t]));
-            m = ni * s / (2.0 * (l + 1));
-        }
-        out[l] = l >= 1 ? m / l : 0.0;
-        out[kMpStride + l] = m;
-        out[2 * kMpStride + l] = (l + 1) * m;
-        out[3 * kMpStride + l] = (l + 1.0) * (l + 2.0) * m;
-    }
-    __syncthreads();
-}
-
-// Grid (coils, kMpChunks): block (c, k) sums the orders [64 k, 64 k + 64) of coil c, or zeroes them when the call's
-// series of that coil stops below them (mp_terms).
+// Moments of coil blockIdx.x. Thread j steps the recurrences of the sheet at thickness node j (squared half-length z2,
+// c2 = rho^2 + z2, in units of r_max) over 32 odd orders, then four threads an order add the sheets. With U_l, V_l of
+// multipole.hpp at height h, E_l = U_l (even l), O_l = U_l / h and G_(l+1) = V_(l+1) / h (odd l) contain no odd power
+// of h, so that a flat sheet (h = 0, also a slow-rule coil's) needs no case of its own; the length average of V_l is
+// G_(l+1) / (l + 2). Bound by the recurrence's latency, some 25 cycles an order; 63 length nodes for each thickness
+// node, summed over the wave at every order, took 90 us for 128 coils and 1.96 ms for 8,192, this 13 and 50 us.
 __global__ __launch_bounds__(kMomThreads) void multipole_moments_kernel(const CoilDev *coils, Tables tab, double *mp)
 {
-    static_assert(kMomWaves == 8, "chunk_moments sums eight wave partials");
-    __shared__ double part[kMomWaves][64];
-    const int ci = blockIdx.x, chunk = blockIdx.y, t = threadIdx.x;
-    if (ci == 0 && chunk == 0 && t < kMpStride) {   // recurrence coefficients of the Legendre polynomials
-        mp[t] = (2.0 * t + 5.0) / (t + 3.0);
-        mp[kMpStride + t] = (t + 2.0) / (t + 3.0);
-        mp[2 * kMpStride + t] = 2.0 * t + 5.0;
-    }
+    __shared__ double inv[kMpStride + 1];                 // 1 / l
+    __shared__ double term[kMomOrders][kMomStride];       // per order and sheet
+    __shared__ double part[4][kMomOrders];
+    const int ci = blockIdx.x, t = threadIdx.x;
+    if (ci == 0)
+        for (int l = t; l < kMpStride; l += kMomThreads) {   // recurrence coefficients of the Legendre polynomials
+            mp[l] = (2.0 * l + 5.0) / (l + 3.0);
+            mp[kMpStride + l] = (l + 2.0) / (l + 3.0);
+            mp[2 * kMpStride + l] = 2.0 * l + 5.0;
+        }
     const CoilDev &c = coils[ci];
     double *out = mp + kMpHeader + (size_t)ci * kMpCoil;
-    const int l0 = 64 * chunk;
-    if (!(c.far_d2 > 0.0) || (chunk > 0 && c.mp_terms < l0)) {   // no series, or none of these orders
-        const int l = l0 + t;
-        if (t < 64 && l < kMpStride)
-            for (int k = 0; k < 4; ++k) out[k * kMpStride + l] = 0.0;
-        return;
+    for (int l = t; l <= kMpStride; l += kMomThreads) inv[l] = l > 0 ? 1.0 / l : 0.0;
+    const int nt = c.n_thk, terms = c.far_d2 > 0.0 ? (c.mp_terms < kMpTerms ? c.mp_terms : kMpTerms) : 0;
+    const double scale = 1.0 / c.rmax, h = c.use_fast ? 0.5 * c.b * scale : 0.0, z2 = h * h;
+    double c2 = 0.0, w = 0.0;
+    if (t < nt) {
+        const double *xt = tab.x + table_offset(nt), *wt = tab.w + table_offset(nt);
+        const double rho = (c.R + 0.5 * c.a * (1.0 + xt[t])) * scale;
+        c2 = rho * rho + z2;
+        w = 0.5 * wt[t] * rho * rho;   // its share of the current (the weights sum to 1), times rho^2
     }
-    if (chunk == 0) chunk_moments<0>(c, tab, out, part);
-    else if (chunk == 1) chunk_moments<64>(c, tab, out, part);
-    else if (chunk == 2) chunk_moments<128>(c, tab, out, part);
-    else chunk_moments<192>(c, tab, out, part);
+    double E = 1.0, O = 1.0, G = 3.0;   // E_(l-1), O_l, G_(l+1) at l = 1
+    const double ni = c.ni * (4.0 * kPi * kMuReduced);   // m_l = mu0 N I sum / (2 (l + 1)), mu0 = 4 pi 1e-7
+    __syncthreads();
+    for (int l0 = 0; l0 < kMpStride; l0 += 2 * kMomOrders) {
+        if (l0 >= terms) {   // no series, or none of these orders
+            for (int k = t; k < 8 * kMomOrders; k += kMomThreads)
+                out[(k / (2 * kMomOrders)) * kMpStride + l0 + k % (2 * kMomOrders)] = 0.0;
+            continue;
+        }
+        if (t < nt)
+#pragma unroll 4
+            for (int i = 0; i < kMomOrders; ++i) {
+                const int l = l0 + 2 * i + 1;
+                const double fl = l;
+                term[i][t] = w * G;
+                E = ((2.0 * fl + 1.0) * z2 * O - fl * c2 * E) * inv[l + 1];
+                O = ((2.0 * fl + 3.0) * E - (fl + 1.0) * c2 * O) * inv[l + 2 <= kMpStride ? l + 2 : 0];
+                G = c2 * G + (2.0 * fl + 5.0) * O;
+            }
+        __syncthreads();
+        const int i = t % kMomOrders, q = t / kMomOrders;
+        double sum = 0.0;
+#pragma unroll 4
+        for (int j = q; j < nt; j += 4) sum += term[i][j];
+        part[q][i] = sum;
+        __syncthreads();
+        if (t < 2 * kMomOrders) {
+            // the moments of even order are zero: V_l(rho, -z0) = (-1)^(l-1) V_l(rho, z0)
+            const int l = l0 + t, k = t / 2;
+            double m = 0.0;
+            if (t % 2 == 1 && l <= kMpTerms)
+                m = ni * (((part[0][k] + part[1][k]) + (part[2][k] + part[3][k])) * inv[l + 2]) / (2.0 * (l + 1));
+            out[l] = l >= 1 ? m / l : 0.0;
+            out[kMpStride + l] = m;
+            out[2 * kMpStride + l] = (l + 1) * m;
+            out[3 * kMpStride + l] = (l + 1.0) * (l + 2.0) * m;
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -218,8 +182,7 @@ __global__ __launch_bounds__(256) void cell_place_kernel(const uint32_t *cell, i
 void launch_multipole_moments(hipStream_t s, const CoilDev *coils, int n_coils, const Tables &tab, double *mp)
 {
     if (n_coils > 0)
-        hipLaunchKernelGGL(multipole_moments_kernel, dim3(n_coils, kMpChunks), dim3(kMomThreads), 0, s, coils, tab,
-                           mp);
+        hipLaunchKernelGGL(multipole_moments_kernel, dim3(n_coils), dim3(kMomThreads), 0, s, coils, tab, mp);
 }
 
 size_t visit_order_bytes(int64_t n, int bits, size_t scan_bytes)

@@ -84,6 +84,33 @@ def test_records_match_the_own_rule(ctx, coil, n):
     print(f"\n{coil} n={n}: worst error over tolerance {check(ctx, _row(*coil), n, abi.FP64, abi.FAR_FIELD, 5)}")
 
 
+LONG = [("RECTANGULAR", 0.02, 0.01, 0.6, 80, 20), ("THIN", 0.02, 0.0, 1.0, 100, 1), ("FLAT", 0.01, 0.3, 0.0, 100, 100),
+        ("RECTANGULAR", 0.1, 0.05, 1e-4, 80, 2), ("RECTANGULAR", 0.3, 0.3, 0.3, 100, 100)]
+
+
+@pytest.mark.parametrize("coil", LONG, ids=lambda c: f"{c[0]}-{c[2]}x{c[3]}")
+def test_series_matches_the_own_rule(ctx, coil):
+    """The series' moments of sheets from none to 99 % of r_max in half-length, 1 to 100 sheets, few orders to all: on
+    shells of 1.3 to 40 r_max, relative to the field's largest value on the shell, the series' 1e-13 with the own rule's
+    rounding of terms that cancel with the distance in radii."""
+    row = _row(*coil)
+    rng = np.random.default_rng(13)
+    y = np.repeat(np.array([1.3, 1.6, 2.0, 3.0, 5.0, 12.0, 40.0]), 300)
+    d = rng.normal(size=(y.size, 3))
+    rmax = np.hypot(row["R"] + row["a"], 0.5 * row["b"])
+    D = y * rmax
+    pts = np.asarray(row["pos"]) + d / np.linalg.norm(d, axis=1)[:, None] * D[:, None]
+    cs = abi.CoilSet.from_rows([row])
+    ref, _ = ctx.fields(cs, pts, abi.A | abi.B | abi.G, abi.FP64_IEEE)
+    got, _ = ctx.fields(cs, pts, abi.A | abi.B | abi.G, abi.FP64, abi.FAR_FIELD)
+    for k, ulps in (("A", 2e-14), ("B", 2e-14), ("G", 2e-13)):
+        err, ref_k = np.linalg.norm(got[k] - ref[k], axis=1), np.linalg.norm(ref[k], axis=1)
+        for v in np.unique(y):
+            s = y == v
+            tol = 1e-13 + ulps * (1.0 + v * rmax / (row["R"] + row["a"])) ** 2
+            assert np.max(err[s]) <= tol * np.max(ref_k[s]), (k, v, np.max(err[s]) / np.max(ref_k[s]), tol)
+
+
 @pytest.mark.parametrize("n,split", [(300, 16), (600, 64), (5000, 16), (20000, 4), (70000, 1)])
 @pytest.mark.parametrize("coil", COILS, ids=lambda c: f"{c[0]}-{c[4]}x{c[5]}")
 def test_field_kernel_matches_the_own_rule(ctx, coil, n, split):
