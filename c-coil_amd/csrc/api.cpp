@@ -226,6 +226,7 @@ Tables ctx_tables(ccoil_ctx ctx)
     t.ws = ctx->gl_ws;
     t.ws2 = ctx->gl_ws2;
     t.wcs = ctx->gl_wcs;
+    t.leg = ctx->gl_leg;
     t.wcsf = ctx->gl_wcsf;
     t.rsin = ctx->gl_rsin;
     return t;
@@ -272,8 +273,8 @@ ccoil_status ccoil_create(int device, ccoil_ctx *out)
     if ((e = scratch_address(device, &ctx->scratch)) != hipSuccess) return bail(e, "hipGetSymbolAddress(scratch)");
     if (const char *tf = std::getenv("CCOIL_TUNING_FILE")) load_tuning_file(ctx, tf);
     const size_t nf = sizeof(float) * kTableSize;
-    double **dp[11] = {&ctx->gl_x, &ctx->gl_w, &ctx->gl_cos, &ctx->gl_omc, &ctx->gl_rcos, &ctx->gl_rsin, &ctx->gl_wcos,
-                       &ctx->gl_opc, &ctx->gl_ws, &ctx->gl_ws2, &ctx->gl_wcs};
+    double **dp[12] = {&ctx->gl_x, &ctx->gl_w, &ctx->gl_cos, &ctx->gl_omc, &ctx->gl_rcos, &ctx->gl_rsin, &ctx->gl_wcos,
+                       &ctx->gl_opc, &ctx->gl_ws, &ctx->gl_ws2, &ctx->gl_wcs, &ctx->gl_leg};
     float **fp[7] = {&ctx->gl_xf, &ctx->gl_wf, &ctx->gl_cosf, &ctx->gl_omcf, &ctx->gl_wcosf, &ctx->gl_opcf,
                      &ctx->gl_wcsf};
     // w and the angular tables also hold the reduced rules (kTableSizeAng)
@@ -297,6 +298,10 @@ ccoil_status ccoil_create(int device, ccoil_ctx *out)
         if ((e = hipMemcpyAsync(t.first + kRedOffset, t.second, sizeof(double) * kRedNodes, hipMemcpyHostToDevice,
                                 ctx->stream)) != hipSuccess)
             return bail(e, "hipMemcpy(reduced rules)");
+    const std::vector<double> leg = legendre_rows();
+    if ((e = hipMemcpyAsync(ctx->gl_leg, leg.data(), sizeof(double) * leg.size(), hipMemcpyHostToDevice, ctx->stream)) !=
+        hipSuccess)
+        return bail(e, "hipMemcpy(legendre_rows)");
     if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return bail(e, "gl_table_kernel");
     *out = ctx;
     return CCOIL_OK;
@@ -307,8 +312,8 @@ ccoil_status ccoil_destroy(ccoil_ctx ctx)
     if (!ctx) return CCOIL_OK;
     (void)hipSetDevice(ctx->device);
     if (ctx->own_stream) (void)hipStreamSynchronize(ctx->own_stream);
-    double *dp[11] = {ctx->gl_x, ctx->gl_w, ctx->gl_cos, ctx->gl_omc, ctx->gl_rcos, ctx->gl_rsin, ctx->gl_wcos,
-                      ctx->gl_opc, ctx->gl_ws, ctx->gl_ws2, ctx->gl_wcs};
+    double *dp[12] = {ctx->gl_x, ctx->gl_w, ctx->gl_cos, ctx->gl_omc, ctx->gl_rcos, ctx->gl_rsin, ctx->gl_wcos,
+                      ctx->gl_opc, ctx->gl_ws, ctx->gl_ws2, ctx->gl_wcs, ctx->gl_leg};
     float *fp[7] = {ctx->gl_xf, ctx->gl_wf, ctx->gl_cosf, ctx->gl_omcf, ctx->gl_wcosf, ctx->gl_opcf, ctx->gl_wcsf};
     for (auto p : dp)
         if (p) (void)hipFree(p);

@@ -88,6 +88,7 @@ struct Tables {
     const double *ws2;    // w (1 - cos)^2
     const double *wcs;    // w cos (1 - cos)
     const float *wcsf;
+    const double *leg;    // the far-field series' Legendre coefficients (multipole.hpp)
 };
 
 // Quantity bits (mirror of the C ABI enum).
@@ -155,50 +156,46 @@ __device__ inline void to_local(const CoilDev &c, double px, double py, double p
 }
 
 // Local cylindrical -> global Cartesian, accumulated into out (CalculateFieldsMethods.cxx:16-19,
-// :33-36, :58-83; FieldGGroup.cu:134-174 for the GPU on-axis threshold).
+// :33-36, :58-83; FieldGGroup.cu:134-174 for the GPU on-axis threshold). With the radial unit vector e = (cph, sph, 0),
+// the axis z and E = T e, n = T z, the local gradient is (RR - RP) e e^T + RP (I - z z^T) + RZ (e z^T + z e^T) + ZZ z z^T:
+// its product with T needs E, n and one more vector, 31 operations where the two matrix products took 53.
 __device__ inline void accumulate_global(const CoilDev &c, const Local &L, double r, double cph, double sph,
                                          uint32_t q, Cart &out)
 {
+    const double *T = c.T;
     if (q & (Q_A | Q_E)) {
-        double v[3] = {-L.A * sph, L.A * cph, 0.0}, g[3];
-        mat_vec(c.T, v, g);
-        if (q & Q_A)
-            for (int k = 0; k < 3; ++k) out.A[k] += g[k];
-        if (q & Q_E)
-            for (int k = 0; k < 3; ++k) out.E[k] += c.omega * g[k];
-    }
-    if (q & Q_B) {
-        double v[3] = {L.Bh * cph, L.Bh * sph, L.Bz}, g[3];
-        mat_vec(c.T, v, g);
-        for (int k = 0; k < 3; ++k) out.B[k] += g[k];
-    }
-    if (q & (Q_G | Q_GJ)) {
-        double g[9];
-        if (r <= kGpuAxisRatio * c.R) {   // r / R <= 1e-5 without the division
-            g[0] = L.RR; g[1] = 0.0; g[2] = 0.0;
-            g[3] = 0.0; g[4] = L.RR; g[5] = 0.0;
-            g[6] = 0.0; g[7] = 0.0; g[8] = L.ZZ;
-        } else {
-            double xx = L.RR * cph * cph + L.RP * sph * sph;
-            double yy = L.RR * sph * sph + L.RP * cph * cph;
-            double xy = cph * sph * (L.RR - L.RP);   // 0.5 sin(2 phi) (RR - RP)
-            double xz = L.RZ * cph, yz = L.RZ * sph;
-            g[0] = xx; g[1] = xy; g[2] = xz;
-            g[3] = xy; g[4] = yy; g[5] = yz;
-            g[6] = xz; g[7] = yz; g[8] = L.ZZ;
+        const double ac = L.A * cph, as = L.A * sph;
+        for (int k = 0; k < 3; ++k) {
+            const double g = T[3 * k + 1] * ac - T[3 * k] * as;
+            if (q & Q_A) out.A[k] += g;
+            if (q & Q_E) out.E[k] += c.omega * g;
         }
-        double tg[9];
-        for (int i = 0; i < 3; ++i)
-            for (int j = 0; j < 3; ++j)
-                tg[3 * i + j] = c.T[3 * i] * g[j] + c.T[3 * i + 1] * g[3 + j] + c.T[3 * i + 2] * g[6 + j];
+    }
+    if (!(q & (Q_B | Q_G | Q_GJ))) return;
+    double E[3];
+    for (int k = 0; k < 3; ++k) E[k] = T[3 * k] * cph + T[3 * k + 1] * sph;
+    if (q & Q_B)
+        for (int k = 0; k < 3; ++k) out.B[k] += L.Bh * E[k] + L.Bz * T[3 * k + 2];
+    if (q & (Q_G | Q_GJ)) {
+        const bool axis = r <= kGpuAxisRatio * c.R;   // r / R <= 1e-5 without the division: diag(RR, RR, ZZ)
+        const double RP = axis ? L.RR : L.RP, RZ = axis ? 0.0 : L.RZ, d = axis ? 0.0 : L.RR - L.RP;
+        double w[3], v[3];   // T G = w e^T + RP T (I - z z^T) + v z^T
+        for (int k = 0; k < 3; ++k) {
+            w[k] = d * E[k] + RZ * T[3 * k + 2];
+            v[k] = RZ * E[k] + L.ZZ * T[3 * k + 2];
+        }
         if (q & Q_GJ) {
             // (T G) T^T
             for (int i = 0; i < 3; ++i)
                 for (int j = 0; j < 3; ++j)
-                    out.G[3 * i + j] += tg[3 * i] * c.T[3 * j] + tg[3 * i + 1] * c.T[3 * j + 1] +
-                                        tg[3 * i + 2] * c.T[3 * j + 2];
+                    out.G[3 * i + j] += w[i] * E[j] + v[i] * T[3 * j + 2] +
+                                        RP * (T[3 * i] * T[3 * j] + T[3 * i + 1] * T[3 * j + 1]);
         } else {
-            for (int k = 0; k < 9; ++k) out.G[k] += tg[k];
+            for (int k = 0; k < 3; ++k) {
+                out.G[3 * k] += w[k] * cph + RP * T[3 * k];
+                out.G[3 * k + 1] += w[k] * sph + RP * T[3 * k + 1];
+                out.G[3 * k + 2] += v[k];
+            }
         }
     }
 }

@@ -61,6 +61,7 @@ struct ccoil_ctx_s {
     double *gl_rcos = nullptr, *gl_rsin = nullptr, *gl_wcos = nullptr;
     float *gl_wcosf = nullptr;
     double *gl_opc = nullptr, *gl_ws = nullptr, *gl_ws2 = nullptr, *gl_wcs = nullptr;
+    double *gl_leg = nullptr;
     float *gl_opcf = nullptr, *gl_wcsf = nullptr;
     ccoil::DevBuf coils, pts, outA, outB, outE, outG, fpartial;
     ccoil::DevBuf ncounts, noffsets, nhist, nstate, nkeys, nrecs, nvals, ntemp;   // FP32C near-winding pass
@@ -132,6 +133,7 @@ struct RedTables {
     double w[kRedNodes], omc[kRedNodes], opc[kRedNodes], wcos[kRedNodes], ws[kRedNodes], ws2[kRedNodes], wcs[kRedNodes];
 };
 void reduced_tables(RedTables &t);
+std::vector<double> legendre_rows();   // Tables::leg
 // Nodes of the rule class that serves every point at least dist from the coil's centre (the coil's own rule within the
 // sphere that holds its winding).
 int64_t rule_nodes_beyond(const CoilDev &c, double dist);

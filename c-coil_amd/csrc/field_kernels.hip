@@ -195,7 +195,7 @@ void field_kernel(FieldParams p)
                                                       PREC == kFP64 ? kMpLogTolFP64 : kMpLogTolFP32C) : 0;
                 const int terms = wave_max_small(own), lo = wave_min_small(own, far);
                 if (far && lane == 0)
-                    eval_multipole<WA, WB, WG>(p.mp + kMpHeader + (size_t)ci * kMpCoil, p.mp, c.rmax, z, r, terms,
+                    eval_multipole<WA, WB, WG>(p.mp + (size_t)ci * kMpCoil, p.tab.leg, c.rmax, z, r, terms,
                                                lo, own, L);
             }
         }
@@ -275,7 +275,7 @@ void field_series_kernel(FieldParams p)
             const int terms = wave_max_small(own), lo = wave_min_small(own, far);
             if (far) {
                 Local L;
-                eval_multipole<WA, WB, WG>(p.mp + kMpHeader + (size_t)ci * kMpCoil, p.mp, c.rmax, z, r, terms, lo,
+                eval_multipole<WA, WB, WG>(p.mp + (size_t)ci * kMpCoil, p.tab.leg, c.rmax, z, r, terms, lo,
                                            own, L);
                 accumulate_global(c, L, r, cph, sph, p.q, acc);
             }

@@ -339,7 +339,7 @@ ccoil_status fields_prepare(ccoil_ctx ctx, const ccoil_coils *coils, const doubl
         p.partial = (double *)partial;
     }
     if (far) {   // the series' moments
-        const size_t mb = sizeof(double) * ((size_t)kMpHeader + (size_t)kMpCoil * hc.size());
+        const size_t mb = sizeof(double) * (size_t)kMpCoil * hc.size();
         L.far_bytes = mb + 256;
         void *mp = nullptr;
         st = call_buffer(ctx, ctx->fmp, arena, mb, &mp);

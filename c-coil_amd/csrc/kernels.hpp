@@ -35,8 +35,7 @@ struct FieldParams {
     int32_t float_records;
     int32_t n_slots;       // key slots of a coil's FP64 records: kRuleClasses, 4 or 2 (record_slot)
     int32_t n_keys;
-    // FP32C far field: the recurrence header and each coil's moments (kMpHeader + n_coils * kMpCoil doubles,
-    // multipole.hpp); a coil with CoilDev::far_d2 > 0 takes its series beyond that distance. NULL: no coil does.
+    // FP32C far field: each coil's moments (n_coils * kMpCoil doubles, multipole.hpp); a coil with CoilDev::far_d2 > 0 takes its series beyond that distance. NULL: no coil does.
     const double *mp;
     // The order the points are visited in (a spatial sort, so the points of a wave lie close together and a wave
     // mostly takes one branch per coil); NULL: index order. No result depends on it.

@@ -30,14 +30,24 @@
 
 namespace ccoil {
 
+//
+// The loops hold P_n as the monic polynomial p_n = P_n / k_n, k_n = (2n)! / (2^n n!^2), whose recurrence p_(n+1) =
+// c p_n - n^2 / (4n^2 - 1) p_(n-1) has one coefficient, with k_n in the moments and in P'_(n+1) = P'_(n-1) + (2n + 1)
+// k_n p_n. The moments of even order are zero, so a term holds one odd order l: q_l steps by (r_max / D)^2, and the
+// eight numbers a term takes lie in two rows of 32 bytes, of the coil and of all coils, for two scalar loads a term.
+// Bound by FP64 issue (70 % of it) with 15 instructions a term for B and gradient and some 190 around the loop; with 17
+// instructions, and loads from seven arrays that the loop waited for five times in two terms, 128 coils x 2^20 points
+// took 2.39 ms, this 2.00 (loads a term ahead, held there by scheduling barriers: the same).
 constexpr int kMpTerms = 250;               // highest order l (below 256, the range of wave_max_small)
-constexpr int kMpStride = 256;              // doubles per coefficient array (index l), one per thread of a block
-constexpr int kMpCoil = 4 * kMpStride;      // per coil: m_l / l, m_l, (l + 1) m_l, (l + 1)(l + 2) m_l
-constexpr int kMpHeader = 3 * kMpStride;    // recurrence coefficients (2l + 5) / (l + 3), (l + 2) / (l + 3), 2l + 5
-static_assert(kMpTerms < 256 && kMpTerms < kMpStride && kMpStride <= 256, "series orders and their arrays");
-// Every coil's winding is symmetric about its mid-plane (a slow-rule coil is a mid-plane sheet), so its moments of even order are zero: multipole_moments_kernel writes them as exact
-// zeros, and the series loops add only the odd orders.
-constexpr bool kMpEvenZero = true;
+constexpr int kMpOdd = 128;                 // odd orders l = 2 i + 1 of the tables (a row more than is summed)
+// Per coil: rows of m_l, (l + 1) m_l k_(l+1), (l + 1)(l + 2) m_l k_(l+2), (l + 1) m_l; then m_l / l.
+constexpr int kMpCoil = 5 * kMpOdd;
+// Tables::leg: rows of n^2 / (4n^2 - 1) and (2n + 1) k_n at n = l + 2 and at n = l + 3; then k_n, n < kMpLegK.
+constexpr int kMpLegK = 2 * kMpOdd + 2;
+static_assert(kMpTerms < 256 && kMpTerms + 2 < 2 * kMpOdd, "series orders and their arrays");
+static_assert(4 * kMpOdd + kMpLegK <= kTableSizeAng, "Tables::leg is allocated with the angular tables");
+// Every coil's winding is symmetric about its mid-plane (a slow-rule coil is a mid-plane sheet), so its moments of even
+// order are zero and have no place in the tables.
 
 // Number of terms for a point at distance D from a coil whose winding lies within r_max: the truncation falls like
 // (r_max / D)^L with a constant below 2, so L = ln(2 / tol) / ln(D / r_max), between 4 and kMpTerms; log_tol =
@@ -47,8 +57,9 @@ constexpr float kMpLogTolFP64 = 35.2319f;
 constexpr float kMpLogTolFP32C = 30.6267f;
 __device__ inline int multipole_terms(double D2, double inv_rmax2, float log_tol)
 {
-    const float lg = __logf((float)(D2 * inv_rmax2));   // 2 ln(D / r_max) > 2 ln 1.17
-    const int L = (int)(2.0f * log_tol * __builtin_amdgcn_rcpf(lg)) + 2;
+    // D^2 / r_max^2 > 1.17^2, a normal number: the bare logarithm (base 2) and reciprocal serve
+    const float lg = __builtin_amdgcn_logf((float)(D2 * inv_rmax2));
+    const int L = (int)(2.0f / 0.69314718f * log_tol * __builtin_amdgcn_rcpf(lg)) + 2;
     return L < 4 ? 4 : (L > kMpTerms ? kMpTerms : L);
 }
 
@@ -61,124 +72,113 @@ __device__ inline int wave_min_small(int v, bool active)
     return 255 - wave_max_small(active ? 255 - v : 0);
 }
 
-// Local (A_phi, B_rho, B_z, B_rho / r, dB_rho/drho, dB_rho/dz, dB_z/dz) of one coil at local (z, r) from its series
-// (mp: the coil's kMpCoil doubles, rec: the shared recurrence coefficients, rmax: the coil's r_max): the loop runs L
-// terms (wave-uniform), and terms beyond own add exact zeros, so the value is that of own terms. The first lo terms
-// (the least own count among the lanes that call; wave-uniform) need no such test.
+// The rows of a term: mp, leg at the term's, ma at its m_l / l.
+template <bool WA, bool WB>
+struct MpTerm {
+    double m, zk, zzk, mz, a, b0, k0, b1, k1;
+    __device__ inline void load(const double *mp, const double *ma, const double *leg)
+    {
+        if (WA) a = ma[0];
+        if (WB) {
+            m = mp[0];
+            zk = mp[1];
+            zzk = mp[2];
+            mz = mp[3];
+        }
+        b0 = leg[0];
+        k0 = leg[1];
+        b1 = leg[2];
+        k1 = leg[3];
+    }
+};
+
+// The series' sums at one point: SA = sum m_l q_l P'_l / l, SZ = sum (l + 1) m_l q_l P_(l+1), SB = sum m_l q_l P'_(l+1),
+// SZZ = sum (l + 1)(l + 2) m_l q_l P_(l+2), SRZ = sum (l + 1) m_l q_l P'_(l+2); c = cos theta, qr = r_max / D. The loop
+// runs L terms (wave-uniform), and terms beyond own add exact zeros, so the value is that of own terms. The first lo
+// terms (the least own count among the lanes that call; wave-uniform) need no such test.
+struct MpSums { double A, Z, B, ZZ, RZ; };
 template <bool WA, bool WB, bool WG>
-__device__ inline void eval_multipole(const double *mp, const double *rec, double rmax, double z, double r, int L,
+__device__ inline MpSums multipole_sums(const double *mp, const double *leg, double c, double qr, int L, int lo, int own)
+{
+    const double c2 = c * c, q2 = qr * qr;
+    // p_(l+1), p_(l+2) and P'_l, P'_(l+1), P'_(l+2), from l = 1
+    double p1 = c2 - 1.0 / 3.0, p2 = c * (c2 - 0.6);
+    double d0 = 1.0, d1 = 3.0 * c, d2 = 1.5 * (5.0 * c2 - 1.0);
+    double q = q2;   // q_l
+    MpSums S = {0.0, 0.0, 0.0, 0.0, 0.0};
+    MpTerm<WA, WB || WG> t0, t1;   // in turn: the term summed and the one loaded meanwhile
+    const double *ma = mp + 4 * kMpOdd;
+    t0.load(mp, ma, leg);
+    auto add = [&](const MpTerm<WA, WB || WG> &t, MpTerm<WA, WB || WG> &next, double ql) {
+        mp += 4;
+        ma += 1;
+        leg += 4;
+        next.load(mp, ma, leg);
+        if (WA) S.A = fma(t.a * ql, d0, S.A);
+        if (WB || WG) {
+            S.Z = fma(t.zk * ql, p1, S.Z);
+            S.B = fma(t.m * ql, d1, S.B);
+        }
+        if (WG) {
+            S.ZZ = fma(t.zzk * ql, p2, S.ZZ);
+            S.RZ = fma(t.mz * ql, d2, S.RZ);
+        }
+        // p_(l+3), p_(l+4), P'_(l+3), P'_(l+4)
+        const double p3 = fma(c, p2, -t.b0 * p1), d3 = fma(t.k0, p2, d1);
+        const double p4 = fma(c, p3, -t.b1 * p2), d4 = fma(t.k1, p3, d2);
+        d0 = d2;
+        p1 = p3;
+        p2 = p4;
+        d1 = d3;
+        d2 = d4;
+        q *= q2;
+    };
+    int l = 1;
+    for (; l + 2 <= lo; l += 4) {
+        add(t0, t1, q);
+        add(t1, t0, q);
+    }
+    for (; l <= L; l += 4) {
+        add(t0, t1, l <= own ? q : 0.0);
+        if (l + 2 > L) break;
+        add(t1, t0, l + 2 <= own ? q : 0.0);
+    }
+    return S;
+}
+
+// Local (A_phi, B_rho, B_z, B_rho / r, dB_rho/drho, dB_rho/dz, dB_z/dz) of one coil at local (z, r) from its series
+// (mp: the coil's kMpCoil doubles, leg: Tables::leg, rmax: the coil's r_max; L, lo, own: multipole_sums).
+template <bool WA, bool WB, bool WG>
+__device__ inline void eval_multipole(const double *mp, const double *leg, double rmax, double z, double r, int L,
                                       int lo, int own, Local &out)
 {
     const double D2 = r * r + z * z;
     const double u = rsqrt_newton(D2);
-    const double c = z * u, s = r * u, qr = rmax * u;
-    const double *mA = mp, *mB = mp + kMpStride, *mZ = mp + 2 * kMpStride, *mZZ = mp + 3 * kMpStride;
-    // P_(l+1), P_(l+2) and P'_l, P'_(l+1), P'_(l+2), advanced together from l = 1
-    double P1 = 0.5 * (3.0 * c * c - 1.0), P2 = 0.5 * c * (5.0 * c * c - 3.0);
-    double d0 = 1.0, d1 = 3.0 * c, d2 = 1.5 * (5.0 * c * c - 1.0);
-    double q = qr;   // q_l = (r_max / D)^(l + 1)
-    double SA = 0.0, SZ = 0.0, SB = 0.0, SZZ = 0.0, SRZ = 0.0;
-    auto accumulate = [&](int l, double ql) {
-        if (WA) SA = fma(mA[l] * ql, d0, SA);
-        if (WB || WG) {
-            SZ = fma(mZ[l] * ql, P1, SZ);
-            SB = fma(mB[l] * ql, d1, SB);
-        }
-        if (WG) {
-            SZZ = fma(mZZ[l] * ql, P2, SZZ);
-            SRZ = fma(mZ[l] * ql, d2, SRZ);
-        }
-    };
-    auto step = [&](int l) {
-        // P_(l+3) = ((2l + 5) c P_(l+2) - (l + 2) P_(l+1)) / (l + 3), P'_(l+3) = P'_(l+1) + (2l + 5) P_(l+2)
-        const double P3 = fma(rec[l] * c, P2, -rec[kMpStride + l] * P1);
-        const double d3 = fma(rec[2 * kMpStride + l], P2, d1);
-        P1 = P2;
-        P2 = P3;
-        d0 = d1;
-        d1 = d2;
-        d2 = d3;
-    };
-    // The moments of even order are exactly zero (kMpEvenZero), so only odd l accumulate while the recurrences and
-    // the powers q_l step through every l: the same operations on the same values as summing every term.
-    int l = 1;
-#pragma unroll 2
-    for (; l <= lo; l += 2) {
-        q *= qr;
-        accumulate(l, q);
-        step(l);
-        q *= qr;
-        step(l + 1);
-    }
-#pragma unroll 2
-    for (; l <= L; l += 2) {
-        q *= qr;
-        accumulate(l, l <= own ? q : 0.0);
-        step(l);
-        q *= qr;
-        step(l + 1);
-    }
-    out.A = s * SA;
-    out.Bz = u * SZ;
-    out.Bh = s * u * SB;
-    out.RP = u * u * SB;
-    out.ZZ = -u * u * SZZ;
-    out.RZ = -s * u * u * SRZ;
+    const double s = r * u;
+    const MpSums S = multipole_sums<WA, WB, WG>(mp, leg, z * u, rmax * u, L, lo, own);
+    out.A = s * S.A;
+    out.Bz = u * S.Z;
+    out.Bh = s * u * S.B;
+    out.RP = u * u * S.B;
+    out.ZZ = -u * u * S.ZZ;
+    out.RZ = -s * u * u * S.RZ;
     out.RR = -(out.RP + out.ZZ);
 }
 
 // The pair kernel's view of the series at a secondary node: A_phi (WA), B_rho and B_z (WB), and A_phi / r = u sum
-// m_l q_l P'_l / l (also on the axis, where it is the limit), for dA_phi/dr = B_z - A_phi / r. Loop as in
-// eval_multipole: L terms, the first lo without the test, the lane's own count own.
+// m_l q_l P'_l / l (also on the axis, where it is the limit), for dA_phi/dr = B_z - A_phi / r.
 template <bool WA, bool WB>
-__device__ inline void eval_multipole_pair(const double *mp, const double *rec, double rmax, double z, double r, int L,
+__device__ inline void eval_multipole_pair(const double *mp, const double *leg, double rmax, double z, double r, int L,
                                            int lo, int own, Local &out, double &a_over_r)
 {
     const double D2 = r * r + z * z;
     const double u = rsqrt_newton(D2);
-    const double c = z * u, s = r * u, qr = rmax * u;
-    const double *mA = mp, *mB = mp + kMpStride, *mZ = mp + 2 * kMpStride;
-    double P1 = 0.5 * (3.0 * c * c - 1.0), P2 = 0.5 * c * (5.0 * c * c - 3.0);
-    double d0 = 1.0, d1 = 3.0 * c, d2 = 1.5 * (5.0 * c * c - 1.0);
-    double q = qr;
-    double SA = 0.0, SZ = 0.0, SB = 0.0;
-    auto accumulate = [&](int l, double ql) {
-        if (WA) SA = fma(mA[l] * ql, d0, SA);
-        if (WB) {
-            SZ = fma(mZ[l] * ql, P1, SZ);
-            SB = fma(mB[l] * ql, d1, SB);
-        }
-    };
-    auto step = [&](int l) {
-        const double P3 = fma(rec[l] * c, P2, -rec[kMpStride + l] * P1);
-        const double d3 = fma(rec[2 * kMpStride + l], P2, d1);
-        P1 = P2;
-        P2 = P3;
-        d0 = d1;
-        d1 = d2;
-        d2 = d3;
-    };
-    int l = 1;   // odd l only, as in eval_multipole
-#pragma unroll 2
-    for (; l <= lo; l += 2) {
-        q *= qr;
-        accumulate(l, q);
-        step(l);
-        q *= qr;
-        step(l + 1);
-    }
-#pragma unroll 2
-    for (; l <= L; l += 2) {
-        q *= qr;
-        accumulate(l, l <= own ? q : 0.0);
-        step(l);
-        q *= qr;
-        step(l + 1);
-    }
-    out.A = s * SA;
-    out.Bz = u * SZ;
-    out.Bh = s * u * SB;
-    a_over_r = u * SA;
+    const double s = r * u;
+    const MpSums S = multipole_sums<WA, WB, false>(mp, leg, z * u, rmax * u, L, lo, own);
+    out.A = s * S.A;
+    out.Bz = u * S.Z;
+    out.Bh = s * u * S.B;
+    a_over_r = u * S.A;
 }
 
 }  // namespace ccoil

@@ -16,7 +16,7 @@ namespace ccoil {
 constexpr int kMomThreads = 128;   // one sheet a thread
 constexpr int kMomOrders = 32;     // odd orders summed at a time
 constexpr int kMomStride = kMaxOrder + 1;   // odd, so that a column of orders crosses the LDS banks
-static_assert(kMaxOrder <= kMomThreads && kMomStride % 2 == 1 && kMpStride % (2 * kMomOrders) == 0, "moments block");
+static_assert(kMaxOrder <= kMomThreads && kMomStride % 2 == 1 && kMpOdd % kMomOrders == 0, "moments block");
 
 // Moments of coil blockIdx.x. Thread j steps the recurrences of the sheet at thickness node j (squared half-length z2,
 // c2 = rho^2 + z2, in units of r_max) over 32 odd orders, then four threads an order add the sheets. With U_l, V_l of
@@ -26,19 +26,14 @@ static_assert(kMaxOrder <= kMomThreads && kMomStride % 2 == 1 && kMpStride % (2 
 // node, summed over the wave at every order, took 90 us for 128 coils and 1.96 ms for 8,192, this 13 and 50 us.
 __global__ __launch_bounds__(kMomThreads) void multipole_moments_kernel(const CoilDev *coils, Tables tab, double *mp)
 {
-    __shared__ double inv[kMpStride + 1];                 // 1 / l
+    __shared__ double inv[2 * kMpOdd + 2];                // 1 / l
     __shared__ double term[kMomOrders][kMomStride];       // per order and sheet
     __shared__ double part[4][kMomOrders];
     const int ci = blockIdx.x, t = threadIdx.x;
-    if (ci == 0)
-        for (int l = t; l < kMpStride; l += kMomThreads) {   // recurrence coefficients of the Legendre polynomials
-            mp[l] = (2.0 * l + 5.0) / (l + 3.0);
-            mp[kMpStride + l] = (l + 2.0) / (l + 3.0);
-            mp[2 * kMpStride + l] = 2.0 * l + 5.0;
-        }
     const CoilDev &c = coils[ci];
-    double *out = mp + kMpHeader + (size_t)ci * kMpCoil;
-    for (int l = t; l <= kMpStride; l += kMomThreads) inv[l] = l > 0 ? 1.0 / l : 0.0;
+    double *out = mp + (size_t)ci * kMpCoil;
+    const double *kn = tab.leg + 4 * kMpOdd;
+    for (int l = t; l < 2 * kMpOdd + 2; l += kMomThreads) inv[l] = l > 0 ? 1.0 / l : 0.0;
     const int nt = c.n_thk, terms = c.far_d2 > 0.0 ? (c.mp_terms < kMpTerms ? c.mp_terms : kMpTerms) : 0;
     const double scale = 1.0 / c.rmax, h = c.use_fast ? 0.5 * c.b * scale : 0.0, z2 = h * h;
     double c2 = 0.0, w = 0.0;
@@ -51,10 +46,11 @@ __global__ __launch_bounds__(kMomThreads) void multipole_moments_kernel(const Co
     double E = 1.0, O = 1.0, G = 3.0;   // E_(l-1), O_l, G_(l+1) at l = 1
     const double ni = c.ni * (4.0 * kPi * kMuReduced);   // m_l = mu0 N I sum / (2 (l + 1)), mu0 = 4 pi 1e-7
     __syncthreads();
-    for (int l0 = 0; l0 < kMpStride; l0 += 2 * kMomOrders) {
+    for (int i0 = 0; i0 < kMpOdd; i0 += kMomOrders) {
+        const int l0 = 2 * i0;
         if (l0 >= terms) {   // no series, or none of these orders
-            for (int k = t; k < 8 * kMomOrders; k += kMomThreads)
-                out[(k / (2 * kMomOrders)) * kMpStride + l0 + k % (2 * kMomOrders)] = 0.0;
+            for (int k = t; k < 4 * kMomOrders; k += kMomThreads) out[4 * i0 + k] = 0.0;
+            if (t < kMomOrders) out[4 * kMpOdd + i0 + t] = 0.0;
             continue;
         }
         if (t < nt)
@@ -64,7 +60,7 @@ __global__ __launch_bounds__(kMomThreads) void multipole_moments_kernel(const Co
                 const double fl = l;
                 term[i][t] = w * G;
                 E = ((2.0 * fl + 1.0) * z2 * O - fl * c2 * E) * inv[l + 1];
-                O = ((2.0 * fl + 3.0) * E - (fl + 1.0) * c2 * O) * inv[l + 2 <= kMpStride ? l + 2 : 0];
+                O = ((2.0 * fl + 3.0) * E - (fl + 1.0) * c2 * O) * inv[l + 2];
                 G = c2 * G + (2.0 * fl + 5.0) * O;
             }
         __syncthreads();
@@ -74,16 +70,17 @@ __global__ __launch_bounds__(kMomThreads) void multipole_moments_kernel(const Co
         for (int j = q; j < nt; j += 4) sum += term[i][j];
         part[q][i] = sum;
         __syncthreads();
-        if (t < 2 * kMomOrders) {
-            // the moments of even order are zero: V_l(rho, -z0) = (-1)^(l-1) V_l(rho, z0)
-            const int l = l0 + t, k = t / 2;
+        if (t < kMomOrders) {
+            const int l = l0 + 2 * t + 1;
             double m = 0.0;
-            if (t % 2 == 1 && l <= kMpTerms)
-                m = ni * (((part[0][k] + part[1][k]) + (part[2][k] + part[3][k])) * inv[l + 2]) / (2.0 * (l + 1));
-            out[l] = l >= 1 ? m / l : 0.0;
-            out[kMpStride + l] = m;
-            out[2 * kMpStride + l] = (l + 1) * m;
-            out[3 * kMpStride + l] = (l + 1.0) * (l + 2.0) * m;
+            if (l <= kMpTerms)
+                m = ni * (((part[0][t] + part[1][t]) + (part[2][t] + part[3][t])) * inv[l + 2]) / (2.0 * (l + 1));
+            double *row = out + 4 * (i0 + t);
+            row[0] = m;
+            row[1] = (l + 1) * m * kn[l + 1];
+            row[2] = (l + 1.0) * (l + 2.0) * m * kn[l + 2];
+            row[3] = (l + 1) * m;
+            out[4 * kMpOdd + i0 + t] = m / l;
         }
     }
 }

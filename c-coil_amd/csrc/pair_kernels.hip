@@ -305,7 +305,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPairWaves<P
                 const int terms = wave_max_small(own), lo = wave_min_small(own, far);
                 if (far) {
                     double aor = 0.0;
-                    eval_multipole_pair<kA, kB>(p.mp + kMpHeader + (size_t)pd.prim * kMpCoil, p.mp, pc.rmax, n.z, n.r,
+                    eval_multipole_pair<kA, kB>(p.mp + (size_t)pd.prim * kMpCoil, p.tab.leg, pc.rmax, n.z, n.r,
                                                 terms, lo, own, L, aor);
                     q = {0.0, 0.0, 0.0, L.Bz - aor};   // dA_phi/dr = B_z - A_phi / r
                 }

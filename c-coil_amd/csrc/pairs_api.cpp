@@ -194,9 +194,9 @@ ccoil_status pairs_setup(ccoil_ctx ctx, const PairBuild &pb, uint32_t what, int3
     CC_HIP(ctx, hipSetDevice(ctx->device));
     const std::vector<CoilDev> &hp = pb.hp, &hs = pb.hs;
     const std::vector<PairDev> &sorted = pb.sorted;
-    // primary records, then (series) the moments: kMpHeader + kMpCoil per primary
+    // primary records, then (series) the moments: kMpCoil per primary
     const size_t prim_bytes = (sizeof(CoilDev) * hp.size() + 255) & ~(size_t)255;
-    const size_t mp_bytes = pb.far ? sizeof(double) * ((size_t)kMpHeader + (size_t)kMpCoil * hp.size()) : 0;
+    const size_t mp_bytes = pb.far ? sizeof(double) * (size_t)kMpCoil * hp.size() : 0;
     CC_HIP(ctx, ensure(*bufs[0], prim_bytes + mp_bytes));
     CC_HIP(ctx, ensure(*bufs[1], sizeof(CoilDev) * hs.size()));
     CC_HIP(ctx, ensure(*bufs[2], sizeof(PairDev) * sorted.size()));

@@ -23,6 +23,7 @@
 // the far-field bound, exp(2 eta) for the node terms that cancel far from the coil), its thickness rule where
 // 200 rho_B^(-2 n_thk) <= 1e-15.
 #include "context.hpp"
+#include "multipole.hpp"
 
 #include <algorithm>
 #include <array>
@@ -138,6 +139,23 @@ int64_t rule_nodes_beyond(const CoilDev &c, double dist)
     const RuleSel s = class_rule(c, class_of(c, (float)(gap * gap), (float)(2.0 * dist * (c.R + c.a)),
                                              (float)(2.0 * gap) * c.ia2f));
     return (int64_t)s.na * s.nt;
+}
+
+std::vector<double> legendre_rows()
+{
+    std::vector<double> v(4 * kMpOdd + kMpLegK);
+    std::vector<ld> k(kMpLegK + 1, 1.0L);   // the leading coefficient of P_n
+    for (int n = 0; n < kMpLegK; ++n) {
+        v[(size_t)(4 * kMpOdd + n)] = (double)k[(size_t)n];
+        k[(size_t)n + 1] = k[(size_t)n] * (2 * n + 1) / (n + 1);
+    }
+    for (int i = 0; i < kMpOdd; ++i)
+        for (int h = 0; h < 2; ++h) {
+            const int n = 2 * i + 3 + h;
+            v[(size_t)(4 * i + 2 * h)] = (double)((ld)n * n / (4.0L * n * n - 1.0L));
+            v[(size_t)(4 * i + 2 * h + 1)] = (double)((2 * n + 1) * k[(size_t)n]);
+        }
+    return v;
 }
 
 void reduced_tables(RedTables &t)
