@@ -130,6 +130,9 @@ __global__ __launch_bounds__(kKeyScanThreads) void near_key_scan_kernel(FieldPar
     if (k_split / 4 % kKeyScanThreads == t) p.near_state->split = p.near_cursor[k_split];
 }
 
+// Coils of a block row of near_fill_kernel: a multiple of record_candidates' eight.
+__host__ __device__ inline int fill_coils_per_row(int n_coils, int rows) { return ((n_coils + rows - 1) / rows + 7) / 8 * 8; }
+
 __global__ __launch_bounds__(256) void near_fill_kernel(FieldParams p)
 {
     if (p.near_state->overflow) return;
@@ -146,8 +149,16 @@ __global__ __launch_bounds__(256) void near_fill_kernel(FieldParams p)
     const int lane = threadIdx.x & 63;
     bool bad = false;
     // coils in ascending order (a point's slots follow its coils), skipping those no point of the wave can be a
-    // record of
-    for (int c0 = 0; c0 < p.n_coils; c0 += 8) {
+    // record of. Block row y takes its share of the coils; the slots before it are counted again, a fifth of the work
+    const int per = fill_coils_per_row(p.n_coils, gridDim.y), first = blockIdx.y * per, last = min(first + per, p.n_coils);
+    for (int c0 = 0; c0 < first; c0 += 8)
+        for (uint32_t cand = record_candidates(p.coils, p.n_coils, c0, px, py, pz); cand; cand &= cand - 1) {
+            const CoilDev &c = p.coils[c0 + __builtin_ctz(cand)];
+            double z, r, cph, sph;
+            to_local(c, px, py, pz, z, r, cph, sph);
+            slot += record_kind(p, c, z, r, p.q & (Q_G | Q_GJ)) >= 0 ? 1 : 0;
+        }
+    for (int c0 = first; c0 < last; c0 += 8) {
         for (uint32_t cand = record_candidates(p.coils, p.n_coils, c0, px, py, pz); cand; cand &= cand - 1) {
             const CoilDev &c = p.coils[c0 + __builtin_ctz(cand)];
             double z, r, cph, sph;
@@ -181,7 +192,7 @@ __global__ __launch_bounds__(256) void near_fill_kernel(FieldParams p)
             }
         }
     }
-    if (bad || slot != end) atomicOr(&p.near_state->mismatch, 1u);
+    if (bad || (last == p.n_coils && slot != end)) atomicOr(&p.near_state->mismatch, 1u);
 }
 
 // Sum over the S lanes of a record by a fixed xor butterfly, so every lane of the group holds the same sum.
@@ -449,7 +460,13 @@ void launch_near_count(hipStream_t s, const FieldParams &p)
 void launch_near_fill(hipStream_t s, const FieldParams &p)
 {
     if (p.n_pts <= 0) return;
-    hipLaunchKernelGGL(near_fill_kernel, dim3((unsigned)((p.n_pts + 255) / 256)), dim3(256), 0, s, p);
+    // A wave takes its coils in turn, about half a microsecond each, so that few points leave the chip to that chain:
+    // rows of at least 8 coils up to eight blocks a CU (128 coils x 16,411 points: 74 us in one row, 34 in eight;
+    // 262,145 points, FP32C: 81 in one, 73 in two).
+    const int64_t blocks = (p.n_pts + 255) / 256;
+    const int64_t most = std::max<int64_t>(1, std::min<int64_t>({8, (p.n_coils + 7) / 8, (2048 + blocks - 1) / blocks}));
+    const int per = fill_coils_per_row(p.n_coils, (int)most);
+    hipLaunchKernelGGL(near_fill_kernel, dim3((unsigned)blocks, (unsigned)((p.n_coils + per - 1) / per)), dim3(256), 0, s, p);
 }
 
 template <bool FLOAT>

@@ -84,6 +84,24 @@ def test_records_match_the_own_rule(ctx, coil, n):
     print(f"\n{coil} n={n}: worst error over tolerance {check(ctx, _row(*coil), n, abi.FP64, abi.FAR_FIELD, 5)}")
 
 
+@pytest.mark.parametrize("n_coils,n", [(1, 300), (8, 300), (9, 5000), (65, 5000), (130, 300), (23, 70000), (40, 270000)])
+def test_records_of_many_coils(ctx, n_coils, n):
+    """Every point next to every coil, at coil counts around the rows of eight that the records are placed in, one row and
+    several: the series mode against the rule alone, which differ by the order of their sums and by rounding (1e-12 of
+    the field's largest value)."""
+    rng = np.random.default_rng(17)
+    rows = []
+    for k in range(n_coils):
+        row = _row(*COILS[k % 8])
+        row.update(pos=tuple(rng.normal(scale=0.02, size=3)), alpha=float(rng.uniform(0, 3)), beta=float(rng.uniform(0, 6)))
+        rows.append(row)
+    cs = abi.CoilSet.from_rows(rows)
+    pts = rng.normal(scale=0.12, size=(n, 3))
+    ref, _ = ctx.fields(cs, pts, abi.B, abi.FP64)
+    got, _ = ctx.fields(cs, pts, abi.B, abi.FP64, abi.FAR_FIELD)
+    assert np.max(np.abs(got["B"] - ref["B"])) <= 1e-12 * np.max(np.abs(ref["B"]))
+
+
 LONG = [("RECTANGULAR", 0.02, 0.01, 0.6, 80, 20), ("THIN", 0.02, 0.0, 1.0, 100, 1), ("FLAT", 0.01, 0.3, 0.0, 100, 100),
         ("RECTANGULAR", 0.1, 0.05, 1e-4, 80, 2), ("RECTANGULAR", 0.3, 0.3, 0.3, 100, 100)]
 
