@@ -8,6 +8,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <system_error>
 #include <thread>
 
 using namespace ccoil;
@@ -66,10 +67,9 @@ ccoil_status call_buffer(ccoil_ctx ctx, DevBuf &b, Arena *arena, size_t bytes, v
 }
 
 // Transformation matrices of Coil::calculateTransformationMatrices (CalculateAttributes.cxx:63-78).
-void rotation(double alpha, double beta, double *T, double *Ti)
+void rotation(const Angles &g, double *T, double *Ti)
 {
-    const double cosY = std::cos(alpha), sinY = std::sin(alpha);
-    const double cosZ = std::cos(beta), sinZ = std::sin(beta);
+    const double cosY = g.ca, sinY = g.sa, cosZ = g.cb, sinZ = g.sb;
     const double t[9] = {cosZ * cosZ * cosY - sinZ * sinZ, -sinZ * cosZ * cosY - sinZ * cosZ, cosZ * sinY,
                          sinZ * cosZ * cosY + sinZ * cosZ, cosZ * cosZ - sinZ * sinZ * cosY, sinZ * sinY,
                          -sinY * cosZ, sinY * sinZ, cosY};
@@ -86,11 +86,9 @@ namespace ccoil {
 
 // Axial vectors of Omega = T^T dT/dtheta for theta = alpha, beta, with T of rotation() differentiated entry by
 // entry (the antisymmetric part is read off; T^T dT is antisymmetric because T is orthogonal).
-void rotation_generators(double alpha, double beta, double *om_a, double *om_b)
+void rotation_generators(const Angles &g, const double *T, double *om_a, double *om_b)
 {
-    const double cY = std::cos(alpha), sY = std::sin(alpha), cZ = std::cos(beta), sZ = std::sin(beta);
-    double T[9], Ti[9];
-    rotation(alpha, beta, T, Ti);
+    const double cY = g.ca, sY = g.sa, cZ = g.cb, sZ = g.sb;
     const double dA[9] = {-cZ * cZ * sY, sZ * cZ * sY, cZ * cY,
                           -sZ * cZ * sY, sZ * sZ * sY, sZ * cY,
                           -cY * cZ, cY * sZ, -sY};
@@ -154,12 +152,13 @@ std::string pack_coils(const ccoil_coils *c, bool need_len, bool need_freq, std:
         double w = std::fmax(std::fmax(d.a, d.b), 1e-3 * d.R);
         d.near_w2 = w * w;
         for (int k = 0; k < 3; ++k) d.pos[k] = c->pos[3 * i + k];
-        rotation(c->alpha[i], c->beta[i], d.T, d.Tinv);
-        d.sa = std::sin(c->alpha[i]);
-        d.ca = std::cos(c->alpha[i]);
-        d.sb = std::sin(c->beta[i]);
-        d.cb = std::cos(c->beta[i]);
-        rotation_generators(c->alpha[i], c->beta[i], d.om_a, d.om_b);
+        const Angles g = {std::sin(c->alpha[i]), std::cos(c->alpha[i]), std::sin(c->beta[i]), std::cos(c->beta[i])};
+        rotation(g, d.T, d.Tinv);
+        d.sa = g.sa;
+        d.ca = g.ca;
+        d.sb = g.sb;
+        d.cb = g.cb;
+        rotation_generators(g, d.T, d.om_a, d.om_b);
         d.cur_used = d.current;
         d.adj_scale = 1.0;
         d.ni = c->J[i] * d.a * d.b;
@@ -190,7 +189,9 @@ std::string pack_coils(const ccoil_coils *c, bool need_len, bool need_freq, std:
 
 void host_parallel_for(int64_t n, const std::function<void(int64_t, int64_t)> &fn)
 {
-    constexpr int64_t kPerThread = 8192;
+    // a thread starts in some 20 us, the loops take 0.1 to 0.3 us a coil (8,192 pairs: 7.4 ms on the host with 8,192
+    // coils a thread, 2.4 with 1,024 and the trigonometry of a coil done once)
+    constexpr int64_t kPerThread = 1024;
     const int64_t hw = std::max<int64_t>(1, (int64_t)std::thread::hardware_concurrency());
     const int64_t parts = std::min<int64_t>(std::min<int64_t>(16, hw), (n + kPerThread - 1) / kPerThread);
     if (parts <= 1) {
@@ -201,7 +202,12 @@ void host_parallel_for(int64_t n, const std::function<void(int64_t, int64_t)> &f
     const int64_t per = (n + parts - 1) / parts;
     for (int64_t k = 1; k < parts; ++k) {
         const int64_t i0 = k * per, i1 = std::min(n, i0 + per);
-        if (i0 < i1) pool.emplace_back(fn, i0, i1);
+        if (i0 >= i1) continue;
+        try {
+            pool.emplace_back(fn, i0, i1);
+        } catch (const std::system_error &) {   // no thread to be had: the range is done here
+            fn(i0, i1);
+        }
     }
     fn(0, std::min(n, per));
     for (auto &t : pool) t.join();

@@ -43,8 +43,9 @@ struct Arena {
     }
 };
 
-void rotation(double alpha, double beta, double *T, double *Ti);
-void rotation_generators(double alpha, double beta, double *om_a, double *om_b);
+struct Angles { double sa, ca, sb, cb; };   // sines and cosines of a coil's alpha and beta
+void rotation(const Angles &g, double *T, double *Ti);
+void rotation_generators(const Angles &g, const double *T, double *om_a, double *om_b);
 std::string pack_coils(const ccoil_coils *c, bool need_len, bool need_freq, std::vector<CoilDev> &out);
 
 }  // namespace ccoil

@@ -6,7 +6,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <complex>
 #include <cstring>
 
 using namespace ccoil;
@@ -72,13 +71,12 @@ FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n, int64_t n_coils, uint32_t 
 // holds.
 double far_threshold(int n_ang, double q, double tol, double ylo)
 {
+    const double log_c = std::log(1000.0 / tol);
     auto g = [&](double y) {
         const double d = y - 1.0;
-        const double eta = std::acosh(1.0 + d * d * q / (2.0 * y));
-        const std::complex<double> xs(-1.0, 2.0 * eta / kPi);
-        const std::complex<double> sq = std::sqrt(xs * xs - 1.0);
-        const double rho = std::max(std::abs(xs + sq), std::abs(xs - sq));
-        return std::log(1000.0 / tol) + 2.0 * std::log(y) - 2.0 * n_ang * std::log(rho);
+        const double t = 2.0 / kPi * std::acosh(1.0 + d * d * q / (2.0 * y));
+        // log(rho_B) is the hyperbolic arc cosine of the ellipse's half axis, (|x_s - 1| + |x_s + 1|) / 2
+        return log_c + 2.0 * std::log(y) - 2.0 * n_ang * std::acosh(0.5 * (std::sqrt(4.0 + t * t) + t));
     };
     if (n_ang < 5) return 0.0;
     double lo = ylo, hi = 100.0, glo = g(lo), ghi = g(hi);

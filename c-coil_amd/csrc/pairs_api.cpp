@@ -118,6 +118,7 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
     std::vector<PairDev> pd((size_t)n_pairs);
     const bool reduced = precision == CCOIL_FP64;
     std::vector<int64_t> prim_nodes((size_t)n_pairs);   // that an item evaluates per secondary node
+    std::vector<uint8_t> series((size_t)n_pairs);       // series_only of each pair
     int64_t node_pairs = 0, work = 0;
     const bool ref_scale = flags & CCOIL_FORCE_REFERENCE_SCALE;
     for (int64_t k = 0; k < n_pairs; ++k) {
@@ -127,7 +128,8 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
         const CoilDev &p = hp[(size_t)pi], &s = hs[(size_t)si];
         const int64_t sec_nodes = (int64_t)s.blk_ang * s.n_ang * s.blk_thk * s.n_thk * s.blk_len * s.n_len;
         node_pairs += sec_nodes * p.n_ang * p.n_thk;
-        prim_nodes[(size_t)k] = series_only(p, s) ? kSeriesNodes : reduced ? rule_nodes_of(p, s) : (int64_t)p.n_ang * p.n_thk;
+        series[(size_t)k] = series_only(p, s);
+        prim_nodes[(size_t)k] = series[(size_t)k] ? kSeriesNodes : reduced ? rule_nodes_of(p, s) : (int64_t)p.n_ang * p.n_thk;
         work += sec_nodes * (reduced ? prim_nodes[(size_t)k] : (int64_t)p.n_ang * p.n_thk);
     }
     const int64_t target = target_override > 0 ? target_override : lane_target(work, reduced);
@@ -142,7 +144,7 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
         d.sec = (int32_t)si;
         d.out = (int32_t)k;
         d.n_nodes = (int64_t)s.blk_ang * s.n_ang * s.blk_thk * s.n_thk * s.blk_len * s.n_len;
-        decompose(target, prim_nodes[(size_t)k], series_only(p, s) ? 1 : p.n_thk, d.nodes_per_item, d.row_groups);
+        decompose(target, prim_nodes[(size_t)k], series[(size_t)k] ? 1 : p.n_thk, d.nodes_per_item, d.row_groups);
         max_row_groups = std::max(max_row_groups, d.row_groups);
         d.ring_offset = ring_offset ? ring_offset[k] : 0.0;
         d.half_ring = half_ring ? (half_ring[k] ? 1 : 0) : 0;
@@ -160,7 +162,7 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
         const CoilDev &p = hp[(size_t)d.prim];
         cost[(size_t)k] = std::min<int64_t>(d.nodes_per_item, d.n_nodes) *
                           ((prim_nodes[(size_t)k] + d.row_groups - 1) / d.row_groups) *
-                          (p.use_fast && !series_only(p, hs[(size_t)d.sec]) ? 2 : 1);
+                          (p.use_fast && !series[(size_t)k] ? 2 : 1);
     }
     std::vector<int32_t> order((size_t)n_pairs);
     std::iota(order.begin(), order.end(), 0);
