@@ -373,6 +373,25 @@ void launch_fill_zero(hipStream_t s, void *p, int64_t n_words)
     hipLaunchKernelGGL(fill_zero_kernel, dim3(blocks), dim3(256), 0, s, (unsigned long long *)p, n_words);
 }
 
+// Four launches of some microseconds, gaps included, each cleared a few kilobytes of a call with the series.
+__global__ void fill_zero_ranges_kernel(ZeroRanges z)
+{
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    for (int k = 0; k < 4; ++k) {
+        if (i < z.n[k]) {
+            ((unsigned long long *)z.p[k])[i] = 0ull;
+            return;
+        }
+        i -= z.n[k];
+    }
+}
+
+void launch_fill_zero(hipStream_t s, const ZeroRanges &z)
+{
+    const int64_t n = z.n[0] + z.n[1] + z.n[2] + z.n[3];
+    if (n > 0) hipLaunchKernelGGL(fill_zero_ranges_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, z);
+}
+
 template <int PREC, bool WA, bool WB, bool WG>
 static void launch_field_q(hipStream_t s, const FieldParams &p, int split)
 {

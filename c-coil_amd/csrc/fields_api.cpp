@@ -205,15 +205,25 @@ void enqueue_fields(hipStream_t s, const FieldLaunch &L, hipEvent_t evm0, hipEve
                     hipEvent_t evr0, hipEvent_t evr1)
 {
     const FieldParams &p = L.p;
+    ZeroRanges zero;
+    std::memset(&zero, 0, sizeof zero);
+    if (p.order) {
+        zero.p[0] = visit_order_counts(L.order_temp, p.n_pts);
+        zero.n[0] = (int64_t)1 << (3 * L.order_bits);
+    }
+    if (L.near) {
+        zero.p[1] = p.near_counts;
+        zero.n[1] = p.n_pts;
+        zero.p[2] = p.near_hist;
+        zero.n[2] = ((int64_t)p.n_keys + 2) / 2;
+        zero.p[3] = p.near_state;
+        zero.n[3] = sizeof(NearState) / 8;
+    }
+    launch_fill_zero(s, zero);
     if (p.mp) launch_multipole_moments(s, p.coils, p.n_coils, p.tab, const_cast<double *>(p.mp));
     if (p.order)
         (void)launch_visit_order(s, p.pts, p.n_pts, L.order_bits, L.order_temp, L.order_scan_bytes,
                                  const_cast<uint32_t *>(p.order));
-    if (L.near) {
-        launch_fill_zero(s, p.near_counts, p.n_pts);
-        launch_fill_zero(s, p.near_hist, ((int64_t)p.n_keys + 2) / 2);
-        launch_fill_zero(s, p.near_state, sizeof(NearState) / 8);
-    }
     if (evm0) (void)hipEventRecord(evm0, s);
     launch_field(s, p, L.precision, L.split);
     if (evm1) (void)hipEventRecord(evm1, s);

@@ -149,6 +149,11 @@ void launch_angular_tables(hipStream_t s, const double *x, const double *w, cons
 // split: 1, 4 or 16 lanes per point.
 // Zeroes n_words 8-byte words with a kernel (no hipMemsetAsync, so callers may capture it in a graph).
 void launch_fill_zero(hipStream_t s, void *p, int64_t n_words);
+struct ZeroRanges {       // up to four ranges of words to zero with one launch
+    void *p[4];
+    int64_t n[4];
+};
+void launch_fill_zero(hipStream_t s, const ZeroRanges &z);
 void launch_field(hipStream_t s, const FieldParams &p, int precision, int split);
 void launch_field_reduce(hipStream_t s, const FieldParams &p);   // after launch_field when n_chunks > 1
 // Resident 256-thread blocks per CU of the field kernel instance (0 if the runtime cannot tell).
@@ -181,6 +186,7 @@ void launch_multipole_moments(hipStream_t s, const CoilDev *coils, int n_coils, 
 // The visit order: points counting-sorted by the Morton cell of a 2^bits-per-axis grid over their bounding box.
 // temp: visit_order_bytes(n, bits, scan_bytes) bytes, scan_bytes from near_scan for 2^(3 bits) counts.
 size_t visit_order_bytes(int64_t n, int bits, size_t scan_bytes);
+int64_t *visit_order_counts(void *temp, int64_t n);   // the cells' 2^(3 bits) counts, zeroed before the launch
 hipError_t launch_visit_order(hipStream_t s, const double *pts, int64_t n, int bits, void *temp, size_t scan_bytes,
                               uint32_t *order);
 

@@ -189,6 +189,13 @@ size_t visit_order_bytes(int64_t n, int bits, size_t scan_bytes)
            scan_bytes + 6 * 256;
 }
 
+int64_t *visit_order_counts(void *temp, int64_t n)
+{
+    auto align = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    return (int64_t *)((char *)temp + align(sizeof(double) * 6 * kBoxBlocks) + align(sizeof(double) * 8) +
+                       align(sizeof(uint32_t) * (size_t)n));
+}
+
 hipError_t launch_visit_order(hipStream_t s, const double *pts, int64_t n, int bits, void *temp, size_t scan_bytes,
                               uint32_t *order)
 {
@@ -201,7 +208,7 @@ hipError_t launch_visit_order(hipStream_t s, const double *pts, int64_t n, int b
     t += align(sizeof(double) * 8);
     uint32_t *cell = (uint32_t *)t;
     t += align(sizeof(uint32_t) * (size_t)n);
-    int64_t *count = (int64_t *)t;
+    int64_t *count = visit_order_counts(temp, n);
     t += align(sizeof(int64_t) * cells);
     int64_t *cursor = (int64_t *)t;
     t += align(sizeof(int64_t) * cells);
@@ -209,7 +216,6 @@ hipError_t launch_visit_order(hipStream_t s, const double *pts, int64_t n, int b
     const int blocks = (int)((n + 255) / 256 < kBoxBlocks ? (n + 255) / 256 : kBoxBlocks);
     hipLaunchKernelGGL(box_partial_kernel, dim3(blocks), dim3(256), 0, s, pts, n, part);
     hipLaunchKernelGGL(box_final_kernel, dim3(1), dim3(256), 0, s, part, blocks, box);
-    launch_fill_zero(s, count, (int64_t)cells);
     const unsigned grid = (unsigned)((n + 255) / 256);
     hipLaunchKernelGGL(cell_count_kernel, dim3(grid), dim3(256), 0, s, pts, n, box, bits, cell,
                        (unsigned long long *)count);

@@ -410,10 +410,19 @@ __global__ __launch_bounds__(256) void scan_sums_kernel(int64_t *sums, int64_t n
     }
 }
 
-__global__ __launch_bounds__(256) void scan_tiles_kernel(const int64_t *counts, int64_t n, const int64_t *sums,
+// sums: the tiles' sums, scanned already or (raw) each tile's block adding those before it.
+__global__ __launch_bounds__(256) void scan_tiles_kernel(const int64_t *counts, int64_t n, const int64_t *sums, int raw,
                                                          int64_t *offsets)
 {
     __shared__ int64_t lds[256];
+    int64_t before = 0;
+    if (raw && blockIdx.x > 0) {
+        int64_t v = 0;
+        for (unsigned i = threadIdx.x; i < blockIdx.x; i += 256) v += sums[i];
+        (void)block_exclusive_scan(v, lds, before);
+    } else if (!raw) {
+        before = sums[blockIdx.x];
+    }
     const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanPerThread;
     int64_t v[kScanPerThread], t = 0;
     for (int k = 0; k < kScanPerThread; ++k) {
@@ -421,7 +430,7 @@ __global__ __launch_bounds__(256) void scan_tiles_kernel(const int64_t *counts, 
         t += v[k];
     }
     int64_t total;
-    int64_t run = sums[blockIdx.x] + block_exclusive_scan(t, lds, total);
+    int64_t run = before + block_exclusive_scan(t, lds, total);
     for (int k = 0; k < kScanPerThread; ++k) {
         if (base + k < n) offsets[base + k] = run;
         run += v[k];
@@ -438,9 +447,13 @@ hipError_t near_scan(hipStream_t s, const int64_t *counts, int64_t *offsets, int
     }
     if (n <= 0) return hipSuccess;
     int64_t *sums = (int64_t *)temp;
-    hipLaunchKernelGGL(scan_tile_sums_kernel, dim3((unsigned)nb), dim3(256), 0, s, counts, n, sums);
-    hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(256), 0, s, sums, nb);
-    hipLaunchKernelGGL(scan_tiles_kernel, dim3((unsigned)nb), dim3(256), 0, s, counts, n, (const int64_t *)sums,
+    // Up to kScanRaw tiles (eight loads a thread) a tile's block adds the sums before it itself, and one tile needs none:
+    // two launches or one in place of three, some 4 us each.
+    constexpr int64_t kScanRaw = 2048;
+    const int raw = nb <= kScanRaw ? 1 : 0;
+    if (nb > 1) hipLaunchKernelGGL(scan_tile_sums_kernel, dim3((unsigned)nb), dim3(256), 0, s, counts, n, sums);
+    if (!raw) hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(256), 0, s, sums, nb);
+    hipLaunchKernelGGL(scan_tiles_kernel, dim3((unsigned)nb), dim3(256), 0, s, counts, n, (const int64_t *)sums, raw,
                        offsets);
     return hipGetLastError();
 }

@@ -84,10 +84,11 @@ def test_records_match_the_own_rule(ctx, coil, n):
     print(f"\n{coil} n={n}: worst error over tolerance {check(ctx, _row(*coil), n, abi.FP64, abi.FAR_FIELD, 5)}")
 
 
-@pytest.mark.parametrize("n_coils,n", [(1, 300), (8, 300), (9, 5000), (65, 5000), (130, 300), (23, 70000), (40, 270000)])
+@pytest.mark.parametrize("n_coils,n", [(1, 300), (8, 300), (9, 5000), (65, 5000), (130, 300), (23, 70000), (40, 270000),
+                                       (1, 8400000)])
 def test_records_of_many_coils(ctx, n_coils, n):
     """Every point next to every coil, at coil counts around the rows of eight that the records are placed in, one row and
-    several: the series mode against the rule alone, which differ by the order of their sums and by rounding (1e-12 of
+    several, and one, a few and over 2,048 tiles of the scans: the series mode against the rule, which differ by the order of their sums and by rounding (1e-12 of
     the field's largest value)."""
     rng = np.random.default_rng(17)
     rows = []
