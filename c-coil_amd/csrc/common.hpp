@@ -61,7 +61,7 @@ struct alignas(64) CoilDev {
     int32_t near_key; // FP32C near pass: the coil's place in the evaluation order (most nodes first)
     int32_t mp_terms; // highest order of the far-field series a pair of this call can use (0: no series)
     // Reduced rules: the least cosh(eta) - 1 and the least ellipse parameter sum (d1 + d2) / (a / 2) at which the
-    // coil's angular and thickness rules may be replaced (FLT_MAX: never), and the winding's geometry in float
+    // coil's angular and thickness rules may be replaced (NaN: never), and the winding's geometry in float
     // (inner and outer radius, half length, 2 / a).
     float red_x, red_s;
     float r0f, r1f, hbf, ia2f;

@@ -29,11 +29,16 @@
 #include <array>
 #include <cfloat>
 #include <cmath>
+#include <limits>
 #include <complex>
 
 namespace ccoil {
 
 namespace {
+
+// No measure of a point reaches it, also none that overflowed.
+constexpr float kNever = std::numeric_limits<float>::quiet_NaN();
+
 
 typedef long double ld;
 
@@ -77,16 +82,16 @@ double log_ellipse(double eta)
     return std::log(std::max(std::abs(xs + sq), std::abs(xs - sq)));
 }
 
-// Least cosh(eta) - 1 at which the n-node angular rule may be replaced (FLT_MAX: never).
+// Least cosh(eta) - 1 at which the n-node angular rule may be replaced (kNever: never).
 float ang_threshold(int n)
 {
     int first = 0;
     while (first < kRedAng && kRedAngN[first] >= n) ++first;
-    if (first == kRedAng) return FLT_MAX;
+    if (first == kRedAng) return kNever;
     auto g = [&](double eta) { return std::log(1000.0 / 1e-15) + 2.0 * eta - 2.0 * n * log_ellipse(eta); };
     double lo = kRedEta[first], hi = 20.0;
     if (g(lo) > 0.0) {
-        if (g(hi) > 0.0) return FLT_MAX;
+        if (g(hi) > 0.0) return kNever;
         for (int it = 0; it < 60; ++it) {
             const double m = 0.5 * (lo + hi);
             (g(m) > 0.0 ? lo : hi) = m;
@@ -96,12 +101,12 @@ float ang_threshold(int n)
     return (float)((std::cosh(lo) - 1.0) * (1.0 + 1e-5));
 }
 
-// Least ellipse distance sum at which the n-node thickness rule may be replaced (FLT_MAX: never).
+// Least ellipse distance sum at which the n-node thickness rule may be replaced (kNever: never).
 float thk_threshold(int n)
 {
     int first = 0;
     while (first < kRedThk && kRedThkN[first] >= n) ++first;
-    if (first == kRedThk) return FLT_MAX;
+    if (first == kRedThk) return kNever;
     const double own = std::log(kRedThkC / 1e-15) / (2.0 * n), red = std::log(kRedThkC / kRedTol) / (2.0 * kRedThkN[first]);
     return (float)(2.0 * std::cosh(std::max(own, red)) * (1.0 + 1e-4));
 }
@@ -122,8 +127,11 @@ struct Thresholds {
 void set_rule_limits(CoilDev &c)
 {
     static const Thresholds t;
-    c.red_x = t.ang[(size_t)c.n_ang];
-    c.red_s = t.thk[(size_t)c.n_thk];
+    // The classes are found in float, to some 1e-7 of the larger of a point's coordinates and the winding's: that must
+    // not overflow nor underflow when squared, and be small against R (angular) and against a (thickness).
+    const bool fits = c.R >= 1e-15 && c.R + c.a <= 1e15 && (!c.use_fast || 0.5 * c.b <= 1e4 * c.R);
+    c.red_x = fits ? t.ang[(size_t)c.n_ang] : kNever;
+    c.red_s = fits && c.a >= 1e-4 * (c.R + c.a) ? t.thk[(size_t)c.n_thk] : kNever;
     c.r0f = (float)c.R;
     c.r1f = (float)(c.R + c.a);
     c.hbf = c.use_fast ? (float)(0.5 * c.b) : 0.0f;

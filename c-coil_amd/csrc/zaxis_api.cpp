@@ -39,7 +39,7 @@ PairRule pair_rule(double Rp, double ap, double hp, double Rs, double as, double
     PairRule rule = {0, 0, 0, 0, 0};
     const double g = std::fmax(0.0, std::fabs(c) - hp - hs);
     const double q = std::fmax(0.0, std::fmax(Rp - (Rs + as), Rs - (Rp + ap)));
-    if (!(q + g > 0.0)) return rule;
+    if (!(q + g > 0.0) || !(Rs >= 1e-15 && Rs + as <= 1e15)) return rule;   // (set_rule_limits: the primary's range)
     CoilDev d;
     d.R = Rp;
     d.a = ap;
@@ -53,9 +53,12 @@ PairRule pair_rule(double Rp, double ap, double hp, double Rs, double as, double
     const int k = cls / (kRedThk + 1), t = cls % (kRedThk + 1);
     const double H = std::fmax(hp, hs), h = std::fmin(hp, hs), x0 = -c + H, x1 = -c - H;
     d.n_thk = n_rad;
+    d.R = Rs;
+    d.a = as;
     set_rule_limits(d);
     const int r = class_of(d, num, den, (float)ellipse_sum(Rs, as, Rp, Rp + ap, g)) % (kRedThk + 1);
     d.n_thk = kMaxOrder;
+    d.a = d.R;
     set_rule_limits(d);
     const double sl = std::fmin(ellipse_sum(-h, 2.0 * h, x0, x0, q), ellipse_sum(-h, 2.0 * h, x1, x1, q));
     const int l = class_of(d, num, den, (float)sl) % (kRedThk + 1);

@@ -88,8 +88,8 @@ def test_records_match_the_own_rule(ctx, coil, n):
                                        (1, 8400000)])
 def test_records_of_many_coils(ctx, n_coils, n):
     """Every point next to every coil, at coil counts around the rows of eight that the records are placed in, one row and
-    several, and one, a few and over 2,048 tiles of the scans: the series mode against the rule, which differ by the order of their sums and by rounding (1e-12 of
-    the field's largest value)."""
+    several, and one, a few and over 2,048 tiles of the scans: the series mode against the rule, which differ by the
+    order of their sums and by rounding (1e-12 of the field's largest value)."""
     rng = np.random.default_rng(17)
     rows = []
     for k in range(n_coils):
@@ -238,3 +238,23 @@ def test_coaxial_pairs(ctx, i, apart):
         lost = 2.0 ** -60 * 20.0 * 2e-7 * np.pi ** 2 * abs(p.J * s.J) * p.a * s.a * (p.R + p.a) * (s.R + s.a)
         assert abs(out["M"][k] - m) <= 1e-12 * abs(m) + lost * gaps[k] / abs(p.I * s.I), (k, gaps[k])
         assert abs(out["Fz"][k] - f) <= 1e-12 * abs(f) + lost, (k, gaps[k])
+
+
+@pytest.mark.parametrize("R,a,b", [(1e21, 1e21, 1e21), (1e-22, 1e-22, 1e-22), (1e-3, 0.0, 1e5), (1.0, 1e-7, 0.5), (2.0, 1e-3, 1e5)])
+def test_classes_out_of_floats_range(ctx, R, a, b):
+    """Coils whose points' classes float cannot tell: too large or small to square, far longer than wide, far thinner. At
+    points in and around the winding, and at its end, CCOIL_FP64 and CCOIL_FP64_IEEE differ by the rounding of their node
+    terms: 1e-11 of the largest value."""
+    row = _row("RECTANGULAR" if a else "THIN", R, a, b, 80, 20 if a else 1)
+    row.update(pos=(0.0, 0.0, 0.0), alpha=0.0, beta=0.0)
+    rng = np.random.default_rng(19)
+    n, phi = 1000, rng.uniform(0, 2 * np.pi, 1000)
+    r = np.where(np.arange(n) % 2, R + max(a, 1e-3 * R) * rng.uniform(-1, 2, n), R * rng.uniform(0.5, 3, n))
+    z = np.where(np.arange(n) % 3, b * rng.uniform(-0.5, 0.5, n), 0.5 * b + R * rng.uniform(-1, 1, n))
+    pts = np.stack([r * np.cos(phi), r * np.sin(phi), z], axis=1)
+    cs = abi.CoilSet.from_rows([row])
+    ref, _ = ctx.fields(cs, pts, abi.A | abi.B, abi.FP64_IEEE)
+    got, _ = ctx.fields(cs, pts, abi.A | abi.B, abi.FP64)
+    for k in ("A", "B"):
+        assert np.all(np.isfinite(ref[k]))
+        assert np.max(np.abs(got[k] - ref[k])) <= 1e-11 * np.max(np.abs(ref[k])), k
