@@ -233,7 +233,8 @@ def main():
                 works[name] = ({"series": (0.0, w["series_flops"], w["series_special"]), "records": rec}, w)
             else:
                 f32 = prec in (abi.FP32C, abi.FP32)
-                works[name] = ({"field": (flops if f32 else 0.0, 0.0 if f32 else flops, trans)}, None)
+                fl, tr = RM.reduced_field_work(rows, pts, with_gradient=True) if prec == abi.FP64 else (flops, trans)
+                works[name] = ({"field": (fl if f32 else 0.0, 0.0 if f32 else fl, tr)}, None)
         return works[name]
 
     def part_roofline(kernel, work, ms):
@@ -357,8 +358,9 @@ def main():
         what = abi.PAIR_M | abi.PAIR_FT
         pf, ptrans, pnodes = RM.pair_work(prow, srow)
         pres = {}
-        # the rule at every node (fp64, fp32c_direct: node-pair rates and algorithmic flops are the rule's), and the
-        # primaries' series beyond their far-field distance (fp64_far_field, fp32c: pairs/s)
+        # the rule at every node (fp64, which sums most of them by reduced rules: node-pair rates are the planned
+        # rule's; fp32c_direct, also algorithmic flops), and the primaries' series beyond their far-field distance
+        # (fp64_far_field, fp32c: pairs/s)
         for name, prec, flags in (("fp64", abi.FP64, 0), ("fp64_far_field", abi.FP64, abi.FAR_FIELD),
                                   ("fp32c", abi.FP32C, 0), ("fp32c_direct", abi.FP32C, abi.DIRECT)):
             ctx.pairs(P, S, len(prow), what, prec, flags)
@@ -369,9 +371,9 @@ def main():
                           "kernel_ms": prep.main_kernel_ms, "out": o}
             if name in ("fp64", "fp32c_direct"):
                 pres[name]["node_pairs_per_s"] = pnodes / (prep.main_kernel_ms * 1e-3)
+            if name == "fp32c_direct":
                 pres[name]["tflops_algorithmic"] = pf / (prep.main_kernel_ms * 1e-3) / 1e12
-                peak = RM.PEAK_FP64_TFLOPS if prec == abi.FP64 else RM.PEAK_FP32_TFLOPS
-                pres[name]["frac"] = pres[name]["tflops_algorithmic"] / peak
+                pres[name]["frac"] = pres[name]["tflops_algorithmic"] / RM.PEAK_FP32_TFLOPS
             log(f"pairs {name}: {dt_p * 1e3:.1f} ms/step, kernel {prep.main_kernel_ms:.1f} ms")
         o64, o32 = pres["fp64"].pop("out"), pres["fp32c"].pop("out")
         ofar, o32d = pres["fp64_far_field"].pop("out"), pres["fp32c_direct"].pop("out")

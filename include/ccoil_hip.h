@@ -53,8 +53,10 @@ enum {
 /* Arithmetic of the quadrature. */
 enum {
     CCOIL_FP64 = 0,           /* cancellation-free integrands in double; reciprocals and reciprocal square roots
-                                 from the hardware FP64 approximations refined by one Newton step (a few ulp):
-                                 the accurate mode */
+                                 from the hardware FP64 approximations refined by one Newton step (a few ulp);
+                                 a coil's angular and thickness sums take fewer nodes than its increments where
+                                 both have converged to rounding (1e-15 of the sum of the terms): the accurate
+                                 mode */
     CCOIL_FP32C = 1,          /* the same integrands with FP32 per-node arithmetic, FP64 per-row work and row
                                  accumulation, re-evaluation with CCOIL_FP64's arithmetic of near-winding (coil,
                                  point) pairs and, for outputs that divide by r (the gradient, the pair position
@@ -63,7 +65,7 @@ enum {
     CCOIL_FP64_REFERENCE = 3, /* the reference's integrands verbatim in double (a TYPE=double build): the
                                  parity mode and the plain-FP64 throughput comparator; its gradient terms
                                  lose up to ~3e-5 relative to cancellation near the winding */
-    CCOIL_FP64_IEEE = 4       /* CCOIL_FP64's integrands with IEEE division and square root */
+    CCOIL_FP64_IEEE = 4       /* CCOIL_FP64's integrands with IEEE division and square root, at all the increments */
 };
 
 /* Flags. */
@@ -80,8 +82,8 @@ enum {
                                   the fastest. A cached shape is replayed as is, so results are bitwise
                                   reproducible for a given cache. */
     CCOIL_DIRECT = 16,         /* FP32C fields: evaluate every (coil, point) pair with the rule. By default a pair
-                                  beyond the coil's far-field distance (at least twice the radius of the sphere that
-                                  holds the winding, more for coils of few angular increments) takes the coil's
+                                  beyond the coil's far-field distance (ccoil_far_field_radius: at least 1.17 times the
+                                  radius of the sphere that holds the winding, more for coils of few increments) takes the coil's
                                   exterior zonal-harmonic series in FP64 instead, with moments summed over the rule's
                                   own thickness nodes: it departs from the FP64 rule by less than 1e-11 of the coil's
                                   field there (the angular rule's error bound) and from the float rule it replaces
@@ -120,7 +122,8 @@ typedef struct {
 
 /* Per-call report (any pointer argument may be NULL). */
 typedef struct {
-    int64_t node_evaluations;  /* sum over (coil, point) of quadrature nodes, or (pair) node-pairs */
+    int64_t node_evaluations;  /* sum over (coil, point) of the increments' quadrature nodes, or (pair) node-pairs,
+                                  whatever a mode sums in their place */
     int64_t near_pairs;        /* FP32C: (coil, point) pairs re-evaluated in FP64 */
     double kernel_ms;          /* device time of the compute kernels of this call (hipEvent) */
     int32_t block_size;        /* threads per workgroup of the main kernel */
@@ -174,7 +177,8 @@ ccoil_status ccoil_fields(ccoil_ctx ctx, const ccoil_coils *coils, const double 
  * fixed 64 MiB scratch array per device, held from the library's load until the process ends. Points and outputs
  * must be device pointers (flags must hold CCOIL_DEVICE_POINTERS). A call whose buffers do not fit, or whose FP32C
  * near pass finds more near pairs than the scratch holds, returns CCOIL_ERR_ARGUMENT (in the second case the
- * outputs lack the near contributions): split the points. Results are bitwise those of ccoil_fields. All calls on
+ * outputs lack the near contributions): split the points. Results are bitwise those of ccoil_fields; from 16,384
+ * points on, in the modes that take the series, they agree to the rounding of the rule's sums. All calls on
  * one device share its scratch, which keeps the last call's contents: calls that overlap on one device (from two
  * contexts or threads) race. */
 ccoil_status ccoil_fields_noalloc(ccoil_ctx ctx, const ccoil_coils *coils, const double *points, int64_t n_points,
@@ -221,7 +225,8 @@ ccoil_status ccoil_field_gradient(ccoil_ctx ctx, const ccoil_coils *coils, const
  * writes M (what & CCOIL_PAIR_M) and Fz, the axial force on the secondary (what & CCOIL_PAIR_FT; the transverse
  * force and the torque of a coaxial pair are zero). Only pos[2] of each coil enters. Primary rule: n_ang, n_thk
  * and the angular and thickness blocks; secondary rule: n_thk and the thickness blocks (blocks NULL = 1). Needs
- * J, current (M divides by I1 I2) and turns. Evaluated in FP64 with the reference's per-node expressions.
+ * J, current (M divides by I1 I2) and turns. Evaluated in FP64 with the reference's per-node expressions, or, for
+ * windings clear of each other, to rounding by fewer cancellation-free nodes.
  * Replaces Coil::calculateMutualInductanceZAxisFast (CalculateMInductanceZAxis.cxx:84-221) and
  * Coil::calculateAmpereForceZAxisFast (CalculateForceZAxis.cxx:82-219). */
 ccoil_status ccoil_pairs_zaxis(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coils *sec,
