@@ -333,12 +333,14 @@ __global__ __launch_bounds__(256) void near_eval_group_kernel(FieldParams p)
     }
 }
 
+// Adds each point's slots to its outputs, in slot order. Points in index order: slots and outputs lie in that order, so
+// that a wave reads and writes whole lines (in the visit order each point's took lines of their own: 128 coils x 2^20
+// points 0.20 ms, this 0.14; 262,145 points FP32C 45 us, this 28).
 __global__ __launch_bounds__(256) void near_add_kernel(FieldParams p)
 {
     if (p.near_state->overflow) return;
-    const int64_t vi = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (vi >= p.n_pts) return;
-    const int64_t pi = p.order ? (int64_t)p.order[vi] : vi;
+    const int64_t pi = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (pi >= p.n_pts) return;
     const int64_t count = p.near_counts[pi];
     if (count == 0) return;
     const int64_t e0 = p.near_offsets[pi];
