@@ -90,8 +90,10 @@ struct FieldShape {
 // The fixed rule (few points: split rows over lanes; few waves: chunk the coils; large: fill the last round).
 // series_only: the call's record pass takes every pair inside the far-field distances, so the launch is the
 // series-only kernel (one lane per point).
-FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n_points, int64_t n_coils, uint32_t q, int precision,
+FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n_points, const std::vector<CoilDev> &coils, uint32_t q, int precision,
                             bool series_only = false);
+// Whether a CCOIL_FP64 call without rule records sums the coils' own nodes (kFP64Own) instead of reduced rules.
+bool field_own_rule(const std::vector<CoilDev> &coils, int64_t n_points, int split, uint32_t q);
 
 // Everything a field call launches, with its buffers already sized.
 struct FieldLaunch {

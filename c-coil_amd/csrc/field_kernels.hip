@@ -184,6 +184,8 @@ void field_kernel(FieldParams p)
             const int kind = record_kind(p, c, z, r, WG);
             if constexpr (PREC == kFP64) {
                 eval_classes<WA, WB, WG, SPLIT>(c, p.tab, z, r, !far && kind < 0, L);
+            } else if constexpr (PREC == kFP64Own) {
+                if (!far && kind < 0) eval_stable<f64s, WA, WB, WG>(c, p.tab, full_rule(c), z, r, lane, SPLIT, 0, 1, L);
             } else if (!far && kind < 0) {
                 eval_stable<float, WA, WB, WG>(c, p.tab, full_rule(c), z, r, lane, SPLIT, 0, 1, L);
             }
@@ -192,7 +194,7 @@ void field_kernel(FieldParams p)
                 // the loop runs to the wave's largest term count (uniform bounds and coefficient loads); each lane
                 // stops adding at its own count, so its value does not depend on the other points of its wave
                 const int own = far ? multipole_terms(r * r + z * z, c.inv_rmax2,
-                                                      PREC == kFP64 ? kMpLogTolFP64 : kMpLogTolFP32C) : 0;
+                                                      PREC == kFP32C ? kMpLogTolFP32C : kMpLogTolFP64) : 0;
                 const int terms = wave_max_small(own), lo = wave_min_small(own, far);
                 if (far && lane == 0)
                     eval_multipole<WA, WB, WG>(p.mp + (size_t)ci * kMpCoil, p.tab.leg, c.rmax, z, r, terms,
@@ -431,7 +433,7 @@ static void launch_series_p(hipStream_t s, const FieldParams &p)
 template <int PREC>
 static void launch_field_p(hipStream_t s, const FieldParams &p, int split)
 {
-    if constexpr (PREC == kFP64 || PREC == kFP32C) {
+    if constexpr (PREC == kFP64 || PREC == kFP32C) {   // (kFP64Own: never with rule records)
         if (p.rule_records) {   // the record pass takes every pair inside the far-field distances
             launch_series_p<PREC>(s, p);
             return;
@@ -508,6 +510,7 @@ int field_series_blocks_per_cu(uint32_t q, int precision)
 int field_blocks_per_cu(uint32_t q, int precision, int split)
 {
     if (precision == kFP64) return blocks_per_cu_p<kFP64>(q, split);
+    if (precision == kFP64Own) return blocks_per_cu_p<kFP64Own>(q, split);
     if (precision == kFP64IEEE) return blocks_per_cu_p<kFP64IEEE>(q, split);
     if (precision == kFP64Reference) return blocks_per_cu_p<kFP64Reference>(q, split);
     if (precision == kFP32) return blocks_per_cu_p<kFP32>(q, split);
@@ -518,6 +521,7 @@ void launch_field(hipStream_t s, const FieldParams &p, int precision, int split)
 {
     if (p.n_pts <= 0) return;
     if (precision == kFP64) launch_field_p<kFP64>(s, p, split);
+    else if (precision == kFP64Own) launch_field_p<kFP64Own>(s, p, split);
     else if (precision == kFP64IEEE) launch_field_p<kFP64IEEE>(s, p, split);
     else if (precision == kFP64Reference) launch_field_p<kFP64Reference>(s, p, split);
     else if (precision == kFP32) launch_field_p<kFP32>(s, p, split);

@@ -23,9 +23,11 @@ namespace ccoil {
 // the launch still has fewer than about 8 waves per SIMD. Large launches take 1-4 chunks, whichever makes the last
 // round of resident waves fullest: every wave does the same work, so with R rounds of resident waves the launch
 // runs ceil(R) rounds.
-FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n, int64_t n_coils, uint32_t q, int precision, bool series_only)
+FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n, const std::vector<CoilDev> &coils, uint32_t q, int precision,
+                            bool series_only)
 {
     FieldShape sh;
+    const int64_t n_coils = (int64_t)coils.size();
     const int64_t target = (int64_t)256 * 4 * 8;
     sh.split = n < (precision == CCOIL_FP64 ? kSortedPoints : (int64_t)256 * 4 * 64 * 4) ? 4 : 1;
     if (sh.split == 4 && (n * 4 + 63) / 64 * n_coils < (int64_t)256 * 4) sh.split = 16;
@@ -34,8 +36,8 @@ FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n, int64_t n_coils, uint32_t 
     const int64_t waves = std::max<int64_t>(1, (n * sh.split + 63) / 64);
     int64_t chunks = waves >= target ? 1 : std::min<int64_t>(n_coils, (target + waves - 1) / waves);
     if (waves >= target && n * 18 < ((int64_t)1 << 31)) {   // the reduction grid stays below 2^31 threads
-        const int bpc = series_only ? field_series_blocks_per_cu(q, precision)
-                                    : field_blocks_per_cu(q, precision, sh.split);
+        const int kernel = precision == CCOIL_FP64 && field_own_rule(coils, n, sh.split, q) ? kFP64Own : precision;
+        const int bpc = series_only ? field_series_blocks_per_cu(q, precision) : field_blocks_per_cu(q, kernel, sh.split);
         const double slots = (double)ctx->cu_count * bpc * (kFieldBlock / 64);
         if (slots > 0) {
             double best = 0.0;
@@ -50,6 +52,59 @@ FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n, int64_t n_coils, uint32_t 
     }
     sh.chunks = (int)std::max<int64_t>(1, std::min<int64_t>(chunks, 65535));
     return sh;
+}
+
+// CCOIL_FP64's kernels: reduced rules by class (kFP64), or the coils' own nodes, the same for all lanes (kFP64Own). Reduced
+// rules save most of a long rule's nodes, but choosing them, the registers of two ways to sum, the classes that a wave
+// takes in turn, the points that it sums one at a time and (one lane per point) the visit order cost more than a short
+// rule takes in all: 128 coils of 20 x 7 slow nodes at 40,000 points took 2.07 ms by reduced rules and 0.55 by their own,
+// coils of 80 x 20 1.05 and 3.4.
+//
+// The costs, for B, are those measured with coils of 14 to 100 angular by 1 to 27 thickness nodes, 1 to 128 of them, at
+// 16,384 to 2^20 points in a normal and in a uniform cloud (reduced rules: the mean of the two, which lie up to a fifth
+// either side of it).
+//  - 16 lanes per point, in nodes of a lane's chain: the own rule those of a row of 16, the reduced ones a share of the
+//    whole rule (such calls' points are mostly few coils' and near) or, from 512 nodes on, a wave's.
+//  - 4 lanes, in ps per coil and point: the own rule 5.2 (1.6 slow) for each node of a lane's rows; the reduced ones by
+//    the number of rows, most for 15 to 29 angular nodes, of which most points keep all. With the gradient the nodes cost
+//    1.4 times as much, the reduced rules, half of which is their choice, 1.2 times.
+//  - 1 lane, in ps likewise: the own rule 1.35 (0.45) a node and as much again for the SIMDs that idle in the last
+//    round of waves; the reduced ones 33 to 38 (10 to 15) a row, less in the smaller cells of more points. Per call they
+//    add the visit order, 50 us and 0.3 ns a point, and the longest rule once more, which the waves next to its winding
+//    end with.
+bool field_own_rule(const std::vector<CoilDev> &coils, int64_t n, int split, uint32_t q)
+{
+    if (split > 16) return false;
+    const bool fine = n >= (int64_t)1 << 19;   // the visit order's cells
+    double own = 0.0, red = 0.0, tail = 0.0;
+    for (const CoilDev &c : coils) {
+        const int na = c.n_ang, nt = c.n_thk, nodes = na * nt;
+        const bool fast = c.use_fast != 0;
+        if (split == 16) {
+            own += na * ((nt + 15) / 16);
+            red += nodes < 512 ? 8.0 + 0.1 * nodes : 40.0;
+        } else if (split == 4) {
+            static constexpr double kRed[2][3][5] = {   // slow, fast; below 15, 15 to 29, from 30 angular nodes on
+                {{92, 120, 120, 190, 260}, {92, 160, 150, 530, 600}, {92, 170, 145, 265, 350}},
+                {{120, 165, 165, 275, 520}, {130, 240, 235, 700, 850}, {140, 300, 230, 450, 600}}};
+            const int rows = nt == 1 ? 0 : nt < 4 ? 1 : nt < 8 ? 2 : nt < 16 ? 3 : 4;
+            own += 30.0 + (fast ? 5.2 : 1.6) * na * ((nt + 3) / 4);
+            red += rows == 1 && na >= 64 ? (fast ? 215.0 : 130.0) : kRed[fast][na < 15 ? 0 : na < 30 ? 1 : 2][rows];
+        } else {
+            const int rows = std::min(nt, 17);
+            const double r = fast ? 12.0 + (fine ? 33.0 : 38.0) * rows : fine ? 8.0 + 10.5 * rows : 16.0 + 14.5 * rows;
+            own += 10.0 + (fast ? 1.35 : 0.45) * nodes;
+            red += na < 15 ? (fast ? 0.75 : 0.55) * r : r;
+            tail = std::max(tail, fast ? std::min(0.13 * nodes, 80.0 + 0.08 * nodes) : 0.065 * nodes);
+        }
+    }
+    const bool grad = (q & (CCOIL_G | CCOIL_G_JACOBIAN)) != 0;
+    if (split > 1) return own * (grad ? 1.4 : 1.0) < red * (grad ? 1.2 : 1.0);
+    const double waves = (double)n / 65536.0 * std::min<double>((double)coils.size(), 8.0);   // per SIMD
+    own *= std::max(std::ceil(waves), 1.2) / waves;
+    const int kinds = (q & (CCOIL_A | CCOIL_E) ? 1 : 0) + (q & CCOIL_B ? 1 : 0) + (grad ? 1 : 0);
+    const double per = 0.5e-6 * (1 + kinds) * (double)n;   // us per ps of B
+    return own * per < red * per + 50.0 + 0.3e-3 * (double)n + tail;
 }
 
 // Distance, in units of the coil's r_max, beyond which the far-field series replaces the rule (0: never), at least
@@ -290,11 +345,12 @@ ccoil_status fields_prepare(ccoil_ctx ctx, const ccoil_coils *coils, const doubl
     out.nodes = 0;
     for (auto &c : hc) out.nodes += (int64_t)c.n_ang * c.n_thk;
     if (n == 0 || hc.empty()) return CCOIL_OK;   // nothing to evaluate, or every field zero
-    const FieldShape sh = shape ? *shape : field_shape_rule(ctx, n, (int64_t)hc.size(), quantities, precision,
-                                                            rule_records);
+    const FieldShape sh = shape ? *shape : field_shape_rule(ctx, n, hc, quantities, precision, rule_records);
     if (shape && sh.split != 1 && sh.split != 4 && sh.split != 16)
         return fail(ctx, CCOIL_ERR_ARGUMENT, "split must be 1, 4 or 16");
     L.split = rule_records ? 1 : sh.split;   // the series-only kernel runs one lane per point
+    const bool own_rule = precision == CCOIL_FP64 && !rule_records && field_own_rule(hc, n, L.split, quantities);
+    if (own_rule) L.precision = kFP64Own;
     if (far)
         for (auto &c : hc) {
             // the cost floor holds for one lane per point; a launch that splits the rows runs the series on one
@@ -356,7 +412,8 @@ ccoil_status fields_prepare(ccoil_ctx ctx, const ccoil_coils *coils, const doubl
     }
     // The visit order, when there are enough points for the spatial sort to pay: the series modes, and the FP64 rule
     // with one lane per point (no result depends on it, so the fixed scratch, which has no room to spare, goes without)
-    const bool sorted_rule = precision == CCOIL_FP64 && L.split == 1 && n >= kSortedPoints && !(arena && arena->fixed);
+    const bool sorted_rule = precision == CCOIL_FP64 && !own_rule && L.split == 1 && n >= kSortedPoints &&
+                             !(arena && arena->fixed);
     if ((far && n >= kOrderMinPoints) || sorted_rule) {
         // about 16-32 points per cell: 2^bits cells per axis, bits = log8(n / 16), between 3 and 6
         int bits = 3;

@@ -69,7 +69,7 @@ ccoil_status tune_fields(ccoil_ctx ctx, const ccoil_coils *coils, const double *
     // candidates around the rule: every lane count that can fill the chip, 1-4 coil chunks and the rule's chunks
     // with its halves and doubles
     const int64_t nc = (int64_t)hc.size();
-    const FieldShape rule = field_shape_rule(ctx, n_points, nc, quantities, precision);
+    const FieldShape rule = field_shape_rule(ctx, n_points, hc, quantities, precision);
     std::set<std::pair<int, int>> cand;
     std::vector<int> splits = {1, 4};
     if (n_points < 65536) splits.push_back(16);

@@ -1,0 +1,58 @@
+"""CCOIL_FP64's choice between reduced rules and the coils' own nodes (field_own_rule), at every launch shape.
+
+Values: against CCOIL_FP64_IEEE, which sums the own nodes whatever the call, per point and relative to the coils' own
+field, with the tolerances of test_gpu_reduced_rules.py (its points, its reasons; a sum of identical coils scales both).
+
+Times: the choice is there so that no call takes longer than the own nodes with IEEE division and square root, which
+cost about twice CCOIL_FP64's arithmetic. The least of several device times, so that a neighbour's load drops out.
+"""
+import numpy as np
+import pytest
+
+import ccoil_abi as abi
+from test_gpu_reduced_rules import _points, _row
+
+pytestmark = pytest.mark.gpu
+
+RECT16 = ("RECTANGULAR", 0.1, 0.1, 0.1, 16, 16)
+RECT59 = ("RECTANGULAR", 0.1, 0.1, 0.1, 59, 27)
+FLAT20 = ("FLAT", 0.1, 0.05, 0.0, 20, 7)
+THIN12 = ("THIN", 0.05, 0.0, 0.05, 12, 1)
+
+
+# own nodes by 16, 4 and 1 lanes per point, chunks of coils among them; reduced rules by one lane in the visit order
+@pytest.mark.parametrize("coil,copies,n,split", [(RECT16, 1, 300, 16), (THIN12, 3, 20001, 4), (FLAT20, 9, 40001, 4),
+                                                 (RECT16, 2, 70001, 1), (THIN12, 40, 262145, 1), (RECT59, 24, 65537, 1)])
+def test_values(ctx, coil, copies, n, split):
+    row = _row(*coil)
+    pts, r, z = _points(np.random.default_rng(23), row, n)
+    cs = abi.CoilSet.from_rows([row] * copies)
+    q = abi.A | abi.B | abi.G
+    ref, _ = ctx.fields(cs, pts, q, abi.FP64_IEEE)
+    got, rep = ctx.fields(cs, pts, q, abi.FP64)
+    assert rep.split == split
+    R, a, hb = row["R"], row["a"], 0.5 * row["b"] if row["use_fast"] else 0.0
+    zd = np.maximum(np.abs(z) - hb, 0.0)
+    rho = np.clip(np.hypot(r, zd), R, R + a)
+    eta = np.arccosh(1.0 + ((rho - r) ** 2 + zd * zd) / (2.0 * rho * r))
+    y = np.hypot(r, z) / np.hypot(R + a, hb)
+    b = np.linalg.norm(ref["B"], axis=1)
+    for k, near, far in (("A", 1e-11, 2e-14), ("B", 1e-11, 2e-14), ("G", 1e-6, 2e-13)):
+        scale = np.linalg.norm(ref[k], axis=1) + (b * R if k == "A" else b / np.maximum(r, 1e-5 * R) if k == "G" else 0.0)
+        tol = np.where(eta > 0.1, far * (1.0 + y) ** 2, near)
+        assert np.all(np.linalg.norm(got[k] - ref[k], axis=1) <= tol * scale), k
+
+
+@pytest.mark.parametrize("coil,copies,n", [(RECT16, 40, 40000), (FLAT20, 128, 40000), (THIN12, 1, 1 << 20), (RECT59, 1, 65536)])
+def test_no_slower_than_ieee(ctx, coil, copies, n):
+    rng = np.random.default_rng(3)
+    rows = []
+    for _ in range(copies):
+        row = _row(*coil)
+        row.update(pos=tuple(rng.normal(scale=0.3, size=3)), alpha=float(rng.uniform(0, 3)), beta=float(rng.uniform(0, 6)))
+        rows.append(row)
+    cs = abi.CoilSet.from_rows(rows)
+    pts = rng.normal(scale=0.4, size=(n, 3))
+    ms = {p: min(ctx.fields(cs, pts, abi.B, p)[1].kernel_ms for _ in range(7)) for p in (abi.FP64, abi.FP64_IEEE)}
+    print(f"\n{coil} {copies} coils {n} points: {1e3 * ms[abi.FP64]:.0f} us, IEEE {1e3 * ms[abi.FP64_IEEE]:.0f}")
+    assert ms[abi.FP64] <= ms[abi.FP64_IEEE]
