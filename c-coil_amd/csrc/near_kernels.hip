@@ -54,32 +54,47 @@ __device__ inline uint32_t record_candidates(const CoilDev *coils, int n_coils, 
 // Calls with fewer points than kNearSplitPoints split each float record's thickness rows over kRecordSplit lanes.
 constexpr int64_t kNearSplitPoints = (int64_t)1 << 17;
 
-// Per coil key, the near points (points with near pairs only; the coil loop is wave-uniform, so each coil's count
-// in a wave is one ballot and one atomic).
+// The records of each key (points with near pairs only; the coil loop is wave-uniform, so each key's count in a wave is
+// one ballot and one atomic). A block counts its points' keys in LDS where they fit (near_count_keys) and adds them up
+// at its end, in some thousand blocks: an atomic on the key per wave made 16,000 on one coil's few keys wait for one
+// another (a thin coil of 48 nodes, 2^20 points: counting and placing 542 us; now 270).
+constexpr int kCountBlocks = 1024;
+__host__ __device__ inline bool near_count_keys(const FieldParams &p) { return p.n_keys <= 10240; }   // 40 KB
 __global__ __launch_bounds__(256) void near_count_kernel(FieldParams p)
 {
-    const int64_t vi = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (vi >= p.n_pts) return;
-    const int64_t pi = p.order ? (int64_t)p.order[vi] : vi;   // the field kernel's visit order
-    if (p.near_counts[pi] == 0) return;
-    const double px = p.pts[3 * pi], py = p.pts[3 * pi + 1], pz = p.pts[3 * pi + 2];
+    extern __shared__ uint32_t key_counts[];
+    const bool lds = near_count_keys(p);
+    if (lds) {
+        for (int i = threadIdx.x; i < p.n_keys; i += 256) key_counts[i] = 0u;
+        __syncthreads();
+    }
+    uint32_t *hist = lds ? key_counts : p.near_hist;
     const int lane = threadIdx.x & 63;
-    // coils in ascending order, skipping those no point of the wave can be a record of
-    for (int c0 = 0; c0 < p.n_coils; c0 += 8)
-        for (uint32_t cand = record_candidates(p.coils, p.n_coils, c0, px, py, pz); cand; cand &= cand - 1) {
-            const CoilDev &c = p.coils[c0 + __builtin_ctz(cand)];
-            double z, r, cph, sph;
-            to_local(c, px, py, pz, z, r, cph, sph);
-            const int kind = record_kind(p, c, z, r, p.q & (Q_G | Q_GJ));   // the field kernel's test, bitwise
-            const uint32_t key = kind < 0 ? 0u : record_key(p, c, kind, z, r);
-            uint64_t todo = __ballot(kind >= 0);
-            while (todo) {
-                const uint32_t k = __builtin_amdgcn_readfirstlane(__shfl(key, __builtin_ctzll(todo)));
-                const uint64_t m = __ballot(kind >= 0 && key == k);
-                if (lane == __builtin_ctzll(m)) atomicAdd(&p.near_hist[k], (unsigned)__popcll(m));
-                todo &= ~m;
+    for (int64_t vi = (int64_t)blockIdx.x * 256 + threadIdx.x; vi < p.n_pts; vi += (int64_t)gridDim.x * 256) {
+        const int64_t pi = p.order ? (int64_t)p.order[vi] : vi;   // the field kernel's visit order
+        if (p.near_counts[pi] == 0) continue;
+        const double px = p.pts[3 * pi], py = p.pts[3 * pi + 1], pz = p.pts[3 * pi + 2];
+        // coils in ascending order, skipping those no point of the wave can be a record of
+        for (int c0 = 0; c0 < p.n_coils; c0 += 8)
+            for (uint32_t cand = record_candidates(p.coils, p.n_coils, c0, px, py, pz); cand; cand &= cand - 1) {
+                const CoilDev &c = p.coils[c0 + __builtin_ctz(cand)];
+                double z, r, cph, sph;
+                to_local(c, px, py, pz, z, r, cph, sph);
+                const int kind = record_kind(p, c, z, r, p.q & (Q_G | Q_GJ));   // the field kernel's test, bitwise
+                const uint32_t key = kind < 0 ? 0u : record_key(p, c, kind, z, r);
+                uint64_t todo = __ballot(kind >= 0);
+                while (todo) {
+                    const uint32_t k = __builtin_amdgcn_readfirstlane(__shfl(key, __builtin_ctzll(todo)));
+                    const uint64_t m = __ballot(kind >= 0 && key == k);
+                    if (lane == __builtin_ctzll(m)) atomicAdd(&hist[k], (unsigned)__popcll(m));
+                    todo &= ~m;
+                }
             }
-        }
+    }
+    if (!lds) return;
+    __syncthreads();
+    for (int i = threadIdx.x; i < p.n_keys; i += 256)
+        if (key_counts[i]) atomicAdd(&p.near_hist[i], key_counts[i]);
 }
 
 // One workgroup: cursor = exclusive prefix sum of near_hist over the keys, and the call's total. Four keys per thread
@@ -469,7 +484,12 @@ void launch_near_key_scan(hipStream_t s, const FieldParams &p)
 void launch_near_count(hipStream_t s, const FieldParams &p)
 {
     if (p.n_pts <= 0) return;
-    hipLaunchKernelGGL(near_count_kernel, dim3((unsigned)((p.n_pts + 255) / 256)), dim3(256), 0, s, p);
+    const unsigned blocks = (unsigned)((p.n_pts + 255) / 256);
+    if (near_count_keys(p))
+        hipLaunchKernelGGL(near_count_kernel, dim3(std::min<unsigned>(blocks, kCountBlocks)), dim3(256),
+                           sizeof(uint32_t) * (size_t)p.n_keys, s, p);
+    else
+        hipLaunchKernelGGL(near_count_kernel, dim3(blocks), dim3(256), 0, s, p);
 }
 
 void launch_near_fill(hipStream_t s, const FieldParams &p)

@@ -1,0 +1,51 @@
+"""The record pass (near pairs of CCOIL_FP32C, rule pairs of the series modes): its key counts, its padding and its grid.
+
+Values are compared with those of calls below 2^17 points, which sort and sum their records another way; the two differ
+by the rounding of FP64 sums, 1e-12 of the field's largest value. Times are the least of several device times, and their
+bounds are ratios within one run.
+"""
+import numpy as np
+import pytest
+import torch
+
+import ccoil_abi as abi
+from test_gpu_reduced_rules import COILS, _row
+
+pytestmark = pytest.mark.gpu
+
+FLAT80 = ("FLAT", 0.1, 0.05, 0.0, 80, 20)
+RECT40 = ("RECTANGULAR", 0.1, 0.1, 0.1, 40, 10)
+THIN48 = ("THIN", 0.3, 0.0, 0.2, 48, 1)
+
+
+def _set(kinds, n, rng, spread=0.3):
+    rows = []
+    for k in range(n):
+        row = _row(*kinds[k % len(kinds)])
+        row.update(pos=tuple(rng.normal(scale=spread, size=3)), alpha=float(rng.uniform(0, 3)), beta=float(rng.uniform(0, 6)))
+        rows.append(row)
+    return abi.CoilSet.from_rows(rows)
+
+
+# keys counted in LDS (up to 10,240: 208 coils of 49 slots) and in memory, and above 2,048 coils two slots instead of 49
+@pytest.mark.parametrize("n_coils", [1, 3, 208, 209, 2100])
+def test_many_keys(ctx, n_coils):
+    rng = np.random.default_rng(31)
+    cs = _set(COILS[:8] if n_coils > 1 else [FLAT80], n_coils, rng)
+    pts = rng.normal(scale=0.4, size=(131100, 3))
+    got, _ = ctx.fields(cs, pts, abi.B, abi.FP32C, abi.DIRECT)
+    ref, _ = ctx.fields(cs, pts[:100000], abi.B, abi.FP32C, abi.DIRECT)
+    assert np.max(np.abs(got["B"][:100000] - ref["B"])) <= 1e-12 * np.max(np.abs(ref["B"]))
+
+
+def test_one_coil_bookkeeping(ctx):
+    """Counting and placing the records of one coil, whose few keys every wave counts on, takes at most eight times as
+    long as its field kernel."""
+    cs = abi.CoilSet.from_rows([_row(*THIN48)])
+    pts = torch.from_numpy(np.random.default_rng(1).normal(scale=0.4, size=(1 << 20, 3))).cuda()
+    out = {"B": torch.empty_like(pts)}
+    reps = [ctx.fields(cs, pts, abi.B, abi.FP32C, abi.DIRECT | abi.DEVICE_POINTERS, out=out)[1] for _ in range(7)]
+    main = min(r.main_kernel_ms for r in reps)
+    rest = min(r.kernel_ms - r.main_kernel_ms - r.record_ms for r in reps)
+    print(f"\nfield kernel {1e3 * main:.0f} us, bookkeeping {1e3 * rest:.0f}")
+    assert rest <= 8 * main
