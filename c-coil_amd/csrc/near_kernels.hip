@@ -210,6 +210,19 @@ __global__ __launch_bounds__(256) void near_fill_kernel(FieldParams p)
     if (bad || (last == p.n_coils && slot != end)) atomicOr(&p.near_state->mismatch, 1u);
 }
 
+// Pointers to data that no kernel writes, in the constant address space: what a wave loads through them uniformly is a
+// scalar load also where the kernel stores in between.
+template <typename T> __device__ inline const T *constant(const T *p)
+{
+    return (const T *)(const T __attribute__((address_space(4))) *)(uintptr_t)p;
+}
+__device__ inline Tables constant(const Tables &t)
+{
+    return {constant(t.x), constant(t.w), constant(t.cosv), constant(t.omc), constant(t.xf), constant(t.wf), constant(t.cosf),
+            constant(t.omcf), constant(t.rcos), constant(t.rsin), constant(t.wcos), constant(t.wcosf), constant(t.opc),
+            constant(t.opcf), constant(t.ws), constant(t.ws2), constant(t.wcs), constant(t.wcsf), constant(t.leg)};
+}
+
 // Sum over the S lanes of a record by a fixed xor butterfly, so every lane of the group holds the same sum.
 __device__ inline void reduce_record(Local &L, int S)
 {
@@ -225,75 +238,81 @@ __device__ inline void reduce_record(Local &L, int S)
 }
 
 // Records sorted by rule class and coil. S consecutive lanes of a wave take one record (thickness rows sub, sub + S,
-// ...); its value goes to the record's slot. FLOAT: the kind-1 records [fp64, total) by the float rule, at 5 waves per
-// SIMD as field_kernel's float instances, S = kRecordSplit in calls with few points, where the records are too few to
-// fill the chip one lane each; else the kind-0 records [0, fp64) by the FP64 rule, S = kRecordSplit for the first
-// `split` of them (record_slot) and 1 for the others, whose reduced rules have at most a few hundred nodes. S follows
-// from the record and the call's shape alone, so a record's value does not depend on its wave.
+// ...); its value goes to the record's slot. FLOAT: the kind-1 records by the float rule, at 5 waves per SIMD as
+// field_kernel's float instances, S = kRecordSplit in calls with few points, where the records are too few to fill the
+// chip one lane each; else the kind-0 records by the FP64 rule, S = kRecordSplit for the split ones (record_slot) and 1
+// for the others, whose rules have at most a few hundred nodes. S follows from the record and the call's shape alone, so
+// a record's value does not depend on its wave.
 template <bool WA, bool WB, bool WG, bool FLOAT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FLOAT ? 5 : 1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FLOAT ? 5 : WA && (WB || WG) ? 2 : 3)))
 void near_eval_kernel(FieldParams p)
 {
     if (p.near_state->overflow) return;
-    const int64_t total = (int64_t)p.near_state->total, fp64 = (int64_t)p.near_state->fp64;
-    const int64_t hi = FLOAT ? total : fp64;
-    // waves of split records first; a split wave at the end of its range is part empty
-    const int64_t wave = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6;
-    const int64_t first = FLOAT ? fp64 : 0;
-    const int64_t n_split = FLOAT ? (p.n_pts < kNearSplitPoints ? total - fp64 : 0) : (int64_t)p.near_state->split;
+    const CoilDev *coils = constant(p.coils);
+    const uint32_t *near_coil = constant(p.near_coil);
+    const Tables tab = constant(p.tab);
+    const int64_t total = (int64_t)p.near_state->total, fp64_end = (int64_t)p.near_state->fp64;
+    // places [first, first + n_split) hold split records, those from there to hi one a lane; the waves of split records
+    // come first, and the last wave of either is part empty
+    const int64_t first = FLOAT ? fp64_end : 0, hi = FLOAT ? total : fp64_end;
+    const int64_t n_split = FLOAT ? (p.n_pts < kNearSplitPoints ? hi - first : 0) : (int64_t)p.near_state->split;
     const int64_t split_waves = (n_split * kRecordSplit + 63) >> 6;
-    const int S = __builtin_amdgcn_readfirstlane(wave < split_waves ? kRecordSplit : 1);
-    const int lane = (int)(threadIdx.x & 63), sub = lane % S;
-    const int64_t e = S > 1 ? first + wave * (64 / kRecordSplit) + lane / kRecordSplit
-                            : first + n_split + ((wave - split_waves) << 6) + lane;
-    if (e >= (S > 1 ? first + n_split : hi)) return;
-    const uint32_t key = p.near_keys[e];
-    const uint64_t rec = p.near_recs[e];
-    const int64_t pi = (int64_t)(rec >> 32), slot = (int64_t)(rec & 0xffffffffu);
-    // only a near_fill that reported a mismatch leaves records unwritten; never follow one out of bounds
-    if (pi >= p.n_pts || slot >= total) return;
-    double *o = p.near_vals + slot * p.near_width;
-    // A wave holds one coil's records, or two or more at the boundaries of the sorted keys: it takes its keys one at a
-    // time (the key of the lowest lane still to do, read into a scalar register), and every lane evaluates that coil
-    // at its point, keeping the value only if the key is its own. The control flow stays uniform and no store
-    // precedes the loads, so the coil's fields and the quadrature tables are scalar loads, as in field_kernel; a
-    // divergent branch would take the same issue time. todo is wave-uniform and loses at least one lane on every pass;
-    // a group's lanes share their key, so a group is always active as a whole.
-    const double px = p.pts[3 * pi], py = p.pts[3 * pi + 1], pz = p.pts[3 * pi + 2];
-    Cart acc;
-    for (int j = 0; j < 3; ++j) { acc.A[j] = 0.0; acc.E[j] = 0.0; acc.B[j] = 0.0; }
-    for (int j = 0; j < 9; ++j) acc.G[j] = 0.0;
-    uint64_t todo = __ballot(1);
-    while (todo) {
-        const uint32_t k = __builtin_amdgcn_readfirstlane(__shfl(key, __builtin_ctzll(todo)));
-        const bool mine = key == k;
-        todo &= ~(uint64_t)__ballot(mine);
-        // only a reported mismatch can leave a key outside the range's kind
-        const uint32_t slot_of = k / (uint32_t)p.n_coils;
-        if (k >= (uint32_t)p.n_keys || (slot_of == (uint32_t)p.n_slots) != FLOAT) continue;
-        const CoilDev &c = p.coils[p.near_coil[k - slot_of * (uint32_t)p.n_coils]];
-        double z, r, cph, sph;
-        to_local(c, px, py, pz, z, r, cph, sph);
-        // FP64 records take their rule classes one at a time too (a slot holds one class, but for the coils of few
-        // rows): the rule's node sets stay uniform, hence scalar loads
-        const int cls = FLOAT ? 0 : rule_class(c, z, r);
-        uint64_t left = __ballot(mine);
-        while (left) {
-            const int q = FLOAT ? 0 : __builtin_amdgcn_readfirstlane(__shfl(cls, __builtin_ctzll(left)));
-            const bool sel = mine && cls == q;
-            left &= ~(uint64_t)__ballot(sel);
-            Local L;
-            if (FLOAT) eval_stable<float, WA, WB, WG>(c, p.tab, full_rule(c), z, r, sub, S, 0, 1, L);
-            else eval_stable<f64s, WA, WB, WG>(c, p.tab, class_rule(c, q), z, r, sub, S, 0, 1, L);
-            reduce_record(L, S);
-            if (sel) accumulate_global(c, L, r, cph, sph, p.q, acc);
+    const int64_t waves = split_waves + ((hi - first - n_split + 63) >> 6);
+    const int lane = (int)(threadIdx.x & 63);
+    // the bounded grid strides over the waves' worth of records there are; the bounds are wave-uniform
+    for (int64_t wave = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 6; wave < waves; wave += (int64_t)gridDim.x * 4) {
+        const int S = __builtin_amdgcn_readfirstlane(wave < split_waves ? kRecordSplit : 1), sub = lane % S;
+        const int64_t e = S > 1 ? first + wave * (64 / kRecordSplit) + lane / kRecordSplit
+                                : first + n_split + ((wave - split_waves) << 6) + lane;
+        if (e >= (S > 1 ? first + n_split : hi)) continue;
+        const uint32_t key = p.near_keys[e];
+        const uint64_t rec = p.near_recs[e];
+        const int64_t pi = (int64_t)(rec >> 32), slot = (int64_t)(rec & 0xffffffffu);
+        // only a near_fill that reported a mismatch leaves records unwritten; never follow one out of bounds
+        if (pi >= p.n_pts || slot >= total) continue;
+        // A wave holds one coil's records, or two or more at the boundaries of the sorted keys: it takes its keys one at a
+        // time (the key of the lowest lane still to do, read into a scalar register), and every lane evaluates that
+        // coil at its point, keeping the value only if the key is its own. The control flow stays uniform and the coils
+        // and tables are in constant memory to the compiler, so that their loads are scalar, as in field_kernel,
+        // whatever the loop stores; a divergent branch would take the same issue time. todo is wave-uniform and loses
+        // at least one lane on every pass; a group's lanes share their key, so a group is always active as a whole.
+        const double px = p.pts[3 * pi], py = p.pts[3 * pi + 1], pz = p.pts[3 * pi + 2];
+        Cart acc;
+        for (int j = 0; j < 3; ++j) { acc.A[j] = 0.0; acc.E[j] = 0.0; acc.B[j] = 0.0; }
+        for (int j = 0; j < 9; ++j) acc.G[j] = 0.0;
+        uint64_t todo = __ballot(1);
+        while (todo) {
+            const uint32_t k = __builtin_amdgcn_readfirstlane(__shfl(key, __builtin_ctzll(todo)));
+            const bool mine = key == k;
+            todo &= ~(uint64_t)__ballot(mine);
+            // only a reported mismatch can leave a key outside the range's kind
+            const uint32_t slot_of = k / (uint32_t)p.n_coils;
+            if (k >= (uint32_t)p.n_keys || (slot_of == (uint32_t)p.n_slots) != FLOAT) continue;
+            const CoilDev &c = coils[near_coil[k - slot_of * (uint32_t)p.n_coils]];
+            double z, r, cph, sph;
+            to_local(c, px, py, pz, z, r, cph, sph);
+            // FP64 records take their rule classes one at a time too (a slot holds one class, but for the coils of few
+            // rows): the rule's node sets stay uniform, hence scalar loads
+            const int cls = FLOAT ? 0 : rule_class(c, z, r);
+            uint64_t left = __ballot(mine);
+            while (left) {
+                const int q = FLOAT ? 0 : __builtin_amdgcn_readfirstlane(__shfl(cls, __builtin_ctzll(left)));
+                const bool sel = mine && cls == q;
+                left &= ~(uint64_t)__ballot(sel);
+                Local L;
+                if (FLOAT) eval_stable<float, WA, WB, WG>(c, tab, full_rule(c), z, r, sub, S, 0, 1, L);
+                else eval_stable<f64s, WA, WB, WG>(c, tab, class_rule(c, q), z, r, sub, S, 0, 1, L);
+                reduce_record(L, S);
+                if (sel) accumulate_global(c, L, r, cph, sph, p.q, acc);
+            }
         }
-    }
-    if (sub == 0) {
-        if (p.A) { for (int j = 0; j < 3; ++j) o[j] = acc.A[j]; o += 3; }
-        if (p.E) { for (int j = 0; j < 3; ++j) o[j] = acc.E[j]; o += 3; }
-        if (p.B) { for (int j = 0; j < 3; ++j) o[j] = acc.B[j]; o += 3; }
-        if (p.G) for (int j = 0; j < 9; ++j) o[j] = acc.G[j];
+        if (sub == 0) {
+            double *o = p.near_vals + slot * p.near_width;
+            if (p.A) { for (int j = 0; j < 3; ++j) o[j] = acc.A[j]; o += 3; }
+            if (p.E) { for (int j = 0; j < 3; ++j) o[j] = acc.E[j]; o += 3; }
+            if (p.B) { for (int j = 0; j < 3; ++j) o[j] = acc.B[j]; o += 3; }
+            if (p.G) for (int j = 0; j < 9; ++j) o[j] = acc.G[j];
+        }
     }
 }
 
@@ -535,16 +554,22 @@ static void launch_near_eval_group(hipStream_t s, const FieldParams &p, unsigned
     }
 }
 
-// Each grid covers the capacity with every record split (float records of large calls: none); the waves beyond the
-// records there are (read on the device) return at once.
+// The grid covers the capacity at `lanes` lanes a place up to kEvalBlocks blocks, some eight times what the chip holds at
+// once, and strides beyond. (A wave that finds no record costs a nanosecond: 75,000 of them, for the default
+// capacity of 262,145 points and hardly any record, took 75 us. And the capacity can pass the 2^32 threads of a launch:
+// 2^29 records split over eight lanes.)
+constexpr int64_t kEvalBlocks = 16384;
+static unsigned near_eval_blocks(const FieldParams &p, int lanes)
+{
+    return (unsigned)std::min<int64_t>((p.near_cap * lanes + 255) / 256, kEvalBlocks);
+}
+
 void launch_near_eval(hipStream_t s, const FieldParams &p)
 {
     if (p.near_cap <= 0) return;
-    const unsigned split = (unsigned)((p.near_cap * kRecordSplit + 255) / 256 + 1);
-    if (uniform_records(p)) launch_near_eval_g<false>(s, p, split);
+    if (uniform_records(p)) launch_near_eval_g<false>(s, p, near_eval_blocks(p, kRecordSplit));
     else launch_near_eval_group(s, p, (unsigned)std::min<int64_t>((p.near_cap + 3) / 4, 8192));
-    if (p.float_records)
-        launch_near_eval_g<true>(s, p, p.n_pts < kNearSplitPoints ? split : (unsigned)((p.near_cap + 255) / 256));
+    if (p.float_records) launch_near_eval_g<true>(s, p, near_eval_blocks(p, p.n_pts < kNearSplitPoints ? kRecordSplit : 1));
 }
 
 void launch_near_add(hipStream_t s, const FieldParams &p)

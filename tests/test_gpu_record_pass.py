@@ -49,3 +49,23 @@ def test_one_coil_bookkeeping(ctx):
     rest = min(r.kernel_ms - r.main_kernel_ms - r.record_ms for r in reps)
     print(f"\nfield kernel {1e3 * main:.0f} us, bookkeeping {1e3 * rest:.0f}")
     assert rest <= 8 * main
+
+
+def test_capacity_beyond_a_launch():
+    """2^28 points and two coils: room for 2^29 records, which split over eight lanes would be 2^32 threads in one
+    dimension. (A context of its own, which gives some 40 GB back.)"""
+    ctx = abi.Context(0)
+    try:
+        cs = _set([("FILAMENT", 0.25, 0.0, 0.0, 6, 1)], 2, np.random.default_rng(2), 0.1)
+        n = 1 << 28
+        g = torch.Generator(device="cuda").manual_seed(7)
+        pts = torch.rand((n, 3), dtype=torch.float64, device="cuda", generator=g) - 0.5
+        out = {"B": torch.empty_like(pts)}
+        ctx.fields(cs, pts, abi.B, abi.FP32C, abi.DIRECT | abi.DEVICE_POINTERS, out=out)
+        some = torch.cat([pts[:1000], pts[-1000:]])
+        ref, _ = ctx.fields(cs, some.cpu().numpy(), abi.B, abi.FP32C, abi.DIRECT)
+        got = torch.cat([out["B"][:1000], out["B"][-1000:]]).cpu().numpy()
+        assert np.max(np.abs(got - ref["B"])) <= 1e-5 * np.max(np.abs(ref["B"]))   # float nodes, by other lanes
+    finally:
+        ctx.close()
+        torch.cuda.empty_cache()
