@@ -213,11 +213,12 @@ ccoil_status near_buffers(ccoil_ctx ctx, FieldLaunch &L, int64_t cap, int width,
         return st;
     if ((st = call_buffer(ctx, ctx->nstate, arena, sizeof(NearState), &state)) != CCOIL_OK) return st;
     if ((st = call_buffer(ctx, ctx->ntemp, arena, tb > 0 ? tb : 1, &temp)) != CCOIL_OK) return st;
-    const size_t per_record = sizeof(uint32_t) + sizeof(uint64_t) + sizeof(double) * (size_t)width;
-    if (arena) cap = std::min<int64_t>(cap, (int64_t)((arena->left() > 768 ? arena->left() - 768 : 0) / per_record));
+    const size_t per_record = kRecordBytes + sizeof(double) * (size_t)width;
+    const size_t pad = (size_t)record_places(p, 0);
+    if (arena) cap = std::min<int64_t>(cap, (int64_t)((arena->left() > 768 + pad * kRecordBytes ? arena->left() - 768 - pad * kRecordBytes : 0) / per_record));
     cap = std::max<int64_t>(cap, 1);
-    if ((st = call_buffer(ctx, ctx->nkeys, arena, sizeof(uint32_t) * (size_t)cap, &keys)) != CCOIL_OK) return st;
-    if ((st = call_buffer(ctx, ctx->nrecs, arena, sizeof(uint64_t) * (size_t)cap, &recs)) != CCOIL_OK) return st;
+    if ((st = call_buffer(ctx, ctx->nkeys, arena, sizeof(uint32_t) * ((size_t)cap + pad), &keys)) != CCOIL_OK) return st;
+    if ((st = call_buffer(ctx, ctx->nrecs, arena, sizeof(uint64_t) * ((size_t)cap + pad), &recs)) != CCOIL_OK) return st;
     if ((st = call_buffer(ctx, ctx->nvals, arena, sizeof(double) * (size_t)width * (size_t)cap, &vals)) != CCOIL_OK)
         return st;
     if (!arena) ctx->near_cap = std::max(ctx->near_cap, cap);

@@ -16,7 +16,9 @@ struct NearState {
     unsigned int overflow;      // total > near_cap: the pass was skipped
     unsigned int mismatch;      // near_fill classified a pair differently from field_kernel
     unsigned long long fp64;    // records of kind 0 (FP64 rule)
-    unsigned long long split;   // records of kind 0 that are split over more lanes (the first ones)
+    // places in the record arrays (the keys' padding counts): the ends of the records of kind 0 that are split over more
+    // lanes (the first ones), of kind 0, and of all
+    unsigned long long split_end, fp64_end, end;
 };
 
 struct FieldParams {
@@ -58,7 +60,7 @@ struct FieldParams {
     uint32_t *near_cursor;    // [n_keys + 1] next free record of each key
     NearState *near_state;
     int64_t near_cap;
-    uint32_t *near_keys;
+    uint32_t *near_keys;      // record_places(near_cap) keys and records
     const uint32_t *near_coil;               // near_key -> coil index
     uint64_t *near_recs;
     double *near_vals;
@@ -98,8 +100,8 @@ __host__ __device__ inline bool uniform_records(const FieldParams &p)
 // the rest of the launch come first, and near_eval splits them over more lanes; with two slots that is all. Else
 // uniform records are sorted by rule class, the costliest first, so that a wave holds one coil's records of one
 // class: the split ones, with the coil's own angular rule and at least kRecordSplit thickness rows, take the first
-// kSplitSlots slots. Grouped records are sorted by their node count in steps of four, the split ones with kGroupSplit
-// nodes or more. Float records follow by coil.
+// kSplitSlots slots. Grouped records are sorted by their node count in steps of four, the split ones with kGroupSplit nodes or more.
+// Float records follow by coil.
 constexpr int kRecordSplit = 8;
 constexpr int kSplitSlots = kRedThk;
 constexpr int kGroupSplit = 640;
@@ -111,13 +113,28 @@ __device__ inline uint32_t record_slot(const FieldParams &p, const CoilDev &c, i
     if (uniform_records(p)) {
         const int k = cls / (kRedThk + 1), t = cls - k * (kRedThk + 1);
         const bool rows = t == 0 ? c.n_thk >= kRecordSplit : t < kRedThk;   // at least kRecordSplit
-        if (p.n_slots == 2) return k == 0 && rows ? 0u : 1u;
-        return (uint32_t)(rows ? cls : k * (kRedThk + 1) + kRedThk);
+        const bool split = k == 0 && rows;
+        if (p.n_slots == 2) return split ? 0u : 1u;
+        return (uint32_t)(split || (k > 0 && rows) ? cls : k * (kRedThk + 1) + kRedThk);
     }
     const RuleSel s = class_rule(c, cls);
     const int n = s.na * s.nt;
     if (p.n_slots == 2) return n >= kGroupSplit ? 0u : 1u;
     return n >= kGroupSplit ? 0u : n >= kGroupSplit / 4 ? 1u : n >= kGroupSplit / 16 ? 2u : 3u;
+}
+// Uniform records of all slots start each key at a wave of its own: a wave whose records are of several keys takes them
+// in turn, and where classes are rare a wave of a dozen keys and rules outlasted the rest of the launch (40 coils of
+// 80 x 20 slow nodes, 131,072 points, series mode: 443 us; in waves of one key 28). key_align: the places that a key's
+// records are padded to (near_key_scan marks the padding kNoKey); record_places: the places that n records may take.
+constexpr uint32_t kNoKey = 0xffffffffu;
+constexpr size_t kRecordBytes = sizeof(uint32_t) + sizeof(uint64_t);   // of one place: its key and its record
+__host__ __device__ inline uint32_t key_align(const FieldParams &p, int key)
+{
+    return p.n_slots != kRuleClasses ? 1u : key < kSplitSlots * p.n_coils ? 64u / kRecordSplit : 64u;
+}
+__host__ __device__ inline int64_t record_places(const FieldParams &p, int64_t n)
+{
+    return n + (p.n_slots != kRuleClasses ? 0 : (int64_t)64 * p.n_keys);
 }
 __device__ inline uint32_t record_key(const FieldParams &p, const CoilDev &c, int kind, double z, double r)
 {

@@ -97,20 +97,29 @@ __global__ __launch_bounds__(256) void near_count_kernel(FieldParams p)
         if (key_counts[i]) atomicAdd(&p.near_hist[i], key_counts[i]);
 }
 
-// One workgroup: cursor = exclusive prefix sum of near_hist over the keys, and the call's total. Four keys per thread
-// and iteration, scanned by waves: a call's few thousand keys (coils x rule classes) take two iterations.
+// One workgroup: cursor = exclusive prefix sum of near_hist over the keys, each padded to key_align, and the call's
+// total. Four keys per thread and iteration, scanned by waves: a call's few thousand keys (coils x rule classes) take two
+// iterations.
 constexpr int kKeyScanThreads = 1024;
 __global__ __launch_bounds__(kKeyScanThreads) void near_key_scan_kernel(FieldParams p)
 {
     __shared__ uint32_t wsum[kKeyScanThreads / 64];
+    __shared__ uint32_t n_fp64;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nk = p.n_keys + 1;
-    uint32_t carry = 0;
+    const int k_fp64 = p.n_slots * p.n_coils;   // the kind-0 keys come first, and of those the split ones
+    const int k_split = (p.n_slots == kRuleClasses ? kSplitSlots : 1) * p.n_coils;
+    const unsigned long long total = (unsigned long long)(p.near_offsets[p.n_pts - 1] + p.near_counts[p.n_pts - 1]);
+    const bool overflow = total > (unsigned long long)p.near_cap;
+    if (t == 0) n_fp64 = 0u;
+    uint32_t carry = 0, fp64 = 0;
     for (int base = 0; base < nk; base += 4 * kKeyScanThreads) {
         const int i0 = base + 4 * t;
-        uint32_t v[4], own = 0;
+        uint32_t v[4], pad[4], own = 0;
         for (int k = 0; k < 4; ++k) {
             v[k] = i0 + k < p.n_keys ? p.near_hist[i0 + k] : 0u;
-            own += v[k];
+            pad[k] = (0u - v[k]) & (key_align(p, i0 + k) - 1u);
+            own += v[k] + pad[k];
+            if (i0 + k < k_fp64) fp64 += v[k];
         }
         uint32_t incl = own;   // inclusive scan of the wave's threads
         for (int d = 1; d < 64; d <<= 1) {
@@ -126,23 +135,25 @@ __global__ __launch_bounds__(kKeyScanThreads) void near_key_scan_kernel(FieldPar
         }
         uint32_t run = carry + before + incl - own;
         for (int k = 0; k < 4; ++k) {
+            if (i0 + k == k_split) p.near_state->split_end = run;
+            if (i0 + k == k_fp64) p.near_state->fp64_end = run;
             if (i0 + k < nk) p.near_cursor[i0 + k] = run;
             run += v[k];
+            if (!overflow)   // else the arrays may not reach there, and nothing reads them
+                for (uint32_t i = 0; i < pad[k]; ++i) p.near_keys[run + i] = kNoKey;
+            run += pad[k];
         }
         carry += all;
         __syncthreads();
     }
+    if (fp64) atomicAdd(&n_fp64, fp64);
+    __syncthreads();
     if (t == 0) {
-        const unsigned long long total =
-            (unsigned long long)(p.near_offsets[p.n_pts - 1] + p.near_counts[p.n_pts - 1]);
         p.near_state->total = total;
-        p.near_state->overflow = total > (unsigned long long)p.near_cap ? 1u : 0u;
+        p.near_state->overflow = overflow ? 1u : 0u;
+        p.near_state->fp64 = n_fp64;
+        p.near_state->end = carry;
     }
-    // the threads that wrote these cursors: the kind-0 keys come first, and of those the split ones
-    const int64_t k_fp64 = (int64_t)p.n_slots * p.n_coils;
-    const int64_t k_split = (int64_t)(p.n_slots == kRuleClasses ? kSplitSlots : 1) * p.n_coils;
-    if (k_fp64 / 4 % kKeyScanThreads == t) p.near_state->fp64 = p.near_cursor[k_fp64];
-    if (k_split / 4 % kKeyScanThreads == t) p.near_state->split = p.near_cursor[k_split];
 }
 
 // Coils of a block row of near_fill_kernel: a multiple of record_candidates' eight.
@@ -156,7 +167,7 @@ __global__ __launch_bounds__(256) void near_fill_kernel(FieldParams p)
     const int64_t pi = p.order ? (int64_t)p.order[vi] : vi;
     const int64_t count = p.near_counts[pi];
     if (count == 0) return;
-    const uint64_t total = p.near_state->total;
+    const uint64_t places = p.near_state->end;
     const double px = p.pts[3 * pi], py = p.pts[3 * pi + 1], pz = p.pts[3 * pi + 2];
     int64_t slot = p.near_offsets[pi];
     const int64_t end = slot + count;
@@ -197,7 +208,7 @@ __global__ __launch_bounds__(256) void near_fill_kernel(FieldParams p)
             if (kind >= 0) {
                 const uint64_t pos = base + (uint64_t)__popcll(same & ((1ull << lane) - 1ull));
                 // a pair classified differently from the series or field kernel: report it, write nothing
-                if (slot >= end || pos >= total) {
+                if (slot >= end || pos >= places) {
                     bad = true;
                     continue;
                 }
@@ -251,11 +262,11 @@ void near_eval_kernel(FieldParams p)
     const CoilDev *coils = constant(p.coils);
     const uint32_t *near_coil = constant(p.near_coil);
     const Tables tab = constant(p.tab);
-    const int64_t total = (int64_t)p.near_state->total, fp64_end = (int64_t)p.near_state->fp64;
+    const int64_t total = (int64_t)p.near_state->total, fp64_end = (int64_t)p.near_state->fp64_end;
     // places [first, first + n_split) hold split records, those from there to hi one a lane; the waves of split records
     // come first, and the last wave of either is part empty
-    const int64_t first = FLOAT ? fp64_end : 0, hi = FLOAT ? total : fp64_end;
-    const int64_t n_split = FLOAT ? (p.n_pts < kNearSplitPoints ? hi - first : 0) : (int64_t)p.near_state->split;
+    const int64_t first = FLOAT ? fp64_end : 0, hi = FLOAT ? (int64_t)p.near_state->end : fp64_end;
+    const int64_t n_split = FLOAT ? (p.n_pts < kNearSplitPoints ? hi - first : 0) : (int64_t)p.near_state->split_end;
     const int64_t split_waves = (n_split * kRecordSplit + 63) >> 6;
     const int64_t waves = split_waves + ((hi - first - n_split + 63) >> 6);
     const int lane = (int)(threadIdx.x & 63);
@@ -266,11 +277,12 @@ void near_eval_kernel(FieldParams p)
                                 : first + n_split + ((wave - split_waves) << 6) + lane;
         if (e >= (S > 1 ? first + n_split : hi)) continue;
         const uint32_t key = p.near_keys[e];
+        if (key == kNoKey) continue;
         const uint64_t rec = p.near_recs[e];
         const int64_t pi = (int64_t)(rec >> 32), slot = (int64_t)(rec & 0xffffffffu);
         // only a near_fill that reported a mismatch leaves records unwritten; never follow one out of bounds
         if (pi >= p.n_pts || slot >= total) continue;
-        // A wave holds one coil's records, or two or more at the boundaries of the sorted keys: it takes its keys one at a
+        // A wave holds one key's records or, where keys are not padded, those of several: it takes its keys one at a
         // time (the key of the lowest lane still to do, read into a scalar register), and every lane evaluates that
         // coil at its point, keeping the value only if the key is its own. The control flow stays uniform and the coils
         // and tables are in constant memory to the compiler, so that their loads are scalar, as in field_kernel,
@@ -324,7 +336,7 @@ template <bool WA, bool WB, bool WG>
 __global__ __launch_bounds__(256) void near_eval_group_kernel(FieldParams p)
 {
     if (p.near_state->overflow) return;
-    const int64_t n_split = (int64_t)p.near_state->split, fp64 = (int64_t)p.near_state->fp64;
+    const int64_t n_split = (int64_t)p.near_state->split_end, fp64 = (int64_t)p.near_state->fp64_end;   // no padding
     const int64_t waves = n_split + (fp64 - n_split + 64 / kRecordSplit - 1) / (64 / kRecordSplit);
     const int lane = (int)(threadIdx.x & 63);
     // a bounded grid strides over the waves' worth of records; the bound is wave-uniform
@@ -561,7 +573,7 @@ static void launch_near_eval_group(hipStream_t s, const FieldParams &p, unsigned
 constexpr int64_t kEvalBlocks = 16384;
 static unsigned near_eval_blocks(const FieldParams &p, int lanes)
 {
-    return (unsigned)std::min<int64_t>((p.near_cap * lanes + 255) / 256, kEvalBlocks);
+    return (unsigned)std::min<int64_t>((record_places(p, p.near_cap) * lanes + 255) / 256, kEvalBlocks);
 }
 
 void launch_near_eval(hipStream_t s, const FieldParams &p)

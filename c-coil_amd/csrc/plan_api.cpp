@@ -119,8 +119,8 @@ ccoil_status ccoil_fields_plan(ccoil_ctx ctx, const ccoil_coils *coils, const do
     bytes += probe.L.far_bytes;
     if (probe.L.near) {
         bytes += 2 * sizeof(int64_t) * (size_t)probe.n + 2 * sizeof(uint32_t) * ((size_t)pp.n_keys + 2) + sizeof(NearState) +
-                 probe.L.scan_bytes + (size_t)pp.near_cap * (sizeof(uint32_t) + sizeof(uint64_t) +
-                                                             sizeof(double) * (size_t)probe.width) + 8 * 256;
+                 probe.L.scan_bytes + (size_t)record_places(pp, pp.near_cap) * kRecordBytes +
+                 (size_t)pp.near_cap * sizeof(double) * (size_t)probe.width + 8 * 256;
         plan->near = true;
         plan->fp32c = precision == CCOIL_FP32C;
         plan->near_cap = pp.near_cap;

@@ -69,3 +69,20 @@ def test_capacity_beyond_a_launch():
     finally:
         ctx.close()
         torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("coil,mode,flags", [(FLAT80, abi.FP64, abi.FAR_FIELD), (RECT40, abi.FP32C, 0)])
+def test_time_where_the_layout_changes(ctx, coil, mode, flags):
+    """40 coils in a cloud that meets most classes rarely: 2^17 points, the least whose records are summed by waves of one
+    key, take no longer than 1.6 times those of an eighth fewer. (Float records change their lanes there too, one where
+    there were eight, so that long rules' are left out.)"""
+    rng = np.random.default_rng(1)
+    cs = _set([coil], 40, rng)
+    pts = torch.from_numpy(rng.uniform(-0.8, 0.8, size=(1 << 17, 3))).cuda()
+    out = {"B": torch.empty_like(pts)}
+    ms = {}
+    for n in (114688, 1 << 17):
+        ms[n] = min(ctx.fields(cs, pts[:n], abi.B, mode, flags | abi.DEVICE_POINTERS, out={"B": out["B"][:n]})[1].record_ms
+                    for _ in range(7))
+    print(f"\n{coil}: " + ", ".join(f"{n} points {1e3 * v:.0f} us" for n, v in ms.items()))
+    assert ms[1 << 17] <= 1.6 * ms[114688]
