@@ -118,22 +118,6 @@ __device__ inline double scalar(double v)
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
-// x / d for a wave-uniform d, leaving the remainder in x: the float quotient is within one of it (x < 2^24, or x < 2 d).
-__device__ inline uint32_t divide(uint32_t &x, uint32_t d)
-{
-    uint32_t q = (uint32_t)((float)x * __builtin_amdgcn_rcpf((float)d));
-    int64_t r = (int64_t)x - (int64_t)q * d;
-    if (r < 0) {
-        --q;
-        r += d;
-    } else if (r >= (int64_t)d) {
-        ++q;
-        r -= d;
-    }
-    x = (uint32_t)r;
-    return q;
-}
-
 // Minimum waves per SIMD: the FP64 kernels' short rules leave the spills of node generation in the way (8,192 pairs,
 // M and F: 16.3 ms at four waves, 15.5 at three, 15.7 at two; the gradient of 256 pairs 2.22, 1.84, 1.72 ms).
 template <int PREC, bool GR> constexpr int kPairWaves = PREC != 0 ? 4 : GR ? 2 : 3;
@@ -181,6 +165,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPairWaves<P
         const int64_t first_rest = n0 / NA;
         const uint32_t ia0 = (uint32_t)(n0 % NA), it0 = (uint32_t)(first_rest % NT), il0 = (uint32_t)(first_rest / NT);
         const int n_item = (int)(n1 - n0);
+        const bool wide = max(max((uint32_t)NA, (uint32_t)NT), il0) + (uint32_t)pd.nodes_per_item >= kFloatDigits;
+        auto divide = [&](uint32_t &x, uint32_t d) {   // d, wide: wave-uniform
+            return divide_digit(x, d, __builtin_amdgcn_rcpf((float)d), wide);
+        };
         auto node = [&](int j0, Node &n) {
             uint32_t ia = ia0 + (uint32_t)j0, it, il, ba = 0, bt = 0, bl = 0;
             it = it0 + divide(ia, (uint32_t)NA);

@@ -20,6 +20,29 @@ struct PairDev {
     double f_scale;        // 2 pi N2 I2 / blocks, or 2 pi N2 / I1 (reference arrangement scale)
 };
 
+// x / d, leaving the remainder in x; inv: about 1 / d, within an ulp. The float quotient of an x below kFloatDigits is
+// within one of the exact one; wide: x may be larger (a ring of millions of nodes in blocks), the integer division.
+constexpr uint32_t kFloatDigits = 1u << 22;
+__host__ __device__ inline uint32_t divide_digit(uint32_t &x, uint32_t d, float inv, bool wide)
+{
+    if (wide) {
+        const uint32_t q = x / d;
+        x -= q * d;
+        return q;
+    }
+    uint32_t q = (uint32_t)((float)x * inv);
+    int64_t r = (int64_t)x - (int64_t)q * d;
+    if (r < 0) {
+        --q;
+        r += d;
+    } else if (r >= (int64_t)d) {
+        ++q;
+        r -= d;
+    }
+    x = (uint32_t)r;
+    return q;
+}
+
 struct PairParams {
     const CoilDev *prim;
     const CoilDev *sec;
