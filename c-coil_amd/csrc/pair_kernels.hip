@@ -23,14 +23,18 @@ __device__ inline double wave_sum(double v)
     return v;
 }
 
-// PREC: 0 FP64 (stable integrands, refined hardware reciprocals), 1 FP32C (stable in FP32, near-winding
+// PREC: 0 FP64 (stable integrands, refined hardware reciprocals; reduced rules), 5 the same at the primary's own nodes
+// (kPairOwn), 1 FP32C (stable in FP32, near-winding
 // nodes as in FP64), 2 FP32 (reference integrands in float), 3 FP64 reference integrands, 4 FP64 with IEEE
 // division and square root.
 template <int PREC, bool WM, bool WF, bool GR>
 __device__ inline void eval_prim(const CoilDev &pc, const Tables &tab, double z, double r, int row0, int rstep,
                                  Local &L, AdjA *ada)
 {
-    if constexpr (PREC == 4) {
+    if constexpr (PREC == kPairOwn) {
+        if constexpr (GR) eval_stable<f64s, true, true, false, false, true>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L, nullptr, ada);
+        else eval_stable<f64s, WM, WF, false, false, false, true>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L);
+    } else if constexpr (PREC == 4) {
         if constexpr (GR) eval_stable<double, true, true, false, false, true>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L, nullptr, ada);
         else eval_stable<double, WM, WF, false>(pc, tab, full_rule(pc), z, r, row0, rstep, 0, 1, L);
     } else if constexpr (PREC == 2) {
@@ -387,8 +391,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPairWaves<P
                 node(k, n);
                 Local L = {0, 0, 0, 0, 0, 0, 0};
                 AdjA q;
-                eval_prim<PREC, kA, kB, kAda>(pc, p.tab, n.z, n.r, rg, pd.row_groups, L, &q);
-                add(n, L, q);
+                const bool far = PREC == kPairOwn && !GR && p.mp && is_far(pc, n.z, n.r);
+                if (!far) eval_prim<PREC, kA, kB, kAda>(pc, p.tab, n.z, n.r, rg, pd.row_groups, L, &q);
+                if (PREC == kPairOwn) series(n, far, L, q);
+                if (!far || rg == 0) add(n, L, q);
             }
         }
         if constexpr (GR) {
@@ -487,6 +493,7 @@ void launch_pairs(hipStream_t s, const PairParams &p)
     if (p.n_items <= 0) return;
     if (p.mp) launch_multipole_moments(s, p.prim, p.n_prim, p.tab, p.mp);
     if (p.precision == 0) launch_pairs_p<0>(s, p);
+    else if (p.precision == kPairOwn) launch_pairs_p<kPairOwn>(s, p);
     else if (p.precision == 4) launch_pairs_p<4>(s, p);
     else if (p.precision == 2) launch_pairs_p<2>(s, p);
     else if (p.precision == 3) launch_pairs_p<3>(s, p);

@@ -51,7 +51,7 @@ struct PairParams {
     int64_t n_items;
     double *partial;                 // kPairTerms doubles per item: M, F[3], T[3], dM/dp[3]
     uint32_t what;                   // 1: M, 2: F and T, 4: dM/d(secondary position), 8: the full gradient of M
-    int32_t precision;
+    int32_t precision;               // of the call, or kPairOwn
     Tables tab;
     double *M, *F, *T, *dM;          // outputs (device), indexed by PairDev::out
     double *grad;                    // what & 8: kPairGradOut doubles per pair
@@ -61,6 +61,7 @@ struct PairParams {
     int32_t n_prim;
 };
 constexpr int kPairTerms = 10;
+constexpr int kPairOwn = 5;          // CCOIL_FP64's arithmetic at the primaries' own nodes (build_pairs)
 // The gradient of M (what & 8): per item M and 13 derivative sums, dM/d(secondary x, y, z, alpha, beta, R, a, b,
 // primary alpha, beta, R, a, b); per pair 16 outputs, the secondary's 8 then the primary's 8 (x, y, z, alpha, beta,
 // R, a, b), the primary's position derivative being minus the secondary's.

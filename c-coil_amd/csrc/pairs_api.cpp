@@ -14,7 +14,7 @@ namespace {
 // Primary-node evaluations per lane and work item. Large batches give every lane about 8192 of the planned rule's
 // (each item's fixed costs, the wave reduction and the partial, stay small); a batch with too little work to give the
 // 1,024 SIMDs about 4 waves each at that size lowers it, down to 256, so that a single pair or a few pairs still spread
-// over the chip instead of running one long chain per lane. Powers of two only. The FP64 kernels, which evaluate
+// over the chip instead of running one long chain per lane. Powers of two only. The FP64 kernels, where they evaluate
 // reduced rules, count those rules' nodes (rule_nodes_of), of which a lane takes up to 2048 and down to 16.
 int64_t lane_target(int64_t node_pairs, bool reduced)
 {
@@ -65,6 +65,36 @@ bool series_only(const CoilDev &p, const CoilDev &s)
     return gap > 0.0 && gap * gap > p.far_d2;
 }
 
+int64_t node_count(const CoilDev &s)   // of a secondary
+{
+    return (int64_t)s.blk_ang * s.n_ang * s.blk_thk * s.n_thk * s.blk_len * s.n_len;
+}
+
+// Flat primaries of few angular and all in all few nodes: most of a secondary's nodes keep all of them, and classes, queues,
+// nodes made twice and the registers of it all cost more than the rest saves. (The fast method's nodes cost three times as
+// much: 20 x 4 of them are even.)
+bool short_rule(const CoilDev &c) { return !c.use_fast && c.n_ang < 30 && c.n_ang * c.n_thk <= 200; }
+
+// Whether a batch takes its primaries' own nodes (kPairOwn): nine tenths of its node pairs are of short rules, and they
+// give every SIMD a wave of items of 256 nodes a lane; smaller batches are faster in the finer items of the reduced
+// rules. 2,048 pairs of 20 x 7 slow nodes, M and F: 391 us of kernels by reduced rules, 198 by their own nodes; of 16 x 16
+// the two are even. (Indexes out of range: build_pairs reports them.)
+bool own_rule_pairs(const std::vector<CoilDev> &hp, const std::vector<CoilDev> &hs, const int64_t *prim_index,
+                    const int64_t *sec_index, int64_t n_pairs)
+{
+    if (std::none_of(hp.begin(), hp.end(), short_rule)) return false;
+    double all = 0.0, brief = 0.0;
+    for (int64_t k = 0; k < n_pairs; ++k) {
+        const int64_t pi = prim_index ? prim_index[k] : k, si = sec_index ? sec_index[k] : k;
+        if (pi < 0 || pi >= (int64_t)hp.size() || si < 0 || si >= (int64_t)hs.size()) return false;
+        const CoilDev &p = hp[(size_t)pi];
+        const double w = (double)node_count(hs[(size_t)si]) * p.n_ang * p.n_thk;
+        all += w;
+        if (short_rule(p)) brief += w;
+    }
+    return brief >= 0.9 * all && all >= 64.0 * 1024.0 * 256.0;
+}
+
 }  // namespace
 
 namespace ccoil {
@@ -98,6 +128,7 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
     if (n_pairs == 0) return CCOIL_OK;
     if (hp.empty() || hs.empty()) return fail(ctx, CCOIL_ERR_ARGUMENT, "pairs given but a coil array is empty");
     // the primaries' far-field series: FP32C by default, FP64 with CCOIL_FAR_FIELD; never for the gradient of M
+    out.own = precision == CCOIL_FP64 && own_rule_pairs(hp, hs, prim_index, sec_index, n_pairs);
     out.far = !(what & kPairGrad) && ((precision == CCOIL_FP32C && !(flags & CCOIL_DIRECT)) ||
                                       (precision == CCOIL_FP64 && (flags & CCOIL_FAR_FIELD)));
     if (out.far)
@@ -107,7 +138,7 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
                 // the slow method's reduced rules take no longer than its series at any distance (18 operations a node;
                 // flat primaries measured 10.6k cycles per 64 nodes either way at three radii, filaments 7.4k against
                 // 9.0k), so FP64 keeps the rule there and saves the moments
-                const bool rule = precision == CCOIL_FP64 && !c.use_fast && c.red_x < 1e30f;
+                const bool rule = precision == CCOIL_FP64 && !out.own && !c.use_fast && c.red_x < 1e30f;
                 const double y = rule ? 0.0 : far_distance(c, precision == CCOIL_FP64, true);
                 c.far_d2 = y > 0.0 ? (y * c.rmax) * (y * c.rmax) : 0.0;
                 c.mp_terms = far_terms(y, precision == CCOIL_FP64);
@@ -116,7 +147,7 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
 
     // Pair table, longest work item first (LPT order of the persistent queue).
     std::vector<PairDev> pd((size_t)n_pairs);
-    const bool reduced = precision == CCOIL_FP64;
+    const bool reduced = precision == CCOIL_FP64 && !out.own;
     std::vector<int64_t> prim_nodes((size_t)n_pairs);   // that an item evaluates per secondary node
     std::vector<uint8_t> series((size_t)n_pairs);       // series_only of each pair
     int64_t node_pairs = 0, work = 0;
@@ -126,7 +157,7 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
         if (pi < 0 || pi >= (int64_t)hp.size() || si < 0 || si >= (int64_t)hs.size())
             return fail(ctx, CCOIL_ERR_ARGUMENT, "pair " + std::to_string(k) + ": coil index out of range");
         const CoilDev &p = hp[(size_t)pi], &s = hs[(size_t)si];
-        const int64_t sec_nodes = (int64_t)s.blk_ang * s.n_ang * s.blk_thk * s.n_thk * s.blk_len * s.n_len;
+        const int64_t sec_nodes = node_count(s);
         node_pairs += sec_nodes * p.n_ang * p.n_thk;
         series[(size_t)k] = series_only(p, s);
         prim_nodes[(size_t)k] = series[(size_t)k] ? kSeriesNodes : reduced ? rule_nodes_of(p, s) : (int64_t)p.n_ang * p.n_thk;
@@ -143,7 +174,7 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
         d.prim = (int32_t)pi;
         d.sec = (int32_t)si;
         d.out = (int32_t)k;
-        d.n_nodes = (int64_t)s.blk_ang * s.n_ang * s.blk_thk * s.n_thk * s.blk_len * s.n_len;
+        d.n_nodes = node_count(s);
         decompose(target, prim_nodes[(size_t)k], series[(size_t)k] ? 1 : p.n_thk, d.nodes_per_item, d.row_groups);
         max_row_groups = std::max(max_row_groups, d.row_groups);
         d.ring_offset = ring_offset ? ring_offset[k] : 0.0;
@@ -218,7 +249,7 @@ ccoil_status pairs_setup(ccoil_ctx ctx, const PairBuild &pb, uint32_t what, int3
     pp.n_items = pb.items;
     pp.partial = (double *)bufs[3]->p;
     pp.what = what;
-    pp.precision = precision;
+    pp.precision = pb.own ? kPairOwn : precision;
     pp.tab = ctx_tables(ctx);
     return CCOIL_OK;
 }

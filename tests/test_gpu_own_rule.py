@@ -56,3 +56,41 @@ def test_no_slower_than_ieee(ctx, coil, copies, n):
     ms = {p: min(ctx.fields(cs, pts, abi.B, p)[1].kernel_ms for _ in range(7)) for p in (abi.FP64, abi.FP64_IEEE)}
     print(f"\n{coil} {copies} coils {n} points: {1e3 * ms[abi.FP64]:.0f} us, IEEE {1e3 * ms[abi.FP64_IEEE]:.0f}")
     assert ms[abi.FP64] <= ms[abi.FP64_IEEE]
+
+
+# pairs: batches of short slow rules, just above and below the size from which they sum their own nodes
+@pytest.mark.parametrize("n", [110, 125, 2048])
+def test_pairs(ctx, n):
+    rng = np.random.default_rng(41)
+    prims, secs = [], []
+    for _ in range(n):
+        prims.append(_row(*FLAT20))
+        s = _row(*RECT16)
+        s.update(pos=tuple(rng.normal(scale=0.7, size=3)), alpha=float(rng.uniform(0, 3)), beta=float(rng.uniform(0, 6)), n_len=4)
+        secs.append(s)
+    P, S = abi.CoilSet.from_rows(prims), abi.CoilSet.from_rows(secs)
+    what = abi.PAIR_M | abi.PAIR_FT | abi.PAIR_DM
+    ref, _ = ctx.pairs(P, S, n, what, abi.FP64_IEEE)
+    for flags in (0, abi.FAR_FIELD):
+        got, _ = ctx.pairs(P, S, n, what, abi.FP64, flags)
+        for k, v in ref.items():   # some nodes lie next to the winding: rounding of terms up to a thousand times the sum
+            assert np.max(np.abs(got[k] - v)) <= 1e-10 * np.max(np.abs(v)), (k, flags)
+    Mr, Gr, _ = ctx.pairs_grad(P, S, n, abi.FP64_IEEE)
+    Mg, Gg, _ = ctx.pairs_grad(P, S, n, abi.FP64)
+    assert np.max(np.abs(Mg - Mr)) <= 1e-10 * np.max(np.abs(Mr)) and np.max(np.abs(Gg - Gr)) <= 1e-10 * np.max(np.abs(Gr))
+
+
+def test_pairs_no_slower_than_ieee(ctx):
+    """2,048 pairs of a short slow rule with filaments, whose few nodes leave the set-up of a node to show."""
+    rng, n = np.random.default_rng(41), 2048
+    prims, secs = [], []
+    for _ in range(n):
+        prims.append(_row(*FLAT20))
+        s = _row("FILAMENT", 0.25, 0.0, 0.0, 80, 1)
+        s.update(pos=tuple(rng.normal(scale=0.2, size=3)), alpha=float(rng.uniform(0, 3)), beta=float(rng.uniform(0, 6)), n_len=1)
+        secs.append(s)
+    P, S = abi.CoilSet.from_rows(prims), abi.CoilSet.from_rows(secs)
+    mf = abi.PAIR_M | abi.PAIR_FT
+    ms = {p: min(ctx.pairs(P, S, n, mf, p)[1].kernel_ms for _ in range(9)) for p in (abi.FP64, abi.FP64_IEEE)}
+    print(f"\n{n} pairs: {1e3 * ms[abi.FP64]:.0f} us, IEEE {1e3 * ms[abi.FP64_IEEE]:.0f}")
+    assert ms[abi.FP64] <= ms[abi.FP64_IEEE]
