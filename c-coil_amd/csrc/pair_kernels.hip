@@ -318,7 +318,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPairWaves<P
             __shared__ int queue[PREC == 1 ? 256 : 128];   // the hard nodes, then FP32C's others
             int h0 = 0, c0 = 0, h1 = 0, c1 = 0;                // head and count of either ring
             const int own = pc.n_ang * ((pc.n_thk + pd.row_groups - 1) / pd.row_groups);
-            const bool reducible = pc.red_x < 1e30f;   // else every node keeps the own rule
+            // else every node keeps the own rule; the gradient's FP32C nodes of primaries of few angular nodes too, in the
+            // one queue: the two end in two partly filled passes (32 pairs of 16 x 16 nodes: 199 us, 172)
+            const bool reducible = pc.red_x < 1e30f && !(PREC == 1 && GR && pc.n_ang < 30);
             auto push = [&](int ring, int head, int &count, bool mine, int k) {
                 const unsigned long long mask = __ballot(mine);
                 if (mine) queue[ring + ((head + count + __popcll(mask & ((1ull << lane) - 1ull))) & 127)] = k;
@@ -326,12 +328,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPairWaves<P
             };
             for (int base = 0;;) {
                 // 0: the next 64 nodes, 1: the hard queue, 2: the other; each queue when it is full, and at the end what
-                // is left but for the last few hard nodes
+                // is left but for the last few hard nodes, which are summed over the wave one by one: some 8 nodes' time
+                // each besides the nodes, for the gradient's 14 sums 32
                 int mode;
                 if (c0 >= 64) mode = 1;
                 else if (PREC == 1 && c1 >= 64) mode = 2;
                 else if (base < n_item) mode = 0;
-                else if (c0 * (own / 64 + 8) > own || (c0 > 0 && own < 256)) mode = 1;
+                else if (c0 * (own / 64 + (GR ? 32 : 8)) > own || (c0 > 0 && own < 256)) mode = 1;
                 else if (PREC == 1 && c1 > 0) mode = 2;
                 else break;
                 int k = base + lane;

@@ -94,3 +94,19 @@ def test_pairs_no_slower_than_ieee(ctx):
     ms = {p: min(ctx.pairs(P, S, n, mf, p)[1].kernel_ms for _ in range(9)) for p in (abi.FP64, abi.FP64_IEEE)}
     print(f"\n{n} pairs: {1e3 * ms[abi.FP64]:.0f} us, IEEE {1e3 * ms[abi.FP64_IEEE]:.0f}")
     assert ms[abi.FP64] <= ms[abi.FP64_IEEE]
+
+
+def test_pairs_grad_fp32c_time(ctx):
+    """32 pairs next to each other's windings: each work item ends with a few nodes for the FP64 rule, after all its nodes
+    in float; half as long again as IEEE arithmetic at all of them is room for both."""
+    rng, n = np.random.default_rng(3), 32
+    prims, secs = [], []
+    for _ in range(n):
+        prims.append(_row(*RECT16))
+        s = _row(*RECT16)
+        s.update(pos=tuple(rng.normal(scale=0.2, size=3)), alpha=float(rng.uniform(0, 3)), beta=float(rng.uniform(0, 6)), n_len=4)
+        secs.append(s)
+    P, S = abi.CoilSet.from_rows(prims), abi.CoilSet.from_rows(secs)
+    ms = {p: min(ctx.pairs_grad(P, S, n, p)[2].kernel_ms for _ in range(9)) for p in (abi.FP32C, abi.FP64_IEEE)}
+    print(f"\n{n} pairs: FP32C {1e3 * ms[abi.FP32C]:.0f} us, IEEE {1e3 * ms[abi.FP64_IEEE]:.0f}")
+    assert ms[abi.FP32C] <= 1.5 * ms[abi.FP64_IEEE]
