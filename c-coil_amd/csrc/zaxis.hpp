@@ -12,7 +12,7 @@ constexpr int kZBlock = 256;   // threads per workgroup of zaxis_kernel
 // batch would otherwise run alone through up to 100 of them.
 constexpr int kZNodes = 8;
 
-constexpr int64_t kZMapped = 1 << 22;
+constexpr int64_t kZBatch = 1 << 22;   // workgroups of a launch, of several items at least
 
 // One coaxial pair (its M, its axial force or both) or one coil's self-inductance, by full or reduced rules. Every
 // workgroup of a quantity covers kZBlock units; each sums over its share of the primary's thickness nodes.
@@ -38,7 +38,7 @@ struct alignas(16) ZItemDev {
 
 struct ZParams {
     const ZItemDev *items;
-    const int32_t *wg_item;   // the item of each workgroup (null beyond kZMapped workgroups: searched for)
+    const int32_t *wg_item;   // the item of each workgroup (null for one item beyond kZBatch workgroups)
     int32_t n_items;
     int32_t mode, n_modes;    // the first quantity and their number (kZMutual and kZForce: two)
     int64_t out_stride;       // between the quantities in out

@@ -94,49 +94,61 @@ void reduce_item(ZItemDev &it, const PairRule &rule)
     }
 }
 
-// Sets the item's units from its rules.
+// Sets the item's units from its rules. An item that fills the chip several times over by itself needs no sharing of its
+// thickness nodes, and so never takes more workgroups than its (radial, angular) nodes.
 void set_units(ZItemDev &it)
 {
-    it.t_split = (int16_t)((it.t_inc + kZNodes - 1) / kZNodes);
-    it.units = (int64_t)it.r_blk * it.r_inc * it.a_blk * it.a_inc * std::max<int>(it.l_inc, 1) * it.t_split;
+    const int64_t units = (int64_t)it.r_blk * it.r_inc * it.a_blk * it.a_inc * std::max<int>(it.l_inc, 1);
+    it.t_split = (int16_t)(units < (int64_t)kZBlock * 16384 ? (it.t_inc + kZNodes - 1) / kZNodes : 1);
+    it.units = units * it.t_split;
     it.n_wg = (it.units + kZBlock - 1) / kZBlock;
 }
 
 bool valid_rule(int32_t blocks, int32_t inc) { return blocks >= 1 && inc >= 1 && inc <= kMaxOrder; }
 
 // Upload the items, run the node kernel and the ordered reduction for `modes` quantities from `mode` on, copy n_out
-// results back.
-ccoil_status run_items(ccoil_ctx ctx, std::vector<ZItemDev> &items, int32_t mode, int32_t modes, size_t n_out,
-                       uint32_t flags, double *out_host, double *out_dev, int64_t node_evals, ccoil_report *report)
+// results back. The items go in batches of kZBatch workgroups (one item at least): a launch of 2^32 threads or more runs
+// what is left over, without an error, and shared thickness nodes make up to 13 workgroups of one of the planned rule's.
+// planned_wg: those of the planned rules, which the documented limit counts.
+ccoil_status run_items(ccoil_ctx ctx, std::vector<ZItemDev> &items, int64_t planned_wg, int32_t mode, int32_t modes,
+                       size_t n_out, uint32_t flags, double *out_host, double *out_dev, int64_t node_evals,
+                       ccoil_report *report)
 {
-    int64_t wg = 0;
-    for (auto &it : items) {
-        it.first_wg = wg;
-        wg += modes * it.n_wg;
-    }
-    if (wg > INT32_MAX) return fail(ctx, CCOIL_ERR_ARGUMENT, "coaxial batch needs more than 2^31 - 1 workgroups");
+    if (planned_wg > INT32_MAX) return fail(ctx, CCOIL_ERR_ARGUMENT, "coaxial batch needs more than 2^31 - 1 workgroups");
     CC_HIP(ctx, hipSetDevice(ctx->device));
-    // the items, then each workgroup's item
-    const size_t n_items = items.size();
-    const bool mapped = wg <= kZMapped;
-    if (mapped) {
-        items.resize(n_items + ((size_t)wg * sizeof(int32_t) + sizeof(ZItemDev) - 1) / sizeof(ZItemDev));
-        int32_t *wg_item = reinterpret_cast<int32_t *>(items.data() + n_items);
-        for (size_t i = 0; i < n_items; ++i) wg_item = std::fill_n(wg_item, modes * items[i].n_wg, (int32_t)i);
+    // each batch: its items, then each workgroup's item
+    struct Batch { std::vector<ZItemDev> rows; size_t n_items; int64_t wg; bool mapped; };
+    std::vector<Batch> batches;
+    size_t max_rows = 0;
+    int64_t max_wg = 0;
+    for (size_t i = 0; i < items.size();) {
+        const size_t i0 = i;
+        int64_t wg = 0;
+        for (; i < items.size() && (i == i0 || wg + modes * items[i].n_wg <= kZBatch); ++i) {
+            items[i].first_wg = wg;
+            wg += modes * items[i].n_wg;
+        }
+        Batch b = {{}, i - i0, wg, wg <= kZBatch};
+        if (i0 == 0 && i == items.size()) b.rows.swap(items);
+        else b.rows.assign(items.begin() + (std::ptrdiff_t)i0, items.begin() + (std::ptrdiff_t)i);
+        if (b.mapped) {
+            b.rows.resize(b.n_items + ((size_t)wg * sizeof(int32_t) + sizeof(ZItemDev) - 1) / sizeof(ZItemDev));
+            int32_t *wg_item = reinterpret_cast<int32_t *>(b.rows.data() + b.n_items);
+            for (size_t k = 0; k < b.n_items; ++k) wg_item = std::fill_n(wg_item, modes * b.rows[k].n_wg, (int32_t)k);
+        }
+        max_rows = std::max(max_rows, b.rows.size());
+        max_wg = std::max(max_wg, wg);
+        batches.push_back(std::move(b));
+        if (batches.back().n_items == i && items.empty()) break;   // the only batch took them all
     }
-    CC_HIP(ctx, ensure(ctx->zitems, sizeof(ZItemDev) * items.size()));
-    CC_HIP(ctx, ensure(ctx->zpartial, sizeof(double) * (size_t)wg));
-    CC_HIP(ctx, hipMemcpyAsync(ctx->zitems.p, items.data(), sizeof(ZItemDev) * items.size(), hipMemcpyHostToDevice,
-                               ctx->stream));
+    CC_HIP(ctx, ensure(ctx->zitems, sizeof(ZItemDev) * max_rows));
+    CC_HIP(ctx, ensure(ctx->zpartial, sizeof(double) * (size_t)max_wg));
     ZParams zp;
     std::memset(&zp, 0, sizeof zp);
     zp.items = (const ZItemDev *)ctx->zitems.p;
-    zp.wg_item = mapped ? (const int32_t *)(zp.items + n_items) : nullptr;
-    zp.n_items = (int32_t)n_items;
     zp.mode = mode;
     zp.n_modes = modes;
     zp.out_stride = modes > 1 ? (int64_t)n_out / modes : 0;
-    zp.n_wg = wg;
     zp.partial = (double *)ctx->zpartial.p;
     zp.tab = ctx_tables(ctx);
     const bool dev = flags & CCOIL_DEVICE_POINTERS;
@@ -146,12 +158,20 @@ ccoil_status run_items(ccoil_ctx ctx, std::vector<ZItemDev> &items, int32_t mode
         CC_HIP(ctx, ensure(ctx->zout, sizeof(double) * n_out));
         zp.out = (double *)ctx->zout.p;
     }
-    CC_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-    launch_zaxis(ctx->stream, zp);
-    CC_HIP(ctx, hipGetLastError());
-    CC_HIP(ctx, hipEventRecord(ctx->evm1, ctx->stream));
-    launch_zaxis_reduce(ctx->stream, zp);
-    CC_HIP(ctx, hipGetLastError());
+    for (size_t k = 0; k < batches.size(); ++k) {   // in stream order, so the next upload waits for the last reduction
+        const Batch &b = batches[k];
+        CC_HIP(ctx, hipMemcpyAsync(ctx->zitems.p, b.rows.data(), sizeof(ZItemDev) * b.rows.size(), hipMemcpyHostToDevice,
+                                   ctx->stream));
+        zp.wg_item = b.mapped ? (const int32_t *)(zp.items + b.n_items) : nullptr;
+        zp.n_items = (int32_t)b.n_items;
+        zp.n_wg = b.wg;
+        if (k == 0) CC_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
+        launch_zaxis(ctx->stream, zp);
+        CC_HIP(ctx, hipGetLastError());
+        if (k + 1 == batches.size()) CC_HIP(ctx, hipEventRecord(ctx->evm1, ctx->stream));
+        launch_zaxis_reduce(ctx->stream, zp);
+        CC_HIP(ctx, hipGetLastError());
+    }
     CC_HIP(ctx, hipEventRecord(ctx->ev1, ctx->stream));
     if (!dev) CC_HIP(ctx, hipMemcpyAsync(out_host, zp.out, sizeof(double) * n_out, hipMemcpyDeviceToHost, ctx->stream));
     CC_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -208,7 +228,7 @@ extern "C" ccoil_status ccoil_pairs_zaxis(ccoil_ctx ctx, const ccoil_coils *prim
     std::vector<ZItemDev> items, reduced;   // full rules are launched first: their workgroups run longest
     items.reserve((size_t)n_pairs + 1);
     reduced.reserve((size_t)n_pairs);
-    int64_t evals = 0;
+    int64_t evals = 0, planned_wg = 0;
     const int modes = (what & CCOIL_PAIR_M ? 1 : 0) + (what & CCOIL_PAIR_FT ? 1 : 0);
     for (int64_t k = 0; k < n_pairs; ++k) {
         const int64_t i = prim_index ? prim_index[k] : k, j = sec_index ? sec_index[k] : k;
@@ -239,6 +259,7 @@ extern "C" ccoil_status ccoil_pairs_zaxis(ccoil_ctx ctx, const ccoil_coils *prim
                                                      "non-zero currents (M = sum * 2 pi / (I1 I2))");
             it.div = prim->current[i] * sec->current[j];
         }
+        planned_wg += modes * (((int64_t)it.r_blk * it.r_inc * it.a_blk * it.a_inc + kZBlock - 1) / kZBlock);
         evals += (int64_t)modes * it.r_blk * it.r_inc * it.a_blk * it.a_inc * it.t_blk * it.t_inc;
         const PairRule rule = pair_rule(it.t_inner, prim->a[i], it.hp, it.r_inner, sec->a[j], it.hs, it.z, it.a_inc,
                                         it.t_inc, it.r_inc);
@@ -256,7 +277,7 @@ extern "C" ccoil_status ccoil_pairs_zaxis(ccoil_ctx ctx, const ccoil_coils *prim
     if (dev) {
         // device outputs are written in place: route M and Fz through one staging buffer, then copy on device
         CC_HIP(ctx, ensure(ctx->zout, sizeof(double) * n_out));
-        ccoil_status st = run_items(ctx, items, mode, modes, n_out, flags, nullptr, (double *)ctx->zout.p, evals, report);
+        ccoil_status st = run_items(ctx, items, planned_wg, mode, modes, n_out, flags, nullptr, (double *)ctx->zout.p, evals, report);
         if (st != CCOIL_OK) return st;
         const size_t s1 = sizeof(double) * (size_t)n_pairs;
         if (what & CCOIL_PAIR_M) CC_HIP(ctx, hipMemcpyAsync(M, ctx->zout.p, s1, hipMemcpyDeviceToDevice, ctx->stream));
@@ -266,7 +287,7 @@ extern "C" ccoil_status ccoil_pairs_zaxis(ccoil_ctx ctx, const ccoil_coils *prim
         return CCOIL_OK;
     }
     std::vector<double> host(n_out);
-    ccoil_status st = run_items(ctx, items, mode, modes, n_out, flags, host.data(), nullptr, evals, report);
+    ccoil_status st = run_items(ctx, items, planned_wg, mode, modes, n_out, flags, host.data(), nullptr, evals, report);
     if (st != CCOIL_OK) return st;
     if (what & CCOIL_PAIR_M) std::memcpy(M, host.data(), sizeof(double) * (size_t)n_pairs);
     if (what & CCOIL_PAIR_FT) std::memcpy(Fz, host.data() + f_at, sizeof(double) * (size_t)n_pairs);
@@ -284,7 +305,7 @@ extern "C" ccoil_status ccoil_self_inductance(ccoil_ctx ctx, const ccoil_coils *
     if (coils->n == 0) return CCOIL_OK;
     if (!radial || !L) return fail(ctx, CCOIL_ERR_ARGUMENT, "radial and L must not be NULL");
     std::vector<ZItemDev> items;
-    int64_t evals = 0;
+    int64_t evals = 0, planned_wg = 0;
     for (int64_t i = 0; i < coils->n; ++i) {
         if (!valid_rule(radial[2 * i], radial[2 * i + 1]))
             return fail(ctx, CCOIL_ERR_ARGUMENT, "coil " + std::to_string(i) + ": radial rule needs blocks >= 1 and "
@@ -312,9 +333,10 @@ extern "C" ccoil_status ccoil_self_inductance(ccoil_ctx ctx, const ccoil_coils *
         it.z = len;
         it.mul = coils->turns[i];
         it.div = coils->current[i] * len;
+        planned_wg += ((int64_t)it.r_blk * it.r_inc * it.a_blk * it.a_inc + kZBlock - 1) / kZBlock;
         evals += (int64_t)it.r_blk * it.r_inc * it.a_blk * it.a_inc * it.t_blk * it.t_inc;
         set_units(it);
         items.push_back(it);
     }
-    return run_items(ctx, items, kZSelf, 1, (size_t)coils->n, flags, L, L, evals, report);
+    return run_items(ctx, items, planned_wg, kZSelf, 1, (size_t)coils->n, flags, L, L, evals, report);
 }
