@@ -568,8 +568,8 @@ static void launch_near_eval_group(hipStream_t s, const FieldParams &p, unsigned
 
 // The grid covers the capacity at `lanes` lanes a place up to kEvalBlocks blocks, some eight times what the chip holds at
 // once, and strides beyond. (A wave that finds no record costs a nanosecond: 75,000 of them, for the default
-// capacity of 262,145 points and hardly any record, took 75 us. And the capacity can pass the 2^32 threads of a launch:
-// 2^29 records split over eight lanes.)
+// capacity of 262,145 points and hardly any record, took 75 us. And the capacity can pass the 2^32 threads of a launch,
+// 2^29 records split over eight lanes, which then runs what is left over, without an error.)
 constexpr int64_t kEvalBlocks = 16384;
 static unsigned near_eval_blocks(const FieldParams &p, int lanes)
 {

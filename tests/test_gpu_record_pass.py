@@ -52,20 +52,23 @@ def test_one_coil_bookkeeping(ctx):
 
 
 def test_capacity_beyond_a_launch():
-    """2^28 points and two coils: room for 2^29 records, which split over eight lanes would be 2^32 threads in one
-    dimension. (A context of its own, which gives some 40 GB back.)"""
+    """2^28 points and two coils: room for 2^29 records, which split over eight lanes would be more than the 2^32 threads
+    of a launch. (A context of its own, which gives some 40 GB back.)"""
     ctx = abi.Context(0)
     try:
-        cs = _set([("FILAMENT", 0.25, 0.0, 0.0, 6, 1)], 2, np.random.default_rng(2), 0.1)
+        cs = _set([("THIN", 0.25, 0.0, 0.05, 6, 1)], 2, np.random.default_rng(2), 0.1)
         n = 1 << 28
         g = torch.Generator(device="cuda").manual_seed(7)
         pts = torch.rand((n, 3), dtype=torch.float64, device="cuda", generator=g) - 0.5
         out = {"B": torch.empty_like(pts)}
-        ctx.fields(cs, pts, abi.B, abi.FP32C, abi.DIRECT | abi.DEVICE_POINTERS, out=out)
-        some = torch.cat([pts[:1000], pts[-1000:]])
+        _, rep = ctx.fields(cs, pts, abi.B, abi.FP32C, abi.DIRECT | abi.DEVICE_POINTERS, out=out)
+        assert rep.near_pairs > 1 << 20
+        some = torch.cat([pts[:20000], pts[-20000:]])
         ref, _ = ctx.fields(cs, some.cpu().numpy(), abi.B, abi.FP32C, abi.DIRECT)
-        got = torch.cat([out["B"][:1000], out["B"][-1000:]]).cpu().numpy()
-        assert np.max(np.abs(got - ref["B"])) <= 1e-5 * np.max(np.abs(ref["B"]))   # float nodes, by other lanes
+        got = torch.cat([out["B"][:20000], out["B"][-20000:]]).cpu().numpy()
+        # each point by itself: a record left out is the coil's whole field there (float nodes by other lanes, 1e-5)
+        err, size = np.linalg.norm(got - ref["B"], axis=1), np.linalg.norm(ref["B"], axis=1)
+        assert np.all(err <= 1e-5 * size + 1e-6 * np.median(size))
     finally:
         ctx.close()
         torch.cuda.empty_cache()
