@@ -394,10 +394,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPairWaves<P
                 node(k, n);
                 Local L = {0, 0, 0, 0, 0, 0, 0};
                 AdjA q;
-                const bool far = PREC == kPairOwn && !GR && p.mp && is_far(pc, n.z, n.r);
-                if (!far) eval_prim<PREC, kA, kB, kAda>(pc, p.tab, n.z, n.r, rg, pd.row_groups, L, &q);
-                if (PREC == kPairOwn) series(n, far, L, q);
-                if (!far || rg == 0) add(n, L, q);
+                eval_prim<PREC, kA, kB, kAda>(pc, p.tab, n.z, n.r, rg, pd.row_groups, L, &q);
+                add(n, L, q);
             }
         }
         if constexpr (GR) {

@@ -75,7 +75,7 @@ int64_t node_count(const CoilDev &s)   // of a secondary
 // much: 20 x 4 of them are even.)
 bool short_rule(const CoilDev &c) { return !c.use_fast && c.n_ang < 30 && c.n_ang * c.n_thk <= 200; }
 
-// Whether a batch takes its primaries' own nodes (kPairOwn): nine tenths of its node pairs are of short rules, and they
+// Whether a batch without the series takes its primaries' own nodes (kPairOwn): nine tenths of its node pairs are of short rules, and they
 // give every SIMD a wave of items of 256 nodes a lane; smaller batches are faster in the finer items of the reduced
 // rules. 2,048 pairs of 20 x 7 slow nodes, M and F: 391 us of kernels by reduced rules, 198 by their own nodes; of 16 x 16
 // the two are even. (Indexes out of range: build_pairs reports them.)
@@ -128,9 +128,9 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
     if (n_pairs == 0) return CCOIL_OK;
     if (hp.empty() || hs.empty()) return fail(ctx, CCOIL_ERR_ARGUMENT, "pairs given but a coil array is empty");
     // the primaries' far-field series: FP32C by default, FP64 with CCOIL_FAR_FIELD; never for the gradient of M
-    out.own = precision == CCOIL_FP64 && own_rule_pairs(hp, hs, prim_index, sec_index, n_pairs);
     out.far = !(what & kPairGrad) && ((precision == CCOIL_FP32C && !(flags & CCOIL_DIRECT)) ||
                                       (precision == CCOIL_FP64 && (flags & CCOIL_FAR_FIELD)));
+    out.own = precision == CCOIL_FP64 && !out.far && own_rule_pairs(hp, hs, prim_index, sec_index, n_pairs);
     if (out.far)
         host_parallel_for((int64_t)hp.size(), [&](int64_t i0, int64_t i1) {
             for (int64_t i = i0; i < i1; ++i) {
@@ -138,7 +138,7 @@ ccoil_status build_pairs(ccoil_ctx ctx, const ccoil_coils *prim, const ccoil_coi
                 // the slow method's reduced rules take no longer than its series at any distance (18 operations a node;
                 // flat primaries measured 10.6k cycles per 64 nodes either way at three radii, filaments 7.4k against
                 // 9.0k), so FP64 keeps the rule there and saves the moments
-                const bool rule = precision == CCOIL_FP64 && !out.own && !c.use_fast && c.red_x < 1e30f;
+                const bool rule = precision == CCOIL_FP64 && !c.use_fast && c.red_x < 1e30f;
                 const double y = rule ? 0.0 : far_distance(c, precision == CCOIL_FP64, true);
                 c.far_d2 = y > 0.0 ? (y * c.rmax) * (y * c.rmax) : 0.0;
                 c.mp_terms = far_terms(y, precision == CCOIL_FP64);
