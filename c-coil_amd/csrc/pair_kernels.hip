@@ -1,7 +1,7 @@
 // Pair kernels: M, F and T of many (primary, secondary) pairs of mixed type and uneven cost in one launch.
 //
 // A work item is (pair, chunk of secondary nodes, group of the primary's thickness rows) and one wave (one
-// 64-lane workgroup) owns one item: item = blockIdx.x. Items are laid out longest-first on the host, and
+// 64-lane workgroup) owns one item: item = blockIdx (rows_of). Items are laid out longest-first on the host, and
 // workgroups are dispatched in index order, so the launch is an LPT schedule without a shared cursor. Each lane
 // evaluates the primary's A or B (over the item's rows) at one secondary node at a time (the primary coil is
 // wave-uniform, so its loops and tables are scalar), the weighted sums (M, F, T and the gradient of M, all linear
@@ -9,12 +9,23 @@
 // adds the partials of each pair in a fixed order, so results are deterministic. The reference instead runs one
 // thread per (configuration, secondary node) and FP32 atomicAdds per configuration (MInductance.cu:157,
 // Force.cu:172-178).
+#include <algorithm>
+
 #include "integrands.hpp"
 #include "kernels.hpp"
 #include "multipole.hpp"
 #include "pairs.hpp"
 
 namespace ccoil {
+
+// One block of 64 threads for each of n things, in rows of 2^22: a launch of 2^32 threads or more in a dimension runs
+// what is left over, without an error, and a batch can have 2^31 - 1 items.
+static dim3 rows_of(int64_t n)
+{
+    constexpr int64_t row = (int64_t)1 << 22;
+    return dim3((unsigned)std::min(n, row), (unsigned)((n + row - 1) / row));
+}
+__device__ inline int64_t block_of_rows() { return (int64_t)blockIdx.y * gridDim.x + blockIdx.x; }
 
 __device__ inline double wave_sum(double v)
 {
@@ -131,7 +142,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPairWaves<P
 {
     static_assert(!GR || (WM && !WF && !WD), "the gradient instance evaluates M and its derivatives");
     const int lane = threadIdx.x;
-    const int64_t item = blockIdx.x;
+    const int64_t item = block_of_rows();
+    if (item >= p.n_items) return;
     {
         int lo = 0, hi = p.n_pairs - 1;
         while (lo < hi) {
@@ -433,7 +445,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kPairWaves<P
 // The gradient of M: one wave per pair, lane l adds items l, l + 64, ..., a fixed butterfly combines the lanes.
 __global__ __launch_bounds__(64) void pair_grad_reduce_kernel(PairParams p)
 {
-    const int k = blockIdx.x, lane = threadIdx.x;
+    const int64_t k = block_of_rows();
+    const int lane = threadIdx.x;
+    if (k >= p.n_pairs) return;
     const PairDev &pd = p.pairs[k];
     const int64_t end = (k + 1 < p.n_pairs) ? p.pairs[k + 1].first_item : p.n_items;
     double s[kPairGradTerms];
@@ -452,7 +466,9 @@ __global__ __launch_bounds__(64) void pair_grad_reduce_kernel(PairParams p)
 
 __global__ __launch_bounds__(64) void pair_reduce_kernel(PairParams p)
 {
-    const int k = blockIdx.x, lane = threadIdx.x;
+    const int64_t k = block_of_rows();
+    const int lane = threadIdx.x;
+    if (k >= p.n_pairs) return;
     const PairDev &pd = p.pairs[k];
     const int64_t end = (k + 1 < p.n_pairs) ? p.pairs[k + 1].first_item : p.n_items;
     double s[kPairTerms];
@@ -474,7 +490,7 @@ template <int PREC>
 static void launch_pairs_p(hipStream_t s, const PairParams &p)
 {
     const bool wm = p.what & 1, wf = p.what & 2, wd = p.what & 4;
-    const dim3 grid((unsigned)p.n_items);
+    const dim3 grid = rows_of(p.n_items);
     if (p.what & kPairGrad) {
         hipLaunchKernelGGL((pair_kernel<PREC, true, false, false, true>), grid, dim3(64), 0, s, p);
     } else if (wd) {
@@ -504,8 +520,8 @@ void launch_pairs(hipStream_t s, const PairParams &p)
 void launch_pair_reduce(hipStream_t s, const PairParams &p)
 {
     if (p.n_pairs <= 0) return;
-    if (p.what & kPairGrad) hipLaunchKernelGGL(pair_grad_reduce_kernel, dim3((unsigned)p.n_pairs), dim3(64), 0, s, p);
-    else hipLaunchKernelGGL(pair_reduce_kernel, dim3((unsigned)p.n_pairs), dim3(64), 0, s, p);
+    if (p.what & kPairGrad) hipLaunchKernelGGL(pair_grad_reduce_kernel, rows_of(p.n_pairs), dim3(64), 0, s, p);
+    else hipLaunchKernelGGL(pair_reduce_kernel, rows_of(p.n_pairs), dim3(64), 0, s, p);
 }
 
 }  // namespace ccoil

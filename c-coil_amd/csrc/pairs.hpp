@@ -69,7 +69,7 @@ constexpr int kPairGradTerms = 14;
 constexpr int kPairGradOut = 16;
 constexpr uint32_t kPairGrad = 8;
 
-// One 64-lane workgroup per work item (grid = n_items, at most 2^31 - 1). A pair's items are its chunks of
+// One 64-lane workgroup per work item (n_items, at most 2^31 - 1). A pair's items are its chunks of
 // secondary nodes times its primary row groups: item i of a pair takes chunk i / row_groups and row group
 // i % row_groups.
 void launch_pairs(hipStream_t s, const PairParams &p);
