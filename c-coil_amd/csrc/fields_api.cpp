@@ -347,8 +347,9 @@ ccoil_status fields_prepare(ccoil_ctx ctx, const ccoil_coils *coils, const doubl
     for (auto &c : hc) out.nodes += (int64_t)c.n_ang * c.n_thk;
     if (n == 0 || hc.empty()) return CCOIL_OK;   // nothing to evaluate, or every field zero
     const FieldShape sh = shape ? *shape : field_shape_rule(ctx, n, hc, quantities, precision, rule_records);
-    if (shape && sh.split != 1 && sh.split != 4 && sh.split != 16)
-        return fail(ctx, CCOIL_ERR_ARGUMENT, "split must be 1, 4 or 16");
+    if (shape && sh.split != 1 && sh.split != 4 && sh.split != 16 &&
+        !(sh.split == 64 && precision == CCOIL_FP64 && n < kSortedPoints))
+        return fail(ctx, CCOIL_ERR_ARGUMENT, "split must be 1, 4, 16 or, in FP64 with few points, 64");
     L.split = rule_records ? 1 : sh.split;   // the series-only kernel runs one lane per point
     const bool own_rule = precision == CCOIL_FP64 && !rule_records && field_own_rule(hc, n, L.split, quantities);
     if (own_rule) L.precision = kFP64Own;

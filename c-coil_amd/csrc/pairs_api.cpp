@@ -322,7 +322,7 @@ ccoil_status pairs_tuned_target(ccoil_ctx ctx, const ccoil_coils *prim, const cc
         if (st != CCOIL_OK) return st;
         ccoil_report rep;
         st = pairs_run(ctx, pb, what, precision, flags, M, F, T, dM, &rep);
-        ms = rep.main_kernel_ms;
+        ms = rep.kernel_ms;
         return st;
     };
     return tune_pairs(ctx, rule, what, precision, run, target);

@@ -60,8 +60,13 @@ ccoil_status tune_fields(ccoil_ctx ctx, const ccoil_coils *coils, const double *
     int64_t nodes = 0;
     for (const auto &c : hc) nodes += (int64_t)c.n_ang * c.n_thk;
     std::ostringstream k;
-    k << "fields n=" << n_points << " coils=" << hc.size() << " nodes=" << nodes << " q=" << quantities
-      << " precision=" << precision << " near=" << ((flags & CCOIL_NO_NEAR_FP64) ? 0 : 1) << " cu=" << ctx->cu_count;
+    // far: the series' calls have kernels of their own. The kernels' version is part of the key: a shape timed with other
+    // kernels is none for these (v2: reduced rules, 64 lanes per point)
+    const bool far = (precision == CCOIL_FP32C && !(flags & CCOIL_DIRECT)) ||
+                     (precision == CCOIL_FP64 && (flags & CCOIL_FAR_FIELD));
+    k << "fields v2 n=" << n_points << " coils=" << hc.size() << " nodes=" << nodes << " q=" << quantities
+      << " precision=" << precision << " far=" << far << " near=" << ((flags & CCOIL_NO_NEAR_FP64) ? 0 : 1)
+      << " cu=" << ctx->cu_count;
     const std::string key = k.str();
     std::string v;
     if (cache_get(ctx, key, v) && std::sscanf(v.c_str(), "split=%d chunks=%d", &out.split, &out.chunks) == 2)
@@ -72,12 +77,13 @@ ccoil_status tune_fields(ccoil_ctx ctx, const ccoil_coils *coils, const double *
     const FieldShape rule = field_shape_rule(ctx, n_points, hc, quantities, precision);
     std::set<std::pair<int, int>> cand;
     std::vector<int> splits = {1, 4};
-    if (n_points < 65536) splits.push_back(16);
+    if (n_points < kSortedPoints) splits.push_back(16);
+    if (n_points < kSortedPoints && precision == CCOIL_FP64) splits.push_back(64);
     for (int s : splits)
         for (int64_t c : {(int64_t)1, (int64_t)2, (int64_t)3, (int64_t)4, (int64_t)rule.chunks,
                           (int64_t)std::max(1, rule.chunks / 2), (int64_t)rule.chunks * 2})
             if (c >= 1 && c <= nc && c <= 65535) cand.insert({s, (int)c});
-    cand.insert({std::min(rule.split, 16), rule.chunks});
+    cand.insert({rule.split, rule.chunks});
     double best = 1e300;
     FieldShape best_shape = rule;   // every candidate is timed, so one of them replaces it
     for (const auto &c : cand) {
@@ -88,8 +94,8 @@ ccoil_status tune_fields(ccoil_ctx ctx, const ccoil_coils *coils, const double *
         const ccoil_status st = fields_call(ctx, coils, points, n_points, quantities, precision, flags, A, B, E, G,
                                             &rep, nullptr, &sh);
         if (st != CCOIL_OK) return st;
-        if (rep.main_kernel_ms < best) {
-            best = rep.main_kernel_ms;
+        if (rep.kernel_ms < best) {   // with what a shape brings along: the visit order, the sum of the chunks
+            best = rep.kernel_ms;
             best_shape = sh;
         }
     }
@@ -104,8 +110,10 @@ ccoil_status tune_pairs(ccoil_ctx ctx, const PairBuild &rule, uint32_t what, int
                         const std::function<ccoil_status(int64_t, double &)> &run, int64_t &target)
 {
     std::ostringstream k;
-    k << "pairs n=" << rule.sorted.size() << " node_pairs=" << rule.node_pairs << " what=" << what
-      << " precision=" << precision << " cu=" << ctx->cu_count;
+    // v2, reduced: what the target counts, nodes of reduced rules or of the planned ones (build_pairs)
+    const bool reduced = precision == CCOIL_FP64 && !rule.own;
+    k << "pairs v2 n=" << rule.sorted.size() << " node_pairs=" << rule.node_pairs << " what=" << what
+      << " precision=" << precision << " far=" << rule.far << " reduced=" << reduced << " cu=" << ctx->cu_count;
     const std::string key = k.str();
     std::string v;
     long long t = 0;
@@ -115,8 +123,10 @@ ccoil_status tune_pairs(ccoil_ctx ctx, const PairBuild &rule, uint32_t what, int
     }
     double best = 1e300;
     target = rule.target;
+    // the rule's own target and its neighbours within the range that is worth a launch (lane_target)
+    const int64_t least = reduced ? 16 : 256, most = reduced ? 8192 : 32768;
     for (int64_t c : {rule.target / 4, rule.target / 2, rule.target, rule.target * 2}) {
-        if (c < 256 || c > 32768) continue;
+        if (c != rule.target && (c < least || c > most)) continue;
         double ms = 0.0;
         const ccoil_status st = run(c, ms);
         if (st != CCOIL_OK) return st;

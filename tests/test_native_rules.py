@@ -33,3 +33,36 @@ int main()
 }
 """)
     assert lines == ["0"]
+
+
+def test_targets_that_the_pair_tuner_times(tmp_path):
+    """tune_pairs times the rule's own target, whatever it is, and its neighbours down to 16 reduced-rule (256 planned)
+    nodes a lane; a file's entry for the same batch whose target counted planned nodes is not replayed."""
+    lines = native.run(tmp_path, r"""
+#include "context.hpp"
+#include <cstdio>
+int main()
+{
+    ccoil_ctx_s ctx;
+    ctx.cu_count = 256;
+    for (int32_t precision : {(int32_t)CCOIL_FP64, (int32_t)CCOIL_FP32C})
+        for (int64_t target : {16, 64, 128, 256, 2048}) {
+            if (precision != CCOIL_FP64 && target < 256) continue;
+            ccoil::PairBuild rule;
+            rule.sorted.resize(3);
+            rule.node_pairs = 1000 * target;
+            rule.target = target;
+            ctx.tuning["pairs n=3 node_pairs=" + std::to_string(rule.node_pairs) + " what=1 precision=0 cu=256"] = "target=8192";
+            int64_t got = 0;
+            std::printf("%d %lld:", precision, (long long)target);
+            ccoil::tune_pairs(&ctx, rule, 1, precision, [](int64_t c, double &ms) {
+                std::printf(" %lld", (long long)c);
+                ms = 1.0;
+                return (ccoil_status)CCOIL_OK;
+            }, got);
+            std::printf("\n");
+        }
+}
+""")
+    assert lines == ["0 16: 16 32", "0 64: 16 32 64 128", "0 128: 32 64 128 256", "0 256: 64 128 256 512",
+                     "0 2048: 512 1024 2048 4096", "1 256: 256 512", "1 2048: 512 1024 2048 4096"]
