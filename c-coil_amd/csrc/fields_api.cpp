@@ -417,9 +417,12 @@ ccoil_status fields_prepare(ccoil_ctx ctx, const ccoil_coils *coils, const doubl
     const bool sorted_rule = precision == CCOIL_FP64 && !own_rule && L.split == 1 && n >= kSortedPoints &&
                              !(arena && arena->fixed);
     if ((far && n >= kOrderMinPoints) || sorted_rule) {
-        // about 16-32 points per cell: 2^bits cells per axis, bits = log8(n / 16), between 3 and 6
+        // 2^bits cells per axis, between 3 and 6 bits, with 2 to 16 points a cell on average (more beyond 2^22 points).
+        // Up to 128 a cell, a cloud dense in its middle had thousands in one cell, whose counters the sort's atomics
+        // queued at, and 64 points of a wave spread over a cell; 2^18 points of a normal cloud, 6 and 24 thin coils of
+        // 100 and 48 nodes: 433 and 809 us with 64 a cell, 260 and 585 with 8 (uniform cloud: 191 and 457, 178 and 420).
         int bits = 3;
-        while (bits < 6 && ((int64_t)1 << (3 * (bits + 1))) * 16 <= n) ++bits;
+        while (bits < 6 && ((int64_t)1 << (3 * (bits + 1))) * 2 <= n) ++bits;
         const int64_t cells = (int64_t)1 << (3 * bits);
         size_t sb = 0;
         CC_HIP(ctx, near_scan(ctx->stream, nullptr, nullptr, cells, nullptr, sb));
