@@ -106,6 +106,7 @@ struct FieldLaunch {
     void *order_temp = nullptr; // FP32C far field: storage of the visit-order sort
     size_t order_scan_bytes = 0;
     int order_bits = 0;
+    int64_t piece = 0;          // points per launch: all, or as many as the order covers (kSortedPiece)
     size_t far_bytes = 0;       // device bytes of the far-field buffers (moments, order, sort storage)
 };
 // Far field: the series replaces the rule where a bound on the angular rule's error is below kFarTolerance
@@ -120,6 +121,7 @@ constexpr int64_t kOrderMinPoints = 16384;
 constexpr int64_t kRecordMaxPoints = (int64_t)1 << 20;
 // CCOIL_FP64 calls of the rule alone take one lane per point, in a spatial visit order, from this many points on.
 constexpr int64_t kSortedPoints = 65536;
+constexpr int64_t kSortedPiece = (int64_t)1 << 24;   // of which one visit order serves at a time
 // Whether a field call of this precision, flags and size has a record pass, and whether it has rule records.
 bool field_record_pass(int32_t precision, uint32_t flags, int64_t n_points, bool fixed_arena, bool *rule_records);
 double far_threshold(int n_ang, double q, double tol, double ylo);
@@ -146,7 +148,7 @@ void host_parallel_for(int64_t n, const std::function<void(int64_t, int64_t)> &f
 int far_terms(double y, bool fp64);
 // Enqueues the field kernel, the chunk reduction and (FP32C) the whole near pass on s, with no host
 // synchronisation and kernel launches and copies only (so it can be captured in a graph); evm0/evm1 (may be NULL)
-// bracket the field kernel. The near pass's outcome is copied to host_state (pinned) when given.
+// bracket the field kernel (of all pieces, with the orders of the later ones). The near pass's outcome is copied to host_state (pinned) when given.
 void enqueue_fields(hipStream_t s, const FieldLaunch &L, hipEvent_t evm0, hipEvent_t evm1, NearState *host_state,
                     hipEvent_t evr0 = nullptr, hipEvent_t evr1 = nullptr);
 // The near pass from the per-coil cursors on (after a grow-on-overflow retry): key scan, fill, eval, add; evr0 / evr1

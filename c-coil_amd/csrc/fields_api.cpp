@@ -264,7 +264,7 @@ void enqueue_fields(hipStream_t s, const FieldLaunch &L, hipEvent_t evm0, hipEve
     ZeroRanges zero;
     std::memset(&zero, 0, sizeof zero);
     if (p.order) {
-        zero.p[0] = visit_order_counts(L.order_temp, p.n_pts);
+        zero.p[0] = visit_order_counts(L.order_temp, L.piece);
         zero.n[0] = (int64_t)1 << (3 * L.order_bits);
     }
     if (L.near) {
@@ -275,15 +275,24 @@ void enqueue_fields(hipStream_t s, const FieldLaunch &L, hipEvent_t evm0, hipEve
         zero.p[3] = p.near_state;
         zero.n[3] = sizeof(NearState) / 8;
     }
-    launch_fill_zero(s, zero);
-    if (p.mp) launch_multipole_moments(s, p.coils, p.n_coils, p.tab, const_cast<double *>(p.mp));
-    if (p.order)
-        (void)launch_visit_order(s, p.pts, p.n_pts, L.order_bits, L.order_temp, L.order_scan_bytes,
-                                 const_cast<uint32_t *>(p.order));
-    if (evm0) (void)hipEventRecord(evm0, s);
-    launch_field(s, p, L.precision, L.split);
-    if (evm1) (void)hipEventRecord(evm1, s);
-    launch_field_reduce(s, p);
+    FieldParams q = p;   // of a piece of points: all of them, except where the order covers fewer
+    for (int64_t s0 = 0; s0 < p.n_pts; s0 += L.piece) {
+        q.n_pts = std::min<int64_t>(L.piece, p.n_pts - s0);
+        q.pts = p.pts + 3 * s0;
+        if (p.A) q.A = p.A + 3 * s0;
+        if (p.B) q.B = p.B + 3 * s0;
+        if (p.E) q.E = p.E + 3 * s0;
+        if (p.G) q.G = p.G + 9 * s0;
+        launch_fill_zero(s, zero);
+        if (p.mp) launch_multipole_moments(s, p.coils, p.n_coils, p.tab, const_cast<double *>(p.mp));
+        if (p.order)
+            (void)launch_visit_order(s, q.pts, q.n_pts, L.order_bits, L.order_temp, L.piece, L.order_scan_bytes,
+                                     const_cast<uint32_t *>(p.order));
+        if (evm0 && s0 == 0) (void)hipEventRecord(evm0, s);
+        launch_field(s, q, L.precision, L.split);
+        if (evm1 && s0 + L.piece >= p.n_pts) (void)hipEventRecord(evm1, s);
+        launch_field_reduce(s, q);
+    }
     if (L.near) {
         size_t tb = L.scan_bytes;
         (void)near_scan(s, p.near_counts, const_cast<int64_t *>(p.near_offsets), p.n_pts, L.scan_temp, tb);
@@ -393,48 +402,59 @@ ccoil_status fields_prepare(ccoil_ctx ctx, const ccoil_coils *coils, const doubl
         if (quantities & CCOIL_E) { CC_HIP(ctx, ensure(ctx->outE, s3)); p.E = (double *)ctx->outE.p; }
         if (quantities & (CCOIL_G | CCOIL_G_JACOBIAN)) { CC_HIP(ctx, ensure(ctx->outG, s9)); p.G = (double *)ctx->outG.p; }
     }
+    const bool sorted_rule = precision == CCOIL_FP64 && !own_rule && L.split == 1 && n >= kSortedPoints &&
+                             !(arena && arena->fixed);
+    L.piece = sorted_rule && !far ? std::min<int64_t>(n, kSortedPiece) : n;
     const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(sh.chunks, (int64_t)hc.size()));
     p.coils_per_chunk = (int32_t)(((int64_t)hc.size() + chunks - 1) / chunks);
     p.n_chunks = (int32_t)(((int64_t)hc.size() + p.coils_per_chunk - 1) / p.coils_per_chunk);
     if (p.n_chunks > 1) {
         p.partial_width = out.width;
         void *partial = nullptr;
-        st = call_buffer(ctx, ctx->fpartial, arena, sizeof(double) * p.partial_width * (size_t)n * (size_t)p.n_chunks,
+        st = call_buffer(ctx, ctx->fpartial, arena, sizeof(double) * p.partial_width * (size_t)L.piece * (size_t)p.n_chunks,
                          &partial);
         if (st != CCOIL_OK) return st;
         p.partial = (double *)partial;
     }
     if (far) {   // the series' moments
         const size_t mb = sizeof(double) * (size_t)kMpCoil * hc.size();
-        L.far_bytes = mb + 256;
+        L.far_bytes += mb + 256;
         void *mp = nullptr;
         st = call_buffer(ctx, ctx->fmp, arena, mb, &mp);
         if (st != CCOIL_OK) return st;
         p.mp = (const double *)mp;
     }
     // The visit order, when there are enough points for the spatial sort to pay: the series modes, and the FP64 rule
-    // with one lane per point (no result depends on it, so the fixed scratch, which has no room to spare, goes without)
-    const bool sorted_rule = precision == CCOIL_FP64 && !own_rule && L.split == 1 && n >= kSortedPoints &&
-                             !(arena && arena->fixed);
+    // with one lane per point. No result depends on it. So the rule's calls of the fixed scratch, which has no room to
+    // spare, go without, those of more than kSortedPiece points run in pieces of them, so that no context keeps more for
+    // it than that takes (0.2 GB), and where even that is not to be had the points go in index order.
     if ((far && n >= kOrderMinPoints) || sorted_rule) {
-        // 2^bits cells per axis, between 3 and 6 bits, with 2 to 16 points a cell on average (more beyond 2^22 points).
+        // 2^bits cells per axis, between 3 and 7 bits, with 2 to 16 points a cell on average.
         // Up to 128 a cell, a cloud dense in its middle had thousands in one cell, whose counters the sort's atomics
         // queued at, and 64 points of a wave spread over a cell; 2^18 points of a normal cloud, 6 and 24 thin coils of
         // 100 and 48 nodes: 433 and 809 us with 64 a cell, 260 and 585 with 8 (uniform cloud: 191 and 457, 178 and 420).
         int bits = 3;
-        while (bits < 6 && ((int64_t)1 << (3 * (bits + 1))) * 2 <= n) ++bits;
+        while (bits < 7 && ((int64_t)1 << (3 * (bits + 1))) * 2 <= L.piece) ++bits;
         const int64_t cells = (int64_t)1 << (3 * bits);
         size_t sb = 0;
         CC_HIP(ctx, near_scan(ctx->stream, nullptr, nullptr, cells, nullptr, sb));
-        const size_t ob = sizeof(uint32_t) * (size_t)n, tb = visit_order_bytes(n, bits, sb);
+        const size_t ob = sizeof(uint32_t) * (size_t)L.piece, tb = visit_order_bytes(L.piece, bits, sb);
         void *order = nullptr, *temp = nullptr;
-        if ((st = call_buffer(ctx, ctx->forder, arena, ob, &order)) != CCOIL_OK) return st;
-        if ((st = call_buffer(ctx, ctx->ftemp, arena, tb, &temp)) != CCOIL_OK) return st;
-        L.far_bytes += ob + tb + 2 * 256;
-        p.order = (const uint32_t *)order;
-        L.order_temp = temp;
-        L.order_scan_bytes = sb;
-        L.order_bits = bits;
+        const std::string err = ctx->err;
+        st = call_buffer(ctx, ctx->forder, arena, ob, &order);
+        if (st == CCOIL_OK) st = call_buffer(ctx, ctx->ftemp, arena, tb, &temp);
+        if (st == CCOIL_OK) {
+            L.far_bytes += ob + tb + 2 * 256;
+            p.order = (const uint32_t *)order;
+            L.order_temp = temp;
+            L.order_scan_bytes = sb;
+            L.order_bits = bits;
+        } else if (far || (st != CCOIL_ERR_OUT_OF_MEMORY && !arena)) {
+            return st;
+        } else {
+            ctx->err = err;
+            (void)hipGetLastError();
+        }
     }
     if (L.near) {
         // Buffers for the records: every (coil, point) pair when that is small, else a capacity kept from earlier

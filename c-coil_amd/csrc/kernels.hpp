@@ -203,11 +203,11 @@ void launch_near_eval(hipStream_t s, const FieldParams &p);
 void launch_near_add(hipStream_t s, const FieldParams &p);
 // Far-field moments of every coil with CoilDev::far_d2 > 0 and the recurrence header, into mp.
 void launch_multipole_moments(hipStream_t s, const CoilDev *coils, int n_coils, const Tables &tab, double *mp);
-// The visit order: points counting-sorted by the Morton cell of a 2^bits-per-axis grid over their bounding box.
-// temp: visit_order_bytes(n, bits, scan_bytes) bytes, scan_bytes from near_scan for 2^(3 bits) counts.
-size_t visit_order_bytes(int64_t n, int bits, size_t scan_bytes);
-int64_t *visit_order_counts(void *temp, int64_t n);   // the cells' 2^(3 bits) counts, zeroed before the launch
-hipError_t launch_visit_order(hipStream_t s, const double *pts, int64_t n, int bits, void *temp, size_t scan_bytes,
-                              uint32_t *order);
+// The visit order: n <= cap points counting-sorted by the Morton cell of a 2^bits-per-axis grid over their bounding box.
+// temp: visit_order_bytes(cap, bits, scan_bytes) bytes, scan_bytes from near_scan for 2^(3 bits) counts.
+size_t visit_order_bytes(int64_t cap, int bits, size_t scan_bytes);
+int64_t *visit_order_counts(void *temp, int64_t cap);   // the cells' 2^(3 bits) counts, zeroed before the launch
+hipError_t launch_visit_order(hipStream_t s, const double *pts, int64_t n, int bits, void *temp, int64_t cap,
+                              size_t scan_bytes, uint32_t *order);
 
 }  // namespace ccoil

@@ -182,22 +182,22 @@ void launch_multipole_moments(hipStream_t s, const CoilDev *coils, int n_coils, 
         hipLaunchKernelGGL(multipole_moments_kernel, dim3(n_coils), dim3(kMomThreads), 0, s, coils, tab, mp);
 }
 
-size_t visit_order_bytes(int64_t n, int bits, size_t scan_bytes)
+size_t visit_order_bytes(int64_t cap, int bits, size_t scan_bytes)
 {
     const size_t cells = (size_t)1 << (3 * bits);
-    return sizeof(double) * (6 * kBoxBlocks + 8) + sizeof(uint32_t) * (size_t)n + 2 * sizeof(int64_t) * cells +
+    return sizeof(double) * (6 * kBoxBlocks + 8) + sizeof(uint32_t) * (size_t)cap + 2 * sizeof(int64_t) * cells +
            scan_bytes + 6 * 256;
 }
 
-int64_t *visit_order_counts(void *temp, int64_t n)
+int64_t *visit_order_counts(void *temp, int64_t cap)
 {
     auto align = [](size_t b) { return (b + 255) & ~(size_t)255; };
     return (int64_t *)((char *)temp + align(sizeof(double) * 6 * kBoxBlocks) + align(sizeof(double) * 8) +
-                       align(sizeof(uint32_t) * (size_t)n));
+                       align(sizeof(uint32_t) * (size_t)cap));
 }
 
-hipError_t launch_visit_order(hipStream_t s, const double *pts, int64_t n, int bits, void *temp, size_t scan_bytes,
-                              uint32_t *order)
+hipError_t launch_visit_order(hipStream_t s, const double *pts, int64_t n, int bits, void *temp, int64_t cap,
+                              size_t scan_bytes, uint32_t *order)
 {
     const size_t cells = (size_t)1 << (3 * bits);
     auto align = [](size_t b) { return (b + 255) & ~(size_t)255; };
@@ -207,8 +207,8 @@ hipError_t launch_visit_order(hipStream_t s, const double *pts, int64_t n, int b
     double *box = (double *)t;
     t += align(sizeof(double) * 8);
     uint32_t *cell = (uint32_t *)t;
-    t += align(sizeof(uint32_t) * (size_t)n);
-    int64_t *count = visit_order_counts(temp, n);
+    t += align(sizeof(uint32_t) * (size_t)cap);
+    int64_t *count = visit_order_counts(temp, cap);
     t += align(sizeof(int64_t) * cells);
     int64_t *cursor = (int64_t *)t;
     t += align(sizeof(int64_t) * cells);

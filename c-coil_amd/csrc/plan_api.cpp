@@ -115,7 +115,7 @@ ccoil_status ccoil_fields_plan(ccoil_ctx ctx, const ccoil_coils *coils, const do
     const FieldParams &pp = probe.L.p;
     const size_t nc = probe.hc.size();
     size_t bytes = (sizeof(CoilDev) + sizeof(uint32_t)) * nc + 4096;
-    if (pp.n_chunks > 1) bytes += sizeof(double) * (size_t)pp.partial_width * (size_t)probe.n * (size_t)pp.n_chunks + 256;
+    if (pp.n_chunks > 1) bytes += sizeof(double) * (size_t)pp.partial_width * (size_t)probe.L.piece * (size_t)pp.n_chunks + 256;
     bytes += probe.L.far_bytes;
     if (probe.L.near) {
         bytes += 2 * sizeof(int64_t) * (size_t)probe.n + 2 * sizeof(uint32_t) * ((size_t)pp.n_keys + 2) + sizeof(NearState) +

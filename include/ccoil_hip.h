@@ -56,7 +56,9 @@ enum {
                                  from the hardware FP64 approximations refined by one Newton step (a few ulp);
                                  a coil's angular and thickness sums take fewer nodes than its increments where
                                  both have converged to rounding (1e-15 of the sum of the terms): the accurate
-                                 mode */
+                                 mode. Field calls of 65,536 points or more may visit them in a spatial order, for
+                                 which the context (or plan) keeps 10 to 20 bytes a point, 0.2 GB at most, and
+                                 which they do without where that cannot be allocated */
     CCOIL_FP32C = 1,          /* the same integrands with FP32 per-node arithmetic, FP64 per-row work and row
                                  accumulation, re-evaluation with CCOIL_FP64's arithmetic of near-winding (coil,
                                  point) pairs and, for outputs that divide by r (the gradient, the pair position
