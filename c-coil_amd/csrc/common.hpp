@@ -28,6 +28,34 @@ constexpr int kRedThk = 6;
 constexpr int kRedThkN[kRedThk] = {22, 17, 13, 10, 8, 6};
 constexpr double kRedThkC = 200.0;
 constexpr double kRedTol = 3e-16;
+// The classes' thresholds, as class_of compares them: the least cosh(eta) - 1 and the least rho_B + 1 / rho_B (the ellipse's
+// distance sum over half the thickness), with margins far above the rounding of class_of's float operations.
+struct RedLimits {
+    float x[kRedAng], s[kRedThk];
+};
+constexpr double cosh_minus_1(double x)
+{
+    double t = 1.0, v = 0.0;
+    for (int k = 2; k <= 60; k += 2) v += t *= x * x / (k * (k - 1));
+    return v;
+}
+constexpr double natural_log(double y)   // y >= 1
+{
+    double k = 0.0, v = 0.0;
+    for (; y >= 2.0; y *= 0.5) k += 1.0;
+    const double u = (y - 1.0) / (y + 1.0);
+    double p = 2.0 * u;
+    for (int i = 1; i <= 79; i += 2, p *= u * u) v += p / i;
+    return 0.69314718055994530942 * k + v;
+}
+constexpr RedLimits red_limits()
+{
+    RedLimits l = {};
+    for (int i = 0; i < kRedAng; ++i) l.x[i] = (float)(cosh_minus_1(kRedEta[i]) * 1.00001);
+    for (int i = 0; i < kRedThk; ++i)
+        l.s[i] = (float)(2.0 * (1.0 + cosh_minus_1(natural_log(kRedThkC / kRedTol) / (2 * kRedThkN[i]))) * 1.0001);
+    return l;
+}
 constexpr int kRuleClasses = (kRedAng + 1) * (kRedThk + 1);   // class = (kRedThk + 1) angular class + thickness class
 constexpr double kPi = 3.14159265358979323846;
 constexpr double kMuReduced = 1e-7;                    // mu0 / (4 pi), g_MiReduced (CalculateFieldsFast.cxx:10)
@@ -268,26 +296,24 @@ __host__ __device__ inline RuleSel class_rule(const CoilDev &c, int cls)
 // ring at radius rho is analytic for |Im phi| < eta, cosh(eta) = 1 + ((rho - r)^2 + zd^2) / (2 rho r), least at the
 // winding's radius nearest to sqrt(r^2 + zd^2); the thickness integrand is analytic outside the point (r, zd) and its
 // mirror, whose ellipse about [R, R + a] has the distance sum d1 + d2. Every operation is a float operation rounded on
-// its own, so every kernel gives a pair the same class; the thresholds carry margins far above float rounding.
+// its own, so every kernel gives a pair the same class; the thresholds (red_limits) carry margins for the rounding.
 //
 // class_of: the class at num = (rho - r)^2 + zd^2, den = 2 rho r and s = (d1 + d2) / (a / 2), or at bounds of them
 // (num / den and s from below).
 __host__ __device__ inline int class_of(const CoilDev &c, float num, float den, float s)
 {
 #pragma clang fp contract(off)
+    constexpr RedLimits kLim = red_limits();
     int k = 0, t = 0;
     if (num >= c.red_x * den) {
-        constexpr float kX[kRedAng] = {0.0050042f, 0.0453385f, 0.2946833f, 0.5430806f, 2.1074632f, 11.2864665f};
         k = 1;   // red_x is at least the first class's threshold
 #pragma unroll
-        for (int i = 1; i < kRedAng; ++i) k += num >= kX[i] * den ? 1 : 0;
+        for (int i = 1; i < kRedAng; ++i) k += num >= kLim.x[i] * den ? 1 : 0;
     }
     if (s >= c.red_s) {
-        // rho_B + 1 / rho_B, rho_B = (kRedThkC / kRedTol)^(1 / (2 n))
-        constexpr float kS[kRedThk] = {2.935256f, 3.643171f, 5.054480f, 7.913130f, 13.079747f, 30.607902f};
         t = 1;
 #pragma unroll
-        for (int i = 1; i < kRedThk; ++i) t += s >= kS[i] ? 1 : 0;
+        for (int i = 1; i < kRedThk; ++i) t += s >= kLim.s[i] ? 1 : 0;
     }
     return (kRedThk + 1) * k + t;
 }

@@ -54,7 +54,7 @@ PEAK_HBM_GBS = 8000.0
 # thickness classes' node counts.
 RED_ANG = (20, 16, 12, 10, 8, 6)
 RED_ETA = (0.1, 0.3, 0.75, 1.0, 1.8, 3.2)
-RED_X = (0.0050042, 0.0453385, 0.2946833, 0.5430806, 2.1074632, 11.2864665)
+RED_X = tuple(math.cosh(e) - 1.0 for e in RED_ETA)
 RED_THK = (22, 17, 13, 10, 8, 6)
 
 

@@ -66,3 +66,46 @@ int main()
 """)
     assert lines == ["0 16: 16 32", "0 64: 16 32 64 128", "0 128: 32 64 128 256", "0 256: 64 128 256 512",
                      "0 2048: 512 1024 2048 4096", "1 256: 256 512", "1 2048: 512 1024 2048 4096"]
+
+
+def test_class_thresholds(tmp_path):
+    """Each reduced class starts at or beyond the eta (the ellipse) that its node set is made for, and at most 1e-4 (2e-4) beyond."""
+    lines = native.run(tmp_path, r"""
+#include "context.hpp"
+#include <cmath>
+#include <cstdio>
+using namespace ccoil;
+// the least float >= 0 whose class, by of(x), is at least cls
+template <typename F> float least(F of, int cls)
+{
+    float lo = 0.0f, hi = 1e4f;
+    while (std::nextafterf(lo, hi) < hi) {
+        const float m = 0.5f * (lo + hi);
+        (of(m) >= cls ? hi : lo) = m;
+    }
+    return hi;
+}
+int main()
+{
+    CoilDev c = {};
+    c.red_x = 0.0f;
+    c.red_s = 0.0f;
+    // class 1 starts where the coil's own rule has converged (red_x)
+    for (int k = 2; k <= kRedAng; ++k)
+        std::printf("%.9g\n", (double)least([&](float x) { return class_of(c, x, 1.0f, 0.0f) / (kRedThk + 1); }, k) / (std::cosh(kRedEta[k - 1]) - 1.0));
+    for (int t = 2; t <= kRedThk; ++t)
+        std::printf("%.9g\n", (double)least([&](float x) { return class_of(c, 0.0f, 1.0f, x) % (kRedThk + 1); }, t) /
+                                  (2.0 * std::cosh(std::log(kRedThkC / kRedTol) / (2 * kRedThkN[t - 1]))));
+    for (int n = 1; n <= kMaxOrder; ++n) {   // and no coil's own threshold lies below its first class's
+        CoilDev d = {};
+        d.R = 0.1;
+        d.a = 0.1;
+        d.n_ang = d.n_thk = n;
+        set_rule_limits(d);
+        const int k = std::isnan(d.red_x) ? 0 : class_of(d, d.red_x, 1.0f, 0.0f) / (kRedThk + 1);
+        if (k > 0 && d.red_x < std::cosh(kRedEta[k - 1]) - 1.0) std::printf("n_ang %d\n", n);
+    }
+}
+""")
+    ratios = [float(v) for v in lines]
+    assert len(ratios) == 10 and min(ratios) >= 1.0 and max(ratios[:5]) <= 1.0001 and max(ratios[5:]) <= 1.0002, lines
