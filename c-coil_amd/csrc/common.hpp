@@ -13,11 +13,12 @@ constexpr int kTableSize = kMaxOrder * (kMaxOrder + 1) / 2;
 // converged to rounding (reduced_rules.cpp: the bounds, the tables and what they measured).
 //
 // Angular class k (1..kRedAng) serves the pairs whose angular integrand is analytic in the strip |Im phi| < eta for an
-// eta of at least kRedEta[k - 1]; its kRedAngN[k - 1] nodes lie in the angular double tables at kRedOffset. Class 0 is
-// the coil's own rule.
+// eta of at least kRedFrom[k - 1]; its kRedAngN[k - 1] nodes, made for the strip of kRedEta[k - 1], lie in the angular
+// double tables at kRedOffset. Class 0 is the coil's own rule.
 constexpr int kRedAng = 6;
 constexpr int kRedAngN[kRedAng] = {20, 16, 12, 10, 8, 6};
 constexpr double kRedEta[kRedAng] = {0.1, 0.3, 0.75, 1.0, 1.8, 3.2};
+constexpr double kRedFrom[kRedAng] = {0.103, 0.3, 0.75, 1.01, 1.8, 3.2};
 constexpr int kRedNodes = 20 + 16 + 12 + 10 + 8 + 6;
 constexpr int kRedOffset = kTableSize;
 constexpr int kTableSizeAng = kRedOffset + kRedNodes;   // the w, omc, wcos, opc, ws, ws2 and wcs tables
@@ -51,7 +52,7 @@ constexpr double natural_log(double y)   // y >= 1
 constexpr RedLimits red_limits()
 {
     RedLimits l = {};
-    for (int i = 0; i < kRedAng; ++i) l.x[i] = (float)(cosh_minus_1(kRedEta[i]) * 1.00001);
+    for (int i = 0; i < kRedAng; ++i) l.x[i] = (float)(cosh_minus_1(kRedFrom[i]) * 1.00001);
     for (int i = 0; i < kRedThk; ++i)
         l.s[i] = (float)(2.0 * (1.0 + cosh_minus_1(natural_log(kRedThkC / kRedTol) / (2 * kRedThkN[i]))) * 1.0001);
     return l;

@@ -11,9 +11,12 @@
 // phi = pi - 2 am(u, k), k' = tanh(eta / 2), the integrand is analytic and 2 K periodic in the strip |Im u| < K'(k)
 // for every point whose eta is at least that one, so the N-point midpoint rule in u errs like exp(-2 pi N K' / K): 20
 // nodes at eta = 0.1 where Gauss-Legendre takes 80. (k', nodes and weights from the arithmetic-geometric mean and
-// Landen's descending transformation, Abramowitz & Stegun 16.4 and 17.6.) Measured in extended precision over rings
-// and sheets with r, z, b over their ranges, 3,000 configurations per class: at most 2e-16 of the sum of the node
-// terms' magnitudes for A, B and the gradient.
+// Landen's descending transformation, Abramowitz & Stegun 16.4 and 17.6.) Where the singularity is one of the fifth power
+// of the distance, the gradient's, that holds a little inside the strip only: in extended precision, over the ring's
+// positions at each eta, A and B have errors below 1e-17 of the sum of the node terms' magnitudes at every class's eta, the
+// gradient 2.8e-15 at eta = 0.1 (20 nodes), 8.0e-16 at 1.0 (10) and below 2e-16 at the others, falling to 1.9e-16 from
+// 0.103 and to 1.1e-16 from 1.01 on, where those two classes begin (kRedFrom). So: at most 2e-16 for A, B and the
+// gradient, and less over the sheets, whose ends alone have the ring's terms.
 //
 // Thickness. The angular sum as a function of the ring radius is singular at rho = r +- i zd (zd: the distance beyond
 // the axial span), so n Gauss-Legendre nodes err like C rho_B^(-2n), rho_B the parameter of the Bernstein ellipse
@@ -89,7 +92,7 @@ float ang_threshold(int n)
     while (first < kRedAng && kRedAngN[first] >= n) ++first;
     if (first == kRedAng) return kNever;
     auto g = [&](double eta) { return std::log(1000.0 / 1e-15) + 2.0 * eta - 2.0 * n * log_ellipse(eta); };
-    double lo = kRedEta[first], hi = 20.0;
+    double lo = kRedFrom[first], hi = 20.0;
     if (g(lo) > 0.0) {
         if (g(hi) > 0.0) return kNever;
         for (int it = 0; it < 60; ++it) {

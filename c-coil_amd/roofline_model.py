@@ -53,7 +53,7 @@ PEAK_HBM_GBS = 8000.0
 # Reduced rules (common.hpp): the angular classes' node counts, least strip half-widths and least cosh(eta) - 1, and the
 # thickness classes' node counts.
 RED_ANG = (20, 16, 12, 10, 8, 6)
-RED_ETA = (0.1, 0.3, 0.75, 1.0, 1.8, 3.2)
+RED_ETA = (0.103, 0.3, 0.75, 1.01, 1.8, 3.2)   # kRedFrom
 RED_X = tuple(math.cosh(e) - 1.0 for e in RED_ETA)
 RED_THK = (22, 17, 13, 10, 8, 6)
 

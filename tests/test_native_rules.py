@@ -69,7 +69,7 @@ int main()
 
 
 def test_class_thresholds(tmp_path):
-    """Each reduced class starts at or beyond the eta (the ellipse) that its node set is made for, and at most 1e-4 (2e-4) beyond."""
+    """Each reduced class starts at or beyond its eta (its ellipse), and at most 1e-4 (2e-4) beyond."""
     lines = native.run(tmp_path, r"""
 #include "context.hpp"
 #include <cmath>
@@ -92,7 +92,7 @@ int main()
     c.red_s = 0.0f;
     // class 1 starts where the coil's own rule has converged (red_x)
     for (int k = 2; k <= kRedAng; ++k)
-        std::printf("%.9g\n", (double)least([&](float x) { return class_of(c, x, 1.0f, 0.0f) / (kRedThk + 1); }, k) / (std::cosh(kRedEta[k - 1]) - 1.0));
+        std::printf("%.9g\n", (double)least([&](float x) { return class_of(c, x, 1.0f, 0.0f) / (kRedThk + 1); }, k) / (std::cosh(kRedFrom[k - 1]) - 1.0));
     for (int t = 2; t <= kRedThk; ++t)
         std::printf("%.9g\n", (double)least([&](float x) { return class_of(c, 0.0f, 1.0f, x) % (kRedThk + 1); }, t) /
                                   (2.0 * std::cosh(std::log(kRedThkC / kRedTol) / (2 * kRedThkN[t - 1]))));
@@ -103,9 +103,82 @@ int main()
         d.n_ang = d.n_thk = n;
         set_rule_limits(d);
         const int k = std::isnan(d.red_x) ? 0 : class_of(d, d.red_x, 1.0f, 0.0f) / (kRedThk + 1);
-        if (k > 0 && d.red_x < std::cosh(kRedEta[k - 1]) - 1.0) std::printf("n_ang %d\n", n);
+        if (k > 0 && d.red_x < std::cosh(kRedFrom[k - 1]) - 1.0) std::printf("n_ang %d\n", n);
     }
 }
 """)
     ratios = [float(v) for v in lines]
     assert len(ratios) == 10 and min(ratios) >= 1.0 and max(ratios[:5]) <= 1.0001 and max(ratios[5:]) <= 1.0002, lines
+
+
+def test_angular_classes_errors(tmp_path):
+    """The reduced angular sums of a ring's A, B and gradient terms, from where class_of takes each class on: within 2e-16 of
+    the sum of the terms' magnitudes, the rule's own error, plus the tables' rounding (half an ulp of each weight and of
+    each 1 - cos(phi), to the power 5/2: 3.5 x 1.1e-16, as if all had one sign)."""
+    lines = native.run(tmp_path, r"""
+#include "context.hpp"
+#include <algorithm>
+#include <cmath>
+#include <cstdio>
+#include <vector>
+using namespace ccoil;
+typedef long double ld;
+struct Rule { std::vector<ld> s, w; };   // 1 - cos(phi), weights
+// the terms of a ring of radius 1 at (r, z): A_phi, B_r, B_z and their derivatives' (integrands.hpp)
+void sums(const Rule &q, ld r, ld z, ld *v, ld *m)
+{
+    std::fill(v, v + 8, 0.0L);
+    std::fill(m, m + 8, 0.0L);
+    for (size_t i = 0; i < q.s.size(); ++i) {
+        const ld s = q.s[i], c = 1 - s, D = (1 - r) * (1 - r) + z * z + 2 * r * s, f = 1 / sqrtl(D), f3 = f / D, f5 = f3 / D;
+        const ld nb = 1 - r + r * s, nr = r - 1 + s;
+        const ld t[8] = {c * f, z * c * f3, nb * f3, z * nb * f5, z * c * nr * f5, c * f3 - 3 * z * z * c * f5, nb * nr * f5, c * f3};
+        for (int k = 0; k < 8; ++k) {
+            v[k] += q.w[i] * t[k];
+            m[k] += q.w[i] * fabsl(t[k]);
+        }
+    }
+}
+int main()
+{
+    RedTables t;
+    reduced_tables(t);
+    CoilDev c = {};
+    c.red_x = red_limits().x[0];
+    for (int k = 0, off = 0; k < kRedAng; off += kRedAngN[k++]) {
+        Rule q;
+        for (int i = 0; i < kRedAngN[k]; ++i) {
+            q.s.push_back(t.omc[off + i]);
+            q.w.push_back(t.w[off + i]);
+        }
+        ld worst = 0;
+        int seen = 0;
+        for (int e = 0; e <= 120; ++e) {
+            const ld eta = (ld)kRedEta[k] * (1 + 0.001L * e), x = coshl(eta) - 1;
+            if (class_of(c, (float)x, 1.0f, 0.0f) / (kRedThk + 1) != k + 1) continue;
+            ++seen;
+            Rule fine;
+            const int n = (int)(60 / eta) + 40;   // midpoints, which err like exp(-2 n eta)
+            for (int i = 0; i < n; ++i) {
+                const ld h = sinl(1.57079632679489661923132169163975L * (i + 0.5L) / n);
+                fine.s.push_back(2 * h * h);
+                fine.w.push_back(2.0L / n);
+            }
+            const ld lo = 1 + x - sqrtl((1 + x) * (1 + x) - 1);   // the radii with this eta: lo to 1 / lo
+            for (int j = 0; j < 60; ++j) {
+                const ld r = powl(lo, cosl(3.14159265358979L * j / 59));
+                const ld z = sqrtl(std::max(2 * r * x - (1 - r) * (1 - r), 0.0L));
+                ld a[8], am[8], b[8], bm[8];
+                sums(q, r, z, a, am);
+                sums(fine, r, z, b, bm);
+                for (int i = 0; i < 8; ++i)
+                    if (bm[i] > 0) worst = std::max(worst, fabsl(a[i] - b[i]) / bm[i]);
+            }
+        }
+        std::printf("%d %d %.3Lg\n", kRedAngN[k], seen, worst);
+    }
+}
+""")
+    for line in lines:
+        n, seen, err = line.split()
+        assert int(seen) > 80 and float(err) <= 2e-16 + 3.5 * 1.11e-16, lines
