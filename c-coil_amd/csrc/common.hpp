@@ -84,16 +84,17 @@ struct alignas(64) CoilDev {
     double rmax;             // radius of the sphere about the centre that holds the winding, |(R + a, b / 2)|
     double far_d2;           // squared distance beyond which the far-field series replaces the rule (0: never)
     double inv_rmax2;        // 1 / rmax^2
+    double hb;               // half the winding's length, 0 where the slow integrands take it for flat
     int32_t use_fast;
     int32_t n_ang, n_thk, n_len;
     int32_t blk_ang, blk_thk, blk_len;
     int32_t near_key; // FP32C near pass: the coil's place in the evaluation order (most nodes first)
     int32_t mp_terms; // highest order of the far-field series a pair of this call can use (0: no series)
     // Reduced rules: the least cosh(eta) - 1 and the least ellipse parameter sum (d1 + d2) / (a / 2) at which the
-    // coil's angular and thickness rules may be replaced (NaN: never), and the winding's geometry in float
-    // (inner and outer radius, half length, 2 / a).
+    // coil's angular and thickness rules may be replaced (NaN: never), and the winding's geometry in float (inner
+    // and outer radius, 2 / a).
     float red_x, red_s;
-    float r0f, r1f, hbf, ia2f;
+    float r0f, r1f, ia2f;
 };
 
 // Gauss-Legendre tables for orders 1..100 at offset table_offset(n), generated in FP64 on the device (w and the double
@@ -296,8 +297,9 @@ __host__ __device__ inline RuleSel class_rule(const CoilDev &c, int cls)
 // (reduced_rules.cpp). With zd the point's distance beyond the winding's axial span, the angular integrand of the
 // ring at radius rho is analytic for |Im phi| < eta, cosh(eta) = 1 + ((rho - r)^2 + zd^2) / (2 rho r), least at the
 // winding's radius nearest to sqrt(r^2 + zd^2); the thickness integrand is analytic outside the point (r, zd) and its
-// mirror, whose ellipse about [R, R + a] has the distance sum d1 + d2. Every operation is a float operation rounded on
-// its own, so every kernel gives a pair the same class; the thresholds (red_limits) carry margins for the rounding.
+// mirror, whose ellipse about [R, R + a] has the distance sum d1 + d2. zd is formed in double (next to the end of a coil
+// thousands of radii long float coordinates are as coarse as its thickness), and every other operation is a float
+// operation rounded on its own, so every kernel gives a pair the same class; the thresholds (red_limits) carry margins for the rounding.
 //
 // class_of: the class at num = (rho - r)^2 + zd^2, den = 2 rho r and s = (d1 + d2) / (a / 2), or at bounds of them
 // (num / den and s from below).
@@ -318,14 +320,22 @@ __host__ __device__ inline int class_of(const CoilDev &c, float num, float den, 
     }
     return (kRedThk + 1) * k + t;
 }
-__device__ inline int rule_class(const CoilDev &c, double z, double r)
+__host__ __device__ inline float class_sqrt(float x)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_sqrtf(x);   // within an ulp
+#else
+    return __builtin_sqrtf(x);
+#endif
+}
+__host__ __device__ inline int rule_class(const CoilDev &c, double z, double r)
 {
 #pragma clang fp contract(off)
-    const float rf = (float)r, zd = fmaxf((float)fabs(z) - c.hbf, 0.0f), zd2 = zd * zd;
-    const float rho = fminf(fmaxf(__builtin_amdgcn_sqrtf(rf * rf + zd2), c.r0f), c.r1f);
+    const float rf = (float)r, zd = fmaxf((float)(fabs(z) - c.hb), 0.0f), zd2 = zd * zd;
+    const float rho = fminf(fmaxf(class_sqrt(rf * rf + zd2), c.r0f), c.r1f);
     const float dr = rho - rf, num = dr * dr + zd2, den = 2.0f * rho * rf;
     const float e0 = rf - c.r0f, e1 = rf - c.r1f;
-    const float s = (__builtin_amdgcn_sqrtf(e0 * e0 + zd2) + __builtin_amdgcn_sqrtf(e1 * e1 + zd2)) * c.ia2f;
+    const float s = (class_sqrt(e0 * e0 + zd2) + class_sqrt(e1 * e1 + zd2)) * c.ia2f;
     return class_of(c, num, den, s);
 }
 

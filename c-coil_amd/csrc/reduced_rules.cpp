@@ -130,14 +130,16 @@ struct Thresholds {
 void set_rule_limits(CoilDev &c)
 {
     static const Thresholds t;
-    // The classes are found in float, to some 1e-7 of the larger of a point's coordinates and the winding's: that must
-    // not overflow nor underflow when squared, and be small against R (angular) and against a (thickness).
+    // The classes are found in float, to some 1e-7 of the winding's radius and the point's distance from its span: that
+    // must not overflow nor underflow when squared, and be small against R (angular) and against a (thickness: 1e-3 of it
+    // at the least a, a tenth more of an error that the constant 200 overstates by four). A point's own coordinate z is
+    // good to 1e-16 of a coil's half length, and so is the distance: 1e-8 of the least a at the greatest length.
     const bool fits = c.R >= 1e-15 && c.R + c.a <= 1e15 && (!c.use_fast || 0.5 * c.b <= 1e4 * c.R);
     c.red_x = fits ? t.ang[(size_t)c.n_ang] : kNever;
     c.red_s = fits && c.a >= 1e-4 * (c.R + c.a) ? t.thk[(size_t)c.n_thk] : kNever;
     c.r0f = (float)c.R;
     c.r1f = (float)(c.R + c.a);
-    c.hbf = c.use_fast ? (float)(0.5 * c.b) : 0.0f;
+    c.hb = c.use_fast ? 0.5 * c.b : 0.0;
     c.ia2f = c.red_s < FLT_MAX ? (float)(2.0 / c.a) : 0.0f;
 }
 

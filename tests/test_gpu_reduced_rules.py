@@ -258,3 +258,20 @@ def test_classes_out_of_floats_range(ctx, R, a, b):
     for k in ("A", "B"):
         assert np.all(np.isfinite(ref[k]))
         assert np.max(np.abs(got[k] - ref[k])) <= 1e-11 * np.max(np.abs(ref[k])), k
+
+
+@pytest.mark.parametrize("a,b", [(1e-3, 1e4), (1e-2, 200.0)])
+def test_end_of_a_long_thin_coil(ctx, a, b):
+    """Where float coordinates are as coarse as the winding is thick: points within two thicknesses of its end. The FP64
+    rules agree there to the rounding of their node terms, as above: 1e-11 of the largest value."""
+    row = _row("RECTANGULAR", 1.0, a, b, 80, 30)
+    row.update(pos=(0.0, 0.0, 0.0), alpha=0.0, beta=0.0)
+    rng = np.random.default_rng(29)
+    n = 1000
+    phi, r, z = rng.uniform(0, 2 * np.pi, n), 1.0 + a * rng.uniform(-1, 2, n), 0.5 * b + a * rng.uniform(-2, 2, n)
+    pts = np.stack([r * np.cos(phi), r * np.sin(phi), z], axis=1)
+    cs = abi.CoilSet.from_rows([row])
+    ref, _ = ctx.fields(cs, pts, abi.A | abi.B, abi.FP64_IEEE)
+    got, _ = ctx.fields(cs, pts, abi.A | abi.B, abi.FP64)
+    for k in ("A", "B"):
+        assert np.max(np.abs(got[k] - ref[k])) <= 1e-11 * np.max(np.abs(ref[k])), k

@@ -182,3 +182,45 @@ int main()
     for line in lines:
         n, seen, err = line.split()
         assert int(seen) > 80 and float(err) <= 2e-16 + 3.5 * 1.11e-16, lines
+
+
+def test_classes_of_long_thin_coils(tmp_path):
+    """rule_class never takes a cheaper rule than the geometry in double gives with the thresholds lowered by class_of's
+    float rounding: 3e-7 of the outer radius against a (ellipse), 1e-5 (angular). Points about the winding's end."""
+    lines = native.run(tmp_path, r"""
+#include "context.hpp"
+#include <algorithm>
+#include <cmath>
+#include <cstdio>
+#include <random>
+using namespace ccoil;
+int main()
+{
+    std::mt19937_64 g(7);
+    std::uniform_real_distribution<double> u(0, 1);
+    for (double a : {1e-3, 1e-2, 0.5})
+        for (double hb : {0.3, 700.1, 5000.3}) {
+            CoilDev c = {};
+            c.R = 1.0;
+            c.a = a;
+            c.b = 2 * hb;
+            c.use_fast = 1;
+            c.n_ang = 60;
+            c.n_thk = 30;
+            set_rule_limits(c);
+            long bad = 0, reduced = 0;
+            for (int i = 0; i < 100000; ++i) {
+                const double far = i % 2 ? a : 2.0, z = hb + far * (4 * u(g) - 1), r = std::fabs(1 + 0.5 * a + far * (4 * u(g) - 2));
+                const double zd = std::max(std::fabs(z) - hb, 0.0), rho = std::min(std::max(std::hypot(r, zd), 1.0), 1 + a);
+                const double num = (rho - r) * (rho - r) + zd * zd, den = 2 * rho * r;
+                const double s = (std::hypot(r - 1, zd) + std::hypot(r - 1 - a, zd)) * 2 / a;
+                const int got = rule_class(c, z, r);
+                const int most = class_of(c, (float)(num * (1 + 1e-5)), (float)den, (float)(s * (1 + 3e-7 * (1 + a) / a)));
+                if (got / (kRedThk + 1) > most / (kRedThk + 1) || got % (kRedThk + 1) > most % (kRedThk + 1)) ++bad;
+                if (got) ++reduced;
+            }
+            std::printf("%g %g %ld %d\n", a, hb, bad, reduced > 50000);
+        }
+}
+""")
+    assert len(lines) == 9 and all(line.split()[2:] == ["0", "1"] for line in lines), lines
