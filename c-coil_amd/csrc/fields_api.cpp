@@ -16,10 +16,12 @@ namespace ccoil {
 // every SIMD of the 256 CUs several waves, and over 16 lanes when even one chunk per coil would leave the launch
 // below one wave per SIMD (few points and few coils: then each lane's serial chain of nodes, not the issue rate,
 // sets the kernel's duration; one coil at 4,096 points measured 46 us at 4 lanes and 25 us at 16, while at 65,536
-// points 16 lanes were slower). The FP64 kernel takes a whole wave per point where that is at most four waves per SIMD:
-// a point next to the winding has 20 times the nodes of the others, and four points of a wave would wait for one
-// another (one coil at 4,096 points around it: 30 us at 16 lanes, 20 us at 64; below 512 points there is nothing
-// to gain). Split the coils into chunks (grid y, summed in order by field_reduce_kernel) while
+// points 16 lanes were slower). The FP64 kernel takes a whole wave per point where that is at most two waves per SIMD, or
+// four where every coil has a thousand fast nodes: a point next to the winding has 20 times the nodes of the others, and
+// four points of a wave would wait for one another. One coil at 2,048 and 4,096 points around it, us by 16 and by 64
+// lanes: 59 x 27 fast nodes 34 / 22 and 34 / 29, 80 x 20 slow 22 / 18 and 22 / 22, 40 x 10 21 / 18 and 21 / 23, 20 x 7 slow
+// 17 / 17 and 17 / 20 (at 6,144: 42 / 36, 24 / 26, 24 / 27, 17 / 23, in a cloud three times as wide 26 / 28 for the first;
+// below 512 points there is nothing to gain). Split the coils into chunks (grid y, summed in order by field_reduce_kernel) while
 // the launch still has fewer than about 8 waves per SIMD. Large launches take 1-4 chunks, whichever makes the last
 // round of resident waves fullest: every wave does the same work, so with R rounds of resident waves the launch
 // runs ceil(R) rounds.
@@ -31,7 +33,12 @@ FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n, const std::vector<CoilDev>
     const int64_t target = (int64_t)256 * 4 * 8;
     sh.split = n < (precision == CCOIL_FP64 ? kSortedPoints : (int64_t)256 * 4 * 64 * 4) ? 4 : 1;
     if (sh.split == 4 && (n * 4 + 63) / 64 * n_coils < (int64_t)256 * 4) sh.split = 16;
-    if (sh.split == 16 && precision == CCOIL_FP64 && n >= 512 && n * n_coils <= (int64_t)256 * 4 * 4) sh.split = 64;
+    if (sh.split == 16 && precision == CCOIL_FP64 && n >= 512 && n * n_coils <= (int64_t)256 * 4 * 4) {
+        const bool large = std::all_of(coils.begin(), coils.end(), [](const CoilDev &c) {
+            return c.use_fast && c.n_ang * c.n_thk >= 1000;
+        });
+        if (large || n * n_coils <= (int64_t)256 * 4 * 2) sh.split = 64;
+    }
     if (series_only) sh.split = 1;   // no rows to split
     const int64_t waves = std::max<int64_t>(1, (n * sh.split + 63) / 64);
     int64_t chunks = waves >= target ? 1 : std::min<int64_t>(n_coils, (target + waves - 1) / waves);

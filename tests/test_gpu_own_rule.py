@@ -110,3 +110,14 @@ def test_pairs_grad_fp32c_time(ctx):
     ms = {p: min(ctx.pairs_grad(P, S, n, p)[2].kernel_ms for _ in range(9)) for p in (abi.FP32C, abi.FP64_IEEE)}
     print(f"\n{n} pairs: FP32C {1e3 * ms[abi.FP32C]:.0f} us, IEEE {1e3 * ms[abi.FP64_IEEE]:.0f}")
     assert ms[abi.FP32C] <= 1.5 * ms[abi.FP64_IEEE]
+
+
+# the most points (times coils) that a wave each could serve, and one more: short rules, whose points have few nodes
+# wherever they lie, were 1.2 times slower a wave each. Five per cent for the card
+@pytest.mark.parametrize("coil,copies,n", [(FLAT20, 1, 4096), (RECT16, 2, 2048), (THIN12, 1, 2048), (RECT59, 1, 4096)])
+def test_time_at_the_whole_wave_limit(ctx, coil, copies, n):
+    cs = abi.CoilSet.from_rows([_row(*coil)] * copies)
+    pts = np.random.default_rng(2).normal(scale=0.3, size=(n + 1, 3))
+    us = [1e3 * min(ctx.fields(cs, pts[:m], abi.B, abi.FP64)[1].kernel_ms for _ in range(25)) for m in (n, n + 1)]
+    print(f"\n{coil} {copies} coils: {n} points {us[0]:.1f} us, {n + 1} points {us[1]:.1f}")
+    assert us[0] <= 1.05 * us[1]
