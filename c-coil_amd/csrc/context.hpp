@@ -92,8 +92,10 @@ struct FieldShape {
 // series-only kernel (one lane per point).
 FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n_points, const std::vector<CoilDev> &coils, uint32_t q, int precision,
                             bool series_only = false);
-// Whether a CCOIL_FP64 call without rule records sums the coils' own nodes (kFP64Own) instead of reduced rules.
-bool field_own_rule(const std::vector<CoilDev> &coils, int64_t n_points, int split, uint32_t q);
+// What a CCOIL_FP64 call without rule records sums: reduced rules (points in index order, or with one lane per point in
+// a visit order), or the coils' own nodes (kFP64Own).
+enum class FieldRule { reduced, sorted, own };
+FieldRule field_rule(const std::vector<CoilDev> &coils, int64_t n_points, int split, uint32_t q);
 
 // Everything a field call launches, with its buffers already sized.
 struct FieldLaunch {

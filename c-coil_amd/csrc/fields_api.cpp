@@ -43,7 +43,7 @@ FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n, const std::vector<CoilDev>
     const int64_t waves = std::max<int64_t>(1, (n * sh.split + 63) / 64);
     int64_t chunks = waves >= target ? 1 : std::min<int64_t>(n_coils, (target + waves - 1) / waves);
     if (waves >= target && n * 18 < ((int64_t)1 << 31)) {   // the reduction grid stays below 2^31 threads
-        const int kernel = precision == CCOIL_FP64 && field_own_rule(coils, n, sh.split, q) ? kFP64Own : precision;
+        const int kernel = precision == CCOIL_FP64 && field_rule(coils, n, sh.split, q) == FieldRule::own ? kFP64Own : precision;
         const int bpc = series_only ? field_series_blocks_per_cu(q, precision) : field_blocks_per_cu(q, kernel, sh.split);
         const double slots = (double)ctx->cu_count * bpc * (kFieldBlock / 64);
         if (slots > 0) {
@@ -65,7 +65,8 @@ FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n, const std::vector<CoilDev>
 // rules save most of a long rule's nodes, but choosing them, the registers of two ways to sum, the classes that a wave
 // takes in turn, the points that it sums one at a time and (one lane per point) the visit order cost more than a short
 // rule takes in all: 128 coils of 20 x 7 slow nodes at 40,000 points took 2.07 ms by reduced rules and 0.55 by their own,
-// coils of 80 x 20 1.05 and 3.4.
+// coils of 80 x 20 1.05 and 3.4. And with few waves the visit order, which gathers the points next to the winding in a
+// few of them, costs more than it saves: one coil of 100 x 27 nodes at 65,536 points 455 us with it and 255 without.
 //
 // The costs, for B, are those measured with coils of 14 to 100 angular by 1 to 27 thickness nodes, 1 to 128 of them, at
 // 16,384 to 2^20 points in a normal and in a uniform cloud (reduced rules: the mean of the two, which lie up to a fifth
@@ -73,17 +74,20 @@ FieldShape field_shape_rule(ccoil_ctx ctx, int64_t n, const std::vector<CoilDev>
 //  - 16 lanes per point, in nodes of a lane's chain: the own rule those of a row of 16, the reduced ones a share of the
 //    whole rule (such calls' points are mostly few coils' and near) or, from 512 nodes on, a wave's.
 //  - 4 lanes, in ps per coil and point: the own rule 5.2 (1.6 slow) for each node of a lane's rows; the reduced ones by
-//    the number of rows, most for 15 to 29 angular nodes, of which most points keep all. With the gradient the nodes cost
-//    1.4 times as much, the reduced rules, half of which is their choice, 1.2 times.
+//    the number of rows, most for 15 to 29 angular nodes, of which most points keep all. Two or three rows cost less from
+//    128 nodes on, which the whole wave sums (40 coils of 48 x 2: 1.2 times their own rule's time, of 48 x 3: 0.83); with
+//    fewer the waves of near points end some 12 us after the others (one coil of 63 x 2 at 16,384 points: 34 us, 24 by
+//    its own nodes). With the gradient the nodes cost 1.4 times as much, the reduced rules, half of which is their choice,
+//    1.2 times.
 //  - 1 lane, in ps likewise: the own rule 1.35 (0.45) a node and as much again for the SIMDs that idle in the last
-//    round of waves; the reduced ones 33 to 38 (10 to 15) a row, less in the smaller cells of more points. Per call they
-//    add the visit order, 50 us and 0.3 ns a point, and the longest rule once more, which the waves next to its winding
-//    end with.
-bool field_own_rule(const std::vector<CoilDev> &coils, int64_t n, int split, uint32_t q)
+//    round of waves; the reduced ones in the visit order 33 to 38 (10 to 15) a row, less in the smaller cells of more
+//    points, and per call the order, 50 us and 0.3 ns a point, and the longest rule once more, which the waves next to
+//    its winding end with; in index order 170 (80) a row up to 16 and the near points' own nodes.
+FieldRule field_rule(const std::vector<CoilDev> &coils, int64_t n, int split, uint32_t q)
 {
-    if (split > 16) return false;
+    if (split > 16) return FieldRule::reduced;
     const bool fine = n >= (int64_t)1 << 19;   // the visit order's cells
-    double own = 0.0, red = 0.0, tail = 0.0;
+    double own = 0.0, red = 0.0, raw = 0.0, tail = 0.0;
     for (const CoilDev &c : coils) {
         const int na = c.n_ang, nt = c.n_thk, nodes = na * nt;
         const bool fast = c.use_fast != 0;
@@ -93,25 +97,36 @@ bool field_own_rule(const std::vector<CoilDev> &coils, int64_t n, int split, uin
         } else if (split == 4) {
             static constexpr double kRed[2][3][5] = {   // slow, fast; below 15, 15 to 29, from 30 angular nodes on
                 {{92, 120, 120, 190, 260}, {92, 160, 150, 530, 600}, {92, 170, 145, 265, 350}},
-                {{120, 165, 165, 275, 520}, {130, 240, 235, 700, 850}, {140, 300, 230, 450, 600}}};
+                {{120, 165, 165, 275, 520}, {130, 240, 235, 700, 850}, {140, 330, 230, 450, 600}}};
             const int rows = nt == 1 ? 0 : nt < 4 ? 1 : nt < 8 ? 2 : nt < 16 ? 3 : 4;
             own += 30.0 + (fast ? 5.2 : 1.6) * na * ((nt + 3) / 4);
-            red += rows == 1 && na >= 64 ? (fast ? 215.0 : 130.0) : kRed[fast][na < 15 ? 0 : na < 30 ? 1 : 2][rows];
+            const bool wave = rows == 1 && nodes >= 128;
+            red += wave ? (fast ? 215.0 : 130.0) : kRed[fast][na < 15 ? 0 : na < 30 ? 1 : 2][rows];
+            if (rows == 1 && !wave && na >= 30 && fast) tail = 12.0;
         } else {
             const int rows = std::min(nt, 17);
             const double r = fast ? 12.0 + (fine ? 33.0 : 38.0) * rows : fine ? 8.0 + 10.5 * rows : 16.0 + 14.5 * rows;
             own += 10.0 + (fast ? 1.35 : 0.45) * nodes;
             red += na < 15 ? (fast ? 0.75 : 0.55) * r : r;
-            tail = std::max(tail, fast ? std::min(0.13 * nodes, 80.0 + 0.08 * nodes) : 0.065 * nodes);
+            raw += 0.008 * nodes + (nt >= 16 ? (fast ? 2850.0 : 1300.0) : fast ? 170.0 * nt : 80.0 * nt);
+            tail = std::max(tail, !fast ? 0.065 * nodes : nodes < 1600 ? std::min(0.13 * nodes, 80.0 + 0.08 * nodes) : 0.167 * nodes - 59.0);
         }
     }
     const bool grad = (q & (CCOIL_G | CCOIL_G_JACOBIAN)) != 0;
-    if (split > 1) return own * (grad ? 1.4 : 1.0) < red * (grad ? 1.2 : 1.0);
+    if (split > 1) {
+        own *= grad ? 1.4 : 1.0;
+        red *= grad ? 1.2 : 1.0;
+        tail *= (grad ? 1.5e6 : 1e6) / (double)n;
+        return own < red + tail ? FieldRule::own : FieldRule::reduced;
+    }
     const double waves = (double)n / 65536.0 * std::min<double>((double)coils.size(), 8.0);   // per SIMD
-    own *= std::max(std::ceil(waves), 1.2) / waves;
+    const double round = std::max(std::ceil(waves), 1.2) / waves;
     const int kinds = (q & (CCOIL_A | CCOIL_E) ? 1 : 0) + (q & CCOIL_B ? 1 : 0) + (grad ? 1 : 0);
     const double per = 0.5e-6 * (1 + kinds) * (double)n;   // us per ps of B
-    return own * per < red * per + 50.0 + 0.3e-3 * (double)n + tail;
+    own *= per * round;
+    raw *= per * round;
+    red = red * per + 50.0 + 0.3e-3 * (double)n + tail;
+    return own < std::min(red, raw) ? FieldRule::own : raw < red ? FieldRule::reduced : FieldRule::sorted;
 }
 
 // Distance, in units of the coil's r_max, beyond which the far-field series replaces the rule (0: never), at least
@@ -367,8 +382,9 @@ ccoil_status fields_prepare(ccoil_ctx ctx, const ccoil_coils *coils, const doubl
         !(sh.split == 64 && precision == CCOIL_FP64 && n < kSortedPoints))
         return fail(ctx, CCOIL_ERR_ARGUMENT, "split must be 1, 4, 16 or, in FP64 with few points, 64");
     L.split = rule_records ? 1 : sh.split;   // the series-only kernel runs one lane per point
-    const bool own_rule = precision == CCOIL_FP64 && !rule_records && field_own_rule(hc, n, L.split, quantities);
-    if (own_rule) L.precision = kFP64Own;
+    FieldRule rule = FieldRule::reduced;
+    if (precision == CCOIL_FP64 && !rule_records) rule = field_rule(hc, n, L.split, quantities);
+    if (rule == FieldRule::own) L.precision = kFP64Own;
     if (far)
         for (auto &c : hc) {
             // the cost floor holds for one lane per point; a launch that splits the rows runs the series on one
@@ -409,8 +425,7 @@ ccoil_status fields_prepare(ccoil_ctx ctx, const ccoil_coils *coils, const doubl
         if (quantities & CCOIL_E) { CC_HIP(ctx, ensure(ctx->outE, s3)); p.E = (double *)ctx->outE.p; }
         if (quantities & (CCOIL_G | CCOIL_G_JACOBIAN)) { CC_HIP(ctx, ensure(ctx->outG, s9)); p.G = (double *)ctx->outG.p; }
     }
-    const bool sorted_rule = precision == CCOIL_FP64 && !own_rule && L.split == 1 && n >= kSortedPoints &&
-                             !(arena && arena->fixed);
+    const bool sorted_rule = rule == FieldRule::sorted && n >= kSortedPoints && !(arena && arena->fixed);
     L.piece = sorted_rule && !far ? std::min<int64_t>(n, kSortedPiece) : n;
     const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(sh.chunks, (int64_t)hc.size()));
     p.coils_per_chunk = (int32_t)(((int64_t)hc.size() + chunks - 1) / chunks);

@@ -7,7 +7,7 @@ namespace ccoil {
 
 // Arithmetic of the quadrature (values of the C ABI precision argument).
 enum { kFP64 = 0, kFP32C = 1, kFP32 = 2, kFP64Reference = 3, kFP64IEEE = 4 };
-constexpr int kFP64Own = 5;   // field kernels: kFP64's arithmetic at the coils' own nodes (field_own_rule)
+constexpr int kFP64Own = 5;   // field kernels: kFP64's arithmetic at the coils' own nodes (field_rule)
 constexpr int kFieldBlock = 256;
 
 // Device-side outcome of the FP32C near pass (read back by the host once the call's work is done).

@@ -1,4 +1,4 @@
-"""CCOIL_FP64's choice between reduced rules and the coils' own nodes (field_own_rule), at every launch shape.
+"""CCOIL_FP64's choice between reduced rules and the coils' own nodes (field_rule), at every launch shape.
 
 Values: against CCOIL_FP64_IEEE, which sums the own nodes whatever the call, per point and relative to the coils' own
 field, with the tolerances of test_gpu_reduced_rules.py (its points, its reasons; a sum of identical coils scales both).
@@ -121,3 +121,23 @@ def test_time_at_the_whole_wave_limit(ctx, coil, copies, n):
     us = [1e3 * min(ctx.fields(cs, pts[:m], abi.B, abi.FP64)[1].kernel_ms for _ in range(25)) for m in (n, n + 1)]
     print(f"\n{coil} {copies} coils: {n} points {us[0]:.1f} us, {n + 1} points {us[1]:.1f}")
     assert us[0] <= 1.05 * us[1]
+
+
+# few coils of two rows, whose reduced rules end in a few long waves, and one coil of the longest rules at the fewest points
+# of one lane each, which the visit order gathered in a few waves: 0.69, 0.48 and 0.29 of IEEE's time that way, and 0.59,
+# 0.16 and 0.12 by own nodes and in index order
+@pytest.mark.parametrize("coil,copies,n,share", [(("RECTANGULAR", 0.2, 0.02, 0.3, 63, 2), 6, 16384, 0.65),
+                                                 (("RECTANGULAR", 0.1, 0.1, 0.1, 100, 100), 1, 65536, 0.3),
+                                                 (("FLAT", 0.1, 0.05, 0.0, 100, 100), 1, 65536, 0.2)])
+def test_time_of_few_coils(ctx, coil, copies, n, share):
+    rng = np.random.default_rng(3)
+    rows = []
+    for _ in range(copies):
+        row = _row(*coil)
+        row.update(pos=tuple(rng.normal(scale=0.3 if copies > 1 else 0.0, size=3)), alpha=float(rng.uniform(0, 3)))
+        rows.append(row)
+    cs = abi.CoilSet.from_rows(rows)
+    pts = rng.normal(scale=0.4, size=(n, 3))
+    ms = {p: min(ctx.fields(cs, pts, abi.B, p)[1].kernel_ms for _ in range(9)) for p in (abi.FP64, abi.FP64_IEEE)}
+    print(f"\n{coil} {copies} coils {n} points: {1e3 * ms[abi.FP64]:.0f} us, IEEE {1e3 * ms[abi.FP64_IEEE]:.0f}")
+    assert ms[abi.FP64] <= share * ms[abi.FP64_IEEE]
