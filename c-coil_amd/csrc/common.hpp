@@ -299,7 +299,8 @@ __host__ __device__ inline RuleSel class_rule(const CoilDev &c, int cls)
 // winding's radius nearest to sqrt(r^2 + zd^2); the thickness integrand is analytic outside the point (r, zd) and its
 // mirror, whose ellipse about [R, R + a] has the distance sum d1 + d2. zd is formed in double (next to the end of a coil
 // thousands of radii long float coordinates are as coarse as its thickness), and every other operation is a float
-// operation rounded on its own, so every kernel gives a pair the same class; the thresholds (red_limits) carry margins for the rounding.
+// operation rounded on its own, so every kernel gives a pair the same class; the thresholds (red_limits) carry margins
+// for the rounding.
 //
 // class_of: the class at num = (rho - r)^2 + zd^2, den = 2 rho r and s = (d1 + d2) / (a / 2), or at bounds of them
 // (num / den and s from below).

@@ -82,7 +82,7 @@ struct ccoil_ctx_s {
 
 namespace ccoil {
 
-// Launch shape of a field call: lanes per point (1, 4 or 16) and coil chunks (grid rows summed in order).
+// Launch shape of a field call: lanes per point (1, 4 or 16, FP64 also 64) and coil chunks (grid rows summed in order).
 struct FieldShape {
     int split = 1;
     int chunks = 1;
@@ -150,10 +150,11 @@ void host_parallel_for(int64_t n, const std::function<void(int64_t, int64_t)> &f
 int far_terms(double y, bool fp64);
 // Enqueues the field kernel, the chunk reduction and (FP32C) the whole near pass on s, with no host
 // synchronisation and kernel launches and copies only (so it can be captured in a graph); evm0/evm1 (may be NULL)
-// bracket the field kernel (of all pieces, with the orders of the later ones). The near pass's outcome is copied to host_state (pinned) when given.
+// bracket the field kernel (of all pieces, with the orders of the later ones). The near pass's outcome is copied to
+// host_state (pinned) when given.
 void enqueue_fields(hipStream_t s, const FieldLaunch &L, hipEvent_t evm0, hipEvent_t evm1, NearState *host_state,
                     hipEvent_t evr0 = nullptr, hipEvent_t evr1 = nullptr);
-// The near pass from the per-coil cursors on (after a grow-on-overflow retry): key scan, fill, eval, add; evr0 / evr1
+// The record pass from the keys' cursors on (after a grow-on-overflow retry): key scan, fill, eval, add; evr0 / evr1
 // (may be NULL) bracket the evaluation kernels.
 void enqueue_near_tail(hipStream_t s, const FieldLaunch &L, NearState *host_state, hipEvent_t evr0 = nullptr,
                        hipEvent_t evr1 = nullptr);

@@ -109,7 +109,8 @@ FieldRule field_rule(const std::vector<CoilDev> &coils, int64_t n, int split, ui
             own += 10.0 + (fast ? 1.35 : 0.45) * nodes;
             red += na < 15 ? (fast ? 0.75 : 0.55) * r : r;
             raw += 0.008 * nodes + (nt >= 16 ? (fast ? 2850.0 : 1300.0) : fast ? 170.0 * nt : 80.0 * nt);
-            tail = std::max(tail, !fast ? 0.065 * nodes : nodes < 1600 ? std::min(0.13 * nodes, 80.0 + 0.08 * nodes) : 0.167 * nodes - 59.0);
+            const double last = nodes < 1600 ? std::min(0.13 * nodes, 80.0 + 0.08 * nodes) : 0.167 * nodes - 59.0;
+            tail = std::max(tail, fast ? last : 0.065 * nodes);
         }
     }
     const bool grad = (q & (CCOIL_G | CCOIL_G_JACOBIAN)) != 0;
@@ -237,7 +238,10 @@ ccoil_status near_buffers(ccoil_ctx ctx, FieldLaunch &L, int64_t cap, int width,
     if ((st = call_buffer(ctx, ctx->ntemp, arena, tb > 0 ? tb : 1, &temp)) != CCOIL_OK) return st;
     const size_t per_record = kRecordBytes + sizeof(double) * (size_t)width;
     const size_t pad = (size_t)record_places(p, 0);
-    if (arena) cap = std::min<int64_t>(cap, (int64_t)((arena->left() > 768 + pad * kRecordBytes ? arena->left() - 768 - pad * kRecordBytes : 0) / per_record));
+    if (arena) {
+        const size_t fixed = 768 + pad * kRecordBytes, left = arena->left();
+        cap = std::min<int64_t>(cap, (int64_t)((left > fixed ? left - fixed : 0) / per_record));
+    }
     cap = std::max<int64_t>(cap, 1);
     if ((st = call_buffer(ctx, ctx->nkeys, arena, sizeof(uint32_t) * ((size_t)cap + pad), &keys)) != CCOIL_OK) return st;
     if ((st = call_buffer(ctx, ctx->nrecs, arena, sizeof(uint64_t) * ((size_t)cap + pad), &recs)) != CCOIL_OK) return st;

@@ -33,27 +33,28 @@ struct FieldParams {
     // Rule records (the series modes, large calls): field_kernel evaluates only the series and defers every other
     // (coil, point) pair to the record pass below, which runs the rule on waves of one coil each. A record's kind is
     // 0 for the FP64 rule (FP32C's near pairs; every rule pair in FP64) and 1 for the float rule (FP32C's others);
-    // its key is record_key below; n_keys = n_coils * (n_slots + float_records).
+    // its key, a slot and a coil, is record_key below; n_keys = n_coils * (n_slots + float_records).
     int32_t rule_records;
     int32_t float_records;
     int32_t n_slots;       // key slots of a coil's FP64 records: kRuleClasses, 4 or 2 (record_slot)
     int32_t n_keys;
-    // FP32C far field: each coil's moments (n_coils * kMpCoil doubles, multipole.hpp); a coil with CoilDev::far_d2 > 0 takes its series beyond that distance. NULL: no coil does.
+    // The far field (FP32C, FP64 with CCOIL_FAR_FIELD): each coil's moments (n_coils * kMpCoil doubles, multipole.hpp); a
+    // coil with CoilDev::far_d2 > 0 takes its series beyond that distance. NULL: no coil does.
     const double *mp;
     // The order the points are visited in (a spatial sort, so the points of a wave lie close together and a wave
     // mostly takes one branch per coil); NULL: index order. No result depends on it.
     const uint32_t *order;
-    // FP32C near-winding pass, stream-ordered with no host readback (so a caller may capture it in a graph):
-    // field_kernel counts each point's near coils (near_counts); an exclusive scan of near_counts gives each point's
-    // slots (near_offsets); near_count counts each coil's near points (near_hist, indexed by CoilDev::near_key, so
-    // the costliest coils come first); near_key_scan turns near_hist into per-coil cursors, and stores the total and whether
-    // it exceeds near_cap in near_state; near_fill places one record per (coil, point) pair at its coil's cursor:
-    // the coil key (near_keys) and point << 32 | slot (near_recs); near_eval writes each record's FP64
-    // contribution into its slot of near_vals (near_width doubles: the requested A, E, B, G in that order);
-    // near_add adds a point's slots in slot (coil) order. The order of records within a coil varies from run to
-    // run, but a slot's value depends only on its (coil, point) and every sum has a fixed order, so FP32C results
-    // are bitwise reproducible. When the total exceeds near_cap, near_fill, near_eval and near_add do nothing and
-    // the host grows the buffers and runs them again.
+    // Record pass, stream-ordered with no host readback (so a caller may capture it in a graph): field_kernel counts
+    // each point's records (near_counts); an exclusive scan of near_counts gives each point's places in near_vals
+    // (near_offsets); near_count, or the series kernel, counts the records of each key (near_hist; coils by
+    // CoilDev::near_key, those with the most nodes first); near_key_scan turns near_hist into cursors per key, and stores
+    // the total and whether it exceeds near_cap in near_state; near_fill places one record per (coil, point) pair at
+    // its key's cursor: the key (near_keys) and point << 32 | place (near_recs); near_eval writes each record's
+    // contribution into its place of near_vals (near_width doubles: the requested A, E, B, G in that order);
+    // near_add adds a point's values in the order of their places, which is the coils'. The order of records within a
+    // key varies from run to run, but a value depends only on its (coil, point) and every sum has a fixed order, so
+    // results are bitwise reproducible. When the total exceeds near_cap, near_fill, near_eval and near_add do nothing
+    // and the host grows the buffers and runs them again.
     int64_t *near_counts;
     const int64_t *near_offsets;
     uint32_t *near_hist;      // [n_keys + 1] counts per key
@@ -99,10 +100,10 @@ __host__ __device__ inline bool uniform_records(const FieldParams &p)
 // The sort key of a record: slot, then coil (most nodes first). FP64 records whose serial chain of nodes would outlast
 // the rest of the launch come first, and near_eval splits them over more lanes; with two slots that is all. Else
 // uniform records are sorted by rule class, the costliest first, so that a wave holds one coil's records of one
-// class: the split ones, with the coil's own angular rule and at least kRecordSplit thickness rows of a coil's kSplitRows,
-// take the first kSplitSlots slots. (One row a lane leaves more to the set-up and the sum over the lanes than it saves:
-// 40 coils of 40 x 10 nodes, 131,072 points, FP32C: 114 us split, 98 not.) Grouped records are sorted by their node count in steps of four, the split ones with kGroupSplit nodes or more.
-// Float records follow by coil.
+// class: the split ones, with the coil's own angular rule and at least kRecordSplit thickness rows of a coil's
+// kSplitRows, take the first kSplitSlots slots. (One row a lane leaves more to the set-up and the sum over the lanes than
+// it saves: 40 coils of 40 x 10 nodes, 131,072 points, FP32C: 114 us split, 98 not.) Grouped records are sorted by their
+// node count in steps of four, the split ones with kGroupSplit nodes or more. Float records follow by coil.
 constexpr int kRecordSplit = 8;
 constexpr int kSplitRows = 13;
 constexpr int kSplitSlots = kRedThk;
@@ -166,7 +167,6 @@ void launch_gl_tables(hipStream_t s, double *x, double *w, double *cosv, double 
 void launch_angular_tables(hipStream_t s, const double *x, const double *w, const double *cosv, const double *omc,
                            double *wc, float *wcf, double *opc, float *opcf, double *ws, double *ws2, double *wcs,
                            float *wcsf);
-// split: 1, 4 or 16 lanes per point.
 // Zeroes n_words 8-byte words with a kernel (no hipMemsetAsync, so callers may capture it in a graph).
 void launch_fill_zero(hipStream_t s, void *p, int64_t n_words);
 struct ZeroRanges {       // up to four ranges of words to zero with one launch
@@ -174,6 +174,7 @@ struct ZeroRanges {       // up to four ranges of words to zero with one launch
     int64_t n[4];
 };
 void launch_fill_zero(hipStream_t s, const ZeroRanges &z);
+// split: 1, 4 or 16 lanes per point, or 64 (kFP64).
 void launch_field(hipStream_t s, const FieldParams &p, int precision, int split);
 void launch_field_reduce(hipStream_t s, const FieldParams &p);   // after launch_field when n_chunks > 1
 // Resident 256-thread blocks per CU of the field kernel instance (0 if the runtime cannot tell).
@@ -194,8 +195,8 @@ int field_series_blocks_per_cu(uint32_t q, int precision);
 // Exclusive prefix sum of n counts into offsets (kernel launches only); with temp == NULL only sets temp_bytes.
 hipError_t near_scan(hipStream_t s, const int64_t *counts, int64_t *offsets, int64_t n, void *temp,
                      size_t &temp_bytes);
-// near_count: per-coil counts into near_hist (zeroed before); near_key_scan: per-coil cursors from near_hist, and
-// near_state's total and overflow (one small kernel).
+// near_count: the records of each key into near_hist (zeroed before); near_key_scan: the keys' cursors from near_hist,
+// and near_state's total, ends and overflow (one small kernel).
 void launch_near_count(hipStream_t s, const FieldParams &p);
 void launch_near_key_scan(hipStream_t s, const FieldParams &p);
 void launch_near_fill(hipStream_t s, const FieldParams &p);

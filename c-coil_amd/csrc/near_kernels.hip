@@ -3,14 +3,15 @@
 // calls) every pair inside the far-field distance is, by the FP64 or the float rule (its record's kind), on waves
 // that share one coil instead of beside the series.
 //
-// field_kernel<kFP32C> skips those pairs and counts them per point; an exclusive scan of the point counts gives each
-// point's slots; near_count_kernel counts each coil's near points and near_key_scan_kernel turns those counts into
-// cursors (a counting sort by coil) and checks the total against the buffers' capacity; near_fill_kernel places one
-// (coil key, point | slot) record per pair at its coil's cursor, so that the lanes of a wave evaluate the same coil
-// (uniform loop bounds, one branch of the fast / slow rule); near_eval_kernel evaluates one record per thread into
-// its slot; near_add_kernel adds a point's slots to the outputs in coil order. A slot's value depends only on its
-// (coil, point), and every sum has a fixed order, so FP32C results are bitwise reproducible although the order of the
-// records within a coil is not. Nothing here is read back by the host before the work is done.
+// field_kernel skips those pairs and counts them per point; an exclusive scan of the point counts gives each point's
+// places; near_count_kernel counts the records of each key (slot and coil, record_slot) and near_key_scan_kernel turns
+// those counts into cursors (a counting sort by key) and checks the total against the buffers' capacity;
+// near_fill_kernel places one (key, point | place) record per pair at its key's cursor, so that the lanes of a wave
+// evaluate the same coil and, in large calls, the same reduced rule (uniform loop bounds and scalar tables);
+// near_eval_kernel (in smaller calls near_eval_group_kernel) evaluates a record per lane or group of lanes into its
+// place; near_add_kernel adds a point's values to the outputs in coil order. A value depends only on its (coil, point),
+// and every sum has a fixed order, so results are bitwise reproducible although the order of the records within a key
+// is not. Nothing here is read back by the host before the work is done.
 #include <algorithm>
 #include <cstddef>
 
