@@ -37,7 +37,8 @@ namespace ccoil {
 // eight numbers a term takes lie in two rows of 32 bytes, of the coil and of all coils, for two scalar loads a term.
 // Bound by FP64 issue (70 % of it) with 15 instructions a term for B and gradient and some 190 around the loop; with 17
 // instructions, and loads from seven arrays that the loop waited for five times in two terms, 128 coils x 2^20 points
-// took 2.39 ms, this 2.00 (loads a term ahead, held there by scheduling barriers: the same).
+// took 2.39 ms, this 2.00 in turn on one card, 2.1 to 2.3 on others (loads a term ahead, held there by scheduling
+// barriers: the same).
 constexpr int kMpTerms = 250;               // highest order l (below 256, the range of wave_max_small)
 constexpr int kMpOdd = 128;                 // odd orders l = 2 i + 1 of the tables (a row more than is summed)
 // Per coil: rows of m_l, (l + 1) m_l k_(l+1), (l + 1)(l + 2) m_l k_(l+2), (l + 1) m_l; then m_l / l.

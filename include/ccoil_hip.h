@@ -81,8 +81,9 @@ enum {
                                   point and coil chunks; pairs: primary-node evaluations per lane and work item)
                                   from the context's tuning cache; the first call of a size not in the cache times
                                   every candidate shape on the device (the call runs once per candidate) and caches
-                                  the fastest. A cached shape is replayed as is, so results are bitwise
-                                  reproducible for a given cache. */
+                                  the one of the least device time. A cached shape is replayed as is, so results
+                                  are bitwise reproducible for a given cache; entries of a library whose kernels
+                                  count or run otherwise have other keys and are not used. */
     CCOIL_DIRECT = 16,         /* FP32C fields: evaluate every (coil, point) pair with the rule. By default a pair
                                   beyond the coil's far-field distance (ccoil_far_field_radius: at least 1.17 times the
                                   radius of the sphere that holds the winding, more for coils of few increments) takes the coil's
